@@ -3,6 +3,8 @@
 // entry points xtb_scf_lds_bytes and xtb_scf.
 #include "scf_kernel.h"
 
+#include <algorithm>
+
 namespace xtb {
 
 __global__ void __launch_bounds__(NT) k_scf(xtb_batch b, xtb_params par, const double* S,
@@ -22,13 +24,16 @@ extern "C" int32_t xtb_scf_lds_bytes(const xtb_batch* batch, int32_t* bytes, int
     const Lay L = make_lay(batch->max_n, batch->max_nsh, batch->max_nat);
     const int budget = 160 * 1024 / 8;
     const int n = batch->max_n;
-    const int want_c = n * (n + 1) / 2 + n * n;
     const int want_a = n * (n + 1) / 2;
     const int avail = budget - L.total_fixed;
     int cap = NGEMM_MFMA_LDS;
-    if (want_c <= avail) cap = want_c > cap ? want_c : cap;
-    else if (want_a <= avail) cap = want_a > cap ? want_a : cap;
-    else cap = NBLOCK_LDS > cap ? NBLOCK_LDS : cap;  // block Jacobi
+    if (want_a <= avail) {
+        // Jacobi in LDS, with the conflict-free row pitch if that fits
+        const int ring = ring_doubles(n, ring_pitch(n, avail));
+        cap = std::max(cap, std::max(want_a, ring));
+    } else {
+        cap = NBLOCK_LDS > cap ? NBLOCK_LDS : cap;  // block Jacobi
+    }
     if (L.total_fixed + cap > budget) return XTB_ETOOBIG;
     *big_cap = cap;
     *bytes = (L.total_fixed + cap) * 8;

@@ -11,12 +11,12 @@
 //   mixed with upstream's Anderson mixer (scf/mixer/anderson.py:163-317).
 //
 // Eigensolver: the generalized problem is reduced once per geometry with the
-// Loewdin orthogonaliser X = S^-1/2 (coupled Newton-Schulz on matrix cores).  Every
-// SCF step transforms F into the basis of the previous step's orbitals,
-// A = C^T F C, which is close to diagonal, and finishes it with a few sweeps
-// of parallel-ordered cyclic Jacobi whose rotations are applied directly to
-// the stored orbitals.  A lives in LDS (packed upper triangle) whenever it
-// fits, and so do the orbitals when both fit.
+// Cholesky factor of S (or the Loewdin S^-1/2 by coupled Newton-Schulz) on
+// matrix cores.  Every SCF step transforms F into the basis of the previous
+// step's orbitals, A = C^T F C, which is close to diagonal, and finishes it
+// with a few sweeps of parallel-ordered cyclic Jacobi whose rotations are
+// applied to the stored orbitals: with A in LDS whenever it fits, by block
+// Jacobi in memory otherwise.
 #pragma once
 
 #include "scf_core.h"
@@ -69,30 +69,14 @@ __device__ __noinline__ int eig_step(const Mol& M, const Shared& sh, int max_swe
     const int npk = n * (n + 1) / 2;
     int sweeps;
     if (npk <= sh.big_cap) {
-        SymPacked A{sh.big, n};
-        for (int i = threadIdx.x / WAVE; i < n; i += NWAVE)
-            for (int j = i + threadIdx.x % WAVE; j < n; j += WAVE) A.at(i, j) = M.F[(size_t)i * n + j];
-        const bool cl = (npk + n * n) <= sh.big_cap;
-        ldsf* cbuf = sh.big + npk;
-        if (cl) {
-            for (int idx = threadIdx.x; idx < n * n; idx += NT) cbuf[idx] = M.Ct[idx];
-        }
-        __syncthreads();
-        if (cl) sweeps = wg_jacobi(A, n, RowsLds{cbuf, n}, max_sweeps, tol, sh.cs, sh.red, cb_lo, cb_hi, intra);
-        else sweeps = wg_jacobi(A, n, RowsGlobal{M.Ct, n}, max_sweeps, tol, sh.cs, sh.red, cb_lo, cb_hi, intra);
-        for (int i = threadIdx.x; i < n; i += NT) sh.ev[i] = A.at(i, i);
-        if (cl) {
-            for (int idx = threadIdx.x; idx < n * n; idx += NT) M.Ct[idx] = cbuf[idx];
-        }
-    } else if (sh.big_cap >= NBLOCK_LDS) {
+        // T is free scratch here and holds a sweep's recorded rotations
+        sweeps = wg_jacobi(M.F, n, sh.big, ring_pitch(n, sh.big_cap), M.Ct, n, M.T, max_sweeps, tol, sh.cs, sh.red,
+                           sh.ev, cb_lo, cb_hi, intra);
+    } else {
         // block Jacobi; T is free scratch here and holds the subproblem rotations
         sweeps = wg_block_jacobi(M.F, n, RowsGlobal{M.Ct, n}, M.T, max_sweeps, tol, sh.big, sh.red,
                                  sh.tacc, inner, cb_lo, cb_hi, intra);
         for (int i = threadIdx.x; i < n; i += NT) sh.ev[i] = M.F[(size_t)i * n + i];
-    } else {
-        SymFull A{M.F, n};
-        sweeps = wg_jacobi(A, n, RowsGlobal{M.Ct, n}, max_sweeps, tol, sh.cs, sh.red, cb_lo, cb_hi, intra);
-        for (int i = threadIdx.x; i < n; i += NT) sh.ev[i] = A.at(i, i);
     }
     __syncthreads();
     return sweeps;

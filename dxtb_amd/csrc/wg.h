@@ -116,6 +116,11 @@ __device__ inline void wg_axpby(size_t len, double a, const glbf* X, double b, c
 // following product: fragments chain without a trip through LDS.
 // ---------------------------------------------------------------------------
 typedef double v4d __attribute__((ext_vector_type(4)));
+typedef double v2d __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) v2d ldsv2;
+// pairs of doubles in global memory need no more than a double's alignment
+typedef double v2d8 __attribute__((ext_vector_type(2), aligned(8)));
+typedef __attribute__((address_space(1))) v2d8 glbv2;
 
 __device__ inline v4d mfma16(double a, double b, v4d c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
@@ -522,29 +527,6 @@ __device__ inline void gemm_sym_mull(int n, int K, const glbf* A, int lda, const
     else wg_gemm_sym_mull<TA, TB, 4>(n, K, A, lda, B, ldb, S, nao, part, out, lds);
 }
 
-// ---------------------------------------------------------------------------
-// Symmetric matrix storage used by the Jacobi eigensolver.  Only the upper
-// triangle (i <= j) is referenced.  Packed form lives in LDS, full form in
-// global memory.
-// ---------------------------------------------------------------------------
-struct SymPacked {
-    ldsf* a;
-    int n;
-    __device__ inline ldsf& at(int i, int j) const {
-        if (i > j) { int t = i; i = j; j = t; }
-        return a[i * n - (i * (i - 1)) / 2 + (j - i)];
-    }
-};
-
-struct SymFull {
-    glbf* a;
-    int n;
-    __device__ inline glbf& at(int i, int j) const {
-        if (i > j) { int t = i; i = j; j = t; }
-        return a[(size_t)i * n + j];
-    }
-};
-
 // Round-robin ("circle method") pairing of n2 (even) players: in round r,
 // pair k matches (n2-1, r) for k = 0 and ((r+k) mod (n2-1), (r-k) mod (n2-1))
 // otherwise.  Every unordered pair meets once in n2-1 rounds.
@@ -554,15 +536,6 @@ __device__ inline void rr_pair(int r, int k, int n2, int& p, int& q) {
     else { p = (r + k) % m; q = (r - k + m) % m; }
 }
 
-// Cyclic two-sided Jacobi with parallel (round-robin) ordering.
-// Diagonalises the symmetric n x n matrix `A` in place (eigenvalues end on
-// the diagonal) and applies every rotation to the rows of Ct (Ct[k][mu],
-// row k = vector k), i.e. C <- C J.  Ct rows have stride `ldc`.
-// `cs` is LDS for 3*(n/2+1) doubles: cos, sin and the packed pair (p, q) of
-// each rotation of the round.  Loops are laid out wave x lane so that no
-// index needs an integer division.  Returns the number of sweeps, or -1
-// when max_sweeps were spent without reaching `tol` (absolute).
-//
 // Occupation classes (cb_lo >= 0): index i has class (i < cb_lo) + (i < cb_hi)
 // (doubly, singly, un-occupied for sorted orbitals).  Mode 1 rotates and
 // tests only pairs of different classes, which decouples the classes without
@@ -574,16 +547,337 @@ __device__ inline bool pair_in_mode(int mode, int ci, int cj) {
     return mode == 0 || ((ci != cj) == (mode == 1));
 }
 
-template <class Sym, class CAcc>
-__device__ int wg_jacobi(Sym A, int n, CAcc Ct, int max_sweeps, double tol, ldsf* cs,
-                         ldsf* red, int cb_lo = -1, int cb_hi = -1, bool intra = false) {
+// ---------------------------------------------------------------------------
+// Cyclic two-sided Jacobi with parallel (round-robin) ordering for matrices
+// that fit in LDS, one workgroup per matrix.
+//
+// Round r of the ordering (rr_pair) pairs position k = 0 as (m, r) and
+// position k > 0 as (p, q) = (r + k, r - k) mod m, with n2 = n rounded up to
+// even, m = n2 - 1 and K = n2 / 2 pairs; m rounds make a sweep.
+//
+// Storage follows the ring of the m moving indices: the element of indices i
+// and j = i + d (mod m), 0 <= d < K, lies at D[d W + i], the elements of the
+// fixed index m in a last row at D[K W + i], its diagonal at D[K W + m].  The
+// difference d of the elements that two pairs (P, R) share is then the same
+// in every round and only the start index moves by one, so an address costs
+// one add and a wrap; the packed triangle took a min, max and multiply per
+// element.  Consecutive lanes (consecutive R) step by W, W + 1 or W - 1
+// doubles: with W = 2 mod 4 at most two of 32 lanes share a bank.
+//
+// The vectors do not enter the elimination, so a sweep first runs all its
+// rounds on D, recording every (c, s) in global memory, and then applies the
+// whole sweep to the vectors (ring_vectors).  Bounds: per round two barriers,
+// the rotation parameters' dependent divide and square roots on K threads,
+// and 8 LDS accesses per 2 x 2 block.  One workgroup, per round with its
+// share of the vector pass: 1.04 us at n = 20, 1.65 at 68, 2.2 at 100, 3.8
+// at 136, 5.5 at 184, half of it the vectors (a packed triangle walked row by
+// row with the vectors rotated in LDS or memory: 2.5 us at n = 20, 5.1 at
+// 68, 17.8 at 136).
+// ---------------------------------------------------------------------------
+struct Ring {
+    ldsf* D;
+    int n, m, K, W;
+    __device__ inline int wrap(int i) const { return i >= m ? i - m : (i < 0 ? i + m : i); }
+    // offset of element (i, j), i != j
+    __device__ inline int at(int i, int j) const {
+        if (i > j) { const int t = i; i = j; j = t; }
+        if (j == m) return K * W + i;
+        const int d = j - i;
+        return d < K ? d * W + i : (m - d) * W + j;
+    }
+    __device__ inline int diag(int i) const { return i == m ? K * W + m : i; }
+};
+
+// doubles that Ring needs for n with row pitch W (the row of the fixed index
+// exists for even n only; it is a dummy otherwise)
+__host__ __device__ inline int ring_pairs(int n) { return (n + 1) / 2; }
+__host__ __device__ inline int ring_doubles(int n, int W) {
+    return ring_pairs(n) * W + (n % 2 == 0 ? n : 0);
+}
+// row pitch: the next W = 2 mod 4 if the matrix then fits in cap doubles
+__host__ __device__ inline int ring_pitch(int n, int cap) {
+    const int m = 2 * ring_pairs(n) - 1;
+    int W = m;
+    while (W % 4 != 2) ++W;
+    return ring_doubles(n, W) <= cap ? W : m;
+}
+
+// lane l <- lane l - 1 (lane 0 <- first) and lane l <- lane l + 1 (lane 63 <- last)
+__device__ inline double wave_up(double v, double first) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(v), 0x138, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(v), 0x138, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ inline double wave_down(double v, double last) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(last), __double2loint(v), 0x130, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(last), __double2hiint(v), 0x130, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ inline double wave_read(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// One recorded sweep applied to C columns of the row-major vectors Ct (row k
+// = vector k) by one wave: lane l (and l + 64 with two sets) holds the two
+// rows paired at its position in registers, rotates them, and then every row
+// moves to its position of the next round: along the top of the ring to the
+// left, along the bottom to the right, the top of position 0 fixed.  After
+// the m rounds every row is back where it started.  Register traffic only:
+// 4 FP64 instructions and 8 moves per column, pair set and round, where
+// rotating rows in memory was bound by the latency of 4 accesses per pair.
+// `rot`: (c, s) of round r and pair k at rot[2 ring_slot(n, r, k)].
+__device__ inline size_t ring_slot(int n, int r, int k) {
+    // the fixed index of an odd n is a dummy: its pair is not recorded, so
+    // that a sweep takes at most n^2 doubles
+    const int K = ring_pairs(n), o = n & 1;
+    return (size_t)r * (K - o) + (k - o);
+}
+
+template <int SETS, int C>
+__device__ __noinline__ void ring_vectors_t(glbf* Ct, int ldc, int n, const glbf* rot, int c0, int ncol) {
+    const int lane = threadIdx.x % WAVE;
+    const int K = ring_pairs(n), m = 2 * K - 1;
+    double top[SETS][C], bot[SETS][C];
+    int rt[SETS], rb[SETS];
+#pragma unroll
+    for (int u = 0; u < SETS; ++u) {
+        const int k = lane + WAVE * u;
+        rt[u] = k == 0 ? m : k;
+        rb[u] = k == 0 ? 0 : m - k;
+        if (k >= K || rt[u] >= n) rt[u] = -1;
+        if (k >= K) rb[u] = -1;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+            const bool in = c < ncol;
+            top[u][c] = (in && rt[u] >= 0) ? Ct[(size_t)rt[u] * ldc + c0 + c] : 0.0;
+            bot[u][c] = (in && rb[u] >= 0) ? Ct[(size_t)rb[u] * ldc + c0 + c] : 0.0;
+        }
+    }
+    // (c, s) four rounds ahead: pairs past the end repeat the last one (their
+    // rows are not stored)
+    constexpr int RB = SETS == 1 ? 4 : 2;
+    v2d cur[RB][SETS], nxt[RB][SETS];
+    auto fetch = [&](int r0, v2d (&x)[RB][SETS]) {
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int u = 0; u < SETS; ++u) {
+                const int r = r0 + b < m ? r0 + b : m - 1;
+                const int k = lane + WAVE * u < K ? lane + WAVE * u : K - 1;
+                const bool none = k == 0 && (n & 1);
+                x[b][u] = *(const glbv2*)(rot + 2 * ring_slot(n, r, none ? 1 : k));
+                if (none) x[b][u] = v2d{1.0, 0.0};
+            }
+    };
+    const bool first = lane == 0;
+    const int kl = (K - 1) % WAVE;
+    fetch(0, cur);
+    for (int r0 = 0; r0 < m; r0 += RB) {
+        fetch(r0 + RB, nxt);
+#pragma unroll
+        for (int b = 0; b < RB; ++b) {
+            if (r0 + b >= m) break;
+#pragma unroll
+            for (int c = 0; c < C; ++c) {
+#pragma unroll
+                for (int u = 0; u < SETS; ++u) {
+                    const double x = top[u][c], y = bot[u][c], cs = cur[b][u].x, sn = cur[b][u].y;
+                    top[u][c] = cs * x - sn * y;
+                    bot[u][c] = sn * x + cs * y;
+                }
+                if constexpr (SETS == 1) {
+                    if (K == 1) continue;  // one pair, nothing moves
+                    const double t = top[0][c], e = bot[0][c];
+                    const double up = wave_down(t, e);  // position k takes k + 1's top
+                    bot[0][c] = wave_up(e, up);         // and k - 1's bottom; 0: the top of 1
+                    top[0][c] = first ? t : (lane == kl ? e : up);
+                } else {
+                    const double t0 = top[0][c], t1 = top[1][c], e0 = bot[0][c], e1 = bot[1][c];
+                    const double up0 = wave_down(t0, wave_read(t1, 0)), up1 = wave_down(t1, e1);
+                    bot[0][c] = wave_up(e0, up0);
+                    bot[1][c] = wave_up(e1, wave_read(e0, WAVE - 1));
+                    top[0][c] = first ? t0 : up0;
+                    top[1][c] = lane == kl ? e1 : up1;
+                }
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int u = 0; u < SETS; ++u) cur[b][u] = nxt[b][u];
+    }
+#pragma unroll
+    for (int u = 0; u < SETS; ++u)
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+            if (c < ncol) {
+                if (rt[u] >= 0) Ct[(size_t)rt[u] * ldc + c0 + c] = top[u][c];
+                if (rb[u] >= 0) Ct[(size_t)rb[u] * ldc + c0 + c] = bot[u][c];
+            }
+}
+
+// A recorded sweep applied to all n columns of Ct: each wave takes runs of C
+// columns.  Up to 64 pairs a lane holds one position, above that two.  C is
+// the wave's share n / 8 rounded up to a compiled size, so that one run covers
+// it (n <= 128) or two even ones do (9 up to n = 144, 12 above; 2 x 16 columns
+// of two positions would not fit the registers).
+__device__ inline void ring_vectors(glbf* Ct, int ldc, int n, const glbf* rot) {
+    const int w = threadIdx.x / WAVE;
+    const int share = (n + NWAVE - 1) / NWAVE;
+#define XTB_RV(S, C)                                        \
+    for (int c0 = w * (C); c0 < n; c0 += NWAVE * (C))       \
+        ring_vectors_t<S, C>(Ct, ldc, n, rot, c0, n - c0)
+    if (ring_pairs(n) <= WAVE) {
+        if (share <= 4) { XTB_RV(1, 4); }
+        else if (share <= 8) { XTB_RV(1, 8); }
+        else if (share <= 12) { XTB_RV(1, 12); }
+        else { XTB_RV(1, 16); }
+    } else {
+        if (share <= 18) { XTB_RV(2, 9); }
+        else { XTB_RV(2, 12); }
+    }
+#undef XTB_RV
+}
+
+// 1 / x and 1 / sqrt(x) for normal positive x: the hardware estimates with
+// Newton steps to full precision (the rotations need no correctly rounded
+// division, whose scaling and fix-up steps double the dependent chain)
+__device__ inline double fast_rcp(double x) {
+    double y = __builtin_amdgcn_rcp(x);
+    y = fma(fma(-x, y, 1.0), y, y);
+    return fma(fma(-x, y, 1.0), y, y);
+}
+__device__ inline double fast_rsq(double x) {
+    double y = __builtin_amdgcn_rsq(x);
+    const double h = 0.5 * x;
+    y = fma(fma(-h * y, y, 0.5), y, y);
+    return fma(fma(-h * y, y, 0.5), y, y);
+}
+
+// The rounds of one sweep on D, every thread holding NB of the K (K - 1) / 2
+// 2 x 2 blocks P < R (rows P and K - 2 - P of the strict triangle joined into
+// runs of K).  A block's four addresses and the rounds in which they wrap
+// around the ring stay in registers.
+template <int NB>
+__device__ __noinline__ void ring_rounds(ldsf* D, int n, int W, glbf* rot, ldsf* cs, double skip, int mode, int cb_lo,
+                                         int cb_hi) {
+    const int K = ring_pairs(n), m = 2 * K - 1, E = K * W;
+    const Ring G{D, n, m, K, W};
+    const bool even = n % 2 == 0;
+    const int nblk = K * (K - 1) / 2;
+    const uint32_t inv = (1u << 22) / (uint32_t)K + 1u;  // e / K = e inv >> 22 for e K < 2^22
+    ldsf* ad[NB][4];
+    ldsf *cp[NB], *cr[NB];
+    uint32_t rw[NB];  // byte u: the round after which address u wraps
+#pragma unroll
+    for (int g = 0; g < NB; ++g) {
+        const int e0 = threadIdx.x + g * NT, e = e0 < nblk ? e0 : (nblk > 0 ? nblk - 1 : 0);
+        const int d = (int)(((uint32_t)e * inv) >> 22), t = e - d * K;
+        const bool lo = t < K - 1 - d;
+        const int P = lo ? d : K - 2 - d, R = lo ? d + 1 + t : t;
+        const int p = P, q = G.wrap(-P), a = R, b = G.wrap(-R);
+        const int dm = R - P, dp = R + P;
+        const bool fold = dp >= K;
+        const int row = (fold ? m - dp : dp) * W;
+        const int s1 = P == 0 ? b : (fold ? p : b), s2 = fold ? a : q;
+        ad[g][0] = D + (P == 0 ? E + a : dm * W + p);  // (p, a)
+        ad[g][1] = D + ((P == 0 ? E : row) + s1);      // (p, b)
+        ad[g][2] = D + (row + s2);                     // (q, a)
+        ad[g][3] = D + (dm * W + b);                   // (q, b)
+        rw[g] = (uint32_t)(m - 1 - (P == 0 ? a : p)) | (uint32_t)(m - 1 - s1) << 8 | (uint32_t)(m - 1 - s2) << 16 |
+                (uint32_t)(m - 1 - b) << 24;
+        cp[g] = cs + 2 * P;
+        cr[g] = cs + 2 * R;
+    }
+    for (int r = 0; r < m; ++r) {
+        // rotation parameters, and the pairs' own diagonal blocks: with
+        // d = a_qq - a_pp, e = 2 a_pq, t = e sgn(d) / (|d| + sqrt(d^2 + e^2))
+        if ((int)threadIdx.x < K) {
+            const int k = threadIdx.x;
+            const int p = k == 0 ? m : G.wrap(r + k), q = G.wrap(r - k);
+            double c = 1.0, s = 0.0;
+            if (p < n) {
+                const int epq = k == 0 ? E + q : (2 * k < K ? 2 * k * W + q : (m - 2 * k) * W + p);
+                const int epp = k == 0 ? E + m : p;
+                const double apq = D[epq], app = D[epp], aqq = D[q];
+                if (fabs(apq) > skip && pair_in_mode(mode, occ_class(p, cb_lo, cb_hi), occ_class(q, cb_lo, cb_hi))) {
+                    const double dd = aqq - app, ee = 2.0 * apq;
+                    const double h2 = fma(dd, dd, ee * ee);
+                    double t = ee * fast_rcp(fma(h2, fast_rsq(h2), fabs(dd)));
+                    if (dd < 0.0) t = -t;
+                    c = fast_rsq(fma(t, t, 1.0));
+                    s = t * c;
+                    D[epp] = fma(-t, apq, app);
+                    D[q] = fma(t, apq, aqq);
+                    D[epq] = 0.0;
+                }
+            }
+            const v2d v = {c, s};
+            *(ldsv2*)(cs + 2 * k) = v;
+            if (even || k > 0) *(glbv2*)(rot + 2 * ring_slot(n, r, k)) = v;
+        }
+        __syncthreads();
+        // A <- J^T A J on the 2 x 2 blocks, up to three at a time so that
+        // their loads are in flight together
+        constexpr int GB = NB < 3 ? NB : 3;
+#pragma unroll
+        for (int g0 = 0; g0 < NB; g0 += GB) {
+            v2d vp[GB], vr[GB];
+            double x[GB][4];
+#pragma unroll
+            for (int g = 0; g < GB; ++g)
+                if (g0 + g < NB) {
+                    vp[g] = *(ldsv2*)cp[g0 + g];
+                    vr[g] = *(ldsv2*)cr[g0 + g];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        x[g][u] = (u >= 2 || even || cp[g0 + g] != cs) ? *ad[g0 + g][u] : 0.0;
+                }
+#pragma unroll
+            for (int g = 0; g < GB; ++g)
+                if (g0 + g < NB) {
+                    const double c1 = vp[g].x, s1 = vp[g].y, c2 = vr[g].x, s2 = vr[g].y;
+                    const double r00 = c1 * x[g][0] - s1 * x[g][2], r01 = c1 * x[g][1] - s1 * x[g][3];
+                    const double r10 = s1 * x[g][0] + c1 * x[g][2], r11 = s1 * x[g][1] + c1 * x[g][3];
+                    x[g][0] = r00 * c2 - r01 * s2;
+                    x[g][1] = r00 * s2 + r01 * c2;
+                    x[g][2] = r10 * c2 - r11 * s2;
+                    x[g][3] = r10 * s2 + r11 * c2;
+                    if ((int)threadIdx.x + (g0 + g) * NT < nblk && (s1 != 0.0 || s2 != 0.0)) {
+#pragma unroll
+                        for (int u = 0; u < 4; ++u)
+                            if (u >= 2 || even || cp[g0 + g] != cs) *ad[g0 + g][u] = x[g][u];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        ad[g0 + g][u] += ((rw[g0 + g] >> (8 * u)) & 255u) == (uint32_t)r ? 1 - m : 1;
+                }
+        }
+        __syncthreads();
+    }
+}
+
+// Diagonalises the symmetric matrix A (full, global, upper triangle read) of
+// order n <= 256 and applies every rotation to the rows of Ct (Ct[k][mu], row
+// k = vector k), i.e. C <- C J; eigenvalues to `ev`.  `D`: LDS of
+// ring_doubles(n, W); `cs`: 2 K doubles of LDS (16-byte aligned); `rot`:
+// global scratch of n^2 doubles for a sweep's rotations.  Returns the number
+// of sweeps, or -1 when max_sweeps were spent without reaching `tol`
+// (absolute, largest off-diagonal element of a pair in mode).
+__device__ __noinline__ int wg_jacobi(glbf* A, int n, ldsf* D, int W, glbf* Ct, int ldc, glbf* rot, int max_sweeps,
+                                      double tol, ldsf* cs, ldsf* red, ldsf* ev, int cb_lo, int cb_hi, bool intra) {
     const int mode = cb_lo < 0 ? 0 : (intra ? 2 : 1);
-    const int n2 = n + (n & 1);
-    const int npair = n2 / 2;
+    n = __builtin_amdgcn_readfirstlane(n);
+    W = __builtin_amdgcn_readfirstlane(W);
+    const int K = ring_pairs(n), m = 2 * K - 1;
+    const Ring G{D, n, m, K, W};
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    ldsf* cc = cs;
-    ldsf* ss = cs + npair;
-    ldsi* pqs = reinterpret_cast<ldsi*>(cs + 2 * npair);  // p | q << 16
+    for (int i = w; i < n; i += NWAVE)
+        for (int j = i + lane; j < n; j += WAVE) D[i == j ? G.diag(i) : G.at(i, j)] = A[(size_t)i * n + j];
+    __syncthreads();
+    const int per = (K * (K - 1) / 2 + NT - 1) / NT;  // 2 x 2 blocks per thread
+    const double skip = 1e-3 * tol;
     int sweep = 0;
     for (;;) {
         // convergence test: largest off-diagonal element
@@ -591,85 +885,26 @@ __device__ int wg_jacobi(Sym A, int n, CAcc Ct, int max_sweeps, double tol, ldsf
         for (int i = w; i < n; i += NWAVE) {
             const int ci = occ_class(i, cb_lo, cb_hi);
             for (int j = i + 1 + lane; j < n; j += WAVE)
-                if (pair_in_mode(mode, ci, occ_class(j, cb_lo, cb_hi))) off = fmax(off, fabs(A.at(i, j)));
+                if (pair_in_mode(mode, ci, occ_class(j, cb_lo, cb_hi))) off = fmax(off, fabs(D[G.at(i, j)]));
         }
         off = wg_max(off, red);
-        if (off <= tol) return sweep;
-        if (sweep >= max_sweeps) return -1;
-        const double skip = 1e-3 * tol;
-        for (int r = 0; r < n2 - 1; ++r) {
-            // 1. rotation parameters (Rutishauser's stable formulas)
-            for (int k = threadIdx.x; k < npair; k += NT) {
-                int p, q;
-                rr_pair(r, k, n2, p, q);
-                double c = 1.0, s = 0.0;
-                if (p < n && q < n && pair_in_mode(mode, occ_class(p, cb_lo, cb_hi), occ_class(q, cb_lo, cb_hi))) {
-                    const double apq = A.at(p, q);
-                    if (fabs(apq) > skip) {
-                        const double app = A.at(p, p), aqq = A.at(q, q);
-                        const double theta = (aqq - app) / (2.0 * apq);
-                        double t = 1.0 / (fabs(theta) + sqrt(fma(theta, theta, 1.0)));
-                        if (theta < 0.0) t = -t;
-                        c = 1.0 / sqrt(fma(t, t, 1.0));
-                        s = t * c;
-                    }
-                }
-                cc[k] = c;
-                ss[k] = s;
-                pqs[k] = p | (q << 16);
-            }
+        if (off <= tol || sweep >= max_sweeps) {
+            for (int i = threadIdx.x; i < n; i += NT) ev[i] = D[G.diag(i)];
             __syncthreads();
-            // 2a. A <- J^T A J on 2x2 blocks (P <= R): a wave per block row P
-            for (int P = w; P < npair; P += NWAVE) {
-                const int pq = pqs[P];
-                const int p = pq & 0xffff, q = pq >> 16;
-                if (p >= n || q >= n) continue;
-                const double sp = ss[P], cp = cc[P];
-                for (int R = P + lane; R < npair; R += WAVE) {
-                    const double sr = ss[R];
-                    if (sp == 0.0 && sr == 0.0) continue;
-                    const int xy = pqs[R];
-                    const int x = xy & 0xffff, y = xy >> 16;
-                    if (x >= n || y >= n) continue;
-                    const double cr = cc[R];
-                    if (P == R) {
-                        const double apq = A.at(p, q);
-                        const double t = sp / cp;
-                        A.at(p, p) = A.at(p, p) - t * apq;
-                        A.at(q, q) = A.at(q, q) + t * apq;
-                        A.at(p, q) = 0.0;
-                    } else {
-                        const double m00 = A.at(p, x), m01 = A.at(p, y);
-                        const double m10 = A.at(q, x), m11 = A.at(q, y);
-                        // rows: J_P^T M
-                        const double r00 = cp * m00 - sp * m10, r01 = cp * m01 - sp * m11;
-                        const double r10 = sp * m00 + cp * m10, r11 = sp * m01 + cp * m11;
-                        // cols: (.) J_R
-                        A.at(p, x) = r00 * cr - r01 * sr;
-                        A.at(p, y) = r00 * sr + r01 * cr;
-                        A.at(q, x) = r10 * cr - r11 * sr;
-                        A.at(q, y) = r10 * sr + r11 * cr;
-                    }
-                }
-            }
-            // 2b. vectors: rows p, q of Ct, a wave per rotation
-            for (int k = w; k < npair; k += NWAVE) {
-                const double s = ss[k];
-                if (s == 0.0) continue;
-                const int pq = pqs[k];
-                const int p = pq & 0xffff, q = pq >> 16;
-                if (p >= n || q >= n) continue;
-                const double c = cc[k];
-                for (int mu = lane; mu < n; mu += WAVE) {
-                    auto& vp = Ct.at(p, mu);
-                    auto& vq = Ct.at(q, mu);
-                    const double a = vp, b = vq;
-                    vp = c * a - s * b;
-                    vq = s * a + c * b;
-                }
-            }
-            __syncthreads();
+            return off <= tol ? sweep : -1;
         }
+        // the smallest compiled block count that covers the thread's share (1, 2, 3,
+        // 5, 7 or 10: the step between them wastes at most a third of a round)
+#define XTB_RR(NB) ring_rounds<NB>(D, n, W, rot, cs, skip, mode, cb_lo, cb_hi)
+        if (per <= 1) XTB_RR(1);
+        else if (per == 2) XTB_RR(2);
+        else if (per == 3) XTB_RR(3);
+        else if (per <= 5) XTB_RR(5);
+        else if (per <= 7) XTB_RR(7);
+        else XTB_RR(10);
+#undef XTB_RR
+        ring_vectors(Ct, ldc, n, rot);
+        __syncthreads();
         ++sweep;
     }
 }
@@ -1149,12 +1384,6 @@ struct RowsGlobal {
     glbf* a;
     int ld;
     __device__ inline glbf& at(int k, int mu) const { return a[(size_t)k * ld + mu]; }
-};
-
-struct RowsLds {
-    ldsf* a;
-    int ld;
-    __device__ inline ldsf& at(int k, int mu) const { return a[k * ld + mu]; }
 };
 
 // Ascending bitonic sort of (key, idx) pairs in LDS; len is a power of two
