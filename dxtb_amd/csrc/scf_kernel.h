@@ -713,8 +713,8 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
     } else {
         // an intermediate step needs the charges, not P: the Mulliken sums
         // a_i = sum_j P_ij S_ij come from the density product's tiles (P is
-        // never stored; its buffer holds the tiles' partial sums), into q
-        gemm_sym_mull<true, false>(n, kocc, perm ? M.F : M.Ct, n, M.T, n, M.S, M.nao, M.P, M.q, sh.big);
+        // never stored), into q
+        gemm_sym_mull<true, false>(n, kocc, perm ? M.F : M.Ct, n, M.T, n, M.S, n, M.nao, M.q, sh.big);
     }
 #ifdef XTB_PD_TIMERS
     sh.ptacc[8] += now_us() - t0;

@@ -361,170 +361,497 @@ __device__ __forceinline__ void gemm_tile(int m0, int n0, int M, int N, int K, d
             }
 }
 
-// C = alpha op(A) op(B) + beta C on matrix cores, all tiles by one workgroup
-// (see gemm_tile).  With `upper` (M == N, a product known to be symmetric)
-// only the tiles on and above the diagonal are formed; gemm_sym mirrors the
-// rest.
-template <bool TA, bool TB, int FM, int FN, int KP, bool EPI = false>
-__device__ __noinline__ void wg_gemm_mfma(int M, int N, int K, double alpha, const glbf* __restrict__ A,
-                                          int lda, const glbf* __restrict__ B, int ldb, double beta,
-                                          glbf* C, int ldc, ldsf* lds, int upper,
-                                          const glbf* E1 = nullptr,
-                                          const glbf* E2 = nullptr, double s1 = 0.0,
-                                          double s2 = 0.0) {
-    constexpr int TM = 32 * FM, TN = 64 * FN;
-    // arguments of an out-of-line call arrive in vector registers; they are
-    // uniform, and saying so turns the tile and fragment tests into scalar
-    // branches instead of exec-masked code
-    M = __builtin_amdgcn_readfirstlane(M);
-    N = __builtin_amdgcn_readfirstlane(N);
-    K = __builtin_amdgcn_readfirstlane(K);
-    lda = __builtin_amdgcn_readfirstlane(lda);
-    ldb = __builtin_amdgcn_readfirstlane(ldb);
-    ldc = __builtin_amdgcn_readfirstlane(ldc);
-    upper = __builtin_amdgcn_readfirstlane(upper);
-    const int tm = (M + TM - 1) / TM, tn = (N + TN - 1) / TN;
-    for (int tile = 0; tile < tm * tn; ++tile) {
-        if (upper && tile / tn > tile % tn) continue;
-        gemm_tile<TA, TB, FM, FN, KP, EPI>((tile / tn) * TM, (tile % tn) * TN, M, N, K, alpha, A, lda, B,
-                                           ldb, beta, C, ldc, lds, E1, E2, s1, s2);
+// ---------------------------------------------------------------------------
+// Workgroup GEMM: C = alpha op(A) op(B) + beta C, and its fused forms, by one
+// workgroup.
+//
+// What bounds it at these sizes is not the matrix cores (a 16x16x4 FP64 MFMA
+// keeps its SIMD busy for 64 cycles) but fragments without output, and the
+// latency around each k panel.  So
+// * a workgroup tile is cut to the matrix in 16 x 16 fragments (up to 11 x 11):
+//   one tile covers any product up to 176 x 176, larger ones are split evenly;
+// * the fragments are dealt to the 8 waves one by one (wave w takes fragments
+//   w, w + 8, ...; NF of them, compiled for every count 1..16), so all SIMDs
+//   get the same number;
+// * a 16-deep panel of both operands is loaded in pairs of doubles without a
+//   branch (rows past the end repeat the last one), one panel ahead in
+//   registers, and stored to the other LDS stage after three quarters of the
+//   panel's MFMAs: one barrier per panel;
+// * reads of two fragments' next half panel are issued before the MFMAs of
+//   the current one, from addresses kept in registers with the stage and the
+//   half panel in the instruction's offset: FP64 MFMAs run at the vector
+//   FP64 rate on gfx950, and every vector instruction between them costs its
+//   issue time.
+// One workgroup alone / 256 of them, n x n x n, us: n = 68: 9.1 / 10.5, 136: 34
+// / 44, 171: 59 / 81, 300: 287 / 400, 528: 1329 / 1595 (72 % of a CU's peak
+// alone; with all CUs at it the clock falls from 2.4 to 1.85 GHz).  Tiles of
+// 128 x 128 to 64 x 64 with a fixed 2 x 4 wave grid, bounds tests on every
+// load and 8-byte LDS accesses took 11.4 / 13, 64 / 71, 86 / 97, 371 / 448,
+// 1784 / 1904: n = 136 ran four 128-wide tiles at a quarter of their area.
+// ---------------------------------------------------------------------------
+typedef __attribute__((address_space(1))) char glbc;
+
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+template <class T>
+__device__ __forceinline__ T* uniform(T* p) {
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return (T*)(((uint64_t)hi << 32) | lo);
+}
+
+constexpr int GEMM_KP = 16;             // k-panel depth
+constexpr int GEMM_F = 11;              // fragment rows (columns) of a workgroup tile, at most
+constexpr int GEMM_R = 16 * GEMM_F;
+constexpr int GEMM_PITCH = 18;          // row pitch of a panel stored [row][k]: conflict-free 16-byte reads
+constexpr int GEMM_KPITCH = GEMM_R + 8; // k pitch of a panel stored [k][row]: conflict-free 8-byte reads
+constexpr int GEMM_SIDE = GEMM_R * GEMM_PITCH;  // doubles of one operand's panel
+constexpr int GEMM_STAGE = 2 * GEMM_SIDE;
+constexpr int NGEMM_MFMA_LDS = 2 * GEMM_STAGE;
+static_assert(GEMM_KP * GEMM_KPITCH <= GEMM_SIDE, "either layout fits");
+
+// One operand of a workgroup tile: panels of R = 16 F rows.  KM: stored with
+// k contiguous, staged as [row][k]; otherwise staged as [k][row].  Each thread loads GE pairs of doubles per
+// panel (64 GE >= R).  In a partial last panel of `rem` k, those past the end
+// are read at the last valid ones (shift) and zeroed when stored.  Needs K >=
+// 2 (KM) or M >= 2 rows (otherwise).
+template <bool KM, int GE>
+struct GemmSide {
+    const glbc* p;
+    uint32_t step, shift;
+    int R, last, dst;
+    uint32_t off[GE];
+    __device__ __forceinline__ void init(const glbf* X, int ld, int m0, int M, int F, int rem) {
+        const int t = threadIdx.x;
+        const uint32_t ld8 = (uint32_t)ld * 8u;
+        R = 16 * F;
+        last = M - m0 - 1;
+        if (KM) {
+            // one double back, so that a last panel of one k, read as the pair
+            // that ends with it, still has an offset >= 0
+            p = (const glbc*)X + (size_t)m0 * ld8 - 8;
+            step = 8 * GEMM_KP;
+            dst = (t >> 3) * GEMM_PITCH + 2 * (t & 7);
+            const int over = 2 * (t & 7) - (rem - 2);
+            shift = over > 0 ? (uint32_t)over * 8u : 0u;
+#pragma unroll
+            for (int e = 0; e < GE; ++e) {
+                const int row = (t >> 3) + 64 * e;
+                off[e] = (uint32_t)(row < last ? row : last) * ld8 + (uint32_t)(t & 7) * 16u + 8u;
+            }
+        } else {
+            // pairs of rows (m, m + 1): an odd last row is read with the one
+            // before it (which lies in the previous tile when it is alone)
+            const int base = last > 0 ? 0 : -1;
+            p = (const glbc*)X + (ptrdiff_t)(m0 + base) * 8;
+            step = GEMM_KP * ld8;
+            dst = (t >> 5) * GEMM_KPITCH + 2 * (t & 31);
+            const int over = (t >> 5) - (rem - 1);
+            shift = over > 0 ? (uint32_t)over * ld8 : 0u;
+#pragma unroll
+            for (int e = 0; e < GE; ++e) {
+                const int m = 2 * (t & 31) + 64 * e;
+                off[e] = (uint32_t)(t >> 5) * ld8 + (uint32_t)((m < last - 1 ? m : last - 1) - base) * 8u;
+            }
+        }
+    }
+    __device__ __forceinline__ void load(v2d (&st)[GE], bool tail) {
+        const uint32_t sh = tail ? shift : 0u;
+#pragma unroll
+        for (int e = 0; e < GE; ++e) st[e] = *(const glbv2*)(p + (off[e] - sh));
+        p += step;
+    }
+    __device__ __forceinline__ void store(v2d (&st)[GE], ldsf* s, int rem) const {
+        const int t = threadIdx.x;
+        if (rem) {
+#pragma unroll
+            for (int e = 0; e < GE; ++e) {
+                if (KM) {
+                    const int k = 2 * (t & 7);
+                    if (k == rem - 1) st[e].x = st[e].y;  // read one k early
+                    if (k >= rem) st[e].x = 0.0;
+                    if (k + 1 >= rem) st[e].y = 0.0;
+                } else if ((t >> 5) >= rem) {
+                    st[e].x = 0.0;
+                    st[e].y = 0.0;
+                }
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < GE; ++e) {
+            if (KM) {
+                if ((t >> 3) + 64 * e < R) *(ldsv2*)(s + dst + 64 * e * GEMM_PITCH) = st[e];
+            } else {
+                const int m = 2 * (t & 31) + 64 * e;
+                if (m < R) {
+                    v2d v = st[e];
+                    if (m == last) v.x = v.y;  // read one row early
+                    *(ldsv2*)(s + dst + 64 * e) = v;
+                }
+            }
+        }
+    }
+    // this lane's address of fragment row f in stage 0; the k of half panel h
+    // are 8 h + 2 lg + j, j = 0, 1 (both operands deal k to the MFMA steps the
+    // same way)
+    __device__ __forceinline__ const ldsf* at(const ldsf* s, int f, int li, int lg) const {
+        return s + (KM ? (16 * f + li) * GEMM_PITCH + 2 * lg : 2 * lg * GEMM_KPITCH + 16 * f + li);
+    }
+    // stage and half are compile-time constants: they go into the read's offset
+    static __device__ __forceinline__ v2d frag(const ldsf* q, int stage, int h) {
+        q += stage * GEMM_STAGE;
+        if (KM) return *(const ldsv2*)(q + 8 * h);
+        const v2d v = {q[8 * h * GEMM_KPITCH], q[(8 * h + 1) * GEMM_KPITCH]};
+        return v;
+    }
+};
+
+// PLAIN: C = alpha op(A) op(B) + beta C; with `sym` (M == N, a symmetric
+// product, beta unused) only the fragments on and above the diagonal are
+// formed, each also written transposed.  EPI: C = alpha op(A) op(B) + s1 E1 +
+// s2 E2, elementwise (E1, E2 with C's leading dimension; C may be E1 or E2, a
+// thread reads an element and then writes it).  MULL: C not written; the sums
+// a_i = sum_j alpha (op(A) op(B))_ij E1_ij over i, j < nao of a symmetric
+// product go to C[i] (0 for i >= nao), from the fragments on and above the
+// diagonal: the row sums of each, and the column sums for the rows of its
+// mirror image, added per row in a fixed order.  A and B must not overlap C.
+enum { GEMM_PLAIN = 0, GEMM_EPI = 1, GEMM_MULL = 2 };
+
+struct GemmOut {
+    int M, N;
+    double alpha, beta;
+    glbf* C;
+    int ldc;
+    const glbf *E1, *E2;
+    double s1, s2;
+    int nao;
+};
+
+// One workgroup tile of 16 fm x 16 fn at (m0, n0); diag: a diagonal tile of a
+// symmetric product.  All threads have passed a barrier since the LDS
+// stages' last use.
+template <bool TA, bool TB, int NF, int GE, int MODE>
+__device__ __forceinline__ void gemm_wg_tile(const GemmOut& g, int m0, int n0, int fm, int fn, int K,
+                                             const glbf* A, int lda, const glbf* B, int ldb, bool sym, bool diag,
+                                             ldsf* lds) {
+    static_assert(NT == 512, "panel loads assume 512 threads");
+    const int w = uniform((int)threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+    const int li = lane % 16, lg = lane / 16;
+    const int rem = K & 15, np = (K + 15) >> 4;
+    GemmSide<!TA, GE> a;
+    GemmSide<TB, GE> b;
+    a.init(A, lda, m0, g.M, fm, rem);
+    b.init(B, ldb, n0, g.N, fn, rem);
+    // this wave's fragments (row-major; of a diagonal tile's upper triangle
+    // rows d and fm - 1 - d together make a run of fm + 1); idle slots repeat
+    // the last fragment and write nothing
+    const int T = diag ? fm * (fm + 1) / 2 : fm * fn;
+    const int run = diag ? fm + 1 : fn;
+    const uint32_t inv = 65536u / (uint32_t)run + 1u;  // q / run, q < 256, run <= 13
+    int fr[NF], fc[NF];
+    const ldsf *qa[NF], *qb[NF];
+#pragma unroll
+    for (int t = 0; t < NF; ++t) {
+        int q = w + NWAVE * t;
+        q = q < T ? q : T - 1;
+        const int d = (int)(((uint32_t)q * inv) >> 16), r = q - d * run;
+        fr[t] = d;
+        fc[t] = r;
+        if (diag) {
+            const bool lo = r < fm - d;
+            fr[t] = lo ? d : fm - 1 - d;
+            fc[t] = lo ? d + r : r - 1;
+        }
+        qa[t] = a.at(lds, fr[t], li, lg);
+        qb[t] = b.at(lds + GEMM_SIDE, fc[t], li, lg);
+    }
+    v4d acc[NF];
+#pragma unroll
+    for (int t = 0; t < NF; ++t) acc[t] = v4zero();
+    auto load = [&](int p, v2d (&sa)[GE], v2d (&sb)[GE]) {
+        const bool tail = rem && p == np - 1;
+        a.load(sa, tail);
+        b.load(sb, tail);
+    };
+    auto store = [&](int p, int stg, v2d (&sa)[GE], v2d (&sb)[GE]) {
+        ldsf* s = lds + stg * GEMM_STAGE;
+        const int r = p == np - 1 ? rem : 0;
+        a.store(sa, s, r);
+        b.store(sb, s + GEMM_SIDE, r);
+    };
+    // units of two fragments x half a panel (8 k): the reads of a unit are
+    // issued one unit ahead, the MFMAs of its two fragments alternate
+    constexpr int NU = 2 * ((NF + 1) / 2);
+    auto read = [&](int stg, int u, v2d (&x)[2], v2d (&y)[2]) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int t = 2 * (u >> 1) + q;
+            if (t < NF) {
+                x[q] = a.frag(qa[t], stg, u & 1);
+                y[q] = b.frag(qb[t], stg, u & 1);
+            }
+        }
+    };
+    auto multiply = [&](int u, const v2d (&x)[2], const v2d (&y)[2]) {
+        const int t = 2 * (u >> 1);
+        acc[t] = mfma16(x[0].x, y[0].x, acc[t]);
+        if (t + 1 < NF) acc[t + 1] = mfma16(x[1].x, y[1].x, acc[t + 1]);
+        acc[t] = mfma16(x[0].y, y[0].y, acc[t]);
+        if (t + 1 < NF) acc[t + 1] = mfma16(x[1].y, y[1].y, acc[t + 1]);
+    };
+    auto panel = [&](int p, int stg) {
+        __syncthreads();
+        v2d x[2][2], y[2][2], sa[GE], sb[GE];
+        if (p + 1 < np) load(p + 1, sa, sb);
+        read(stg, 0, x[0], y[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr int US = NU - (NU + 3) / 4;
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            if (u == US && p + 1 < np) store(p + 1, 1 - stg, sa, sb);
+            if (u + 1 < NU) {
+                read(stg, u + 1, x[(u + 1) & 1], y[(u + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            multiply(u, x[u & 1], y[u & 1]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    {
+        v2d sa[GE], sb[GE];
+        load(0, sa, sb);
+        store(0, 0, sa, sb);
+    }
+    for (int p = 0; p < np; p += 2) {
+        panel(p, 0);
+        if (p + 1 < np) panel(p + 1, 1);
+    }
+    if constexpr (MODE == GEMM_MULL) {
+        ldsf* rowp = lds;                 // [fn][16 fm] row sums of fragment column c
+        ldsf* colp = lds + 16 * fm * fn;  // [fm][16 fn] column sums of fragment row r
+        __syncthreads();                  // every wave has read the last panel
+#pragma unroll
+        for (int t = 0; t < NF; ++t) {
+            if (w + NWAVE * t >= T) break;
+            const int gn = n0 + 16 * fc[t] + li;
+            double cs = 0.0, rs[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int gm = m0 + 16 * fr[t] + lg + 4 * r;
+                rs[r] = 0.0;
+                if (gm < g.nao && gn < g.nao)
+                    rs[r] = g.alpha * acc[t][r] *
+                            *(const glbf*)((const glbc*)g.E1 + ((uint32_t)gm * (uint32_t)g.ldc + (uint32_t)gn) * 8u);
+                cs += rs[r];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int o = 1; o < 16; o <<= 1) rs[r] += __shfl_xor(rs[r], o, WAVE);
+#pragma unroll
+            for (int o = 16; o < WAVE; o <<= 1) cs += __shfl_xor(cs, o, WAVE);
+            if (li == 0)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) rowp[fc[t] * 16 * fm + 16 * fr[t] + lg + 4 * r] = rs[r];
+            if (lg == 0) colp[fr[t] * 16 * fn + 16 * fc[t] + li] = cs;
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < 16 * fm; i += NT) {
+            if (m0 + i >= g.M) continue;
+            double s = g.C[m0 + i];
+            for (int c = diag ? i / 16 : 0; c < fn; ++c) s += rowp[c * 16 * fm + i];
+            if (diag)
+                for (int r = 0; r < i / 16; ++r) s += colp[r * 16 * fn + i];
+            g.C[m0 + i] = s;
+        }
+        if (!diag)
+            for (int i = threadIdx.x; i < 16 * fn; i += NT) {
+                if (n0 + i >= g.N) continue;
+                double s = g.C[n0 + i];
+                for (int r = 0; r < fm; ++r) s += colp[r * 16 * fn + i];
+                g.C[n0 + i] = s;
+            }
+        __syncthreads();
+        return;
+    }
+    glbc* C = (glbc*)g.C;
+    const uint32_t ldc = (uint32_t)g.ldc * 8u;
+#pragma unroll
+    for (int t = 0; t < NF; ++t) {
+        if (w + NWAVE * t >= T) break;
+        const int gn = n0 + 16 * fc[t] + li;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int gm = m0 + 16 * fr[t] + lg + 4 * r;
+            if (gm < g.M && gn < g.N) {
+                const uint32_t e = (uint32_t)gm * ldc + (uint32_t)gn * 8u;
+                glbf* c0 = (glbf*)(C + e);
+                if (MODE == GEMM_EPI) {
+                    const double e1 = *(const glbf*)((const glbc*)g.E1 + e);
+                    const double e2 = *(const glbf*)((const glbc*)g.E2 + e);
+                    *c0 = fma(g.alpha, acc[t][r], fma(g.s1, e1, g.s2 * e2));
+                } else if (sym) {
+                    const double v = g.alpha * acc[t][r];
+                    *c0 = v;
+                    if (!diag || fr[t] != fc[t]) *(glbf*)(C + ((uint32_t)gn * ldc + (uint32_t)gm * 8u)) = v;
+                } else {
+                    *c0 = g.beta == 0.0 ? g.alpha * acc[t][r] : fma(g.alpha, acc[t][r], g.beta * *c0);
+                }
+            }
+        }
     }
     __syncthreads();
 }
 
-// k-panel depth of the workgroup GEMM
-#ifndef XTB_GEMM_KP
-#define XTB_GEMM_KP 16
-#endif
-constexpr int GEMM_KP = XTB_GEMM_KP;
-constexpr int NGEMM_MFMA_LDS = 2 * GEMM_KP * (128 + 128 + 2);  // largest tile, 128 x 128
-
-// Tile shape for an M x N product: the least padded area, with one 64 x 64
-// tile's worth of area added per tile for its fixed costs; ties keep the
-// larger tile.  Returns FM * 4 + FN (FM in 2..4 fragments of 32 rows, FN in
-// 1..2 of 64 columns).
-__device__ inline int gemm_shape(int M, int N) {
-    int best = 0;
-    long cost = -1;
-    for (int fm = 4; fm >= 2; --fm)
-        for (int fn = 2; fn >= 1; --fn) {
-            const long tm = (M + 32 * fm - 1) / (32 * fm), tn = (N + 64 * fn - 1) / (64 * fn);
-            const long c = tm * tn * (32L * fm * 64 * fn + 4096);
-            if (cost < 0 || c < cost) { cost = c; best = fm * 4 + fn; }
+// `tile`: fm | fn << 8 | sym << 16
+template <bool TA, bool TB, int NF, int GE, int MODE>
+__device__ __noinline__ void wg_gemm(int M, int N, int K, int tile, double alpha, const glbf* A, int lda,
+                                     const glbf* B, int ldb, double beta, glbf* C, int ldc, ldsf* lds,
+                                     const glbf* E1, const glbf* E2, double s1, double s2, int nao) {
+    // arguments of an out-of-line call arrive in vector registers; they are
+    // uniform, and saying so turns the tests into scalar branches and the
+    // addresses into a scalar base plus a 32-bit lane offset
+    M = uniform(M);
+    N = uniform(N);
+    K = uniform(K);
+    lda = uniform(lda);
+    ldb = uniform(ldb);
+    tile = uniform(tile);
+    A = uniform(A);
+    B = uniform(B);
+    GemmOut g{M, N, alpha, beta, uniform(C), uniform(ldc), nullptr, nullptr, s1, s2, 0};
+    if (MODE != GEMM_PLAIN) g.E1 = uniform(E1);
+    if (MODE == GEMM_EPI) g.E2 = uniform(E2);
+    if (MODE == GEMM_MULL) g.nao = uniform(nao);
+    const int fm = tile & 255, fn = (tile >> 8) & 255;
+    const bool sym = MODE == GEMM_MULL || (MODE == GEMM_PLAIN && (tile >> 16));
+    if (MODE == GEMM_MULL) {
+        for (int i = threadIdx.x; i < M; i += NT) g.C[i] = 0.0;
+        __syncthreads();
+    }
+    const int FM = (M + 15) >> 4, FN = (N + 15) >> 4;
+    for (int i = 0; i < FM; i += fm)
+        for (int j = 0; j < FN; j += fn) {
+            if (sym && j < i) continue;
+            gemm_wg_tile<TA, TB, NF, GE, MODE>(g, 16 * i, 16 * j, FM - i < fm ? FM - i : fm, FN - j < fn ? FN - j : fn,
+                                               K, A, lda, B, ldb, sym, sym && i == j, lds);
         }
-    return best;
 }
 
-#define XTB_GEMM_SHAPES(CALL)        \
-    switch (gemm_shape(M, N)) {      \
-        case 2 * 4 + 1: CALL(2, 1); break; \
-        case 2 * 4 + 2: CALL(2, 2); break; \
-        case 3 * 4 + 1: CALL(3, 1); break; \
-        case 3 * 4 + 2: CALL(3, 2); break; \
-        case 4 * 4 + 1: CALL(4, 1); break; \
-        default: CALL(4, 2); break;  \
+// Products that the panel loads do not take (fewer than two k, or fewer than
+// two rows of an operand stored by rows): an element per thread.
+template <bool TA, bool TB, int MODE>
+__device__ __noinline__ void wg_gemm_thin(int M, int N, int K, double alpha, const glbf* A, int lda, const glbf* B,
+                                          int ldb, double beta, glbf* C, int ldc, const glbf* E1, const glbf* E2,
+                                          double s1, double s2, int nao) {
+    auto dot = [&](int i, int j) {
+        double d = 0.0;
+        for (int k = 0; k < K; ++k)
+            d = fma(TA ? A[(size_t)k * lda + i] : A[(size_t)i * lda + k],
+                    TB ? B[(size_t)j * ldb + k] : B[(size_t)k * ldb + j], d);
+        return alpha * d;
+    };
+    if (MODE == GEMM_MULL) {
+        for (int i = threadIdx.x; i < M; i += NT) {
+            double a = 0.0;
+            for (int j = 0; j < nao && i < nao; ++j) a = fma(dot(i, j), E1[(size_t)i * ldc + j], a);
+            C[i] = a;
+        }
+    } else {
+        for (int e = threadIdx.x; e < M * N; e += NT) {
+            const int i = e / N, j = e - i * N;
+            const size_t x = (size_t)i * ldc + j;
+            const double d = dot(i, j);
+            if (MODE == GEMM_EPI) C[x] = d + fma(s1, E1[x], s2 * E2[x]);
+            else C[x] = beta == 0.0 ? d : fma(beta, C[x], d);
+        }
     }
+    __syncthreads();
+}
 
-// dispatch: matrix-core GEMM with a tile shape matched to the size
+// The workgroup tile: the whole product if it fits, otherwise the longer side
+// is split (evenly) until it does; the wave's fragment count and the panel
+// loads per thread follow from it.
+template <bool TA, bool TB, int MODE>
+__device__ inline void gemm_run(int M, int N, int K, double alpha, const glbf* A, int lda, const glbf* B, int ldb,
+                                double beta, glbf* C, int ldc, ldsf* lds, bool sym, const glbf* E1, const glbf* E2,
+                                double s1, double s2, int nao) {
+    M = uniform(M);
+    N = uniform(N);
+    K = uniform(K);
+    if (M <= 0 || N <= 0) return;
+    if (K < 2 || (TA && M < 2) || (!TB && N < 2)) {
+        wg_gemm_thin<TA, TB, MODE>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, E1, E2, s1, s2, nao);
+        return;
+    }
+    const int FM = (M + 15) >> 4, FN = (N + 15) >> 4;
+    int pm = 1, pn = 1, fm = FM, fn = FN;
+    while (fm > GEMM_F || fn > GEMM_F) {
+        if (sym) fm = fn = (FM + pm) / (pm + 1), ++pm;
+        else if (fm > fn) fm = (FM + pm) / (pm + 1), ++pm;
+        else fn = (FN + pn) / (pn + 1), ++pn;
+    }
+    const int T = sym && fm == FM ? fm * (fm + 1) / 2 : fm * fn;
+    const int nf = (T + 7) >> 3, big = fm > fn ? fm : fn;
+    const int tile = fm | fn << 8 | (sym ? 1 : 0) << 16;
+#define XTB_G(NF, GE)                                                                                                \
+    wg_gemm<TA, TB, NF, GE, MODE>(M, N, K, tile, alpha, A, lda, B, ldb, beta, C, ldc, lds, E1, E2, s1, s2, nao)
+#define XTB_G23(NF)             \
+    case NF:                    \
+        if (big <= 8) XTB_G(NF, 2); \
+        else XTB_G(NF, 3);      \
+        break;
+#define XTB_G3(NF)     \
+    case NF:           \
+        XTB_G(NF, 3);  \
+        break;
+    switch (nf) {
+        case 1:
+            if (big <= 4) XTB_G(1, 1);
+            else XTB_G(1, 3);
+            break;
+        case 2:
+            if (big <= 4) XTB_G(2, 1);
+            else XTB_G(2, 3);
+            break;
+        XTB_G23(3) XTB_G23(4) XTB_G23(5) XTB_G23(6) XTB_G23(7) XTB_G23(8)
+        XTB_G3(9) XTB_G3(10) XTB_G3(11) XTB_G3(12) XTB_G3(13) XTB_G3(14) XTB_G3(15)
+        default: XTB_G(16, 3);
+    }
+#undef XTB_G3
+#undef XTB_G23
+#undef XTB_G
+}
+
+// C = alpha op(A) op(B) + beta C
 template <bool TA, bool TB>
 __device__ inline void gemm(int M, int N, int K, double alpha, const glbf* A, int lda,
                             const glbf* B, int ldb, double beta, glbf* C, int ldc, ldsf* lds) {
-#define XTB_G(fm, fn) wg_gemm_mfma<TA, TB, fm, fn, GEMM_KP>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, lds, 0)
-    XTB_GEMM_SHAPES(XTB_G)
-#undef XTB_G
+    gemm_run<TA, TB, GEMM_PLAIN>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, lds, false, nullptr, nullptr, 0.0, 0.0,
+                                 0);
 }
 
 // C = A B + s1 E1 + s2 E2 (row-major, E1 and E2 with C's leading dimension)
 __device__ inline void gemm_epi(int M, int N, int K, const glbf* A, int lda, const glbf* B, int ldb,
                                 glbf* C, int ldc, const glbf* E1, double s1, const glbf* E2, double s2,
                                 ldsf* lds) {
-#define XTB_G(fm, fn) \
-    wg_gemm_mfma<false, false, fm, fn, GEMM_KP, true>(M, N, K, 1.0, A, lda, B, ldb, 0.0, C, ldc, lds, 0, E1, E2, s1, s2)
-    XTB_GEMM_SHAPES(XTB_G)
-#undef XTB_G
+    gemm_run<false, false, GEMM_EPI>(M, N, K, 1.0, A, lda, B, ldb, 0.0, C, ldc, lds, false, E1, E2, s1, s2, 0);
 }
 
-// C (n x n) = alpha op(A) op(B) for a product known to be symmetric: the
-// tiles on and above the diagonal on matrix cores, the others mirrored
-// through LDS in 64 x 64 blocks (coalesced both ways).  `lds` holds
-// >= max(NGEMM_MFMA_LDS, 64 * 65) doubles.
+// C (n x n) = alpha op(A) op(B) for a product known to be symmetric
 template <bool TA, bool TB>
 __device__ inline void gemm_sym(int n, int K, double alpha, const glbf* A, int lda, const glbf* B, int ldb,
                                 glbf* C, int ldc, ldsf* lds) {
-    // square tiles: 64 x 64 for small n, 128 x 128 otherwise
-    const int tile = n <= 64 ? 64 : 128;
-    if (tile == 64) wg_gemm_mfma<TA, TB, 2, 1, GEMM_KP>(n, n, K, alpha, A, lda, B, ldb, 0.0, C, ldc, lds, 1);
-    else wg_gemm_mfma<TA, TB, 4, 2, GEMM_KP>(n, n, K, alpha, A, lda, B, ldb, 0.0, C, ldc, lds, 1);
-    // 64-blocks (bi, bj) whose tile lies below the diagonal: C_bi,bj = C_bj,bi^T
-    const int nb = (n + 63) / 64, per = tile / 64;
-    for (int bi = 1; bi < nb; ++bi)
-        for (int bj = 0; bj < bi; ++bj) {
-            if (bi / per <= bj / per) continue;  // formed by the GEMM
-            for (int e = threadIdx.x; e < 64 * 64; e += NT) {
-                const int r = e / 64, c = e % 64;  // source row bj*64 + r, column bi*64 + c
-                const int gr = bj * 64 + r, gc = bi * 64 + c;
-                lds[r * 65 + c] = (gr < n && gc < n) ? C[(size_t)gr * ldc + gc] : 0.0;
-            }
-            __syncthreads();
-            for (int e = threadIdx.x; e < 64 * 64; e += NT) {
-                const int c = e / 64, r = e % 64;  // destination row bi*64 + c, column bj*64 + r
-                const int gr = bi * 64 + c, gc = bj * 64 + r;
-                if (gr < n && gc < n) C[(size_t)gr * ldc + gc] = lds[r * 65 + c];
-            }
-            __syncthreads();
-        }
+    gemm_run<TA, TB, GEMM_PLAIN>(n, n, K, alpha, A, lda, B, ldb, 0.0, C, ldc, lds, true, nullptr, nullptr, 0.0, 0.0, 0);
 }
 
-// Mulliken sums a_i = sum_{j < nao} P_ij S_ij (0 for i >= nao) of the
-// symmetric n x n product P = op(A) op(B), without forming P: the tiles on
-// and above the diagonal on matrix cores, each reducing P o S in its
-// epilogue per row and per column (a tile above the diagonal stands, by its
-// column sums, for the rows of its mirror image); the partials are added per
-// row in a fixed order.  Square tiles as gemm_sym.  `part`: scratch of
-// 2 T tm^2 doubles (T the tile edge, tm = ceil(n / T)) when n > T; one tile
-// writes its row sums straight to `out`.  S with leading dimension n.
-template <bool TA, bool TB, int FM>
-__device__ __noinline__ void wg_gemm_sym_mull(int n, int K, const glbf* __restrict__ A, int lda,
-                                              const glbf* __restrict__ B, int ldb, const glbf* S, int nao,
-                                              glbf* part, glbf* out, ldsf* lds) {
-    constexpr int FN = FM / 2;
-    constexpr int T = 32 * FM;
-    static_assert(T == 64 * FN, "square tiles");
-    n = __builtin_amdgcn_readfirstlane(n);
-    K = __builtin_amdgcn_readfirstlane(K);
-    lda = __builtin_amdgcn_readfirstlane(lda);
-    ldb = __builtin_amdgcn_readfirstlane(ldb);
-    nao = __builtin_amdgcn_readfirstlane(nao);
-    const int tm = (n + T - 1) / T;
-    if (tm == 1) {
-        gemm_tile<TA, TB, FM, FN, GEMM_KP, false, true>(0, 0, n, n, K, 1.0, A, lda, B, ldb, 0.0, nullptr, n, lds,
-                                                         S, nullptr, 0.0, 0.0, nao, out, n, false);
-        __syncthreads();
-        return;
-    }
-    for (int tile = 0; tile < tm * tm; ++tile) {
-        const int I = tile / tm, J = tile % tm;
-        if (I > J) continue;
-        gemm_tile<TA, TB, FM, FN, GEMM_KP, false, true>(I * T, J * T, n, n, K, 1.0, A, lda, B, ldb, 0.0, nullptr, n,
-                                                         lds, S, nullptr, 0.0, 0.0, nao,
-                                                         part + (size_t)tile * 2 * T, T, I != J);
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += NT) {
-        const int I = i / T, r = i - I * T;
-        double a = 0.0;
-        for (int J = I; J < tm; ++J) a += part[(size_t)(I * tm + J) * 2 * T + r];
-        for (int J = 0; J < I; ++J) a += part[(size_t)(J * tm + I) * 2 * T + T + r];
-        out[i] = a;
-    }
-    __syncthreads();
-}
-
+// Mulliken sums out[i] = sum_{j < nao} P_ij S_ij (0 for i >= nao) of the
+// symmetric n x n product P = op(A) op(B), which is never stored.  S with
+// leading dimension ldS.
 template <bool TA, bool TB>
 __device__ inline void gemm_sym_mull(int n, int K, const glbf* A, int lda, const glbf* B, int ldb, const glbf* S,
-                                     int nao, glbf* part, glbf* out, ldsf* lds) {
-    if (n <= 64) wg_gemm_sym_mull<TA, TB, 2>(n, K, A, lda, B, ldb, S, nao, part, out, lds);
-    else wg_gemm_sym_mull<TA, TB, 4>(n, K, A, lda, B, ldb, S, nao, part, out, lds);
+                                     int ldS, int nao, glbf* out, ldsf* lds) {
+    gemm_run<TA, TB, GEMM_MULL>(n, n, K, 1.0, A, lda, B, ldb, 0.0, out, ldS, lds, true, S, nullptr, 0.0, 0.0, nao);
 }
 
 // Round-robin ("circle method") pairing of n2 (even) players: in round r,
