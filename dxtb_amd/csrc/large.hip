@@ -32,14 +32,6 @@
 namespace xtb {
 namespace big {
 
-// ---------------------------------------------------------------------------
-// Grid GEMM: one 128 x 128 output tile per workgroup (gemm_tile: 8 waves of
-// 64 x 32, 16-deep k panels double-buffered in LDS).  Workgroup b runs on XCD
-// b mod 8; each XCD takes a contiguous run of tiles in row-major order, so
-// the tiles sharing one XCD's L2 share the row panels of op(A).  With
-// `upper` only tiles on and above the diagonal are formed (a product known
-// to be symmetric; k_mirror fills the rest).
-// ---------------------------------------------------------------------------
 // control values the host reads back (slots of the `ctl` array)
 enum {
     C_EFA = 0, C_EFB, C_FOK, C_KOCC, C_PERM, C_GAPA, C_GAPB, C_DMAX,
@@ -47,75 +39,220 @@ enum {
     C_NCTL = 24
 };
 
-constexpr int GT = 128;
-// k-panel depth of the grid GEMM (one workgroup per CU either way: its
-// register use allows three waves per SIMD, fewer than a second workgroup);
-// 32 deep panels keep more loads in flight than 16 (the 600-water single
-// point 577 -> 569 ms)
-#ifndef XTB_GRID_KP
-#define XTB_GRID_KP 32
-#endif
-constexpr int GRID_KP = XTB_GRID_KP;
-constexpr int GEMM_LDS_BYTES = 2 * GRID_KP * (GT + 1 + GT + 1) * 8;
-
-__device__ inline void tile_of(int idx, int tn, int upper, int& ti, int& tj) {
-    if (!upper) {
-        ti = idx / tn;
-        tj = idx % tn;
-        return;
+// ---------------------------------------------------------------------------
+// Grid GEMM, C = alpha op(A) op(B) + beta C: wave tiles of 16 FM x 16 FN whose
+// MFMA operands are loaded straight from memory into registers, several k
+// chunks ahead, with no LDS stage and no barrier in the loop.  (An FP64 MFMA
+// takes 64 cycles here, so the 128-byte row segments that a fragment of a
+// chunk needs arrive well below the caches' rate, and the vector unit, which
+// also runs the FP64 MFMAs, is left alone: a scalar base, 32-bit lane offsets.)
+//
+// With SPLIT the four waves of a workgroup share one tile and take a quarter
+// of k each; their partial sums meet in LDS once, wave w adding and writing
+// element w of every fragment.  That shortens the chain of loads that bounds
+// small products and gives four times the tiles; without it they are 2 x 2
+// tiles with all of k each (large products, where operand re-use counts).
+//
+// Workgroup b runs on XCD b mod 8; each XCD takes a contiguous run of tiles,
+// four tile rows at a time column by column, so that those that run together
+// share row and column panels in its L2.  `sym` (M == N, a symmetric product,
+// beta unused): tiles on and above the diagonal only, written to both
+// triangles.
+//
+// us at n, k = n / 2 (k n k / n n n / symmetric n n k): n = 148: 3.1 / 3.5 /
+// 4, 296: 3.5 / 5.5 / 3.6, 528: 6.2 / 16 / 6.7, 1500: 37 / 130 / 50, 4800: 825
+// / 3460 / 840 (65 TFLOP/s); 64- and 128-wide LDS tiles of 8 waves took 7.2 /
+// 10.5 / 14.7, 10.6 / 18.7 / 17.9, 17 / 31 / 25, 126 / 245 / 134, 1250 / 4610
+// / 1260.
+// ---------------------------------------------------------------------------
+// One operand of a wave tile.  KM: stored with k contiguous; otherwise by
+// rows of k.  A lane's k of a chunk: lg KS + j, j < KS.  Rows past the end
+// repeat the last one (their results are not stored).
+template <bool KM, int F, int KS>
+struct WaveSide {
+    const glbc* p;
+    uint32_t ldb;
+    uint32_t off[F];
+    __device__ __forceinline__ void init(const double* X, int ld, int m0, int M, int li, int lg) {
+        p = (const glbc*)to_glb(X);
+        ldb = (uint32_t)ld * 8u;
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            int m = m0 + 16 * f + li;
+            m = m < M ? m : M - 1;
+            off[f] = KM ? (uint32_t)m * ldb + (uint32_t)(lg * KS * 8) : (uint32_t)(lg * KS) * ldb + (uint32_t)m * 8u;
+        }
     }
-    int r = 0, rem = idx;
-    while (rem >= tn - r) {
-        rem -= tn - r;
-        ++r;
+    __device__ __forceinline__ void fetch(double (&x)[F][KS]) {
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            if constexpr (KM) {
+#pragma unroll
+                for (int j = 0; j < KS; j += 2) {
+                    const v2d8 v = *(const glbv2*)(p + off[f] + j * 8);
+                    x[f][j] = v.x;
+                    x[f][j + 1] = v.y;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < KS; ++j) x[f][j] = *(const glbf*)((p + (size_t)j * ldb) + off[f]);
+            }
+        }
+        p += KM ? (size_t)(4 * KS * 8) : (size_t)(4 * KS) * ldb;
     }
-    ti = r;
-    tj = r + rem;
-}
+    // the last chunk's first rem k; the others are read at the last valid one
+    // and count as zero
+    __device__ __forceinline__ void fetch_tail(double (&x)[F][KS], int rem, int lg) const {
+        const uint32_t unit = KM ? 8u : ldb;
+#pragma unroll
+        for (int j = 0; j < KS; ++j) {
+            const int k = lg * KS + j, kk = k < rem ? k : rem - 1;
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                // off holds lg KS units
+                const double v = *(const glbf*)(p + (off[f] + (uint32_t)kk * unit - (uint32_t)(lg * KS) * unit));
+                x[f][j] = k < rem ? v : 0.0;
+            }
+        }
+    }
+};
 
-// square tiles of TE x TE (128, or 64 for products too small to give a
-// quarter of the CUs a 128-tile)
-template <bool TA, bool TB, bool EPI, int TE>
-__global__ void __launch_bounds__(NT) k_gemm(int M, int N, int K, double alpha, const double* A, int lda,
-                                             const double* B, int ldb, double beta, double* C, int ldc,
-                                             int upper, int ntiles, const double* E1, const double* E2,
-                                             double s1, double s2) {
-    extern __shared__ double lds[];
+template <bool TA, bool TB, bool EPI, bool SPLIT, int FM, int FN, int KS, int NB>
+__global__ void __launch_bounds__(256, 2) k_gemm(int M, int N, int K, double alpha, const double* A, int lda,
+                                                 const double* B, int ldb, double beta, double* C, int ldc,
+                                                 int sym, int ntiles, const double* E1, const double* E2,
+                                                 double s1, double s2) {
+    constexpr int KC = 4 * KS, TM = (SPLIT ? 16 : 32) * FM, TN = (SPLIT ? 16 : 32) * FN;
+    __shared__ double part[SPLIT ? 3 * FM * FN * 256 : 1];
     const int per = gridDim.x / 8;  // the grid is a multiple of 8
     const int idx = (blockIdx.x % 8) * per + blockIdx.x / 8;
     if (idx >= ntiles) return;
-    const int tn = (N + TE - 1) / TE;
+    const int tm = (M + TM - 1) / TM, tn = (N + TN - 1) / TN;
     int ti, tj;
-    tile_of(idx, tn, upper, ti, tj);
-    gemm_tile<TA, TB, TE / 32, TE / 64, GRID_KP, EPI>(ti * TE, tj * TE, M, N, K, alpha, to_glb(A), lda, to_glb(B),
-                                                      ldb, beta, to_glb(C), ldc, to_lds(lds), to_glb(E1),
-                                                      to_glb(E2), s1, s2);
-}
-
-// C[j][i] = C[i][j] for the 64 x 64 blocks below the diagonal whose tile
-// (tile edge `per` x 64) was not formed by an `upper` GEMM; one workgroup
-// per block, through LDS.
-__global__ void __launch_bounds__(256) k_mirror(double* C, int n, int ldc, int per) {
-    __shared__ double t[64 * 65];
-    const int nb = (n + 63) / 64;
-    // block index -> (bi, bj), bi > bj, lower triangle row-major
-    int bi = 1, rem = blockIdx.x;
-    while (rem >= bi) {
-        rem -= bi;
-        ++bi;
+    if (sym) {
+        int r = 0, q = idx;
+        while (q >= tn - r) {
+            q -= tn - r;
+            ++r;
+        }
+        ti = r;
+        tj = r + q;
+    } else {
+        constexpr int G = 4;
+        const int g = idx / (G * tn), r0 = g * G, h = tm - r0 < G ? tm - r0 : G;
+        const int q = idx - g * G * tn;
+        tj = q / h;
+        ti = r0 + (q - tj * h);
     }
-    const int bj = rem;
-    if (bi >= nb || bi / per <= bj / per) return;  // formed by the GEMM
-    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-        const int r = e / 64, c = e % 64;  // source row bj*64 + r, column bi*64 + c
-        const int gr = bj * 64 + r, gc = bi * 64 + c;
-        t[r * 65 + c] = (gr < n && gc < n) ? C[(size_t)gr * ldc + gc] : 0.0;
+    const int lane = threadIdx.x % WAVE, li = lane % 16, lg = lane / 16;
+    const int w = uniform((int)threadIdx.x / WAVE);
+    int m0 = ti * TM, n0 = tj * TN;
+    if (SPLIT) {
+        // this wave's quarter of k, in whole chunks
+        const int q = ((K + KC - 1) / KC + 3) / 4 * KC;
+        const int kb = w * q < K ? w * q : K, ke = kb + q < K ? kb + q : K;
+        A += TA ? (size_t)kb * lda : (size_t)kb;
+        B += TB ? (size_t)kb : (size_t)kb * ldb;
+        K = ke - kb;
+    } else {
+        m0 += (w / 2) * 16 * FM;
+        n0 += (w % 2) * 16 * FN;
+        if (m0 >= M || n0 >= N) return;
     }
-    __syncthreads();
-    for (int e = threadIdx.x; e < 64 * 64; e += 256) {
-        const int c = e / 64, r = e % 64;  // destination row bi*64 + c, column bj*64 + r
-        const int gr = bi * 64 + c, gc = bj * 64 + r;
-        if (gr < n && gc < n) C[(size_t)gr * ldc + gc] = t[r * 65 + c];
+    WaveSide<!TA, FM, KS> a;
+    WaveSide<TB, FN, KS> b;
+    a.init(A, lda, m0, M, li, lg);
+    b.init(B, ldb, n0, N, li, lg);
+    v4d acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = v4zero();
+    double xa[NB][FM][KS], xb[NB][FN][KS];
+    auto get = [&](int u) {
+        a.fetch(xa[u]);
+        b.fetch(xb[u]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](int u) {
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int j = 0; j < FN; ++j) acc[i][j] = mfma16(xa[u][i][k], xb[u][j][k], acc[i][j]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const int nfull = K / KC, rem = K - nfull * KC;
+    int c = 0;
+    if (nfull >= NB) {
+        // NB buffers in a ring, each chunk loaded NB - 1 chunks ahead
+#pragma unroll
+        for (int u = 0; u < NB - 1; ++u) get(u);
+        int left = nfull - (NB - 1);  // not loaded yet
+        for (; left >= NB; left -= NB) {
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+                get((u + NB - 1) % NB);
+                multiply(u);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < NB - 1; ++u) {
+            if (u < left) get((u + NB - 1) % NB);
+            multiply(u);
+        }
+#pragma unroll
+        for (int u = 0; u < NB - 1; ++u)
+            if (u < left) multiply((u + NB - 1) % NB);
+        c = nfull;
+    }
+    for (; c < nfull; ++c) {
+        get(0);
+        multiply(0);
+    }
+    if (rem) {
+        a.fetch_tail(xa[0], rem, lg);
+        b.fetch_tail(xb[0], rem, lg);
+        multiply(0);
+    }
+    auto put = [&](int i, int j, int r, double v) {
+        const int gm = m0 + 16 * i + lg + 4 * r, gn = n0 + 16 * j + li;
+        if (gm >= M || gn >= N) return;
+        const size_t e = (size_t)gm * ldc + gn;
+        if (EPI) C[e] = fma(alpha, v, fma(s1, E1[e], s2 * E2[e]));
+        else if (sym) {
+            C[e] = alpha * v;
+            if (ti != tj) C[(size_t)gn * ldc + gm] = alpha * v;
+        } else C[e] = beta == 0.0 ? alpha * v : fma(alpha, v, beta * C[e]);
+    };
+    if constexpr (SPLIT) {
+        // element r of a fragment is summed by wave r, in wave order; wave s != r
+        // leaves its part in slot s - r - 1 (mod 4)
+        auto slot = [&](int f, int r, int s) { return ((((s - r - 1) & 3) * FM * FN + f) * 4 + r) * WAVE + lane; };
+#pragma unroll
+        for (int f = 0; f < FM * FN; ++f)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (w != r) part[slot(f, r, w)] = acc[f / FN][f % FN][r];
+        __syncthreads();
+#pragma unroll
+        for (int f = 0; f < FM * FN; ++f)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (w == r) {
+                    double v = 0.0;
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) v += s == r ? acc[f / FN][f % FN][r] : part[slot(f, r, s)];
+                    put(f / FN, f % FN, r, v);
+                }
+    } else {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) put(i, j, r, acc[i][j][r]);
     }
 }
 
@@ -812,39 +949,31 @@ void gemm_t(Ctx& c, int M, int N, int K, double alpha, const double* A, int lda,
             double beta, double* C, int ldc, bool upper, const double* E1 = nullptr, const double* E2 = nullptr,
             double s1 = 0.0, double s2 = 0.0) {
     if (M <= 0 || N <= 0) return;
-    static bool attr = false;
-    if (!attr) {
-        chk(c, hipFuncSetAttribute((const void*)k_gemm<TA, TB, EPI, GT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   GEMM_LDS_BYTES));
-        chk(c, hipFuncSetAttribute((const void*)k_gemm<TA, TB, EPI, 64>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   GEMM_LDS_BYTES));
-        attr = true;
-    }
-    auto count = [&](int te) {
-        const int tm = (M + te - 1) / te, tn = (N + te - 1) / te;
+    auto tiles = [&](int t) {
+        const int tm = (M + t - 1) / t, tn = (N + t - 1) / t;
         return upper ? tm * (tm + 1) / 2 : tm * tn;
     };
-    // fewer 128-tiles than a quarter of the CUs: 64-tiles, four times as many
-    const int te = count(GT) < 64 ? 64 : GT;
-    const int ntiles = count(te);
-    const int grid = (ntiles + 7) / 8 * 8;
-    if (te == GT)
-        hipLaunchKernelGGL((k_gemm<TA, TB, EPI, GT>), dim3(grid), dim3(NT), GEMM_LDS_BYTES, c.s, M, N, K, alpha, A,
-                           lda, B, ldb, beta, C, ldc, upper ? 1 : 0, ntiles, E1, E2, s1, s2);
-    else
-        hipLaunchKernelGGL((k_gemm<TA, TB, EPI, 64>), dim3(grid), dim3(NT), GEMM_LDS_BYTES, c.s, M, N, K, alpha, A,
-                           lda, B, ldb, beta, C, ldc, upper ? 1 : 0, ntiles, E1, E2, s1, s2);
-    chk_launch(c);
-    if (upper) {
-        const int nb = (M + 63) / 64;
-        if (nb > 1) {
-            hipLaunchKernelGGL(k_mirror, dim3(nb * (nb - 1) / 2), dim3(256), 0, c.s, C, M, ldc, te / 64);
-            chk_launch(c);
-        }
+#define XTB_GG(SPLIT, F, KS, NB)                                                                                     \
+    {                                                                                                                \
+        const int nt = tiles((SPLIT ? 16 : 32) * F), grid = (nt + 7) / 8 * 8;                                        \
+        hipLaunchKernelGGL((k_gemm<TA, TB, EPI, SPLIT, F, F, KS, NB>), dim3(grid), dim3(256), 0, c.s, M, N, K,       \
+                           alpha, A, lda, B, ldb, beta, C, ldc, upper ? 1 : 0, nt, E1, E2, s1, s2);                  \
     }
+    // the largest tile that still gives the CUs enough workgroups.  us at both
+    // sides of the lines: 48-wide tiles (against 32) from ~220 of them, 750 x
+    // 1500 x 750 (512) 37 / 44, 500 x 1001 x 500 (231) 15.4 / 14.2, 528^3
+    // (121) 15.5 / 15.7; 16-wide below 600 of them, 296^3 (361) 5.4 / 6.8, 350
+    // x 700 x 350 (968) 9.2 / 7.5; all of k per wave from 1000 96-wide tiles,
+    // 2400 x 4800 x 2400 (1250) 821 / 875, 2400^3 (625) 520 / 460
+    if (tiles(96) >= 1000) XTB_GG(false, 3, 2, 2)
+    else if (tiles(48) >= 220) XTB_GG(true, 3, 2, 2)
+    else if (tiles(16) <= 600) XTB_GG(true, 1, 4, 4)
+    else XTB_GG(true, 2, 2, 3)
+#undef XTB_GG
+    chk_launch(c);
 }
 
-// C (n x n, symmetric) = op(A) op(B): the upper tiles, then the mirror
+// C (n x n, symmetric) = op(A) op(B)
 template <bool TA, bool TB>
 void gemm_sym(Ctx& c, int n, int K, const double* A, int lda, const double* B, int ldb, double* C, int ldc) {
     gemm_t<TA, TB, false>(c, n, n, K, 1.0, A, lda, B, ldb, 0.0, C, ldc, true);

@@ -131,236 +131,6 @@ __device__ inline v4d v4zero() {
     return z;
 }
 
-// C = alpha op(A) op(B) + beta C on matrix cores.  Workgroup tile TM x TN =
-// 32 FM x 64 FN, 8 waves as 2 (rows) x 4 (cols) of FM x FN 16x16 fragments
-// each, k panels of KP staged in LDS as As[k][m], Bs[k][n] (row pitches
-// TM+1, TN+1: conflict-free transposed stores), two stages: the next panel
-// is fetched into registers before the current panel's MFMAs and stored to
-// the other stage after them, so one barrier per panel separates the
-// stages.  `lds` holds >= 2*KP*(TM+TN+2) doubles.  Each global load instruction covers contiguous memory: lanes run
-// along m (or n) when the operand is stored that way, along k otherwise.
-// Panel loop per fragment pattern (split) or one loop for both: measured per
-// operand layout under a full chip of workgroups.
-#ifndef XTB_GEMM_SPLIT
-#define XTB_GEMM_SPLIT(TA, TB) (true)
-#endif
-
-// One TM x TN output tile at (m0, n0).  With EPI, C = alpha op(A) op(B) + s1 E1 + s2 E2 (E1, E2 with C's leading
-// dimension; beta unused): an elementwise update fused into the epilogue.  C may
-// be E1 or E2 (each element is read and then written by the same thread, once);
-// A and B must not overlap C.
-//
-// With MULL (C not written): the tile's elements x = alpha (op(A) op(B))_ij
-// E1_ij over rows and columns below `nao` are summed per row (over the
-// tile's columns) and per column (over its rows); part[0..prow) gets the
-// first prow row sums and, with pcol, part[TM..TM+TN) the column sums.
-// Lanes reduce by xor butterflies (the same bits in every lane), waves
-// through LDS in index order: the sums have the same bits on every run.
-template <bool TA, bool TB, int FM, int FN, int KP, bool EPI = false, bool MULL = false>
-__device__ __forceinline__ void gemm_tile(int m0, int n0, int M, int N, int K, double alpha,
-                                          const glbf* __restrict__ A, int lda,
-                                          const glbf* __restrict__ B, int ldb, double beta,
-                                          glbf* C, int ldc, ldsf* lds,
-                                          const glbf* E1, const glbf* E2,
-                                          double s1, double s2, int nao = 0, glbf* part = nullptr,
-                                          int prow = 0, bool pcol = false) {
-    static_assert(NT == 512, "wave layout assumes 8 waves");
-    constexpr int TM = 32 * FM, TN = 64 * FN;
-    constexpr int LDA_S = TM + 1, LDB_S = TN + 1;
-    constexpr int EA = TM * KP / NT, EB = TN * KP / NT;  // staged elements per thread
-    static_assert(EA * NT == TM * KP && EB * NT == TN * KP, "panel split over the threads");
-    constexpr int STAGE = KP * (LDA_S + LDB_S);
-    const int t = threadIdx.x;
-    // wave index made scalar, so that per-wave decisions are scalar branches
-    const int w = __builtin_amdgcn_readfirstlane(t / WAVE);
-    const int lane = t % WAVE, li = lane % 16, lg = lane / 16;
-    const int wm = w / 4, wn = w % 4;
-    // element e of this thread: (row along the contiguous direction)
-    auto a_mk = [&](int e, int& m, int& k) {
-        const int idx = t + e * NT;
-        if (TA) { m = idx % TM; k = idx / TM; }       // A[k][m]: contiguous m
-        else { k = idx % KP; m = idx / KP; }          // A[m][k]: contiguous k
-    };
-    auto b_nk = [&](int e, int& n, int& k) {
-        const int idx = t + e * NT;
-        if (TB) { k = idx % KP; n = idx / KP; }       // B[n][k]: contiguous k
-        else { n = idx % TN; k = idx / TN; }          // B[k][n]: contiguous n
-    };
-    // 16x16 fragments of this wave that hold any output (the last tile
-    // row/column is partial): the others skip their MFMAs
-    const int rrem = M - (m0 + wm * (TM / 2)), crem = N - (n0 + wn * (TN / 4));
-    const int nfm = rrem <= 0 ? 0 : (rrem >= FM * 16 ? FM : (rrem + 15) / 16);
-    const int nfn = crem <= 0 ? 0 : (crem >= FN * 16 ? FN : (crem + 15) / 16);
-    const bool full = nfm == FM && nfn == FN;
-    v4d acc[FM][FN];
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = v4zero();
-    double pa[EA], pb[EB];
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int e = 0; e < EA; ++e) {
-            int m, k;
-            a_mk(e, m, k);
-            const int gm = m0 + m, gk = k0 + k;
-            pa[e] = (gm < M && gk < K) ? (TA ? A[(size_t)gk * lda + gm] : A[(size_t)gm * lda + gk]) : 0.0;
-        }
-#pragma unroll
-        for (int e = 0; e < EB; ++e) {
-            int n, k;
-            b_nk(e, n, k);
-            const int gn = n0 + n, gk = k0 + k;
-            pb[e] = (gn < N && gk < K) ? (TB ? B[(size_t)gn * ldb + gk] : B[(size_t)gk * ldb + gn]) : 0.0;
-        }
-    };
-    auto store = [&](ldsf* st) {
-        ldsf* As = st;
-        ldsf* Bs = st + KP * LDA_S;
-#pragma unroll
-        for (int e = 0; e < EA; ++e) {
-            int m, k;
-            a_mk(e, m, k);
-            As[k * LDA_S + m] = pa[e];
-        }
-#pragma unroll
-        for (int e = 0; e < EB; ++e) {
-            int n, k;
-            b_nk(e, n, k);
-            Bs[k * LDB_S + n] = pb[e];
-        }
-    };
-    // MFMAs of one panel when every fragment of the wave holds output
-    auto panel_full = [&](const ldsf* As, const ldsf* Bs) {
-#pragma unroll
-        for (int kk = 0; kk < KP / 4; ++kk) {
-            double a[FM], b[FN];
-#pragma unroll
-            for (int i = 0; i < FM; ++i) a[i] = As[(4 * kk + lg) * LDA_S + wm * (TM / 2) + i * 16 + li];
-#pragma unroll
-            for (int j = 0; j < FN; ++j) b[j] = Bs[(4 * kk + lg) * LDB_S + wn * (TN / 4) + j * 16 + li];
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
-            __builtin_amdgcn_sched_group_barrier(0x100, FM + FN, 0);  // DS reads
-            __builtin_amdgcn_sched_group_barrier(0x008, FM * FN, 0);  // MFMAs
-        }
-    };
-    // partial tiles: fragments without output skip their MFMAs
-    auto panel_part = [&](const ldsf* As, const ldsf* Bs) {
-#pragma unroll
-        for (int kk = 0; kk < KP / 4; ++kk) {
-            double a[FM], b[FN];
-#pragma unroll
-            for (int i = 0; i < FM; ++i) a[i] = As[(4 * kk + lg) * LDA_S + wm * (TM / 2) + i * 16 + li];
-#pragma unroll
-            for (int j = 0; j < FN; ++j) b[j] = Bs[(4 * kk + lg) * LDB_S + wn * (TN / 4) + j * 16 + li];
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j)
-                    if (i < nfm && j < nfn) acc[i][j] = mfma16(a[i], b[j], acc[i][j]);
-        }
-    };
-    const int np = (K + KP - 1) / KP;
-    if (np > 0) {
-        fetch(0);
-        store(lds);
-        __syncthreads();
-    }
-    if (XTB_GEMM_SPLIT(TA, TB)) {
-        // one panel loop per fragment pattern, so the accumulators are
-        // not merged between the two code paths after every panel
-        if (full) {
-            for (int p = 0; p < np; ++p) {
-                ldsf* cur = lds + (p & 1) * STAGE;
-                if (p + 1 < np) fetch((p + 1) * KP);
-                panel_full(cur, cur + KP * LDA_S);
-                if (p + 1 < np) store(lds + ((p + 1) & 1) * STAGE);
-                __syncthreads();
-            }
-        } else {
-            for (int p = 0; p < np; ++p) {
-                ldsf* cur = lds + (p & 1) * STAGE;
-                if (p + 1 < np) fetch((p + 1) * KP);
-                panel_part(cur, cur + KP * LDA_S);
-                if (p + 1 < np) store(lds + ((p + 1) & 1) * STAGE);
-                __syncthreads();
-            }
-        }
-    } else {
-        for (int p = 0; p < np; ++p) {
-            ldsf* cur = lds + (p & 1) * STAGE;
-            if (p + 1 < np) fetch((p + 1) * KP);
-            if (full) panel_full(cur, cur + KP * LDA_S);
-            else panel_part(cur, cur + KP * LDA_S);
-            if (p + 1 < np) store(lds + ((p + 1) & 1) * STAGE);
-            __syncthreads();
-        }
-    }
-    if constexpr (MULL) {
-        double rs[FM][4], cs[FN];
-#pragma unroll
-        for (int j = 0; j < FN; ++j) cs[j] = 0.0;
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                rs[i][r] = 0.0;
-                const int gm = m0 + wm * (TM / 2) + i * 16 + lg + 4 * r;
-#pragma unroll
-                for (int j = 0; j < FN; ++j) {
-                    const int gn = n0 + wn * (TN / 4) + j * 16 + li;
-                    const double x =
-                        (gm < nao && gn < nao) ? alpha * acc[i][j][r] * E1[(size_t)gm * ldc + gn] : 0.0;
-                    rs[i][r] += x;
-                    cs[j] += x;
-                }
-            }
-#pragma unroll
-        for (int i = 0; i < FM; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int o = 1; o < 16; o <<= 1) rs[i][r] += __shfl_xor(rs[i][r], o, WAVE);
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int o = 16; o < WAVE; o <<= 1) cs[j] += __shfl_xor(cs[j], o, WAVE);
-        ldsf* rred = lds;           // [4 column waves][TM]
-        ldsf* cred = lds + 4 * TM;  // [2 row waves][TN]
-        if (li == 0)
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) rred[wn * TM + wm * (TM / 2) + i * 16 + lg + 4 * r] = rs[i][r];
-        if (lg == 0)
-#pragma unroll
-            for (int j = 0; j < FN; ++j) cred[wm * TN + wn * (TN / 4) + j * 16 + li] = cs[j];
-        __syncthreads();
-        for (int e = t; e < prow; e += NT) part[e] = ((rred[e] + rred[TM + e]) + rred[2 * TM + e]) + rred[3 * TM + e];
-        if (pcol)
-            for (int e = t; e < TN; e += NT) part[TM + e] = cred[e] + cred[TN + e];
-        __syncthreads();  // the LDS stages of the next tile reuse these rows
-        return;
-    }
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int gm = m0 + wm * (TM / 2) + i * 16 + lg + 4 * r;
-                const int gn = n0 + wn * (TN / 4) + j * 16 + li;
-                if (gm < M && gn < N) {
-                    const size_t e = (size_t)gm * ldc + gn;
-                    if (EPI) C[e] = fma(alpha, acc[i][j][r], fma(s1, E1[e], s2 * E2[e]));
-                    else C[e] = (beta == 0.0) ? alpha * acc[i][j][r] : fma(alpha, acc[i][j][r], beta * C[e]);
-                }
-            }
-}
-
 // ---------------------------------------------------------------------------
 // Workgroup GEMM: C = alpha op(A) op(B) + beta C, and its fused forms, by one
 // workgroup.

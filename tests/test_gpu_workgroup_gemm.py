@@ -12,7 +12,7 @@ import pytest
 
 import oracle.gfn1 as og
 from dxtb_amd import workloads
-from tests.helpers import TIGHT_ORACLE, run_native
+from helpers import TIGHT_ORACLE, run_native
 
 pytestmark = pytest.mark.gpu
 
