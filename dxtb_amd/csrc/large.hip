@@ -511,58 +511,19 @@ __global__ void k_set_slot(double* ctl, int slot, double v) {
 // block, and flags Q_k == I; k_japply then applies every Q_k of the round
 // to the off-diagonal tiles of A (Q_k^T A_kl Q_l) and to the orbital rows.
 // ---------------------------------------------------------------------------
-__device__ inline void build_schedules_wave(ldsi* tab) {
-    const int lane = threadIdx.x % WAVE;
-    for (int e = lane; e < (JS - 1) * NPAIR32; e += WAVE) {
-        int p, q;
-        rr32(e / NPAIR32, e % NPAIR32, p, q);
-        tab[e] = p | (q << 8);
-    }
-    for (int e = lane; e < NBLK32; e += WAVE) {
-        int P = 0, rem = e;
-        while (rem >= NPAIR32 - P) {
-            rem -= NPAIR32 - P;
-            ++P;
-        }
-        tab[(JS - 1) * NPAIR32 + e] = P | ((P + rem) << 8);
-    }
-}
-
 // one wave (64-thread workgroup) per block pair k of round r
 __global__ void __launch_bounds__(WAVE) k_jsub(double* A_, int n, int r, int nb2, double* Qbuf, int* ident,
                                                double tol, int inner) {
-    __shared__ double buf[JWAVE_LDS];
-    __shared__ int sched[SCHED_INTS];
+    __shared__ __align__(16) double buf[JWAVE_LDS];
     glbf* A = to_glb(A_);
-    const int k = blockIdx.x, lane = threadIdx.x;
-    ldsf* M = to_lds(buf);
-    ldsf* Q = M + JPK;
-    ldsf* cs = Q + JS * JS;
-    ldsi* sc = to_lds(sched);
-    build_schedules_wave(sc);
+    const int k = blockIdx.x;
+    ldsf* D = to_lds(buf);
     int I, J;
     rr_pair(r, k, nb2, I, J);
-    for (int e = lane; e < JS * JS; e += WAVE) {
-        const int i = e / JS, j = e % JS;
-        if (j >= i) {
-            const int gi = slot_index(I, J, i, n), gj = slot_index(I, J, j, n);
-            double v = 0.0;
-            if (gi >= 0 && gj >= 0) v = A[(size_t)(gi < gj ? gi : gj) * n + (gi < gj ? gj : gi)];
-            pk(M, i, j) = v;
-        }
-    }
-    wave_sync();
-    const int rot = wave_jacobi_sub(M, Q, cs, sc, tol, inner, 0, 0u, 0u);
-    glbf* qg = to_glb(Qbuf) + (size_t)k * JS * JS;
-    if (lane == 0) ident[k] = rot ? 0 : 1;
-    if (rot) {
-        for (int e = lane; e < JS * JS; e += WAVE) {
-            qg[e] = Q[(e % JS) * JS + e / JS];  // Q[i][j] = Qt[j][i]
-            const int i = e / JS, j = e % JS;
-            const int gi = slot_index(I, J, i, n), gj = slot_index(I, J, j, n);
-            if (gi >= 0 && gj >= 0) A[(size_t)gi * n + gj] = pk(M, i, j);
-        }
-    }
+    sub_stage(A, n, I, J, D);
+    const int rot = wave_jacobi_sub(D, D + JD, to_glb(Qbuf) + (size_t)k * JS * JS, tol, inner, 0, 0u, 0u);
+    if (threadIdx.x == 0) ident[k] = rot ? 0 : 1;
+    if (rot) sub_unstage(A, n, I, J, D);
 }
 
 // one wave per work item: the ntile off-diagonal tiles (k < l) of A, then

@@ -32,7 +32,7 @@ extern "C" int32_t xtb_scf_lds_bytes(const xtb_batch* batch, int32_t* bytes, int
         const int ring = ring_doubles(n, ring_pitch(n, avail));
         cap = std::max(cap, std::max(want_a, ring));
     } else {
-        cap = NBLOCK_LDS > cap ? NBLOCK_LDS : cap;  // block Jacobi
+        cap = NMIXED_LDS;  // block Jacobi for the largest
     }
     if (L.total_fixed + cap > budget) return XTB_ETOOBIG;
     *big_cap = cap;

@@ -687,8 +687,8 @@ struct Ring {
 
 // doubles that Ring needs for n with row pitch W (the row of the fixed index
 // exists for even n only; it is a dummy otherwise)
-__host__ __device__ inline int ring_pairs(int n) { return (n + 1) / 2; }
-__host__ __device__ inline int ring_doubles(int n, int W) {
+__host__ __device__ constexpr int ring_pairs(int n) { return (n + 1) / 2; }
+__host__ __device__ constexpr int ring_doubles(int n, int W) {
     return ring_pairs(n) * W + (n % 2 == 0 ? n : 0);
 }
 // row pitch: the next W = 2 mod 4 if the matrix then fits in cap doubles
@@ -1019,23 +1019,20 @@ __device__ __noinline__ int wg_jacobi(glbf* A, int n, ldsf* D, int W, glbf* Ct, 
 // ~3 n^3 bytes instead of the ~32 n^3 of the scalar method.
 // ---------------------------------------------------------------------------
 constexpr int JB = 16;
-constexpr int JS = 2 * JB;                  // subproblem dimension
-constexpr int JPK = JS * (JS + 1) / 2;      // packed subproblem
-constexpr int JWAVE_LDS = JPK + JS * JS + JS;  // M (packed), Q, c/s
-constexpr int NPAIR32 = JS / 2;                      // 16 pairs per round
-constexpr int NBLK32 = NPAIR32 * (NPAIR32 + 1) / 2;  // 136 blocks
-constexpr int SCHED_INTS = (JS - 1) * NPAIR32 + NBLK32;
-constexpr int NBLOCK_LDS = NWAVE * JWAVE_LDS + 64 + (SCHED_INTS + 1) / 2;  // + flags, schedules
+constexpr int JS = 2 * JB;               // subproblem dimension
+constexpr int JW = 34;                   // row pitch of its ring storage
+constexpr int JD = ring_doubles(JS, JW);
+constexpr int JWAVE_LDS = JD + JS;       // D, (c, s)
+constexpr int NBLOCK_LDS = NWAVE * JWAVE_LDS + 64;  // + flags
+// The LDS share of a launch whose largest matrix does not fit: matrices up to
+// 161 orbitals among its molecules still take the LDS Jacobi.
+constexpr int NMIXED_LDS = 13052;
+static_assert(NBLOCK_LDS <= NMIXED_LDS && NGEMM_MFMA_LDS <= NMIXED_LDS, "LDS of the mixed launches");
 
 __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-__device__ inline ldsf& pk(ldsf* M, int i, int j) {
-    if (i > j) { int t = i; i = j; j = t; }
-    return M[i * JS - (i * (i - 1)) / 2 + (j - i)];
 }
 
 // Global index of slot i (0..31) of the subproblem of block pair (I, J):
@@ -1046,176 +1043,174 @@ __device__ inline int slot_index(int I, int J, int i, int n) {
     return g < n ? g : -1;
 }
 
-// Round-robin pair of a 32-slot subproblem (constant modulus).
-__device__ inline void rr32(int r, int k, int& p, int& q) {
-    if (k == 0) { p = 31; q = r; }
-    else { p = (r + k) % 31; q = (r - k + 31) % 31; }
+// lane l of each row of 16 <- lane l - 1 (lane 0 <- first), and <- l + 1 (lane 15 <- last)
+__device__ inline double row_up(double v, double first) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(v), 0x111, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(v), 0x111, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ inline double row_down(double v, double last) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(last), __double2loint(v), 0x101, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(last), __double2hiint(v), 0x101, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
 }
 
-// Schedules of the 32-slot subproblem, built once per block-Jacobi call in
-// LDS: rrtab[r*16+k] = p | q<<8 for pair k of round r, and blktab[e] =
-// P | R<<8 for the e-th 2x2 block (P <= R) of a round.
-
-__device__ inline void build_schedules(ldsi* tab) {
-    for (int e = threadIdx.x; e < (JS - 1) * NPAIR32; e += NT) {
-        int p, q;
-        rr32(e / NPAIR32, e % NPAIR32, p, q);
-        tab[e] = p | (q << 8);
-    }
-    for (int e = threadIdx.x; e < NBLK32; e += NT) {
-        int P = 0, rem = e;
-        while (rem >= NPAIR32 - P) { rem -= NPAIR32 - P; ++P; }
-        tab[(JS - 1) * NPAIR32 + e] = P | ((P + rem) << 8);
-    }
-}
-
-// Wave-level cyclic Jacobi on the packed JS x JS matrix M (slots whose
-// rows/columns are zero are never rotated).  Qt (JS x JS, Qt[col][row])
-// accumulates the rotations so that M_final = Q^T M_0 Q.  Returns 1 if any
-// rotation was applied, 0 if M was already diagonal to `tol` (Q = I).
+// Cyclic Jacobi on a 32 x 32 subproblem by one wavefront, in place on its ring
+// storage D (pitch JW; zero rows and columns are never rotated).  The
+// rotations Q, D_final = Q^T D_0 Q, go to qg (Q[i][j] at qg[i JS + j]) if any
+// was applied; returns 1 then, 0 if D was already diagonal to `tol`.
 //
-// A round is two LDS round trips per lane: the 16 rotation lanes read their
-// pivots and publish (c, s); then every lane gathers the schedule entries,
-// (c, s) and matrix/vector elements of all its work items at once, computes,
-// and stores.  Work items: the 2x2 blocks lane, lane+64, lane+128 (of 136)
-// of the two-sided update, and 8 (pair, row) elements of Qt.  Items touch
-// disjoint elements, so no ordering among them is needed.
-__device__ __noinline__ int wave_jacobi_sub(ldsf* M, ldsf* Qt, ldsf* cs, const ldsi* sched,
-                                            double tol, int max_sweeps, int mode, unsigned lo_mask,
-                                            unsigned hi_mask) {
-    const int lane = threadIdx.x % WAVE;
+// As in the workgroup's rounds, but all in one wave: every lane computes the
+// rotation of position lane % 16 (one LDS trip for its pivots), the lanes hold
+// two of the 120 2 x 2 blocks each, and Q stays in registers, 8 columns per
+// row of 16 lanes, its rows moving around the ring by row shifts of the lanes.
+// A round is bound by that chain.  With n = 296 on the whole GPU a subproblem
+// takes 27 us; looking up a schedule, packed triangle indices and Q's rows in
+// LDS took 62 us.
+__device__ __noinline__ int wave_jacobi_sub(ldsf* D, ldsf* cs, glbf* qg, double tol, int max_sweeps, int mode,
+                                            unsigned lo_mask, unsigned hi_mask) {
+    constexpr int K = JB, m = JS - 1, E = K * JW;
+    const int lane = threadIdx.x % WAVE, k = lane % K, g0 = lane / K * 8;
+    const Ring G{D, JS, m, K, JW};
     // occupation class of a slot (pairs are selected by mode as in wg_jacobi)
     auto scls = [&](int i) { return (int)((lo_mask >> i) & 1u) + (int)((hi_mask >> i) & 1u); };
-    const ldsi* rrtab = sched;
-    const ldsi* blktab = sched + (JS - 1) * NPAIR32;
-    constexpr int NB = (NBLK32 + WAVE - 1) / WAVE;  // 3 block slots per lane
-    constexpr int NQ = NPAIR32 / (WAVE / JS);       // 8 Qt items per lane
-    int bP[NB], bR[NB];
+    ldsf* ad[2][4];
+    ldsf *cp[2], *cr[2];
+    uint32_t rw[2];  // byte u: the round after which address u wraps
 #pragma unroll
-    for (int j = 0; j < NB; ++j) {
-        const int e = lane + WAVE * j;
-        const int PR = (e < NBLK32) ? blktab[e] : -1;
-        bP[j] = (e < NBLK32) ? (PR & 255) : -1;
-        bR[j] = (e < NBLK32) ? (PR >> 8) : -1;
+    for (int g = 0; g < 2; ++g) {
+        const int e = lane + g * WAVE < K * (K - 1) / 2 ? lane + g * WAVE : K * (K - 1) / 2 - 1;
+        const int d = e / K, t = e % K;
+        const bool lo = t < K - 1 - d;
+        const int P = lo ? d : K - 2 - d, R = lo ? d + 1 + t : t;
+        const int q = G.wrap(-P), b = G.wrap(-R);
+        const int dm = R - P, dp = R + P;
+        const bool fold = dp >= K;
+        const int row = (fold ? m - dp : dp) * JW;
+        const int i0 = P == 0 ? R : P, i1 = P == 0 ? b : (fold ? P : b), i2 = fold ? R : q;
+        ad[g][0] = D + (P == 0 ? E : dm * JW) + i0;
+        ad[g][1] = D + (P == 0 ? E : row) + i1;
+        ad[g][2] = D + row + i2;
+        ad[g][3] = D + dm * JW + b;
+        rw[g] = (uint32_t)(m - 1 - i0) | (uint32_t)(m - 1 - i1) << 8 | (uint32_t)(m - 1 - i2) << 16 |
+                (uint32_t)(m - 1 - b) << 24;
+        cp[g] = cs + 2 * P;
+        cr[g] = cs + 2 * R;
     }
-    const int qrow = lane % JS, qk0 = lane / JS;
-    for (int e = lane; e < JS * JS; e += WAVE) Qt[e] = ((e / JS) == (e % JS)) ? 1.0 : 0.0;
-    wave_sync();
+    // rows of Q^T at this lane's position: top (k, or the fixed row 31) and
+    // bottom (31 - k, or 0), columns g0 .. g0 + 7 of the identity
+    const int rt = k == 0 ? m : k, rb = k == 0 ? 0 : m - k;
+    double top[8], bot[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        top[c] = rt == g0 + c ? 1.0 : 0.0;
+        bot[c] = rb == g0 + c ? 1.0 : 0.0;
+    }
     const double skip = 1e-3 * tol;
     int rotated = 0;
     for (int sw = 0; sw < max_sweeps; ++sw) {
         double off = 0.0;
-        for (int e = lane; e < JS * JS; e += WAVE) {
-            const int i = e / JS, j = e % JS;
-            if (j > i && pair_in_mode(mode, scls(i), scls(j))) off = fmax(off, fabs(pk(M, i, j)));
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int d = 1 + 2 * u + (lane >> 5), i = lane & 31;
+            if (d < K && i < m && pair_in_mode(mode, scls(i), scls(G.wrap(i + d)))) off = fmax(off, fabs(D[d * JW + i]));
         }
+        if (lane < m && pair_in_mode(mode, scls(lane), scls(m))) off = fmax(off, fabs(D[E + lane]));
         off = wave_max(off);
         if (off <= tol) break;
         rotated = 1;
-        for (int r = 0; r < JS - 1; ++r) {
-            const ldsi* rr = rrtab + r * NPAIR32;
-            if (lane < NPAIR32) {
-                const int pq = rr[lane];
-                const int p = pq & 255, q = pq >> 8;
-                double c = 1.0, s = 0.0;
-                const double apq = pk(M, p, q), app = pk(M, p, p), aqq = pk(M, q, q);
-                if (fabs(apq) > skip && pair_in_mode(mode, scls(p), scls(q))) {
-                    const double theta = (aqq - app) / (2.0 * apq);
-                    double t = 1.0 / (fabs(theta) + sqrt(fma(theta, theta, 1.0)));
-                    if (theta < 0.0) t = -t;
-                    c = 1.0 / sqrt(fma(t, t, 1.0));
-                    s = t * c;
+        for (int r = 0; r < m; ++r) {
+            const int p = k == 0 ? m : G.wrap(r + k), q = G.wrap(r - k);
+            const int epq = k == 0 ? E + q : (2 * k < K ? 2 * k * JW + q : (m - 2 * k) * JW + p);
+            const int epp = k == 0 ? E + m : p;
+            const double apq = D[epq], app = D[epp], aqq = D[q];
+            double c = 1.0, s = 0.0;
+            if (fabs(apq) > skip && pair_in_mode(mode, scls(p), scls(q))) {
+                const double dd = aqq - app, ee = 2.0 * apq;
+                const double h2 = fma(dd, dd, ee * ee);
+                double t = ee * fast_rcp(fma(h2, fast_rsq(h2), fabs(dd)));
+                if (dd < 0.0) t = -t;
+                c = fast_rsq(fma(t, t, 1.0));
+                s = t * c;
+                if (lane < K) {
+                    D[epp] = fma(-t, apq, app);
+                    D[q] = fma(t, apq, aqq);
+                    D[epq] = 0.0;
                 }
-                cs[lane] = c;
-                cs[JB + lane] = s;
+            }
+            if (lane < K) {
+                const v2d v = {c, s};
+                *(ldsv2*)(cs + 2 * k) = v;
             }
             wave_sync();
-            // gather: schedule entries and rotation parameters
-            int bpq[NB], bxy[NB];
-            double bcp[NB], bsp[NB], bcr[NB], bsr[NB];
+            v2d vp[2], vr[2];
+            double x[2][4];
 #pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                const int P = bP[j] < 0 ? 0 : bP[j], R = bR[j] < 0 ? 0 : bR[j];
-                bpq[j] = rr[P];
-                bxy[j] = rr[R];
-                bcp[j] = cs[P];
-                bsp[j] = cs[JB + P];
-                bcr[j] = cs[R];
-                bsr[j] = cs[JB + R];
+            for (int g = 0; g < 2; ++g) {
+                vp[g] = *(ldsv2*)cp[g];
+                vr[g] = *(ldsv2*)cr[g];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) x[g][u] = *ad[g][u];
             }
-            int qpq[NQ];
-            double qc[NQ], qs[NQ];
 #pragma unroll
-            for (int j = 0; j < NQ; ++j) {
-                const int k = qk0 + 2 * j;
-                qpq[j] = rr[k];
-                qc[j] = cs[k];
-                qs[j] = cs[JB + k];
+            for (int y = 0; y < 8; ++y) {
+                const double a = top[y], b = bot[y];
+                const double t = c * a - s * b, e = s * a + c * b;
+                const double up = row_down(t, e);
+                bot[y] = row_up(e, up);
+                top[y] = k == 0 ? t : up;
             }
-            // gather: matrix and vector elements
-            double m[NB][4];
-            int mi[NB][4];
 #pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                const int p = bpq[j] & 255, q = bpq[j] >> 8, x = bxy[j] & 255, y = bxy[j] >> 8;
-                const bool diag = bP[j] == bR[j];
-                int i0 = diag ? p : p, j0 = diag ? p : x;
-                int i1 = diag ? q : p, j1 = diag ? q : y;
-                int i2 = diag ? p : q, j2 = diag ? q : x;
-                int i3 = diag ? p : q, j3 = diag ? q : y;
-                mi[j][0] = (i0 <= j0) ? i0 * JS - (i0 * (i0 - 1)) / 2 + (j0 - i0)
-                                      : j0 * JS - (j0 * (j0 - 1)) / 2 + (i0 - j0);
-                mi[j][1] = (i1 <= j1) ? i1 * JS - (i1 * (i1 - 1)) / 2 + (j1 - i1)
-                                      : j1 * JS - (j1 * (j1 - 1)) / 2 + (i1 - j1);
-                mi[j][2] = (i2 <= j2) ? i2 * JS - (i2 * (i2 - 1)) / 2 + (j2 - i2)
-                                      : j2 * JS - (j2 * (j2 - 1)) / 2 + (i2 - j2);
-                mi[j][3] = (i3 <= j3) ? i3 * JS - (i3 * (i3 - 1)) / 2 + (j3 - i3)
-                                      : j3 * JS - (j3 * (j3 - 1)) / 2 + (i3 - j3);
-#pragma unroll
-                for (int u = 0; u < 4; ++u) m[j][u] = M[mi[j][u]];
-            }
-            double qa[NQ], qb[NQ];
-#pragma unroll
-            for (int j = 0; j < NQ; ++j) {
-                const int p = qpq[j] & 255, q = qpq[j] >> 8;
-                qa[j] = Qt[p * JS + qrow];
-                qb[j] = Qt[q * JS + qrow];
-            }
-            // compute and store.  Diagonal block (P == R): elements
-            // (p,p), (q,q), (p,q); off-diagonal: (p,x), (p,y), (q,x), (q,y).
-#pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                const double sp = bsp[j], sr = bsr[j], cp = bcp[j], cr = bcr[j];
-                if (bP[j] < 0 || (sp == 0.0 && sr == 0.0)) continue;
-                if (bP[j] == bR[j]) {
-                    const double apq = m[j][2];
-                    const double t = sp / cp;
-                    M[mi[j][0]] = m[j][0] - t * apq;
-                    M[mi[j][1]] = m[j][1] + t * apq;
-                    M[mi[j][2]] = 0.0;
-                } else {
-                    const double m00 = m[j][0], m01 = m[j][1], m10 = m[j][2], m11 = m[j][3];
-                    const double r00 = cp * m00 - sp * m10, r01 = cp * m01 - sp * m11;
-                    const double r10 = sp * m00 + cp * m10, r11 = sp * m01 + cp * m11;
-                    M[mi[j][0]] = r00 * cr - r01 * sr;
-                    M[mi[j][1]] = r00 * sr + r01 * cr;
-                    M[mi[j][2]] = r10 * cr - r11 * sr;
-                    M[mi[j][3]] = r10 * sr + r11 * cr;
+            for (int g = 0; g < 2; ++g) {
+                const double c1 = vp[g].x, s1 = vp[g].y, c2 = vr[g].x, s2 = vr[g].y;
+                const double r00 = c1 * x[g][0] - s1 * x[g][2], r01 = c1 * x[g][1] - s1 * x[g][3];
+                const double r10 = s1 * x[g][0] + c1 * x[g][2], r11 = s1 * x[g][1] + c1 * x[g][3];
+                if ((g == 0 || lane + g * WAVE < K * (K - 1) / 2) && (s1 != 0.0 || s2 != 0.0)) {
+                    *ad[g][0] = r00 * c2 - r01 * s2;
+                    *ad[g][1] = r00 * s2 + r01 * c2;
+                    *ad[g][2] = r10 * c2 - r11 * s2;
+                    *ad[g][3] = r10 * s2 + r11 * c2;
                 }
-            }
 #pragma unroll
-            for (int j = 0; j < NQ; ++j) {
-                const double s = qs[j];
-                if (s == 0.0) continue;
-                const double c = qc[j];
-                const int p = qpq[j] & 255, q = qpq[j] >> 8;
-                Qt[p * JS + qrow] = c * qa[j] - s * qb[j];
-                Qt[q * JS + qrow] = s * qa[j] + c * qb[j];
+                for (int u = 0; u < 4; ++u) ad[g][u] += ((rw[g] >> (8 * u)) & 255u) == (uint32_t)r ? 1 - m : 1;
             }
             wave_sync();
         }
     }
+    if (rotated) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            qg[(g0 + c) * JS + rt] = top[c];
+            qg[(g0 + c) * JS + rb] = bot[c];
+        }
+    }
     return rotated;
+}
+
+// The subproblem of block pair (I, J) of A (full, global, upper triangle
+// read): staged into D (slots beyond n zero), and its diagonalised form
+// written back (every element).
+__device__ inline void sub_stage(const glbf* A, int n, int I, int J, ldsf* D) {
+    const int lane = threadIdx.x % WAVE;
+    const Ring G{D, JS, JS - 1, JB, JW};
+    for (int e = lane; e < JS * JS; e += WAVE) {
+        const int i = e / JS, j = e % JS;
+        if (j < i) continue;
+        const int gi = slot_index(I, J, i, n), gj = slot_index(I, J, j, n);
+        double v = 0.0;
+        if (gi >= 0 && gj >= 0) v = A[(size_t)(gi < gj ? gi : gj) * n + (gi < gj ? gj : gi)];
+        D[i == j ? G.diag(i) : G.at(i, j)] = v;
+    }
+    wave_sync();
+}
+__device__ inline void sub_unstage(glbf* A, int n, int I, int J, ldsf* D) {
+    const int lane = threadIdx.x % WAVE;
+    const Ring G{D, JS, JS - 1, JB, JW};
+    for (int e = lane; e < JS * JS; e += WAVE) {
+        const int i = e / JS, j = e % JS;
+        const int gi = slot_index(I, J, i, n), gj = slot_index(I, J, j, n);
+        if (gi >= 0 && gj >= 0) A[(size_t)gi * n + gj] = D[i == j ? G.diag(i) : G.at(i, j)];
+    }
 }
 
 // Two-sided tile update on matrix cores (one wavefront):
@@ -1345,17 +1340,14 @@ __device__ __noinline__ int wg_block_jacobi(glbf* A, int n, CAcc Ct, glbf* Qbuf,
     // still meets a block of its own class if each class spans two blocks
     const bool skip_cross = mode == 2 && cb_lo >= 2 * JB && n - cb_hi >= 2 * JB;
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    ldsf* M = lds + w * JWAVE_LDS;
-    ldsf* Q = M + JPK;
-    ldsf* cs = Q + JS * JS;
+    ldsf* D = lds + w * JWAVE_LDS;
+    ldsf* cs = D + JD;
     const int nb = (n + JB - 1) / JB;
     const int nb2 = nb + (nb & 1);
     const int npair = nb2 / 2;
     const int ntile = npair * (npair - 1) / 2;
     const int nch = (n + WAVE - 1) / WAVE;
     ldsi* ident = reinterpret_cast<ldsi*>(lds + NWAVE * JWAVE_LDS);  // per pair: Q == I
-    ldsi* sched = ident + 128;                                        // subproblem schedules
-    build_schedules(sched);
     // symmetrise from the upper triangle
     for (int i = w; i < n; i += NWAVE)
         for (int j = lane; j < i; j += WAVE) A[(size_t)i * n + j] = A[(size_t)j * n + i];
@@ -1418,28 +1410,11 @@ __device__ __noinline__ int wg_block_jacobi(glbf* A, int n, CAcc Ct, glbf* Qbuf,
                         continue;
                     }
                 }
-                for (int e = lane; e < JS * JS; e += WAVE) {
-                    const int i = e / JS, j = e % JS;
-                    if (j >= i) {
-                        const int gi = slot_index(I, J, i, n), gj = slot_index(I, J, j, n);
-                        double v = 0.0;
-                        if (gi >= 0 && gj >= 0)
-                            v = A[(size_t)(gi < gj ? gi : gj) * n + (gi < gj ? gj : gi)];
-                        pk(M, i, j) = v;
-                    }
-                }
-                wave_sync();
-                const int rot = wave_jacobi_sub(M, Q, cs, sched, tol, inner, mode, lo_mask, hi_mask);
-                glbf* qg = Qbuf + (size_t)k * JS * JS;
+                sub_stage(A, n, I, J, D);
+                const int rot =
+                    wave_jacobi_sub(D, cs, Qbuf + (size_t)k * JS * JS, tol, inner, mode, lo_mask, hi_mask);
                 if (lane == 0) ident[k] = rot ? 0 : 1;
-                if (rot) {
-                    for (int e = lane; e < JS * JS; e += WAVE) {
-                        qg[e] = Q[(e % JS) * JS + e / JS];  // Q[i][j] = Qt[j][i]
-                        const int i = e / JS, j = e % JS;
-                        const int gi = slot_index(I, J, i, n), gj = slot_index(I, J, j, n);
-                        if (gi >= 0 && gj >= 0) A[(size_t)gi * n + gj] = pk(M, i, j);
-                    }
-                }
+                if (rot) sub_unstage(A, n, I, J, D);
                 wave_sync();
             }
             __syncthreads();
