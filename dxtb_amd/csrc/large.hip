@@ -450,45 +450,11 @@ __global__ void __launch_bounds__(NT) k_dev_identity(int n, const double* T, dou
 // chol_setup in scf.hip), 32-wide panels.  k_chol_diag: one wave factors the
 // diagonal block j0 of the lower triangle of L in place and writes its
 // inverse to Dg (nb x nb, leading dimension nb); a non-positive pivot sets
-// ctl[C_ERR].  With factor = 0 it only inverts the (already factored) block.
+// ctl[C_ERR].
 // ---------------------------------------------------------------------------
-__device__ inline void chol_diag_block(ldsf* D, ldsf* Di, glbf* L, int n, int j0, int factor, glbf* Dg,
-                                       double* ctl, int lane) {
-    constexpr int NB = 32;
-    const int nb = n - j0 < NB ? n - j0 : NB;
-    for (int e = lane; e < NB * NB; e += WAVE) {
-        const int r = e / NB, c = e % NB;
-        D[e] = (r < nb && c < nb) ? ((factor || c <= r) ? L[(size_t)(j0 + r) * n + j0 + c] : 0.0)
-                                  : (r == c ? 1.0 : 0.0);
-    }
-    wave_sync();
-    if (factor) {
-        const bool ok = chol_block_factor(D, lane);
-        if (!ok && lane == 0) ctl[C_ERR] = 1.0;
-        for (int e = lane; e < nb * nb; e += WAVE) {
-            const int r = e / nb, c = e % nb;
-            if (c <= r) L[(size_t)(j0 + r) * n + j0 + c] = D[r * NB + c];
-        }
-        wave_sync();
-    }
-    chol_block_inverse(D, Di, Dg, nb, lane);
-}
-
-__global__ void __launch_bounds__(WAVE) k_chol_diag(double* L_, int n, int j0, int factor, double* Dg_,
-                                                    double* ctl) {
-    __shared__ double dl[32 * 32], dil[32 * 32];
-    chol_diag_block(to_lds(dl), to_lds(dil), to_glb(L_), n, j0, factor, to_glb(Dg_), ctl, threadIdx.x);
-}
-
-// The inverses of all diagonal blocks of a finished factor L at once (they
-// are independent): block j (rows 32 j ..) to Dg + 32 j * 32, nb x nb with
-// leading dimension nb; one wave per block.  Dg holds 32 n doubles (n >= 32)
-// or n^2.
-__global__ void __launch_bounds__(WAVE) k_chol_inv_all(double* L_, int n, double* Dg_) {
-    __shared__ double dl[32 * 32], dil[32 * 32];
-    const int j0 = blockIdx.x * 32;
-    chol_diag_block(to_lds(dl), to_lds(dil), to_glb(L_), n, j0, 0, to_glb(Dg_ + (size_t)j0 * 32), nullptr,
-                    threadIdx.x);
+__global__ void __launch_bounds__(WAVE) k_chol_diag(double* L, int n, int j0, int nb, double* Dg, double* ctl) {
+    const bool ok = chol_block(to_glb(L) + (size_t)j0 * n + j0, n, nb, to_glb(Dg));
+    if (!ok && threadIdx.x == 0) ctl[C_ERR] = 1.0;
 }
 
 // Y[r][c] = X[r][c] for r < rows, c < cols (leading dimensions ldx, ldy)
@@ -1076,7 +1042,7 @@ bool warm_orthonormalise(Ctx& c, const double* pot) {
 // solve and the trailing update are grid GEMMs), then X = L^-1 by the
 // right-looking triangular inverse: block row j of X <- D_j^-1 X_j, rows
 // below -= L_(>j, j) X_j, on the identity.  L in T, X in the orbital buffer,
-// R (rows x 32, leading dimension n) in F, the block inverse in P.  Returns
+// R (rows x 32, leading dimension n) in F, the block inverses in P.  Returns
 // false when S is not numerically positive definite.
 bool ortho_chol(Ctx& c) {
     constexpr int NB = 32;
@@ -1090,12 +1056,13 @@ bool ortho_chol(Ctx& c) {
     chk_launch(c);
     for (int j0 = 0; j0 < n; j0 += NB) {
         const int nb = n - j0 < NB ? n - j0 : NB;
-        hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(WAVE), 0, c.s, L, n, j0, 1, Dg, c.ctl);
+        double* D = Dg + (size_t)j0 * NB;
+        hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(WAVE), 0, c.s, L, n, j0, nb, D, c.ctl);
         chk_launch(c);
         const int mt = n - j0 - nb;
         if (mt > 0) {
             double* Pn = L + (size_t)(j0 + nb) * n + j0;  // panel below the block
-            gemm_t<false, true, false>(c, mt, nb, nb, 1.0, Pn, n, Dg, nb, 0.0, R, n, false);  // b D^-T
+            gemm_t<false, true, false>(c, mt, nb, nb, 1.0, Pn, n, D, nb, 0.0, R, n, false);  // b D^-T
             hipLaunchKernelGGL(k_copy_block, dim3(1, mt), dim3(256), 0, c.s, mt, nb, R, n, Pn, n);
             chk_launch(c);
             gemm_t<false, true, false>(c, mt, mt, nb, -1.0, Pn, n, Pn, n, 1.0, Pn + nb, n, false);
@@ -1103,8 +1070,6 @@ bool ortho_chol(Ctx& c) {
     }
     if (!read_ctl(c) || c.h[C_ERR] != 0.0) return false;
     hipLaunchKernelGGL(k_identity, dim3((n + 255) / 256, n), dim3(256), 0, c.s, n, X);
-    chk_launch(c);
-    hipLaunchKernelGGL(k_chol_inv_all, dim3((n + NB - 1) / NB), dim3(WAVE), 0, c.s, L, n, Dg);
     chk_launch(c);
     for (int j0 = 0; j0 < n; j0 += NB) {
         const int nb = n - j0 < NB ? n - j0 : NB;

@@ -60,52 +60,57 @@ constexpr int PD_EXACT_PASSES = 7;
 constexpr double PD_FINAL_REL = 1e-1;
 
 // ---------------------------------------------------------------------------
-// Diagonal blocks of the blocked Cholesky orthogonaliser (one wave, 32 x 32
-// in LDS, row-major).  chol_block_factor: D <- its lower Cholesky factor in
-// place (the upper triangle is left stale); returns false when a pivot is
-// not positive (the pivot is then taken as 1 and the factor is meaningless).
+// Diagonal blocks of the blocked Cholesky factorisations: one wave, a row per
+// lane in registers.  Lane r < 32 holds row r of the block and lane 32 + j
+// row j of the identity; the column operations that turn the block into its
+// factor L turn the identity into L^-T, so both come out of one pass.  Every
+// step works on register 0 and moves the others down by one (chol_steps: CNT
+// columns are left behind the pivot at most).
+//
+// The pass is bound by its serial chain, the pivot's inverse square root and
+// then two lane reads and an FMA per column left: 13 us a block as a launch
+// of its own.  Factor and inverse through LDS, with the inverse by
+// substitution in one lane per column, took 65 us.
 // ---------------------------------------------------------------------------
-__device__ inline bool chol_block_factor(ldsf* D, int lane) {
-    constexpr int NB = 32;
-    bool ok = true;
-    for (int c = 0; c < NB; ++c) {
-        const double d = D[c * NB + c];
-        wave_sync();
-        const double sd = d > 0.0 ? sqrt(d) : 1.0;
-        if (!(d > 0.0)) ok = false;
-        if (lane == 0) D[c * NB + c] = sd;
-        for (int r = c + 1 + lane; r < NB; r += WAVE) D[r * NB + c] /= sd;
-        wave_sync();
-        const int m = NB - c - 1;
-        for (int e = lane; e < m * m; e += WAVE) {
-            const int rr = c + 1 + e / m, qq = c + 1 + e % m;
-            if (qq <= rr) D[rr * NB + qq] -= D[rr * NB + c] * D[qq * NB + c];
-        }
-        wave_sync();
+template <int CNT>
+__device__ __forceinline__ void chol_steps(double (&x)[32], int c0, int nb, bool& ok, glbf* out, int step) {
+    const int lane = threadIdx.x % WAVE;
+    for (int c = c0; c < c0 + 8; ++c) {
+        const double d = wave_read(x[0], c);
+        const bool pos = d > 0.0;
+        ok = ok && pos;
+        // sqrt(d) and the column over it, each corrected by its residual
+        const double inv = pos ? fast_rsq(d) : 1.0;
+        double sd = d * inv, v = x[0] * inv;
+        sd = pos ? fma(fma(-sd, sd, d), 0.5 * inv, sd) : 1.0;
+        v = fma(fma(-v, sd, x[0]), inv, v);
+#pragma unroll
+        for (int i = 0; i < CNT; ++i) x[i] = fma(-v, wave_read(v, c + 1 + i), x[i + 1]);
+        const int r = lane % 32;
+        if (r < nb && c < nb && (lane >= 32 || r >= c)) out[(size_t)c * step] = lane >= 32 && r > c ? 0.0 : v;
     }
-    return ok;
 }
 
-__device__ inline void chol_block_inverse(ldsf* D, ldsf* Di, glbf* Dg, int nb, int lane) {
-    // lower-triangular D (NB x NB, LDS) -> Di = D^-1 (LDS) and its leading
-    // nb x nb block to Dg (global, leading dimension nb: it must fit in an
-    // n x n buffer when n < NB); lane j forms column j by forward substitution
-    constexpr int NB = 32;
-    if (lane < NB) {
-        const int j = lane;
-        for (int i = 0; i < NB; ++i) {
-            double v;
-            if (i < j) v = 0.0;
-            else if (i == j) v = 1.0 / D[j * NB + j];
-            else {
-                double acc = 0.0;
-                for (int k = j; k < i; ++k) acc = fma(D[i * NB + k], Di[k * NB + j], acc);
-                v = -acc / D[i * NB + i];
-            }
-            Di[i * NB + j] = v;
-            if (i < nb && j < nb) Dg[i * nb + j] = v;
-        }
+// L (leading dimension ld, lower triangle read) <- its lower Cholesky factor
+// in place, the inverse of the factor to Dg (leading dimension nb); nb <= 32.
+// Returns false when a pivot is not positive (taken as 1 then: the factor is
+// meaningless).
+__device__ __noinline__ bool chol_block(glbf* L, int ld, int nb, glbf* Dg) {
+    const int lane = threadIdx.x % WAVE, r = lane % 32;
+    double x[32];
+#pragma unroll
+    for (int c = 0; c < 32; ++c) {
+        const double a = L[(size_t)(r < nb ? r : nb - 1) * ld + (c < nb ? c : nb - 1)];
+        x[c] = lane < 32 && r < nb && c <= r ? a : (r == c ? 1.0 : 0.0);
     }
+    bool ok = true;
+    glbf* out = lane < 32 ? L + (size_t)r * ld : Dg + r;
+    const int step = lane < 32 ? 1 : nb;
+    chol_steps<31>(x, 0, nb, ok, out, step);
+    chol_steps<23>(x, 8, nb, ok, out, step);
+    chol_steps<15>(x, 16, nb, ok, out, step);
+    chol_steps<7>(x, 24, nb, ok, out, step);
+    return ok;
 }
 
 // electronic temperatures below this (0.1 K in Hartree) fill the orbitals

@@ -167,62 +167,31 @@ __device__ __noinline__ int ortho_setup(const Mol& M, const Shared& sh, int* sta
 // In-place blocked right-looking Cholesky L L^T = A of the n x n symmetric
 // positive definite A (lower triangle read and overwritten by L; the strict
 // upper triangle is left as it was), 32-wide panels: one wave factors and
-// inverts each diagonal block in LDS, the panel solve and the trailing
-// update are matrix-core GEMMs.  R (>= n rows x 32, leading dimension n) and
-// Dg (32 x 32) are global scratch.  Returns false when a pivot is not
-// positive.
+// inverts each diagonal block, the panel solve and the trailing update are
+// matrix-core GEMMs.  R (>= n rows x 32, leading dimension n) is
+// global scratch; the inverse of block j0's factor goes to Dg + 32 j0
+// (leading dimension its width; n x 32 doubles, n x n for n < 32).  Returns
+// false when a pivot is not positive.
 __device__ __noinline__ bool chol_factor(glbf* L, int n, glbf* R, glbf* Dg, const Shared& sh) {
     constexpr int NB = 32;
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    // LDS: two 32 x 32 blocks at the end of the GEMM staging area; every GEMM
-    // below runs after the blocks were consumed (the inverse goes through Dg)
-    ldsf* D = sh.big + NGEMM_MFMA_LDS - 2 * NB * NB;
-    ldsf* Di = D + NB * NB;
     bool bad = false;
     for (int j0 = 0; j0 < n; j0 += NB) {
         const int nb = n - j0 < NB ? n - j0 : NB;
-        for (int e = threadIdx.x; e < NB * NB; e += NT) {
-            const int r = e / NB, c = e % NB;
-            D[e] = (r < nb && c < nb) ? L[(size_t)(j0 + r) * n + j0 + c] : (r == c ? 1.0 : 0.0);
-        }
+        glbf* D = Dg + (size_t)j0 * NB;
+        if (w == 0 && !chol_block(L + (size_t)j0 * n + j0, n, nb, D)) bad = true;
         __syncthreads();
-        if (w == 0) {
-            if (!chol_block_factor(D, lane)) bad = true;
-            chol_block_inverse(D, Di, Dg, nb, lane);
-        }
-        __syncthreads();
-        for (int e = threadIdx.x; e < nb * nb; e += NT) {
-            const int r = e / nb, c = e % nb;
-            if (c <= r) L[(size_t)(j0 + r) * n + j0 + c] = D[r * NB + c];
-        }
         const int mt = n - j0 - nb;
         if (mt > 0) {
             glbf* Pn = L + (size_t)(j0 + nb) * n + j0;  // panel below the block
-            gemm<false, true>(mt, nb, nb, 1.0, Pn, n, Dg, nb, 0.0, R, n, sh.big);  // b D^-T
+            gemm<false, true>(mt, nb, nb, 1.0, Pn, n, D, nb, 0.0, R, n, sh.big);  // b D^-T
             for (int r = w; r < mt; r += NWAVE)
                 for (int c = lane; c < nb; c += WAVE) Pn[(size_t)r * n + c] = R[(size_t)r * n + c];
             __syncthreads();
             gemm<false, true>(mt, mt, nb, -1.0, Pn, n, Pn, n, 1.0, Pn + nb, n, sh.big);
-        } else {
-            __syncthreads();
         }
     }
     return !__syncthreads_or(bad);
-}
-
-// Load the lower-triangular diagonal block i0 of L (nb x nb, NB-padded with
-// the identity) and its inverse into Dg (leading dimension nb).
-__device__ inline void chol_diag_inverse(const glbf* L, int n, int i0, int nb, glbf* Dg, const Shared& sh) {
-    constexpr int NB = 32;
-    ldsf* D = sh.big + NGEMM_MFMA_LDS - 2 * NB * NB;
-    ldsf* Di = D + NB * NB;
-    for (int e = threadIdx.x; e < NB * NB; e += NT) {
-        const int r = e / NB, c = e % NB;
-        D[e] = (r < nb && c < nb) ? (c <= r ? L[(size_t)(i0 + r) * n + i0 + c] : 0.0) : (r == c ? 1.0 : 0.0);
-    }
-    __syncthreads();
-    if (threadIdx.x < WAVE) chol_block_inverse(D, Di, Dg, nb, threadIdx.x);
-    __syncthreads();
 }
 
 // Cholesky orthogonaliser: L L^T = S, Ct <- X = L^-1 (rows S-orthonormal).
@@ -235,7 +204,7 @@ __device__ __noinline__ int chol_setup(const Mol& M, const Shared& sh, int* stat
     glbf* L = M.T;
     glbf* X = M.Ct;
     glbf* R = M.F;   // NB x n (and mt x NB) scratch
-    glbf* Dg = M.P;  // NB x NB inverse of the diagonal block
+    glbf* Dg = M.P;  // inverses of the diagonal blocks
     for (int r = w; r < n; r += NWAVE)
         for (int c = lane; c < n; c += WAVE) L[(size_t)r * n + c] = M.S[(size_t)r * n + c];
     __syncthreads();
@@ -250,8 +219,8 @@ __device__ __noinline__ int chol_setup(const Mol& M, const Shared& sh, int* stat
             const int r = e / nb, c = e % nb;
             R[(size_t)r * n + i0 + c] = (r == c) ? 1.0 : 0.0;
         }
-        chol_diag_inverse(L, n, i0, nb, Dg, sh);
-        gemm<false, false>(nb, i0 + nb, nb, 1.0, Dg, nb, R, n, 0.0, X + (size_t)i0 * n, n, sh.big);
+        __syncthreads();
+        gemm<false, false>(nb, i0 + nb, nb, 1.0, Dg + (size_t)i0 * NB, nb, R, n, 0.0, X + (size_t)i0 * n, n, sh.big);
     }
     return 0;
 }
@@ -280,8 +249,7 @@ __device__ __noinline__ bool warm_orthonormalise(const Mol& M, const Shared& sh)
             for (int c = lane; c < n; c += WAVE) R[(size_t)r * n + c] = Ci[(size_t)r * n + c];
         __syncthreads();
         if (i0 > 0) gemm<false, false>(nb, n, i0, -1.0, G + (size_t)i0 * n, n, M.Ct, n, 1.0, R, n, sh.big);
-        chol_diag_inverse(G, n, i0, nb, Dg, sh);
-        gemm<false, false>(nb, n, nb, 1.0, Dg, nb, R, n, 0.0, Ci, n, sh.big);
+        gemm<false, false>(nb, n, nb, 1.0, Dg + (size_t)i0 * NB, nb, R, n, 0.0, Ci, n, sh.big);
     }
     return true;
 }
