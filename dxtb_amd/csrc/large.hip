@@ -537,7 +537,6 @@ __global__ void __launch_bounds__(NT) k_japply(double* A_, double* Ct_, int n, i
 //   ctl[C_PERM]              1 if the sort moved any row
 //   ctl[C_GAPA], ctl[C_GAPB] frontier gaps skey[ia] - skey[ia-1] (ib), +inf
 //                            when the index is outside 1..n-1
-//   ctl[C_DMAX]              max |ev|
 //   ctl[C_FSOFT]             largest f (1 - f) of either channel
 // ---------------------------------------------------------------------------
 
@@ -558,45 +557,26 @@ __global__ void __launch_bounds__(NT) k_sort_fermi(int n, int nao, int npow, con
     sh.skey = ls + 256;
     sh.sidx = reinterpret_cast<ldsi*>(ls + 256 + npow);
     sh.ftot = to_glb(ftot);
-    double dmax = 0.0;
-    for (int j = threadIdx.x; j < npow; j += NT) {
-        const double e = (j < n) ? ev[j] : INFINITY;
-        if (j < n) dmax = fmax(dmax, fabs(e));
-        sh.skey[j] = e;
-        sh.sidx[j] = j;
-    }
-    for (int j = threadIdx.x; j < n; j += NT) ftot[j] = 0.0;
-    dmax = wg_max(dmax, sh.red);
-    __syncthreads();
-    wg_bitonic_sort(sh.skey, sh.sidx, npow);
+    wg_sort(to_glb(ev), sh.skey, sh.sidx, n, npow);
     Mol M;
     M.n = n;
     M.nao = nao;
-    double efa = 0.0, efb = 0.0;
-    bool ok = fermi_channel(M, sh, nel_a, kt, thr, maxiter, false, to_glb(occ), &efa);
-    ok = fermi_channel(M, sh, nel_b, kt, thr, maxiter, false, to_glb(occ) + n, &efb) && ok;
-    int kk = 0, moved = 0;
-    double fs = 0.0;
-    for (int j = threadIdx.x; j < 2 * n; j += NT) fs = fmax(fs, occ[j] * (1.0 - occ[j]));
-    fs = wg_max(fs, sh.red);
+    M.nel_a = nel_a;
+    M.nel_b = nel_b;
+    const Filling fl = fill_orbitals(M, sh, kt, thr, maxiter, false, to_glb(occ), to_glb(occ) + n);
     for (int j = threadIdx.x; j < n; j += NT) {
-        if (ftot[sh.sidx[j]] > 0.0) kk = j + 1;
-        moved |= sh.sidx[j] != j;
         skey_out[j] = sh.skey[j];
         sidx_out[j] = sh.sidx[j];
     }
-    const double kocc = wg_max((double)kk, sh.red);
-    const int perm = __syncthreads_or(moved);
     if (threadIdx.x == 0) {
-        ctl[C_EFA] = efa;
-        ctl[C_EFB] = efb;
-        ctl[C_FOK] = ok ? 1.0 : 0.0;
-        ctl[C_KOCC] = kocc;
-        ctl[C_PERM] = perm ? 1.0 : 0.0;
+        ctl[C_EFA] = fl.ef[0];
+        ctl[C_EFB] = fl.ef[1];
+        ctl[C_FOK] = fl.ok ? 1.0 : 0.0;
+        ctl[C_KOCC] = (double)fl.kocc;
+        ctl[C_PERM] = fl.moved ? 1.0 : 0.0;
         ctl[C_GAPA] = (ia > 0 && ia < n) ? sh.skey[ia] - sh.skey[ia - 1] : INFINITY;
         ctl[C_GAPB] = (ib > 0 && ib < n) ? sh.skey[ib] - sh.skey[ib - 1] : INFINITY;
-        ctl[C_DMAX] = dmax;
-        ctl[C_FSOFT] = fs;
+        ctl[C_FSOFT] = fl.soft;
     }
 }
 

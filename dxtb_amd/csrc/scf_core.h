@@ -119,78 +119,109 @@ __device__ __noinline__ bool chol_block(glbf* L, int ld, int nb, glbf* Dg) {
 constexpr double KT_AUFBAU = 3e-7;
 
 // ---------------------------------------------------------------------------
-// Fermi smearing of one spin channel (src/dxtb/_src/wavefunction/
+// Fermi smearing of the spin channels (src/dxtb/_src/wavefunction/
 // filling.py:201-366): mid-gap start, Newton on the rounded electron count
 // (scf/base.py:879), exponent cutoff 50, threshold on |N - sum f|.  Below
 // KT_AUFBAU the aufbau occupations of the unrounded count instead
 // (filling.py:116-198; base.py:888-889 keeps the initial filling of
 // iterator.py:147-189): orbital j (from 0) is full while j + 1 < nel, the
-// next one takes nel - ceil(nel) + 1.  Sorted eigenvalues in sh.skey.
-// Writes the sorted occupations to occ_out and adds them to sh.ftot.
+// next one takes nel - ceil(nel) + 1.  Sorted eigenvalues in sh.skey, their
+// orbitals in sh.sidx.  Writes the sorted occupations to occ[channel] and
+// the orbitals' sums to sh.ftot.
+//
+// Latency-bound (an exponential and a reduction per Newton step): both
+// channels advance together, and equal ones (closed shells) are one.  With
+// the sort above 13 us a launch at n = 296 (one channel after the other and
+// a bitonic sort: 20 us).
 // ---------------------------------------------------------------------------
+struct Filling {
+    double ef[2];  // Fermi levels
+    double soft;   // largest f (1 - f) of either channel
+    int kocc;      // orbitals with f > 0 (a prefix in sorted order)
+    bool moved;    // the sort moved an orbital
+    bool ok;       // every channel converged
+};
+
 template <class SH>
-__device__ __noinline__ bool fermi_channel(const Mol& M, const SH& sh, double nel, double kt, double thr,
-                              int maxiter, bool padded, glbf* occ_out, double* efermi) {
+__device__ __noinline__ Filling fill_orbitals(const Mol& M, const SH& sh, double kt, double thr, int maxiter,
+                                              bool padded, glbf* occ_a, glbf* occ_b) {
     const int n = M.n;
     const double eps = 2.220446049250313e-16;
-    if (fabs(nel) < eps) {
-        for (int j = threadIdx.x; j < n; j += NT) occ_out[j] = 0.0;
-        *efermi = 0.0;
-        __syncthreads();
-        return true;
+    const int nch = M.nel_a == M.nel_b ? 1 : 2;
+    double ef[2] = {0.0, 0.0}, target[2] = {0.0, 0.0};
+    bool open[2] = {false, false}, smear[2] = {false, false};
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+        double nel = c == 0 ? M.nel_a : M.nel_b;
+        if (c >= nch || fabs(nel) < eps || kt < KT_AUFBAU) continue;
+        nel = rint(nel);
+        int homo = (int)ceil(nel - 5e-15) - 1;
+        if (homo < 0) homo = 0;
+        if (homo > n - 1) homo = n - 1;
+        const int lumo = n - 1 <= homo ? homo : homo + 1;
+        ef[c] = 0.5 * (sh.skey[homo] + sh.skey[lumo]);
+        if (padded && (homo >= M.nao || lumo >= M.nao)) ef[c] *= 2.0;  // filling.py:254-264
+        target[c] = (double)(homo + 1);
+        open[c] = true;
     }
-    if (kt < KT_AUFBAU) {
-        const double frac = nel - ceil(nel) + 1.0;
+    for (int it = 0; it < maxiter && (open[0] || open[1]); ++it) {
+        double acc[4] = {0.0, 0.0, 0.0, 0.0};
         for (int j = threadIdx.x; j < n; j += NT) {
-            const double idx = (double)(j + 1);
-            const double f = idx < nel ? 1.0 : (idx < nel + 1.0 ? frac : 0.0);
-            occ_out[j] = f;
-            sh.ftot[sh.sidx[j]] += f;
+            const double e = sh.skey[j];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                if (!open[c]) continue;
+                const double x = (e - ef[c]) / kt;
+                if (x < 50.0) {
+                    const double et = exp(x), f = 1.0 / (et + 1.0);
+                    acc[2 * c] += f;
+                    acc[2 * c + 1] += et * f * f;
+                } else {
+                    acc[2 * c + 1] += eps * kt;
+                }
+            }
         }
-        *efermi = 0.0;
-        __syncthreads();
-        return true;
-    }
-    nel = rint(nel);
-    int homo = (int)ceil(nel - 5e-15) - 1;
-    if (homo < 0) homo = 0;
-    if (homo > n - 1) homo = n - 1;
-    const bool lumo_missing = (n - 1 <= homo);
-    const int lumo = lumo_missing ? homo : homo + 1;
-    double ef = 0.5 * (sh.skey[homo] + sh.skey[lumo]);
-    if (padded && (homo >= M.nao || lumo >= M.nao)) ef *= 2.0;  // filling.py:254-264
-    const double target = (double)(homo + 1);
-    for (int it = 0; it < maxiter; ++it) {
-        double acc[2] = {0.0, 0.0};
-        for (int j = threadIdx.x; j < n; j += NT) {
-            const double x = (sh.skey[j] - ef) / kt;
-            if (x < 50.0) {
-                const double et = exp(x);
-                acc[0] += 1.0 / (et + 1.0);
-                acc[1] += et / (kt * (et + 1.0) * (et + 1.0));
+        wg_sum_n<4>(acc, sh.red);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            if (!open[c]) continue;
+            const double diff = target[c] - acc[2 * c];
+            if (fabs(diff) <= thr) {
+                open[c] = false;
+                smear[c] = true;
             } else {
-                acc[1] += eps;
+                ef[c] += diff * kt / acc[2 * c + 1];
             }
         }
-        wg_sum_n<2>(acc, sh.red);
-        const double diff = target - acc[0];
-        if (fabs(diff) <= thr) {
-            for (int j = threadIdx.x; j < n; j += NT) {
-                const double x = (sh.skey[j] - ef) / kt;
-                const double f = (x < 50.0) ? 1.0 / (exp(x) + 1.0) : 0.0;
-                occ_out[j] = f;
-                sh.ftot[sh.sidx[j]] += f;
-            }
-            *efermi = ef;
-            __syncthreads();
-            return true;
-        }
-        ef += diff / acc[1];
     }
-    for (int j = threadIdx.x; j < n; j += NT) occ_out[j] = 0.0;
-    *efermi = ef;
-    __syncthreads();
-    return false;
+    const bool ok = !open[0] && !open[1];
+    double red[3] = {0.0, 0.0, 0.0};
+    for (int j = threadIdx.x; j < n; j += NT) {
+        const double e = sh.skey[j];
+        double f[2] = {0.0, 0.0};
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const double nel = c == 0 ? M.nel_a : M.nel_b;
+            if (c >= nch) {
+                f[c] = f[0];
+            } else if (smear[c]) {
+                const double x = (e - ef[c]) / kt;
+                f[c] = x < 50.0 ? 1.0 / (exp(x) + 1.0) : 0.0;
+            } else if (kt < KT_AUFBAU && !(fabs(nel) < eps)) {
+                const double idx = (double)(j + 1);
+                f[c] = idx < nel ? 1.0 : (idx < nel + 1.0 ? nel - ceil(nel) + 1.0 : 0.0);
+            }
+            red[0] = fmax(red[0], f[c] * (1.0 - f[c]));
+        }
+        occ_a[j] = f[0];
+        occ_b[j] = f[1];
+        const int o = sh.sidx[j];
+        sh.ftot[o] = f[0] + f[1];
+        if (f[0] + f[1] > 0.0) red[1] = (double)(j + 1);
+        if (o != j) red[2] = 1.0;
+    }
+    wg_max_n<3>(red, sh.red);
+    return Filling{{ef[0], nch == 1 ? ef[0] : ef[1]}, red[0], (int)red[1], red[2] != 0.0, ok};
 }
 
 // ---------------------------------------------------------------------------
@@ -198,9 +229,8 @@ __device__ __noinline__ bool fermi_channel(const Mol& M, const SH& sh, double ne
 // a ring buffer of G = generations+1 slots.  Returns the convergence flag of
 // the step (mixer/base.py:229-256 on the step's residual).
 // ---------------------------------------------------------------------------
-// largest history (generations) the mixer takes; its Gram system's 27 sums
-// fit one pass of the reduction scratch, and 8 generations (44 sums) grow
-// the kernel's stack by ~0.9 KB per lane for ~1 % fewer iterations
+// largest history (generations) the mixer takes: its system with the right
+// side fits 8 x 8 lanes, and more generations save ~1 % of the iterations
 constexpr int MIX_MAXG = 6;
 
 struct Mixer {
@@ -213,8 +243,12 @@ __device__ __noinline__ bool anderson(Mixer& mx, const Mol& M, const SH& sh, con
                          glbf* hx, glbf* hf, const glbf* xnew, const glbf* xold,
                          glbf* xout, double* resid_inf) {
     const int n = M.n, G = mx.G;
-    auto X = [&](int h) { return hx + (size_t)((mx.head + h) % G) * M.nvec_total + M.vec0; };
-    auto Fh = [&](int h) { return hf + (size_t)((mx.head + h) % G) * M.nvec_total + M.vec0; };
+    auto slot = [&](int h) {  // h < G
+        const int k = mx.head + h;
+        return (size_t)(k < G ? k : k - G) * M.nvec_total + M.vec0;
+    };
+    auto X = [&](int h) { return hx + slot(h); };
+    auto Fh = [&](int h) { return hf + slot(h); };
     if (mx.step == 0) {
         glbf* x0 = X(0);
         for (int i = threadIdx.x; i < n; i += NT) x0[i] = xold[i];
@@ -232,7 +266,7 @@ __device__ __noinline__ bool anderson(Mixer& mx, const Mol& M, const SH& sh, con
         linf = fmax(linf, fabs(f));
     }
     l2 = wg_sum(l2, sh.red);
-    linf = wg_max(linf, sh.red);
+    linf = wg_max(linf, sh.red + NWAVE);
     const bool conv = (sqrt(l2) < o.x_atol) && (linf < o.x_atol_max);
     *resid_inf = linf;
     double theta[MIX_MAXG];
@@ -242,82 +276,69 @@ __device__ __noinline__ bool anderson(Mixer& mx, const Mol& M, const SH& sh, con
     if (mx.step > gen || !mx.soft) nn = (mx.step - 1 < gen) ? mx.step - 1 : gen;  // soft start
     if (nn > 0) {
         // a_hj = (f0 - f_h).(f0 - f_j), b_h = (f0 - f_h).f0 ; h, j = 1..nn.
-        // One pass per h over the elements with at most MIX_MAXG + 1 sums
-        // live; each sum is reduced at once (wave butterfly, then the waves'
-        // partials in LDS added in wave order), so no per-thread array of all
-        // NACC sums stays live (it spilled to scratch on every call)
-        constexpr int NA = MIX_MAXG * (MIX_MAXG + 1) / 2, NACC = NA + MIX_MAXG;
-        static_assert(NACC * NWAVE + NACC <= 256, "reduction scratch");
+        // The nt sums (j = nn + 1: b_h) are dealt to the waves, each over all
+        // elements: no partial sums to combine
         const int wv = threadIdx.x / WAVE, ln = threadIdx.x % WAVE;
-        ldsf* part = sh.red;                 // [NACC][NWAVE]
-        ldsf* tot = sh.red + NACC * NWAVE;   // [NACC]
-        int k0 = 0;
+        constexpr int NACC = MIX_MAXG * (MIX_MAXG + 3) / 2, PER = (NACC + NWAVE - 1) / NWAVE;
+        ldsf* tot = sh.red;
+        const int nt = nn * (nn + 3) / 2;
+        const glbf *ph[PER], *pj[PER];
+        bool rhs[PER];
+        double s[PER];
 #pragma unroll
-        for (int h = 0; h < MIX_MAXG; ++h) {
-            double sj[MIX_MAXG + 1];
+        for (int t = 0; t < PER; ++t) {
+            int e = wv + NWAVE * t < nt ? wv + NWAVE * t : nt - 1, h = 1;
+            while (e >= nn + 2 - h) e -= nn + 2 - h++;
+            ph[t] = Fh(h);
+            rhs[t] = h + e > nn;
+            pj[t] = rhs[t] ? f0 : Fh(h + e);
+            s[t] = 0.0;
+        }
+#pragma unroll 2
+        for (int i = ln; i < n; i += WAVE) {
+            const double fi = f0[i];
 #pragma unroll
-            for (int j = 0; j <= MIX_MAXG; ++j) sj[j] = 0.0;
-            if (h < nn) {
-                for (int i = threadIdx.x; i < n; i += NT) {
-                    const double fi = f0[i];
-                    const double dh = fi - Fh(h + 1)[i];
+            for (int t = 0; t < PER; ++t) {
+                const double a = ph[t][i], b = pj[t][i];
+                s[t] = fma(fi - a, rhs[t] ? b : fi - b, s[t]);
+            }
+        }
 #pragma unroll
-                    for (int j = h; j < MIX_MAXG; ++j)
-                        if (j < nn) sj[j] = fma(dh, fi - Fh(j + 1)[i], sj[j]);
-                    sj[MIX_MAXG] = fma(dh, fi, sj[MIX_MAXG]);
+        for (int t = 0; t < PER; ++t) {
+            s[t] = wave_sum(s[t]);
+            if (ln == 0 && wv + NWAVE * t < nt) tot[wv + NWAVE * t] = s[t];
+        }
+        __syncthreads();
+        // solve (a * diag(1 + off^2)) theta = b by Gauss-Jordan elimination
+        // with partial pivoting: element (r, x) on lane 8 r + x, b in column
+        // 7, the same in every wave.  The mixing step takes 15 us a launch at
+        // n = 296 (every thread with all sums, reduced one by one, and one
+        // thread solving in LDS: 28 us)
+        const int r = ln / 8, x = ln % 8;
+        double a = 0.0;
+        if (r < nn && (x < nn || x == 7)) {
+            const int h = x < r ? x : r, j = x == 7 ? nn : (x < r ? r : x);  // h <= j, from 0
+            a = tot[h * (2 * nn + 3 - h) / 2 + j - h];
+            if (r == x) a *= 1.0 + o.diag_offset * o.diag_offset;
+        }
+        for (int c = 0; c < nn; ++c) {
+            int piv = c;
+            double best = fabs(wave_read(a, 9 * c));
+            for (int q = c + 1; q < nn; ++q) {
+                const double v = fabs(wave_read(a, 8 * q + c));
+                if (v > best) {
+                    best = v;
+                    piv = q;
                 }
             }
+            a = __shfl(a, 8 * (r == c ? piv : (r == piv ? c : r)) + x, WAVE);
+            const double col = __shfl(a, 8 * r + c, WAVE), row = __shfl(a, 8 * c + x, WAVE);
+            const double fct = col / wave_read(a, 9 * c);
+            if (r != c && x >= c) a -= fct * row;
+        }
+        a /= __shfl(a, 9 * r, WAVE);  // column 7: theta
 #pragma unroll
-            for (int j = h; j <= MIX_MAXG; ++j) {
-                const double v = wave_sum(sj[j]);
-                const int e = j < MIX_MAXG ? k0 + (j - h) : NA + h;
-                if (ln == 0) part[e * NWAVE + wv] = v;
-            }
-            k0 += MIX_MAXG - h;
-        }
-        __syncthreads();
-        if (threadIdx.x < NACC) {
-            double v = 0.0;
-            for (int x = 0; x < NWAVE; ++x) v += part[threadIdx.x * NWAVE + x];
-            tot[threadIdx.x] = v;
-        }
-        __syncthreads();
-        // solve (a * diag(1 + off^2)) theta = b by Gaussian elimination with
-        // partial pivoting; one thread, system held in LDS (over the partials)
-        constexpr int W = MIX_MAXG + 1;
-        ldsf* a = sh.red;                  // [MIX_MAXG][W]
-        ldsf* th = sh.red + MIX_MAXG * W;  // [MIX_MAXG]
-        static_assert(MIX_MAXG * W + MIX_MAXG <= NACC * NWAVE, "solver rows below the totals");
-        if (threadIdx.x == 0) {
-            int k = 0;
-            for (int h = 0; h < MIX_MAXG; ++h)
-                for (int j = h; j < MIX_MAXG; ++j) { a[h * W + j] = tot[k]; a[j * W + h] = tot[k]; ++k; }
-            for (int h = 0; h < MIX_MAXG; ++h) a[h * W + MIX_MAXG] = tot[NA + h];
-            for (int h = 0; h < nn; ++h) a[h * W + h] *= 1.0 + o.diag_offset * o.diag_offset;
-            for (int c = 0; c < nn; ++c) {
-                int piv = c;
-                for (int r = c + 1; r < nn; ++r)
-                    if (fabs(a[r * W + c]) > fabs(a[piv * W + c])) piv = r;
-                if (piv != c)
-                    for (int x = 0; x < W; ++x) {
-                        const double t = a[c * W + x];
-                        a[c * W + x] = a[piv * W + x];
-                        a[piv * W + x] = t;
-                    }
-                for (int r = c + 1; r < nn; ++r) {
-                    const double fct = a[r * W + c] / a[c * W + c];
-                    for (int x = c; x < W; ++x) a[r * W + x] -= fct * a[c * W + x];
-                }
-            }
-            for (int r = nn - 1; r >= 0; --r) {
-                double sacc = a[r * W + MIX_MAXG];
-                for (int x = r + 1; x < nn; ++x) sacc -= a[r * W + x] * th[x];
-                th[r] = sacc / a[r * W + r];
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int h = 0; h < MIX_MAXG; ++h) theta[h] = (h < nn) ? th[h] : 0.0;
+        for (int h = 0; h < MIX_MAXG; ++h) theta[h] = (h < nn) ? wave_read(a, 8 * h + 7) : 0.0;
         __syncthreads();
     }
     // new slot for the mixed vector = oldest slot

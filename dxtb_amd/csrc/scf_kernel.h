@@ -259,16 +259,12 @@ __device__ __noinline__ bool warm_orthonormalise(const Mol& M, const Shared& sh)
 // orbitals with f > 0 form a prefix of length kocc; G[j] = C_{sidx[j]} (row
 // j, for j < kocc, or every j when `all_rows`) and H[j] = w_j G[j] (j < kocc)
 // with w = f (or f e when `with_e`).  H may alias Ct: it is written only
-// after every row of G has been gathered.  Returns kocc.
+// after every row of G has been gathered.
 // ---------------------------------------------------------------------------
-__device__ __noinline__ int gather_occupied(const Mol& M, const Shared& sh, glbf* G, glbf* H,
-                                            bool with_e, bool all_rows = false) {
+__device__ __noinline__ void gather_occupied(const Mol& M, const Shared& sh, glbf* G, glbf* H, int kocc, bool with_e,
+                                             bool all_rows = false) {
     const int n = M.n;
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    int k = 0;
-    for (int j = threadIdx.x; j < n; j += NT)
-        if (sh.ftot[sh.sidx[j]] > 0.0) k = j + 1;
-    const int kocc = (int)wg_max((double)k, sh.red);
     for (int j = w; j < (all_rows ? n : kocc); j += NWAVE) {
         const glbf* src = M.Ct + (size_t)sh.sidx[j] * n;
         for (int c = lane; c < n; c += WAVE) G[(size_t)j * n + c] = src[c];
@@ -280,7 +276,6 @@ __device__ __noinline__ int gather_occupied(const Mol& M, const Shared& sh, glbf
         for (int c = lane; c < n; c += WAVE) H[(size_t)j * n + c] = f * G[(size_t)j * n + c];
     }
     __syncthreads();
-    return kocc;
 }
 
 // ---------------------------------------------------------------------------
@@ -347,17 +342,22 @@ __device__ inline void fock_build(const Mol& M, const glbf* vin) {
 // Scratch: T holds C F, then X and Z; P the couplings/amplitudes; F the two
 // Horner accumulators (k x n each, k <= n/2).
 // ---------------------------------------------------------------------------
-// Coefficient of term j of the series in X = K K^T used by the rotation:
-// which 0: cos, (-1)^j / (2j)!; 1: sinc, (-1)^j / (2j+1)!; 2: phi,
-// -(-1)^j / (2j+2)!  ((2j)! by the running product (2t-1)(2t), t <= j)
-__device__ inline double horner_coef(int j, int which) {
-    double f = 1.0;
-    for (int t = 1; t <= j; ++t) f *= (2.0 * t - 1.0) * (2.0 * t);
-    const double sg = (j & 1) ? -1.0 : 1.0;
-    if (which == 0) return sg / f;
-    if (which == 1) return sg / (f * (2.0 * j + 1.0));
-    return -sg / (f * (2.0 * j + 1.0) * (2.0 * j + 2.0));
-}
+// Coefficients of the series in X = K K^T used by the rotation: term j of
+// cos (0): (-1)^j / (2j)!, sinc (1): (-1)^j / (2j+1)!, phi (2): -(-1)^j / (2j+2)!
+struct HornerCoef {
+    double v[3][9];
+    constexpr HornerCoef() : v() {
+        double f = 1.0;  // (2j)!
+        for (int j = 0; j <= 8; ++j) {
+            if (j > 0) f *= (2.0 * j - 1.0) * (2.0 * j);
+            const double sg = (j & 1) ? -1.0 : 1.0;
+            v[0][j] = sg / f;
+            v[1][j] = sg / (f * (2.0 * j + 1.0));
+            v[2][j] = -sg / (f * (2.0 * j + 1.0) * (2.0 * j + 2.0));
+        }
+    }
+};
+__constant__ const HornerCoef horner_coef;
 
 __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_scf_opts& o, int k,
                                     double loose, const glbf* vin) {
@@ -418,8 +418,6 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
         __syncthreads();
         double dmax = 0.0;
         for (int i = threadIdx.x; i < n; i += NT) dmax = fmax(dmax, fabs(sh.ev[i]));
-        dmax = wg_max(dmax, sh.red);
-        const double tol = fmax(o.jacobi_tol * fmax(dmax, 1.0), loose > 0.0 ? loose : PD_FINAL_REL * o.x_atol_max);
         double aov = 0.0, kmax = 0.0, dmin = INFINITY;
         for (int i0 = w * ROWS_PER_WAVE; i0 < k; i0 += NWAVE * ROWS_PER_WAVE) {
             int ii[ROWS_PER_WAVE];
@@ -446,9 +444,12 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
                 }
             }
         }
-        aov = wg_max(aov, sh.red);
-        kmax = wg_max(kmax, sh.red);
-        dmin = -wg_max(-dmin, sh.red);
+        double mx[4] = {dmax, aov, kmax, -dmin};
+        wg_max_n<4>(mx, sh.red);
+        aov = mx[1];
+        kmax = mx[2];
+        dmin = -mx[3];
+        const double tol = fmax(o.jacobi_tol * fmax(mx[0], 1.0), loose > 0.0 ? loose : PD_FINAL_REL * o.x_atol_max);
         if (aov <= tol) return 1;  // decoupled: orbitals stay
         const int fail = pass == 0 ? 0 : -1;
         PD_MARK(sh, 2, tm);
@@ -478,21 +479,17 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
             term *= xf / ((2.0 * J + 1.0) * (2.0 * J + 2.0));
             if (J > 8) return fail;  // F and Ct untouched in this pass
         }
-        // series coefficients of term j (computed where used: arrays indexed
-        // by the run-time j would live in scratch memory)
-        auto cc = [](int j) { return horner_coef(j, 0); };
-        auto ss = [](int j) { return horner_coef(j, 1); };
-        auto ph = [](int j) { return horner_coef(j, 2); };
+        const double(&cc)[9] = horner_coef.v[0], (&ss)[9] = horner_coef.v[1], (&ph)[9] = horner_coef.v[2];
         // Horner steps acc <- X acc + a_j C_occ + b_j Z, the update fused into
         // the GEMM epilogue; the two k x n halves of F alternate
         glbf* cur = M.F;
         glbf* nxt = M.F + (size_t)k * n;
         // R = sinc(X) C_occ + phi(X) Z
-        wg_axpby((size_t)k * n, ss(J), Ct, ph(J), Z, cur);
+        wg_axpby((size_t)k * n, ss[J], Ct, ph[J], Z, cur);
         __syncthreads();
         for (int j = J - 1; j >= 0; --j) {
             PD_MARK(sh, 6, tm);
-            gemm_epi(k, n, k, X, k, cur, n, nxt, n, Ct, ss(j), Z, ph(j), sh.big);
+            gemm_epi(k, n, k, X, k, cur, n, nxt, n, Ct, ss[j], Z, ph[j], sh.big);
             PD_MARK(sh, 5, tm);
             glbf* t = cur;
             cur = nxt;
@@ -506,11 +503,11 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
         // over C_occ itself: each element of C_occ is read (as E1) and
         // written by the same thread, and no product takes C_occ as an
         // operand, so no copy pass follows
-        wg_axpby((size_t)k * n, cc(J), Ct, -ss(J), Z, J == 0 ? Ct : cur);
+        wg_axpby((size_t)k * n, cc[J], Ct, -ss[J], Z, J == 0 ? Ct : cur);
         __syncthreads();
         for (int j = J - 1; j >= 0; --j) {
             PD_MARK(sh, 6, tm);
-            gemm_epi(k, n, k, X, k, cur, n, j == 0 ? Ct : nxt, n, Ct, cc(j), Z, -ss(j), sh.big);
+            gemm_epi(k, n, k, X, k, cur, n, j == 0 ? Ct : nxt, n, Ct, cc[j], Z, -ss[j], sh.big);
             PD_MARK(sh, 5, tm);
             glbf* t = cur;
             cur = nxt;
@@ -613,50 +610,28 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
     // an intermediate step's eigensolve that ran out of sweeps only slows
     // the SCF down; the final step's results would be unreliable
     if (sw < 0 && final_step) *status |= XTB_MOL_JACOBI;
-    // sort eigenvalues
-    for (int j = threadIdx.x; j < sh.npow; j += NT) {
-        sh.skey[j] = (j < n) ? sh.ev[j] : INFINITY;
-        sh.sidx[j] = j;
-    }
-    for (int j = threadIdx.x; j < n; j += NT) sh.ftot[j] = 0.0;
-    __syncthreads();
-    wg_bitonic_sort(sh.skey, sh.sidx, sh.npow);
-    // Fermi occupations, alpha then beta
-    bool ok = fermi_channel(M, sh, M.nel_a, o.kt, o.fermi_thresh, o.fermi_maxiter, o.padded != 0,
-                            M.occ, &ef[0]);
-    ok = fermi_channel(M, sh, M.nel_b, o.kt, o.fermi_thresh, o.fermi_maxiter, o.padded != 0,
-                       M.occ + M.nvec_total, &ef[1]) && ok;
-    if (!ok) *status |= XTB_MOL_FERMI;
-    {
-        // ef[2]: the largest f (1 - f) of either channel.  Above ~1e-6 some
-        // levels lie within ~14 kT of the Fermi level, where the density
-        // depends on rotations among near-degenerate orbitals of different
-        // occupation: the caller then tightens inexact eigensolves by 2 kT,
-        // the bound on |f_i - f_j| / |e_i - e_j| over both channels
-        double fs = 0.0;
-        for (int c = 0; c < 2; ++c)
-            for (int j = threadIdx.x; j < n; j += NT) {
-                const double f = M.occ[c * M.nvec_total + j];
-                fs = fmax(fs, f * (1.0 - f));
-            }
-        ef[2] = wg_max(fs, sh.red);
-    }
+    wg_sort(sh.ev, sh.skey, sh.sidx, n, sh.npow);
+    // Fermi occupations.  ef[2]: the largest f (1 - f).  Above ~1e-6 some
+    // levels lie within ~14 kT of the Fermi level, where the density depends
+    // on rotations among near-degenerate orbitals of different occupation:
+    // the caller then tightens inexact eigensolves by 2 kT, the bound on
+    // |f_i - f_j| / |e_i - e_j| over both channels
+    const Filling fl = fill_orbitals(M, sh, o.kt, o.fermi_thresh, o.fermi_maxiter, o.padded != 0, M.occ,
+                                     M.occ + M.nvec_total);
+    if (!fl.ok) *status |= XTB_MOL_FERMI;
+    ef[0] = fl.ef[0];
+    ef[1] = fl.ef[1];
+    ef[2] = fl.soft;
     // P = C diag(f) C^T over the occupied orbitals (F and T are free here).
     // When the rows of Ct are already in ascending order (the usual case once
     // the SCF settles) they are used in place: no gather into F and no copy
     // back, 4 n^2 doubles of traffic less per step
     t0 = now_us();
-    bool moved = false;
-    for (int j = threadIdx.x; j < n; j += NT) moved |= sh.sidx[j] != j;
-    const bool perm = __syncthreads_or(moved) != 0;
-    int kocc;
+    const bool perm = fl.moved;
+    const int kocc = fl.kocc;
     if (perm) {
-        kocc = gather_occupied(M, sh, M.F, M.T, false, sort_rows);
+        gather_occupied(M, sh, M.F, M.T, kocc, false, sort_rows);
     } else {
-        int k = 0;
-        for (int j = threadIdx.x; j < n; j += NT)
-            if (sh.ftot[j] > 0.0) k = j + 1;
-        kocc = (int)wg_max((double)k, sh.red);
         for (int j0 = w * ROWS_PER_WAVE; j0 < kocc; j0 += NWAVE * ROWS_PER_WAVE) {
             int jj[ROWS_PER_WAVE];
             double f[ROWS_PER_WAVE];

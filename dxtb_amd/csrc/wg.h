@@ -28,66 +28,91 @@ __device__ inline ldsi* to_lds(int* p) { return (ldsi*)p; }
 __device__ inline glbf* to_glb(double* p) { return (glbf*)p; }
 __device__ inline const glbf* to_glb(const double* p) { return (const glbf*)p; }
 
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-    return v;
+// DPP move of a double; lanes without a source keep `old`
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp64(double old, double v) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, ROWS, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+// lane `lane` (uniform) of v, on every lane
+__device__ __forceinline__ double wave_read(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
 }
 
-__device__ inline double wave_max(double v) {
-#pragma unroll
-    for (int o = WAVE / 2; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, WAVE));
-    return v;
+// Reductions over a wave: up the rows of 16 lanes by row shifts 1, 2, 4, 8,
+// then across the rows by row broadcasts; the result, in lane 63, goes to
+// every lane as a uniform value.  Register moves only, ~150 cycles; a
+// butterfly through LDS permutes took ~600.
+__device__ __forceinline__ double wave_sum(double v) {
+    v += dpp64<0x111, 0xf>(0.0, v);
+    v += dpp64<0x112, 0xf>(0.0, v);
+    v += dpp64<0x114, 0xf>(0.0, v);
+    v += dpp64<0x118, 0xf>(0.0, v);
+    v += dpp64<0x142, 0xa>(0.0, v);
+    v += dpp64<0x143, 0xc>(0.0, v);
+    return wave_read(v, WAVE - 1);
 }
 
-// Sum over the workgroup; `red` holds >= NWAVE doubles of LDS.  Result is
-// returned to every thread.
-__device__ inline double wg_sum(double v, ldsf* red) {
-    v = wave_sum(v);
-    const int w = threadIdx.x / WAVE, l = threadIdx.x % WAVE;
-    __syncthreads();
-    if (l == 0) red[w] = v;
-    __syncthreads();
-    double s = 0.0;
-#pragma unroll
-    for (int i = 0; i < NWAVE; ++i) s += red[i];
-    __syncthreads();
-    return s;
+__device__ __forceinline__ double wave_max(double v) {
+    v = fmax(v, dpp64<0x111, 0xf>(v, v));
+    v = fmax(v, dpp64<0x112, 0xf>(v, v));
+    v = fmax(v, dpp64<0x114, 0xf>(v, v));
+    v = fmax(v, dpp64<0x118, 0xf>(v, v));
+    v = fmax(v, dpp64<0x142, 0xa>(v, v));
+    v = fmax(v, dpp64<0x143, 0xc>(v, v));
+    return wave_read(v, WAVE - 1);
 }
 
-__device__ inline double wg_max(double v, ldsf* red) {
-    v = wave_max(v);
-    const int w = threadIdx.x / WAVE, l = threadIdx.x % WAVE;
-    __syncthreads();
-    if (l == 0) red[w] = v;
-    __syncthreads();
-    double s = red[0];
-#pragma unroll
-    for (int i = 1; i < NWAVE; ++i) s = fmax(s, red[i]);
-    __syncthreads();
-    return s;
-}
-
-// Several sums at once: vals[K] per thread -> out[K] on every thread.
-// `red` must hold K*NWAVE doubles.
+// K sums / maxima over the workgroup at once: v[K] per thread -> v[K] on
+// every thread.  `red`: K NWAVE doubles of LDS that no thread still reads
+// (they end with a barrier, so calls may follow one another).
 template <int K>
-__device__ inline void wg_sum_n(double (&vals)[K], ldsf* red) {
+__device__ inline void wg_sum_n(double (&v)[K], ldsf* red) {
     const int w = threadIdx.x / WAVE, l = threadIdx.x % WAVE;
 #pragma unroll
-    for (int k = 0; k < K; ++k) vals[k] = wave_sum(vals[k]);
-    __syncthreads();
-    if (l == 0) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) red[k * NWAVE + w] = vals[k];
+    for (int k = 0; k < K; ++k) {
+        v[k] = wave_sum(v[k]);
+        if (l == 0) red[k * NWAVE + w] = v[k];
     }
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         double s = 0.0;
+#pragma unroll
         for (int i = 0; i < NWAVE; ++i) s += red[k * NWAVE + i];
-        vals[k] = s;
+        v[k] = s;
     }
     __syncthreads();
+}
+template <int K>
+__device__ inline void wg_max_n(double (&v)[K], ldsf* red) {
+    const int w = threadIdx.x / WAVE, l = threadIdx.x % WAVE;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        v[k] = wave_max(v[k]);
+        if (l == 0) red[k * NWAVE + w] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        double s = red[k * NWAVE];
+#pragma unroll
+        for (int i = 1; i < NWAVE; ++i) s = fmax(s, red[k * NWAVE + i]);
+        v[k] = s;
+    }
+    __syncthreads();
+}
+__device__ inline double wg_sum(double v, ldsf* red) {
+    double x[1] = {v};
+    wg_sum_n<1>(x, red);
+    return x[0];
+}
+__device__ inline double wg_max(double v, ldsf* red) {
+    double x[1] = {v};
+    wg_max_n<1>(x, red);
+    return x[0];
 }
 
 // Y[e] = a X[e] + b Z[e] (Z null: a X[e]) over `len` contiguous elements, by
@@ -700,20 +725,8 @@ __host__ __device__ inline int ring_pitch(int n, int cap) {
 }
 
 // lane l <- lane l - 1 (lane 0 <- first) and lane l <- lane l + 1 (lane 63 <- last)
-__device__ inline double wave_up(double v, double first) {
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(v), 0x138, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(v), 0x138, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-__device__ inline double wave_down(double v, double last) {
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(last), __double2loint(v), 0x130, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(last), __double2hiint(v), 0x130, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-__device__ inline double wave_read(double v, int lane) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                            __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
+__device__ __forceinline__ double wave_up(double v, double first) { return dpp64<0x138, 0xf>(first, v); }
+__device__ __forceinline__ double wave_down(double v, double last) { return dpp64<0x130, 0xf>(last, v); }
 
 // One recorded sweep applied to C columns of the row-major vectors Ct (row k
 // = vector k) by one wave: lane l (and l + 64 with two sets) holds the two
@@ -1044,16 +1057,8 @@ __device__ inline int slot_index(int I, int J, int i, int n) {
 }
 
 // lane l of each row of 16 <- lane l - 1 (lane 0 <- first), and <- l + 1 (lane 15 <- last)
-__device__ inline double row_up(double v, double first) {
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(v), 0x111, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(v), 0x111, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-__device__ inline double row_down(double v, double last) {
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(last), __double2loint(v), 0x101, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(last), __double2hiint(v), 0x101, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
+__device__ __forceinline__ double row_up(double v, double first) { return dpp64<0x111, 0xf>(first, v); }
+__device__ __forceinline__ double row_down(double v, double last) { return dpp64<0x101, 0xf>(last, v); }
 
 // Cyclic Jacobi on a 32 x 32 subproblem by one wavefront, in place on its ring
 // storage D (pitch JW; zero rows and columns are never rotated).  The
@@ -1458,12 +1463,46 @@ struct RowsGlobal {
     __device__ inline glbf& at(int k, int mu) const { return a[(size_t)k * ld + mu]; }
 };
 
-// Ascending bitonic sort of (key, idx) pairs in LDS; len is a power of two
-// and entries beyond the valid range must hold +inf keys.
-__device__ inline void wg_bitonic_sort(ldsf* key, ldsi* idx, int len) {
-    for (int size = 2; size <= len; size <<= 1) {
+// Ascending sort of the n keys src[0..n): key[r] = src[idx[r]], in LDS of
+// npow entries each (npow: the next power of two).  src may be key itself.
+//
+// Up to a key per thread each thread counts the keys below its own (equal
+// ones in index order, NaN as +inf): n LDS broadcasts and two barriers, ~1 us
+// at n = 128 and 3 us at 300, where the bitonic network below, a barrier per
+// stage (28 and 45), takes 3 and 5 us.  It stays for the larger n.
+template <class Src>
+__device__ inline void wg_sort(Src src, ldsf* key, ldsi* idx, int n, int npow) {
+    if (n <= NT) {
+        const int j = threadIdx.x, b0 = j - j % WAVE, b1 = b0 + WAVE < n ? b0 + WAVE : n;
+        const double v = j < n ? src[j] : 0.0, e = v == v ? v : INFINITY;
+        __syncthreads();
+        if (j < n) key[j] = e;
+        __syncthreads();
+        int rank = 0;
+        if (b0 < n) {
+#pragma unroll 8
+            for (int i = 0; i < b0; ++i) rank += key[i] <= e;
+#pragma unroll 8
+            for (int i = b0; i < b1; ++i) rank += i < j ? key[i] <= e : key[i] < e;
+#pragma unroll 8
+            for (int i = b1; i < n; ++i) rank += key[i] < e;
+        }
+        __syncthreads();
+        if (j < n) {
+            key[rank] = v;
+            idx[rank] = j;
+        }
+        __syncthreads();
+        return;
+    }
+    for (int j = threadIdx.x; j < npow; j += NT) {
+        key[j] = j < n ? src[j] : INFINITY;
+        idx[j] = j;
+    }
+    __syncthreads();
+    for (int size = 2; size <= npow; size <<= 1) {
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int t = threadIdx.x; t < len / 2; t += NT) {
+            for (int t = threadIdx.x; t < npow / 2; t += NT) {
                 const int lo = 2 * t - (t & (stride - 1));
                 const int hi = lo + stride;
                 const bool up = ((lo & size) == 0);

@@ -14,8 +14,8 @@ from helpers import TIGHT, TIGHT_ORACLE, run_native
 pytestmark = pytest.mark.gpu
 
 
-# water: 6 orbitals a molecule; 198 (13 blocks, 6 in the last), 204 (13), 222
-# (14), 240 (15, full)
+# orbitals: 264 (17 blocks, the last half full), 272 (17), 296 (19, half full)
+# and 320 (20)
 @pytest.mark.parametrize("size", [33, 34, 37, 40])
 def test_orbital_energies_from_full_eigensolves(size):
     """Full eigensolves only; the SCF's 1e-11 threshold leaves energies
