@@ -4,7 +4,8 @@
 // the right shape for streams of molecules and the wrong one for a single
 // system of n ~ 5000 orbitals.  Here every stage of the same SCF is a grid
 // kernel that spreads over all CUs, and the SCF driver runs on the host,
-// stream ordered, reading a few control scalars back once or twice per step:
+// stream ordered; a few control scalars come back once or twice per step
+// through host memory that the kernels write (read_ctl):
 //
 //   setup   Loewdin orthogonaliser X = S^-1/2 by the coupled Newton-Schulz
 //           iteration on matrix-core GEMMs; the orbitals start as the rows
@@ -38,6 +39,27 @@ enum {
     C_AOV, C_KMAX, C_DMIN, C_XF, C_OFF, C_ERR, C_GERSH, C_CONV, C_RESID, C_FSOFT, C_BRANK, C_BDX,
     C_NCTL = 24
 };
+
+// The control values' copy in host memory that the device writes (pinned,
+// coherent): kernels that end a stretch of work post them, `seq` last.
+struct Box {
+    double v[C_NCTL];
+    unsigned long long seq;
+};
+struct Post {
+    Box* box;  // null: nothing to post
+    unsigned long long seq;
+};
+
+// by (at least) the first wave, which has written its values to ctl
+__device__ inline void post(const double* ctl, const Post& p) {
+    if (!p.box || threadIdx.x >= WAVE) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    if (threadIdx.x < C_NCTL)
+        __hip_atomic_store(&p.box->v[threadIdx.x], ctl[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+    if (threadIdx.x == 0) __hip_atomic_store(&p.box->seq, p.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // ---------------------------------------------------------------------------
 // Grid GEMM, C = alpha op(A) op(B) + beta C: wave tiles of 16 FM x 16 FN whose
@@ -117,16 +139,24 @@ struct WaveSide {
     }
 };
 
+// EPI: C = alpha op(A) op(B) + s1 E1 + s2 E2, columns from `half` on
+// + s3 E1 + s4 E2 of column - half (E1, E2: leading dimension lde).
+struct Epi {
+    const double *E1, *E2;
+    int lde, half;
+    double s1, s2, s3, s4;
+};
+
 template <bool TA, bool TB, bool EPI, bool SPLIT, int FM, int FN, int KS, int NB>
 __global__ void __launch_bounds__(256, 2) k_gemm(int M, int N, int K, double alpha, const double* A, int lda,
                                                  const double* B, int ldb, double beta, double* C, int ldc,
-                                                 int sym, int ntiles, const double* E1, const double* E2,
-                                                 double s1, double s2) {
+                                                 int sym, int ntiles, const double* Kd, Epi ep) {
     constexpr int KC = 4 * KS, TM = (SPLIT ? 16 : 32) * FM, TN = (SPLIT ? 16 : 32) * FN;
     __shared__ double part[SPLIT ? 3 * FM * FN * 256 : 1];
     const int per = gridDim.x / 8;  // the grid is a multiple of 8
     const int idx = (blockIdx.x % 8) * per + blockIdx.x / 8;
     if (idx >= ntiles) return;
+    if (Kd) K = uniform((int)*Kd);  // k from device memory
     const int tm = (M + TM - 1) / TM, tn = (N + TN - 1) / TN;
     int ti, tj;
     if (sym) {
@@ -220,8 +250,11 @@ __global__ void __launch_bounds__(256, 2) k_gemm(int M, int N, int K, double alp
         const int gm = m0 + 16 * i + lg + 4 * r, gn = n0 + 16 * j + li;
         if (gm >= M || gn >= N) return;
         const size_t e = (size_t)gm * ldc + gn;
-        if (EPI) C[e] = fma(alpha, v, fma(s1, E1[e], s2 * E2[e]));
-        else if (sym) {
+        if (EPI) {
+            const bool hi = gn >= ep.half;
+            const size_t x = (size_t)gm * ep.lde + (hi ? gn - ep.half : gn);
+            C[e] = fma(alpha, v, fma(hi ? ep.s3 : ep.s1, ep.E1[x], (hi ? ep.s4 : ep.s2) * ep.E2[x]));
+        } else if (sym) {
             C[e] = alpha * v;
             if (ti != tj) C[(size_t)gn * ldc + gm] = alpha * v;
         } else C[e] = beta == 0.0 ? alpha * v : fma(alpha, v, beta * C[e]);
@@ -270,10 +303,16 @@ __global__ void __launch_bounds__(256) k_fock(int n, const double* H0, const dou
     }
 }
 
-// out[i] = sum_c X[i][c] Y[i][c], i < rows
-__global__ void __launch_bounds__(NT) k_rowdot(int rows, int n, const double* X, const double* Y, double* out) {
+// out[i] = sum_c X[i][c] Y[i][c], i < rows; out[i] = tail[i] for the rest up
+// to n
+__global__ void __launch_bounds__(NT) k_rowdot(int rows, int n, const double* X, const double* Y, const double* tail,
+                                               double* out) {
     const int i = blockIdx.x * NWAVE + threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    if (i >= rows) return;
+    if (i >= n) return;
+    if (i >= rows) {
+        if (lane == 0) out[i] = tail[i];
+        return;
+    }
     double d = 0.0;
     for (int c = lane; c < n; c += WAVE) d = fma(X[(size_t)i * n + c], Y[(size_t)i * n + c], d);
     d = wave_sum(d);
@@ -318,31 +357,38 @@ __global__ void __launch_bounds__(NT) k_rowabs(int n, const double* A, double* p
     }
 }
 
-// Reduction of per-workgroup partials: slot s of ctl[s] = op_s over
-// part[b * nslot + s], b < nblk, in a fixed order (deterministic).  op:
-// bits 2s..2s+1 of `ops`: 0 sum, 1 max, 2 min.
-__global__ void __launch_bounds__(NT) k_finish(const double* part, int nblk, int nslot, int ops, double* ctl,
-                                               int ctl0) {
+// Reduction of per-workgroup partials: ctl[slot] = sum (op 0) or max (op 1) of
+// part[b], b < nblk, in a fixed order (deterministic).
+__global__ void __launch_bounds__(NT) k_finish(const double* part, int nblk, int op, double* ctl, int slot, Post p) {
     __shared__ double red[NWAVE];
-    const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    for (int s = 0; s < nslot; ++s) {
-        const int op = (ops >> (2 * s)) & 3;
-        auto comb = [op](double x, double y) { return op == 0 ? x + y : (op == 1 ? fmax(x, y) : fmin(x, y)); };
-        double a = op == 0 ? 0.0 : (op == 1 ? -INFINITY : INFINITY);
-        for (int b = threadIdx.x; b < nblk; b += NT) a = comb(a, part[(size_t)b * nslot + s]);
-        // xor butterfly (each pair combined in the same order in both
-        // lanes: every lane ends with the same bits), then the waves in
-        // index order
-        for (int o = 1; o < WAVE; o <<= 1) a = comb(a, __shfl_xor(a, o, WAVE));
-        if (lane == 0) red[w] = a;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            double r = red[0];
-            for (int k = 1; k < NWAVE; ++k) r = comb(r, red[k]);
-            ctl[ctl0 + s] = r;
-        }
-        __syncthreads();
+    double a = op == 0 ? 0.0 : -INFINITY;
+    for (int b = threadIdx.x; b < nblk; b += NT) a = op == 0 ? a + part[b] : fmax(a, part[b]);
+    a = op == 0 ? wg_sum(a, to_lds(red)) : wg_max(a, to_lds(red));
+    if (threadIdx.x == 0) ctl[slot] = a;
+    post(ctl, p);
+}
+
+// What a perturbative step's host decisions need (one workgroup): max |ev|
+// over n, and over the partials of k_amplitudes max |A_ia|, max |K_ia|, min
+// (e_a - e_i)
+__global__ void __launch_bounds__(NT) k_pd_stats(int n, const double* ev, const double* part, int nblk, double* ctl,
+                                                 Post p) {
+    __shared__ double red[4 * NWAVE];
+    double m[4] = {0.0, 0.0, 0.0, -INFINITY};
+    for (int i = threadIdx.x; i < n; i += NT) m[0] = fmax(m[0], fabs(ev[i]));
+    for (int b = threadIdx.x; b < nblk; b += NT) {
+        m[1] = fmax(m[1], part[3 * b]);
+        m[2] = fmax(m[2], part[3 * b + 1]);
+        m[3] = fmax(m[3], -part[3 * b + 2]);
     }
+    wg_max_n<4>(m, to_lds(red));
+    if (threadIdx.x == 0) {
+        ctl[C_DMAX] = m[0];
+        ctl[C_AOV] = m[1];
+        ctl[C_KMAX] = m[2];
+        ctl[C_DMIN] = -m[3];
+    }
+    post(ctl, p);
 }
 
 // Perturbative amplitudes K_ia <- A_ia / (e_a - e_i) (k x m, row-major);
@@ -399,6 +445,18 @@ __global__ void __launch_bounds__(NT) k_sumsq(size_t len, const double* x, doubl
         double r = 0.0;
         for (int k = 0; k < NWAVE; ++k) r += red[k];
         part[blockIdx.x] = r;
+    }
+}
+
+// First terms of the two series of a perturbative rotation (k x n):
+// R = s1 C + s2 Z and D = s3 C + s4 Z (D may be C itself)
+__global__ void __launch_bounds__(256) k_series0(int n, const double* C, const double* Z, double s1, double s2,
+                                                 double* R, int ldr, double s3, double s4, double* D, int ldd) {
+    const size_t r = blockIdx.y;
+    for (int c = blockIdx.x * 256 + threadIdx.x; c < n; c += gridDim.x * 256) {
+        const double x = C[r * n + c], z = Z[r * n + c];
+        R[r * ldr + c] = s1 * x + s2 * z;
+        D[r * ldd + c] = s3 * x + s4 * z;
     }
 }
 
@@ -464,6 +522,8 @@ __global__ void __launch_bounds__(256) k_copy_block(int rows, int cols, const do
     for (int c = blockIdx.x * 256 + threadIdx.x; c < cols; c += gridDim.x * 256)
         Y[(size_t)r * ldy + c] = X[(size_t)r * ldx + c];
 }
+
+__global__ void k_post(const double* ctl, Post p) { post(ctl, p); }
 
 __global__ void k_set_slot(double* ctl, int slot, double v) {
     if (threadIdx.x == 0) ctl[slot] = v;
@@ -549,7 +609,7 @@ struct SharedG {
 __global__ void __launch_bounds__(NT) k_sort_fermi(int n, int nao, int npow, const double* ev, double* skey_out,
                                                    int* sidx_out, double* ftot, double* occ, double nel_a,
                                                    double nel_b, int ia, int ib, double kt, double thr,
-                                                   int maxiter, double* ctl) {
+                                                   int maxiter, double* ctl, Post p) {
     extern __shared__ double lds[];
     ldsf* ls = to_lds(lds);
     SharedG sh;
@@ -578,23 +638,37 @@ __global__ void __launch_bounds__(NT) k_sort_fermi(int n, int nao, int npow, con
         ctl[C_GAPB] = (ib > 0 && ib < n) ? sh.skey[ib] - sh.skey[ib - 1] : INFINITY;
         ctl[C_FSOFT] = fl.soft;
     }
+    post(ctl, p);
 }
 
-// G[j] = Ct[sidx[j]] (j < rows); one workgroup per row
-__global__ void __launch_bounds__(256) k_gather(int n, const double* Ct, const int* sidx, double* G) {
+// G[j] = Ct[sidx[j]]; one workgroup per row.  With ctl: only if the sort moved
+// a row (when = C_PERM), or only the occupied rows j < ctl[C_KOCC] (when =
+// C_KOCC)
+__global__ void __launch_bounds__(256) k_gather(int n, const double* Ct, const int* sidx, const double* ctl, int when,
+                                                double* G) {
     const int j = blockIdx.x;
+    if (ctl && (when == C_PERM ? ctl[C_PERM] == 0.0 : (double)j >= ctl[C_KOCC])) return;
     const double* src = Ct + (size_t)sidx[j] * n;
     for (int c = threadIdx.x; c < n; c += 256) G[(size_t)j * n + c] = src[c];
 }
 
-// H[j] = w_j G[j], w_j = ftot[sidx[j]] (x ev[sidx[j]] when ev is given;
-// sidx null: the identity); one workgroup per row j < k
-__global__ void __launch_bounds__(256) k_scale_rows(int n, const double* G, const int* sidx, const double* ftot,
-                                                    const double* ev, double* H) {
+// H[j] = w_j X[j] for the occupied rows j < ctl[C_KOCC], w_j = ftot[sidx[j]]
+// (x ev[sidx[j]] when ev is given), one workgroup per row.  With Ct: X are
+// the rows gathered for a sort that moved any, which become Ct's rows; Ct
+// itself is X if it moved none.
+__global__ void __launch_bounds__(256) k_scale_rows(int n, const double* X, const int* sidx, const double* ftot,
+                                                    const double* ev, const double* ctl, double* Ct, double* H) {
     const int j = blockIdx.x;
-    const int o = sidx ? sidx[j] : j;
+    const bool perm = ctl[C_PERM] != 0.0, occ = (double)j < ctl[C_KOCC], back = Ct && perm;
+    if (!occ && !back) return;
+    const int o = sidx[j];
     const double w = ev ? ftot[o] * ev[o] : ftot[o];
-    for (int c = threadIdx.x; c < n; c += 256) H[(size_t)j * n + c] = w * G[(size_t)j * n + c];
+    const double* src = Ct && !perm ? Ct : X;
+    for (int c = threadIdx.x; c < n; c += 256) {
+        const double x = src[(size_t)j * n + c];
+        if (back) Ct[(size_t)j * n + c] = x;
+        if (occ) H[(size_t)j * n + c] = w * x;
+    }
 }
 
 // A'_ij = (f_i + f_j)/2 A_ij for the k x k occupied block, f of row i =
@@ -629,49 +703,40 @@ __global__ void __launch_bounds__(NT) k_mulliken(int n, int nao, const double* P
     }
 }
 
-// shell and atom charges (one workgroup)
-__global__ void __launch_bounds__(NT) k_shell_atom(int nsh, int nat, const int* sh_ao, const int* sh_us,
-                                                   const int* us_l, const int* atom_sh0, const int* atom_nsh,
-                                                   const double* q, double* qsh, double* qat) {
+// Shell and atom charges, ES2 (gamma q_sh) + ES3 (hd q_at^2) shell potential,
+// spread to the orbitals; one wave per shell.  Every workgroup sums all shell
+// charges for itself (LDS, nsh doubles): three launches in one.
+__global__ void __launch_bounds__(NT) k_potential(int nsh, const int* sh_ao, const int* sh_us, const int* us_l,
+                                                  const int* atom_sh0, const int* atom_nsh, const double* q,
+                                                  const double* gam, const int* sh_atom, const int* atom_sp,
+                                                  const double* sp_gam3, double* qsh_out, double* qat, double* gq,
+                                                  double* v) {
+    extern __shared__ double lds[];
+    ldsf* qsh = to_lds(lds);
     for (int s = threadIdx.x; s < nsh; s += NT) {
-        const int o0 = sh_ao[s];
-        const int nl = 2 * us_l[sh_us[s]] + 1;
+        const int o0 = sh_ao[s], nl = 2 * us_l[sh_us[s]] + 1;
         double acc = 0.0;
         for (int x = 0; x < nl; ++x) acc += q[o0 + x];
         qsh[s] = acc;
     }
     __syncthreads();
-    for (int a = threadIdx.x; a < nat; a += NT) {
-        const int s0 = atom_sh0[a], ns = atom_nsh[a];
-        double acc = 0.0;
-        for (int x = 0; x < ns; ++x) acc += qsh[s0 + x];
-        qat[a] = acc;
-    }
-}
-
-// ES2 (gamma q_sh) + ES3 (hd q_at^2) shell potential, one wave per shell
-__global__ void __launch_bounds__(NT) k_shell_pot(int nsh, const double* gam, const double* qsh, const double* qat,
-                                                  const int* sh_atom, const int* atom_sp, const double* sp_gam3,
-                                                  double* gq, double* vsh) {
     const int s = blockIdx.x * NWAVE + threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     if (s >= nsh) return;
     const double* gr = gam + (size_t)s * nsh;
     double acc = 0.0;
     for (int t = lane; t < nsh; t += WAVE) acc = fma(gr[t], qsh[t], acc);
     acc = wave_sum(acc);
+    const int a = sh_atom[s], s0 = atom_sh0[a], ns = atom_nsh[a];
+    double qa = 0.0;
+    for (int x = 0; x < ns; ++x) qa += qsh[s0 + x];
+    const double vs = acc + sp_gam3[atom_sp[a]] * qa * qa;
+    const int o0 = sh_ao[s], nl = 2 * us_l[sh_us[s]] + 1;
+    if (lane < nl) v[o0 + lane] = vs;
     if (lane == 0) {
-        const int a = sh_atom[s];
-        const double hd = sp_gam3[atom_sp[a]];
+        qsh_out[s] = qsh[s];
         gq[s] = acc;
-        vsh[s] = acc + hd * qat[a] * qat[a];
+        if (s == s0) qat[a] = qa;
     }
-}
-
-__global__ void __launch_bounds__(256) k_spread(int n, int nao, const int* ao_sh, const double* vsh, double* v) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const int s = (i < nao) ? ao_sh[i] : -1;
-    v[i] = (s >= 0) ? vsh[s] : 0.0;
 }
 
 // Mixing (one workgroup; the same mixers as the per-molecule kernel):
@@ -679,7 +744,8 @@ __global__ void __launch_bounds__(256) k_spread(int n, int nao, const int* ao_sh
 // ctl[C_RESID] = the residual's max norm; the Broyden memory's rank and last
 // step norm go to ctl[C_BRANK], ctl[C_BDX] for the host's copy of its state
 __global__ void __launch_bounds__(NT) k_mix(Mixer mx, Broyden bm, int n, xtb_scf_opts o, double* hx, double* hf,
-                                            const double* xnew, const double* xold, double* xout, double* ctl) {
+                                            const double* xnew, const double* xold, double* xout, double* ctl,
+                                            Post p) {
     __shared__ double red[256];
     struct { ldsf* red; } sh{to_lds(red)};
     Mol M;
@@ -696,6 +762,7 @@ __global__ void __launch_bounds__(NT) k_mix(Mixer mx, Broyden bm, int n, xtb_scf
         ctl[C_BRANK] = (double)bm.rank;
         ctl[C_BDX] = bm.dxnorm;
     }
+    post(ctl, p);
 }
 
 // energies (scf/base.py:514-623) into the result record (one workgroup)
@@ -759,12 +826,6 @@ __global__ void k_diag(int n, const double* A, double* ev) {
     if (i < n) ev[i] = A[(size_t)i * n + i];
 }
 
-// ev[a] = src[a] for rows <= a < n
-__global__ void k_copy_tail(int rows, int n, const double* src, double* ev) {
-    const int a = rows + blockIdx.x * 256 + threadIdx.x;
-    if (a < n) ev[a] = src[a];
-}
-
 // per-workgroup max |x_i|
 __global__ void __launch_bounds__(NT) k_vec_absmax(int n, const double* x, double* part) {
     __shared__ double red[NWAVE];
@@ -783,7 +844,7 @@ __global__ void __launch_bounds__(NT) k_vec_absmax(int n, const double* x, doubl
 inline size_t al32(size_t d) { return (d + 31) & ~(size_t)31; }
 
 struct Layout {
-    size_t E, Q, ev, skey, ftot, sidx, ident, part, ctl, qat, gq, vsh, total;
+    size_t E, Q, ev, skey, ftot, sidx, ident, part, ctl, qat, gq, total;
 };
 
 Layout make_layout(int n, int nsh, int nat) {
@@ -801,7 +862,6 @@ Layout make_layout(int n, int nsh, int nat) {
     L.ctl = o; o += al32(C_NCTL);
     L.qat = o; o += al32(nat);
     L.gq = o; o += al32(nsh);
-    L.vsh = o; o += al32(nsh);
     L.total = o;
     return L;
 }
@@ -809,6 +869,25 @@ Layout make_layout(int n, int nsh, int nat) {
 // largest orbital count: the sort keeps keys and indices of the next power
 // of two in one workgroup's LDS
 constexpr int LARGE_MAX_N = 8192;
+
+// The calling thread's Box (a call uses it from start to end, so one per
+// thread is enough), kept until the thread ends.
+struct Mail {
+    Box* box = nullptr;
+    unsigned long long seq = 0;  // of the last post asked for
+    hipError_t open() {
+        if (box) return hipSuccess;
+        const hipError_t e = hipHostMalloc((void**)&box, sizeof(Box),
+                                           hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);
+        if (e == hipSuccess) box->seq = 0;
+        else box = nullptr;
+        return e;
+    }
+    ~Mail() {
+        if (box) (void)hipHostFree(box);
+    }
+};
+thread_local Mail thread_mail;
 
 struct Ctx {
     hipStream_t s;
@@ -821,9 +900,10 @@ struct Ctx {
     int ia, ib;
     const double *S, *H0, *gam;
     double *F, *Ct, *T, *P, *E;  // n x n; the roles of F, Ct and E rotate
-    double *ev, *skey, *ftot, *Qbuf, *part, *ctl, *qat, *gq, *vsh;
+    double *ev, *skey, *ftot, *Qbuf, *part, *ctl, *qat, *gq;
     int *sidx, *ident;
-    double h[C_NCTL];
+    double h[C_NCTL];  // control values of the last read_ctl
+    Mail* mail;
     double gap_a = INFINITY, gap_b = INFINITY;  // frontier gaps of the last sort
     int refresh = 0;                            // perturbative steps since fresh eigenvalues
     hipError_t err = hipSuccess;
@@ -840,21 +920,43 @@ inline double now_s() {
     return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 
+constexpr Post NO_POST{nullptr, 0};
+
+// for the kernel launched last before read_ctl
+Post next_post(Ctx& c) { return Post{c.mail->box, ++c.mail->seq}; }
+
+// Waits for the last post and takes its values.  The wait watches host memory
+// for ~200 us, then leaves it to the stream.  (A copy and a stream
+// synchronisation instead left the GPU idle for ~40 us a time: of 8.5 ms at n
+// = 296, 3.1 were such gaps; with fewer reads and fewer, merged kernels the
+// same call takes 5.3.)
 bool read_ctl(Ctx& c) {
-    chk(c, hipMemcpyAsync(c.h, c.ctl, sizeof(c.h), hipMemcpyDeviceToHost, c.s));
-    chk(c, hipStreamSynchronize(c.s));
-    return c.err == hipSuccess;
+    if (c.err != hipSuccess) return false;
+    Box* box = c.mail->box;
+    auto there = [&]() { return __atomic_load_n(&box->seq, __ATOMIC_ACQUIRE) == c.mail->seq; };
+    const auto t0 = std::chrono::steady_clock::now();
+    while (!there()) {
+        for (int i = 0; i < 32 && !there(); ++i) __builtin_ia32_pause();
+        if (std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(200)) {
+            chk(c, hipStreamSynchronize(c.s));
+            if (c.err == hipSuccess && !there()) chk(c, hipErrorUnknown);
+            break;
+        }
+    }
+    if (c.err != hipSuccess) return false;
+    for (int i = 0; i < C_NCTL; ++i) c.h[i] = box->v[i];
+    return true;
 }
 
-void finish(Ctx& c, int nblk, int nslot, int ops, int slot) {
-    hipLaunchKernelGGL(k_finish, dim3(1), dim3(NT), 0, c.s, c.part, nblk, nslot, ops, c.ctl, slot);
+// ctl[slot] = sum / max of nblk partials; posted if it is to be read
+void finish(Ctx& c, int nblk, int op, int slot, Post p = NO_POST) {
+    hipLaunchKernelGGL(k_finish, dim3(1), dim3(NT), 0, c.s, c.part, nblk, op, c.ctl, slot, p);
     chk_launch(c);
 }
 
 template <bool TA, bool TB, bool EPI>
 void gemm_t(Ctx& c, int M, int N, int K, double alpha, const double* A, int lda, const double* B, int ldb,
-            double beta, double* C, int ldc, bool upper, const double* E1 = nullptr, const double* E2 = nullptr,
-            double s1 = 0.0, double s2 = 0.0) {
+            double beta, double* C, int ldc, bool upper, const Epi& ep = Epi{}, const double* Kd = nullptr) {
     if (M <= 0 || N <= 0) return;
     auto tiles = [&](int t) {
         const int tm = (M + t - 1) / t, tn = (N + t - 1) / t;
@@ -864,7 +966,7 @@ void gemm_t(Ctx& c, int M, int N, int K, double alpha, const double* A, int lda,
     {                                                                                                                \
         const int nt = tiles((SPLIT ? 16 : 32) * F), grid = (nt + 7) / 8 * 8;                                        \
         hipLaunchKernelGGL((k_gemm<TA, TB, EPI, SPLIT, F, F, KS, NB>), dim3(grid), dim3(256), 0, c.s, M, N, K,       \
-                           alpha, A, lda, B, ldb, beta, C, ldc, upper ? 1 : 0, nt, E1, E2, s1, s2);                  \
+                           alpha, A, lda, B, ldb, beta, C, ldc, upper ? 1 : 0, nt, Kd, ep);                          \
     }
     // the largest tile that still gives the CUs enough workgroups.  us at both
     // sides of the lines: 48-wide tiles (against 32) from ~220 of them, 750 x
@@ -880,14 +982,23 @@ void gemm_t(Ctx& c, int M, int N, int K, double alpha, const double* A, int lda,
     chk_launch(c);
 }
 
-// C (n x n, symmetric) = op(A) op(B)
+// C (n x n, symmetric) = op(A) op(B); with Kd, k is *Kd at run time
 template <bool TA, bool TB>
-void gemm_sym(Ctx& c, int n, int K, const double* A, int lda, const double* B, int ldb, double* C, int ldc) {
-    gemm_t<TA, TB, false>(c, n, n, K, 1.0, A, lda, B, ldb, 0.0, C, ldc, true);
+void gemm_sym(Ctx& c, int n, int K, const double* A, int lda, const double* B, int ldb, double* C, int ldc,
+              const double* Kd = nullptr) {
+    gemm_t<TA, TB, false>(c, n, n, K, 1.0, A, lda, B, ldb, 0.0, C, ldc, true, Epi{}, Kd);
 }
 
 void fock(Ctx& c, const double* v) {
     hipLaunchKernelGGL(k_fock, dim3((c.n + 255) / 256, c.n), dim3(256), 0, c.s, c.n, c.H0, c.S, v, c.F);
+    chk_launch(c);
+}
+
+void sort_fermi(Ctx& c, Post p) {
+    const size_t lds = (256 + (size_t)c.npow) * 8 + (size_t)c.npow * 4;
+    const xtb_scf_opts& o = c.o;
+    hipLaunchKernelGGL(k_sort_fermi, dim3(1), dim3(NT), lds, c.s, c.n, c.nao, c.npow, c.ev, c.skey, c.sidx, c.ftot,
+                       c.st->occ, c.nel_a, c.nel_b, c.ia, c.ib, o.kt, o.fermi_thresh, o.fermi_maxiter, c.ctl, p);
     chk_launch(c);
 }
 
@@ -906,7 +1017,7 @@ bool ortho(Ctx& c) {
     const int rb = (n + NWAVE - 1) / NWAVE;
     hipLaunchKernelGGL(k_rowabs, dim3(rb), dim3(NT), 0, c.s, n, c.S, c.part);
     chk_launch(c);
-    finish(c, rb, 1, 1, C_GERSH);
+    finish(c, rb, 1, C_GERSH, next_post(c));
     if (!read_ctl(c)) return false;
     const double cg = c.h[C_GERSH] * 1.0001;
     double* Y = c.F;
@@ -923,7 +1034,7 @@ bool ortho(Ctx& c) {
         chk_launch(c);
         hipLaunchKernelGGL(k_dev_identity, dim3(rb), dim3(NT), 0, c.s, n, T, c.part);
         chk_launch(c);
-        finish(c, rb, 1, 1, C_ERR);
+        finish(c, rb, 1, C_ERR, next_post(c));
         if (!read_ctl(c)) return false;
         const double err = c.h[C_ERR];
         if (extra == 0 || err < 1e-15) break;
@@ -976,7 +1087,7 @@ bool warm_orthonormalise(Ctx& c, const double* pot) {
         chk_launch(c);
         hipLaunchKernelGGL(k_dev_identity, dim3(rb), dim3(NT), 0, c.s, n, T, c.part);
         chk_launch(c);
-        finish(c, rb, 1, 1, C_ERR);
+        finish(c, rb, 1, C_ERR, next_post(c));
         if (!read_ctl(c)) return false;
         const double err = c.h[C_ERR];
         // |I - T| = |I - G|/2 at the start: beyond 1/4 the kept orbitals
@@ -1000,14 +1111,10 @@ bool warm_orthonormalise(Ctx& c, const double* pot) {
     // frontier gaps steer the first step's occupied-virtual decoupling
     fock(c, pot);
     gemm_t<false, false, false>(c, n, n, n, 1.0, c.Ct, n, c.F, n, 0.0, T, n, false);
-    hipLaunchKernelGGL(k_rowdot, dim3(rb), dim3(NT), 0, c.s, n, n, T, c.Ct, c.ev);
+    hipLaunchKernelGGL(k_rowdot, dim3(rb), dim3(NT), 0, c.s, n, n, T, c.Ct, (const double*)nullptr, c.ev);
     chk_launch(c);
-    const size_t lds = (256 + (size_t)c.npow) * 8 + (size_t)c.npow * 4;
-    const xtb_scf_opts& o = c.o;
-    hipLaunchKernelGGL(k_sort_fermi, dim3(1), dim3(NT), lds, c.s, n, c.nao, c.npow, c.ev, c.skey, c.sidx, c.ftot,
-                       c.st->occ, c.nel_a, c.nel_b, c.ia, c.ib, o.kt, o.fermi_thresh, o.fermi_maxiter, c.ctl);
-    chk_launch(c);
-    hipLaunchKernelGGL(k_gather, dim3(n), dim3(256), 0, c.s, n, c.Ct, c.sidx, c.F);
+    sort_fermi(c, next_post(c));
+    hipLaunchKernelGGL(k_gather, dim3(n), dim3(256), 0, c.s, n, c.Ct, c.sidx, (const double*)nullptr, 0, c.F);
     chk_launch(c);
     chk(c, hipMemcpyAsync(c.Ct, c.F, sizeof(double) * n * n, hipMemcpyDeviceToDevice, c.s));
     if (!read_ctl(c)) return false;
@@ -1048,6 +1155,8 @@ bool ortho_chol(Ctx& c) {
             gemm_t<false, true, false>(c, mt, mt, nb, -1.0, Pn, n, Pn, n, 1.0, Pn + nb, n, false);
         }
     }
+    hipLaunchKernelGGL(k_post, dim3(1), dim3(WAVE), 0, c.s, c.ctl, next_post(c));
+    chk_launch(c);
     if (!read_ctl(c) || c.h[C_ERR] != 0.0) return false;
     hipLaunchKernelGGL(k_identity, dim3((n + 255) / 256, n), dim3(256), 0, c.s, n, X);
     chk_launch(c);
@@ -1082,13 +1191,13 @@ int eig(Ctx& c, double rel_tol, double loose) {
     chk_launch(c);
     hipLaunchKernelGGL(k_vec_absmax, dim3(1), dim3(NT), 0, c.s, n, c.ev, c.part);
     chk_launch(c);
-    finish(c, 1, 1, 1, C_DMAX);
+    finish(c, 1, 1, C_DMAX);
     double tol = 0.0;
     int sweep = 0;
     for (;;) {
         hipLaunchKernelGGL(k_offmax, dim3(rb), dim3(NT), 0, c.s, n, c.F, c.part);
         chk_launch(c);
-        finish(c, rb, 1, 1, C_OFF);
+        finish(c, rb, 1, C_OFF, next_post(c));
         if (!read_ctl(c)) return -1;
         if (sweep == 0) tol = fmax(rel_tol * fmax(c.h[C_DMAX], 1.0), loose);
         if (c.h[C_OFF] <= tol) break;
@@ -1132,19 +1241,14 @@ int pd(Ctx& c, int k, double loose, const double* vin) {
         if (pass > 0) fock(c, vin);
         gemm_t<false, false, false>(c, rows, n, n, 1.0, c.Ct, n, c.F, n, 0.0, c.T, n, false);  // C F
         gemm_t<false, true, false>(c, k, m, n, 1.0, c.T, n, Cv, n, 0.0, Kb, m, false);        // A_ov
-        hipLaunchKernelGGL(k_rowdot, dim3((rows + NWAVE - 1) / NWAVE), dim3(NT), 0, c.s, rows, n, c.T, c.Ct, c.ev);
+        hipLaunchKernelGGL(k_rowdot, dim3((n + NWAVE - 1) / NWAVE), dim3(NT), 0, c.s, rows, n, c.T, c.Ct, c.skey,
+                           c.ev);
         chk_launch(c);
-        if (rows < n) {
-            hipLaunchKernelGGL(k_copy_tail, dim3((n - rows + 255) / 256), dim3(256), 0, c.s, rows, n, c.skey, c.ev);
-            chk_launch(c);
-        }
-        hipLaunchKernelGGL(k_vec_absmax, dim3(1), dim3(NT), 0, c.s, n, c.ev, c.part);
-        chk_launch(c);
-        finish(c, 1, 1, 1, C_DMAX);
         const int ab = (k + NWAVE - 1) / NWAVE;
         hipLaunchKernelGGL(k_amplitudes, dim3(ab), dim3(NT), 0, c.s, k, m, Kb, c.ev, c.part);
         chk_launch(c);
-        finish(c, ab, 3, 1 | (1 << 2) | (2 << 4), C_AOV);
+        hipLaunchKernelGGL(k_pd_stats, dim3(1), dim3(NT), 0, c.s, n, c.ev, c.part, ab, c.ctl, next_post(c));
+        chk_launch(c);
         if (!read_ctl(c)) return 0;
         const double tol = fmax(c.o.jacobi_tol * fmax(c.h[C_DMAX], 1.0),
                                 loose > 0.0 ? loose : PD_FINAL_REL * c.o.x_atol_max);
@@ -1160,7 +1264,7 @@ int pd(Ctx& c, int k, double loose, const double* vin) {
         gemm_t<false, false, false>(c, k, n, m, 1.0, Kb, m, Cv, n, 0.0, Z, n, false);         // K C_vir
         hipLaunchKernelGGL(k_sumsq, dim3(256), dim3(NT), 0, c.s, (size_t)k * k, X, c.part);
         chk_launch(c);
-        finish(c, 256, 1, 0, C_XF);
+        finish(c, 256, 0, C_XF, next_post(c));
         if (!read_ctl(c)) return 0;
         const double xf = sqrt(c.h[C_XF]);
         const double tolj = loose > 0.0 ? fmin(1e-13, fmax(1e-17, 1e-3 * loose)) : 1e-17;
@@ -1184,30 +1288,45 @@ int pd(Ctx& c, int k, double loose, const double* vin) {
                 ph[j] = -sg / (f * (2.0 * j + 1.0) * (2.0 * j + 2.0));
             }
         }
-        const size_t kn = (size_t)k * n;
+        // R = sinc(X) C_occ + phi(X) Z and D = cos(X) C_occ - sinc(X) Z by
+        // Horner's rule, side by side (columns 0 .. n and n .. 2n) until the
+        // last term, which writes D over C_occ
         double* cur = c.F;
-        double* nxt = c.F + kn;
-        // R = sinc(X) C_occ + phi(X) Z
-        axpby(c, kn, ss[J], c.Ct, ph[J], Z, cur);
-        for (int j = J - 1; j >= 0; --j) {
-            gemm_t<false, false, true>(c, k, n, k, 1.0, X, k, cur, n, 0.0, nxt, n, false, c.Ct, Z, ss[j], ph[j]);
+        double* nxt = c.E;
+        const int n2 = 2 * n;
+        hipLaunchKernelGGL(k_series0, dim3((n + 255) / 256, k), dim3(256), 0, c.s, n, c.Ct, Z, ss[J], ph[J], cur, n2,
+                           cc[J], -ss[J], J == 0 ? c.Ct : cur + n, J == 0 ? n : n2);
+        chk_launch(c);
+        for (int j = J - 1; j > 0; --j) {
+            gemm_t<false, false, true>(c, k, n2, k, 1.0, X, k, cur, n2, 0.0, nxt, n2, false,
+                                       Epi{c.Ct, Z, n, n, ss[j], ph[j], cc[j], -ss[j]});
             double* t = cur; cur = nxt; nxt = t;
         }
-        gemm_t<true, false, false>(c, m, n, k, 1.0, Kb, m, cur, n, 1.0, Cv, n, false);  // C_vir += K^T R
-        // C_occ <- cos(X) C_occ - sinc(X) Z
-        axpby(c, kn, cc[J], c.Ct, -ss[J], Z, cur);
-        for (int j = J - 1; j >= 0; --j) {
-            gemm_t<false, false, true>(c, k, n, k, 1.0, X, k, cur, n, 0.0, nxt, n, false, c.Ct, Z, cc[j], -ss[j]);
-            double* t = cur; cur = nxt; nxt = t;
+        if (J > 0) {
+            gemm_t<false, false, true>(c, k, n, k, 1.0, X, k, cur, n2, 0.0, nxt, n2, false,
+                                       Epi{c.Ct, Z, n, n, ss[0], ph[0], 0.0, 0.0});
+            gemm_t<false, false, true>(c, k, n, k, 1.0, X, k, cur + n, n2, 0.0, c.Ct, n, false,
+                                       Epi{c.Ct, Z, n, n, cc[0], -ss[0], 0.0, 0.0});
+            cur = nxt;
         }
-        axpby(c, kn, 1.0, cur, 0.0, nullptr, c.Ct);
+        gemm_t<true, false, false>(c, m, n, k, 1.0, Kb, m, cur, n2, 1.0, Cv, n, false);  // C_vir += K^T R
         if (loose > 0.0 && kmax * aov <= tol) { ret = 1; break; }
     }
     c.t_pd += now_s() - t0;
     return ret;
 }
 
-// one SCF map vin -> vout (scf_step in scf.hip)
+// F <- the occupied rows in ascending order, H <- f (or f e, with ev) F
+void scaled_occupied(Ctx& c, const double* ev, double* H) {
+    hipLaunchKernelGGL(k_gather, dim3(c.n), dim3(256), 0, c.s, c.n, c.Ct, c.sidx, c.ctl, (int)C_KOCC, c.F);
+    chk_launch(c);
+    hipLaunchKernelGGL(k_scale_rows, dim3(c.n), dim3(256), 0, c.s, c.n, c.F, c.sidx, c.ftot, ev, c.ctl,
+                       (double*)nullptr, H);
+    chk_launch(c);
+}
+
+// one SCF map vin -> vout (scf_step in scf.hip); the sort's control values
+// are posted (!sort_rows) or left for the mixing step's post
 int step(Ctx& c, const double* vin, double* vout, int& status, double loose, bool allow_bd, bool sort_rows,
          bool final_step, int* decoupled, bool last) {
     const int n = c.n;
@@ -1249,64 +1368,47 @@ int step(Ctx& c, const double* vin, double* vout, int& status, double loose, boo
     }
     if (sw < 0 && final_step) status |= XTB_MOL_JACOBI;
     // sort, Fermi occupations, frontier gaps, occupied prefix
-    const size_t lds = (256 + (size_t)c.npow) * 8 + (size_t)c.npow * 4;
-    hipLaunchKernelGGL(k_sort_fermi, dim3(1), dim3(NT), lds, c.s, n, c.nao, c.npow, c.ev, c.skey, c.sidx, c.ftot,
-                       c.st->occ, c.nel_a, c.nel_b, c.ia, c.ib, o.kt, o.fermi_thresh, o.fermi_maxiter, c.ctl);
-    chk_launch(c);
-    if (!read_ctl(c)) return 0;
-    if (c.h[C_FOK] == 0.0) status |= XTB_MOL_FERMI;
-    c.gap_a = c.h[C_GAPA];
-    c.gap_b = c.h[C_GAPB];
-    const int kocc = (int)c.h[C_KOCC];
-    const bool perm = c.h[C_PERM] != 0.0;
-    // density P = C_occ^T diag(f) C_occ in ascending order
-    if (perm) {
-        const int rows = sort_rows ? n : kocc;
-        if (rows > 0) {
-            hipLaunchKernelGGL(k_gather, dim3(rows), dim3(256), 0, c.s, n, c.Ct, c.sidx, c.F);
-            chk_launch(c);
-        }
-        if (kocc > 0) {
-            hipLaunchKernelGGL(k_scale_rows, dim3(kocc), dim3(256), 0, c.s, n, c.F, c.sidx, c.ftot,
-                               (const double*)nullptr, c.T);
-            chk_launch(c);
-        }
-        gemm_sym<true, false>(c, n, kocc, c.F, n, c.T, n, c.P, n);
-        if (sort_rows) {
-            // the gathered rows become the orbitals (ascending order)
-            double* t = c.Ct;
-            c.Ct = c.F;
-            c.F = t;
-        }
+    sort_fermi(c, sort_rows ? NO_POST : next_post(c));
+    // density P = C_occ^T diag(f) C_occ in ascending order.  Which rows the
+    // sort moved and how many are occupied stays on the device.
+    if (sort_rows) {
+        // the orbitals' rows into ascending order
+        hipLaunchKernelGGL(k_gather, dim3(n), dim3(256), 0, c.s, n, c.Ct, c.sidx, c.ctl, (int)C_PERM, c.F);
+        chk_launch(c);
+        hipLaunchKernelGGL(k_scale_rows, dim3(n), dim3(256), 0, c.s, n, c.F, c.sidx, c.ftot, (const double*)nullptr,
+                           c.ctl, c.Ct, c.T);
+        chk_launch(c);
     } else {
-        if (kocc > 0) {
-            hipLaunchKernelGGL(k_scale_rows, dim3(kocc), dim3(256), 0, c.s, n, c.Ct, (const int*)nullptr, c.ftot,
-                               (const double*)nullptr, c.T);
-            chk_launch(c);
-        }
-        gemm_sym<true, false>(c, n, kocc, c.Ct, n, c.T, n, c.P, n);
+        scaled_occupied(c, nullptr, c.T);
     }
+    gemm_sym<true, false>(c, n, 0, sort_rows ? c.Ct : c.F, n, c.T, n, c.P, n, c.ctl + C_KOCC);
     // Mulliken charges, shell/atom charges, ES2 + ES3 potential
     const xtb_batch* b = c.b;
     hipLaunchKernelGGL(k_mulliken, dim3((n + NWAVE - 1) / NWAVE), dim3(NT), 0, c.s, n, c.nao, c.P, c.S, c.H0, b->n0,
                        last ? 1 : 0, c.st->q, c.st->eorb);
     chk_launch(c);
-    hipLaunchKernelGGL(k_shell_atom, dim3(1), dim3(NT), 0, c.s, c.nsh, c.nat, b->sh_ao, b->sh_us, c.par->us_l,
-                       b->atom_sh0, b->atom_nsh, c.st->q, c.st->qsh, c.qat);
-    chk_launch(c);
-    hipLaunchKernelGGL(k_shell_pot, dim3((c.nsh + NWAVE - 1) / NWAVE), dim3(NT), 0, c.s, c.nsh, c.gam, c.st->qsh,
-                       c.qat, b->sh_atom, b->atom_sp, c.par->sp_gam3, c.gq, c.vsh);
-    chk_launch(c);
-    hipLaunchKernelGGL(k_spread, dim3((n + 255) / 256), dim3(256), 0, c.s, n, c.nao, b->ao_sh, c.vsh, vout);
+    hipLaunchKernelGGL(k_potential, dim3((c.nsh + NWAVE - 1) / NWAVE), dim3(NT), sizeof(double) * c.nsh, c.s, c.nsh,
+                       b->sh_ao, b->sh_us, c.par->us_l, b->atom_sh0, b->atom_nsh, c.st->q, c.gam, b->sh_atom,
+                       b->atom_sp, c.par->sp_gam3, c.st->qsh, c.qat, c.gq, vout);
     chk_launch(c);
     return sw < 0 ? 0 : sw;
 }
 
-bool mix(Ctx& c, Mixer& mx, Broyden& bm, const double* xnew, const double* xold, double* xout, double* resid) {
-    hipLaunchKernelGGL(k_mix, dim3(1), dim3(NT), 0, c.s, mx, bm, c.n, c.o, c.st->hist_x, c.st->hist_f, xnew, xold,
-                       xout, c.ctl);
-    chk_launch(c);
+// takes the values of a step's sort
+bool read_step(Ctx& c, int& status) {
     if (!read_ctl(c)) return false;
+    if (c.h[C_FOK] == 0.0) status |= XTB_MOL_FERMI;
+    c.gap_a = c.h[C_GAPA];
+    c.gap_b = c.h[C_GAPB];
+    return true;
+}
+
+bool mix(Ctx& c, Mixer& mx, Broyden& bm, const double* xnew, const double* xold, double* xout, double* resid,
+         int& status) {
+    hipLaunchKernelGGL(k_mix, dim3(1), dim3(NT), 0, c.s, mx, bm, c.n, c.o, c.st->hist_x, c.st->hist_f, xnew, xold,
+                       xout, c.ctl, next_post(c));
+    chk_launch(c);
+    if (!read_step(c, status)) return false;
     // the kernel's own copy of the mixer advanced the same way
     if (c.o.mixer == 1) {
         bm.step += 1;
@@ -1348,6 +1450,8 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
     const double tstart = now_s();
     Ctx c;
     c.s = (hipStream_t)stream;
+    c.mail = &thread_mail;
+    if (c.mail->open() != hipSuccess) return XTB_EHIP;
     c.b = batch;
     c.par = par;
     c.o = *opts;
@@ -1379,7 +1483,6 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
     c.ctl = work + L.ctl;
     c.qat = work + L.qat;
     c.gq = work + L.gq;
-    c.vsh = work + L.vsh;
     static bool attr = false;
     if (!attr) {
         chk(c, hipFuncSetAttribute((const void*)k_sort_fermi, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1406,13 +1509,18 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
         rec.v[slot] = v;
         rec.mask |= 1u << slot;
     };
+    // nothing may post to this thread's box after the call
+    auto fail = [&]() {
+        (void)hipStreamSynchronize(c.s);
+        return XTB_EHIP;
+    };
     // warm start from the orbitals and potential a previous call on this
     // state left (a failed re-orthonormalisation starts cold)
     bool warm = opts->warm_start != 0 && prev_status == 0.0;
     if (warm) warm = warm_orthonormalise(c, state->pot);
     const bool ok_ortho = warm || (opts->ortho == 1 ? ortho_chol(c) : ortho(c));
     const double t_ortho = now_s() - tstart;
-    if (c.err != hipSuccess) return XTB_EHIP;
+    if (c.err != hipSuccess) return fail();
     if (!ok_ortho) {
         status |= XTB_MOL_OVERLAP;
         for (int k = 0; k < XTB_OUT_STRIDE; ++k)
@@ -1421,7 +1529,7 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
         put(XTB_OUT_STATUS, (double)status);
         hipLaunchKernelGGL(k_put, dim3(1), dim3(XTB_OUT_STRIDE), 0, c.s, out, rec);
         chk_launch(c);
-        return c.err == hipSuccess ? XTB_OK : XTB_EHIP;
+        return c.err == hipSuccess ? XTB_OK : fail();
     }
     const int n = c.n;
     if (!warm) chk(c, hipMemsetAsync(state->pot, 0, sizeof(double) * n, c.s));
@@ -1439,9 +1547,12 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
     sweeps += sw_first;
     ++iters;
     if (o.mix_guess || use_broyden) {
-        mix(c, mx, bm, state->vnew, state->pot, state->pot, &resid);
+        mix(c, mx, bm, state->vnew, state->pot, state->pot, &resid, status);
     } else {
         chk(c, hipMemcpyAsync(state->pot, state->vnew, sizeof(double) * n, hipMemcpyDeviceToDevice, c.s));
+        hipLaunchKernelGGL(k_post, dim3(1), dim3(WAVE), 0, c.s, c.ctl, next_post(c));
+        chk_launch(c);
+        read_step(c, status);
     }
     bool converged = false;
     for (int it = 0; it < o.maxiter && c.err == hipSuccess; ++it) {
@@ -1451,7 +1562,7 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
         sweeps += step(c, state->pot, state->vnew, status, o.eig_inexact * resid * soft, o.eig_inexact > 0.0,
                        true, false, nullptr, false);
         ++iters;
-        if (mix(c, mx, bm, state->vnew, state->pot, state->pot, &resid)) {
+        if (mix(c, mx, bm, state->vnew, state->pot, state->pot, &resid, status)) {
             converged = true;
             break;
         }
@@ -1464,6 +1575,7 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
     int kdec = 0;
     const int sw_last = step(c, state->vnew, state->pot, status, 0.0, false, false, o.eig_inexact > 0.0, &kdec, true);
     sweeps += sw_last;
+    read_step(c, status);
     hipLaunchKernelGGL(k_energies, dim3(1), dim3(NT), 0, c.s, n, c.nao, c.nsh, c.nat, state->eorb, state->qsh, c.gq,
                        c.qat, batch->atom_sp, par->sp_gam3, state->occ, o.kt, out);
     chk_launch(c);
@@ -1484,14 +1596,8 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
         gemm_sym<true, false>(c, n, k, c.Ct, n, R, n, c.T, n);
     } else if (o.want_w) {
         // W = C diag(f e) C^T over the occupied orbitals in ascending order
-        const int kocc = (int)c.h[C_KOCC];
-        if (kocc > 0) {
-            hipLaunchKernelGGL(k_gather, dim3(kocc), dim3(256), 0, c.s, n, c.Ct, c.sidx, c.F);
-            chk_launch(c);
-            hipLaunchKernelGGL(k_scale_rows, dim3(kocc), dim3(256), 0, c.s, n, c.F, c.sidx, c.ftot, c.ev, c.E);
-            chk_launch(c);
-        }
-        gemm_sym<true, false>(c, n, kocc, c.F, n, c.E, n, c.T, n);
+        scaled_occupied(c, c.ev, c.E);
+        gemm_sym<true, false>(c, n, 0, c.F, n, c.E, n, c.T, n, c.ctl + C_KOCC);
     }
     chk(c, hipStreamSynchronize(c.s));
     put(XTB_OUT_ITER, (double)iters);
@@ -1508,11 +1614,11 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
     put(XTB_OUT_T_TOTAL, (now_s() - tstart) * 1e6);
     hipLaunchKernelGGL(k_put, dim3(1), dim3(XTB_OUT_STRIDE), 0, c.s, out, rec);
     chk_launch(c);
-    if (c.err != hipSuccess) return XTB_EHIP;
+    if (c.err != hipSuccess) return fail();
     // the state's orbital buffer holds the orbitals, whichever buffer they
     // ended in
     if (c.Ct != state->C) {
         chk(c, hipMemcpyAsync(state->C, c.Ct, sizeof(double) * n * n, hipMemcpyDeviceToDevice, c.s));
     }
-    return c.err == hipSuccess ? XTB_OK : XTB_EHIP;
+    return c.err == hipSuccess ? XTB_OK : fail();
 }
