@@ -24,9 +24,26 @@ struct Shared {
     ldsi* sidx;
     int npow, big_cap;
     double* tacc;  // per-thread stage timers (meaningful on thread 0)
+    // Padding orbitals (padded layout) take no part in the products: see Pad
+    struct Pad* pad;
 #ifdef XTB_PD_TIMERS
     double* ptacc;  // phases of the perturbative step (instrumented builds only)
 #endif
+};
+
+// The padding orbitals of a padded layout have a unit overlap diagonal, zero
+// H0 and zero potential: they stay exact eigenvectors at energy 0, coupled to
+// nothing.  Between the steps the orbitals' rows are the nr real ones in
+// ascending order, then the padding, so that every product of a step runs
+// over nr rows and columns.  An eigensolve pairs rows by their place in the
+// whole spectrum, padding included (the place decides which rotations
+// precede which); for it the padding rows move to row p0, behind the real
+// ones of negative energy.  Without padding (or when the state is kept for
+// the next call) nr = n.
+struct Pad {
+    int nr;   // real orbitals
+    int at;   // first padding row: nr, or p0
+    int p0;   // where they belong in the whole spectrum
 };
 
 #ifdef XTB_PD_TIMERS

@@ -60,7 +60,7 @@ __host__ __device__ inline Lay make_lay(int nmax, int max_nsh, int max_nat) {
 // ---------------------------------------------------------------------------
 __device__ __noinline__ int eig_step(const Mol& M, const Shared& sh, int max_sweeps, double rel_tol,
                                      double loose, int inner, int cb_lo, int cb_hi, bool intra) {
-    const int n = M.n;
+    const int n = M.n, npad = n - sh.pad->nr;
     // scale for the absolute tolerance
     double dmax = 0.0;
     for (int i = threadIdx.x; i < n; i += NT) dmax = fmax(dmax, fabs(M.F[(size_t)i * n + i]));
@@ -70,12 +70,12 @@ __device__ __noinline__ int eig_step(const Mol& M, const Shared& sh, int max_swe
     int sweeps;
     if (npk <= sh.big_cap) {
         // T is free scratch here and holds a sweep's recorded rotations
-        sweeps = wg_jacobi(M.F, n, sh.big, ring_pitch(n, sh.big_cap), M.Ct, n, M.T, max_sweeps, tol, sh.cs, sh.red,
-                           sh.ev, cb_lo, cb_hi, intra);
+        sweeps = wg_jacobi(M.F, n, sh.big, ring_pitch(n, sh.big_cap), M.Ct, n, M.nao, M.T, max_sweeps, tol, sh.cs,
+                           sh.red, sh.ev, cb_lo, cb_hi, intra);
     } else {
         // block Jacobi; T is free scratch here and holds the subproblem rotations
-        sweeps = wg_block_jacobi(M.F, n, RowsGlobal{M.Ct, n}, M.T, max_sweeps, tol, sh.big, sh.red,
-                                 sh.tacc, inner, cb_lo, cb_hi, intra);
+        sweeps = wg_block_jacobi(M.F, n, RowsGlobal{M.Ct, n}, M.nao, sh.pad->at, sh.pad->at + npad, M.T, max_sweeps, tol,
+                                 sh.big, sh.red, sh.tacc, inner, cb_lo, cb_hi, intra);
         for (int i = threadIdx.x; i < n; i += NT) sh.ev[i] = M.F[(size_t)i * n + i];
     }
     __syncthreads();
@@ -165,30 +165,30 @@ __device__ __noinline__ int ortho_setup(const Mol& M, const Shared& sh, int* sta
 // torch.linalg.cholesky raises) sets XTB_MOL_OVERLAP in *status.
 // ---------------------------------------------------------------------------
 // In-place blocked right-looking Cholesky L L^T = A of the n x n symmetric
-// positive definite A (lower triangle read and overwritten by L; the strict
+// positive definite A (leading dimension ld; lower triangle read and overwritten by L; the strict
 // upper triangle is left as it was), 32-wide panels: one wave factors and
 // inverts each diagonal block, the panel solve and the trailing update are
-// matrix-core GEMMs.  R (>= n rows x 32, leading dimension n) is
+// matrix-core GEMMs.  R (>= n rows x 32, leading dimension ld) is
 // global scratch; the inverse of block j0's factor goes to Dg + 32 j0
 // (leading dimension its width; n x 32 doubles, n x n for n < 32).  Returns
 // false when a pivot is not positive.
-__device__ __noinline__ bool chol_factor(glbf* L, int n, glbf* R, glbf* Dg, const Shared& sh) {
+__device__ __noinline__ bool chol_factor(glbf* L, int n, int ld, glbf* R, glbf* Dg, const Shared& sh) {
     constexpr int NB = 32;
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     bool bad = false;
     for (int j0 = 0; j0 < n; j0 += NB) {
         const int nb = n - j0 < NB ? n - j0 : NB;
         glbf* D = Dg + (size_t)j0 * NB;
-        if (w == 0 && !chol_block(L + (size_t)j0 * n + j0, n, nb, D)) bad = true;
+        if (w == 0 && !chol_block(L + (size_t)j0 * ld + j0, ld, nb, D)) bad = true;
         __syncthreads();
         const int mt = n - j0 - nb;
         if (mt > 0) {
-            glbf* Pn = L + (size_t)(j0 + nb) * n + j0;  // panel below the block
-            gemm<false, true>(mt, nb, nb, 1.0, Pn, n, D, nb, 0.0, R, n, sh.big);  // b D^-T
+            glbf* Pn = L + (size_t)(j0 + nb) * ld + j0;  // panel below the block
+            gemm<false, true>(mt, nb, nb, 1.0, Pn, ld, D, nb, 0.0, R, ld, sh.big);  // b D^-T
             for (int r = w; r < mt; r += NWAVE)
-                for (int c = lane; c < nb; c += WAVE) Pn[(size_t)r * n + c] = R[(size_t)r * n + c];
+                for (int c = lane; c < nb; c += WAVE) Pn[(size_t)r * ld + c] = R[(size_t)r * ld + c];
             __syncthreads();
-            gemm<false, true>(mt, mt, nb, -1.0, Pn, n, Pn, n, 1.0, Pn + nb, n, sh.big);
+            gemm<false, true>(mt, mt, nb, -1.0, Pn, ld, Pn, ld, 1.0, Pn + nb, ld, sh.big);
         }
     }
     return !__syncthreads_or(bad);
@@ -199,28 +199,28 @@ __device__ __noinline__ bool chol_factor(glbf* L, int n, glbf* R, glbf* Dg, cons
 // i0 + nb columns of block row i are non-zero.  L in T, R in F, Dg in P.
 __device__ __noinline__ int chol_setup(const Mol& M, const Shared& sh, int* status) {
     constexpr int NB = 32;
-    const int n = M.n;
+    const int n = M.nao, ld = M.n;  // (padding: unit rows and columns)
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     glbf* L = M.T;
     glbf* X = M.Ct;
     glbf* R = M.F;   // NB x n (and mt x NB) scratch
     glbf* Dg = M.P;  // inverses of the diagonal blocks
     for (int r = w; r < n; r += NWAVE)
-        for (int c = lane; c < n; c += WAVE) L[(size_t)r * n + c] = M.S[(size_t)r * n + c];
+        for (int c = lane; c < n; c += WAVE) L[(size_t)r * ld + c] = M.S[(size_t)r * ld + c];
     __syncthreads();
-    if (!chol_factor(L, n, R, Dg, sh)) *status |= XTB_MOL_OVERLAP;
-    for (int r = w; r < n; r += NWAVE)
-        for (int c = lane; c < n; c += WAVE) X[(size_t)r * n + c] = 0.0;
+    if (!chol_factor(L, n, ld, R, Dg, sh)) *status |= XTB_MOL_OVERLAP;
+    for (int r = w; r < ld; r += NWAVE)
+        for (int c = lane; c < ld; c += WAVE) X[(size_t)r * ld + c] = r == c && r >= n ? 1.0 : 0.0;
     __syncthreads();
     for (int i0 = 0; i0 < n; i0 += NB) {
         const int nb = n - i0 < NB ? n - i0 : NB;
-        if (i0 > 0) gemm<false, false>(nb, i0, i0, -1.0, L + (size_t)i0 * n, n, X, n, 0.0, R, n, sh.big);
+        if (i0 > 0) gemm<false, false>(nb, i0, i0, -1.0, L + (size_t)i0 * ld, ld, X, ld, 0.0, R, ld, sh.big);
         for (int e = threadIdx.x; e < nb * nb; e += NT) {
             const int r = e / nb, c = e % nb;
-            R[(size_t)r * n + i0 + c] = (r == c) ? 1.0 : 0.0;
+            R[(size_t)r * ld + i0 + c] = (r == c) ? 1.0 : 0.0;
         }
         __syncthreads();
-        gemm<false, false>(nb, i0 + nb, nb, 1.0, Dg + (size_t)i0 * NB, nb, R, n, 0.0, X + (size_t)i0 * n, n, sh.big);
+        gemm<false, false>(nb, i0 + nb, nb, 1.0, Dg + (size_t)i0 * NB, nb, R, ld, 0.0, X + (size_t)i0 * ld, ld, sh.big);
     }
     return 0;
 }
@@ -241,7 +241,7 @@ __device__ __noinline__ bool warm_orthonormalise(const Mol& M, const Shared& sh)
     glbf* Dg = M.T;
     gemm<false, false>(n, n, n, 1.0, M.Ct, n, M.S, n, 0.0, M.T, n, sh.big);  // C S
     gemm_sym<false, true>(n, n, 1.0, M.T, n, M.Ct, n, G, n, sh.big);         // C S C^T
-    if (!chol_factor(G, n, R, Dg, sh)) return false;
+    if (!chol_factor(G, n, n, R, Dg, sh)) return false;
     for (int i0 = 0; i0 < n; i0 += NB) {
         const int nb = n - i0 < NB ? n - i0 : NB;
         glbf* Ci = M.Ct + (size_t)i0 * n;
@@ -257,29 +257,31 @@ __device__ __noinline__ bool warm_orthonormalise(const Mol& M, const Shared& sh)
 // ---------------------------------------------------------------------------
 // Orbitals in ascending energy order for the density products.  The
 // orbitals with f > 0 form a prefix of length kocc; G[j] = C_{sidx[j]} (row
-// j, for j < kocc, or every j when `all_rows`) and H[j] = w_j G[j] (j < kocc)
+// j, for j < kocc, or j < rows when `all_rows`; rows columns) and H[j] = w_j
+// G[j] (j < kocc, cols columns)
 // with w = f (or f e when `with_e`).  H may alias Ct: it is written only
 // after every row of G has been gathered.
 // ---------------------------------------------------------------------------
-__device__ __noinline__ void gather_occupied(const Mol& M, const Shared& sh, glbf* G, glbf* H, int kocc, bool with_e,
-                                             bool all_rows = false) {
+__device__ __noinline__ void gather_occupied(const Mol& M, const Shared& sh, glbf* G, glbf* H, int rows, int cols, int kocc,
+                                             bool with_e, bool all_rows = false) {
     const int n = M.n;
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    for (int j = w; j < (all_rows ? n : kocc); j += NWAVE) {
+    for (int j = w; j < (all_rows ? rows : kocc); j += NWAVE) {
         const glbf* src = M.Ct + (size_t)sh.sidx[j] * n;
-        for (int c = lane; c < n; c += WAVE) G[(size_t)j * n + c] = src[c];
+        for (int c = lane; c < rows; c += WAVE) G[(size_t)j * n + c] = src[c];
     }
     __syncthreads();
     for (int j = w; j < kocc; j += NWAVE) {
         const int o = sh.sidx[j];
         const double f = with_e ? sh.ftot[o] * sh.ev[o] : sh.ftot[o];
-        for (int c = lane; c < n; c += WAVE) H[(size_t)j * n + c] = f * G[(size_t)j * n + c];
+        for (int c = lane; c < cols; c += WAVE) H[(size_t)j * n + c] = f * G[(size_t)j * n + c];
     }
     __syncthreads();
 }
 
 // ---------------------------------------------------------------------------
-// Fock build F = H0 - 1/2 S o (v_i + v_j) (scf/base.py:817-859)
+// Fock build F = H0 - 1/2 S o (v_i + v_j) (scf/base.py:817-859), its leading
+// d x d block
 // ---------------------------------------------------------------------------
 // Streaming passes over rows run four rows per wave at a time, so that each
 // lane has the loads of four rows in flight (one row per wave left a CU's
@@ -288,18 +290,18 @@ __device__ __noinline__ void gather_occupied(const Mol& M, const Shared& sh, glb
 // for the stores.
 constexpr int ROWS_PER_WAVE = 4;
 
-__device__ inline void fock_build(const Mol& M, const glbf* vin) {
+__device__ inline void fock_build(const Mol& M, const glbf* vin, int d) {
     const int n = M.n;
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    for (int r0 = w * ROWS_PER_WAVE; r0 < n; r0 += NWAVE * ROWS_PER_WAVE) {
+    for (int r0 = w * ROWS_PER_WAVE; r0 < d; r0 += NWAVE * ROWS_PER_WAVE) {
         int rr[ROWS_PER_WAVE];
         double vr[ROWS_PER_WAVE];
 #pragma unroll
         for (int u = 0; u < ROWS_PER_WAVE; ++u) {
-            rr[u] = r0 + u < n ? r0 + u : n - 1;
+            rr[u] = r0 + u < d ? r0 + u : d - 1;
             vr[u] = vin[rr[u]];
         }
-        for (int c = lane; c < n; c += WAVE) {
+        for (int c = lane; c < d; c += WAVE) {
             const double vc = vin[c];
             double h[ROWS_PER_WAVE], sv[ROWS_PER_WAVE];
 #pragma unroll
@@ -309,7 +311,7 @@ __device__ inline void fock_build(const Mol& M, const glbf* vin) {
             }
 #pragma unroll
             for (int u = 0; u < ROWS_PER_WAVE; ++u)
-                if (r0 + u < n) M.F[(size_t)rr[u] * n + c] = h[u] - 0.5 * sv[u] * (vr[u] + vc);
+                if (r0 + u < d) M.F[(size_t)rr[u] * n + c] = h[u] - 0.5 * sv[u] * (vr[u] + vc);
         }
     }
     __syncthreads();
@@ -340,7 +342,8 @@ __device__ inline void fock_build(const Mol& M, const glbf* vin) {
 // last measured coupling is above the tolerance.  On return 1, sh.ev holds the
 // diagonal of C F C^T in the rows' order (occupied rows: of the last pass).
 // Scratch: T holds C F, then X and Z; P the couplings/amplitudes; F the two
-// Horner accumulators (k x n each, k <= n/2).
+// Horner accumulators (k x n each, k <= n/2).  Rows and columns run to d: n,
+// or the real orbitals only (the padding's couplings are exact zeros).
 // ---------------------------------------------------------------------------
 // Coefficients of the series in X = K K^T used by the rotation: term j of
 // cos (0): (-1)^j / (2j)!, sinc (1): (-1)^j / (2j+1)!, phi (2): -(-1)^j / (2j+2)!
@@ -360,9 +363,9 @@ struct HornerCoef {
 __constant__ const HornerCoef horner_coef;
 
 __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_scf_opts& o, int k,
-                                    double loose, const glbf* vin) {
-    const int n = M.n, m = n - k;
-    if (k <= 0 || m <= 0 || 2 * k > n) return 0;
+                                    double loose, const glbf* vin, int d) {
+    const int n = M.n, m = d - k;  // n: leading dimension
+    if (k <= 0 || n - k <= 0 || 2 * k > n) return 0;
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     glbf* Ct = M.Ct;
     glbf* Cv = M.Ct + (size_t)k * n;
@@ -370,7 +373,7 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
     // Virtual orbital energies only scale the amplitudes: an error of a few
     // SCF steps in them leaves a second-order coupling, so they are formed
     // (all rows of C F) every XTB_PD_REFRESH-th perturbative step only; the
-    // others reuse the last values (sh.skey, in the rows' order) and form
+    // others reuse the last values (sh.ev, in the rows' order) and form
     // the occupied rows of C F.  Every 4th step costs no SCF iterations on
     // 500-orbital molecules; never refreshing them costs two.
 #ifndef XTB_PD_REFRESH
@@ -379,26 +382,26 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
     // sh.tacc[7] counts the steps since the last refresh (>= 1)
     const bool refresh = sh.tacc[7] == 0.0 || sh.tacc[7] >= XTB_PD_REFRESH;
     sh.tacc[7] = refresh ? 1.0 : sh.tacc[7] + 1.0;
-    const int rows = refresh ? n : k;
+    const int rows = refresh ? d : k;
     double tm = now_us();
     (void)tm;
     const int npass = loose > 0.0 ? PD_INEXACT_PASSES : PD_EXACT_PASSES;
     for (int pass = 0; pass < npass; ++pass) {
-        if (pass > 0) fock_build(M, vin);
+        if (pass > 0) fock_build(M, vin, d);
         // T = C F (rows: all, or the occupied ones); A_ov = T_occ C_vir^T
-        gemm<false, false>(rows, n, n, 1.0, Ct, n, M.F, n, 0.0, M.T, n, sh.big);
+        gemm<false, false>(rows, d, d, 1.0, Ct, n, M.F, n, 0.0, M.T, n, sh.big);
         PD_MARK(sh, 0, tm);
-        gemm<false, true>(k, m, n, 1.0, M.T, n, Cv, n, 0.0, Kb, m, sh.big);
+        gemm<false, true>(k, m, d, 1.0, M.T, n, Cv, n, 0.0, Kb, m, sh.big);
         PD_MARK(sh, 1, tm);
         for (int i0 = w * ROWS_PER_WAVE; i0 < rows; i0 += NWAVE * ROWS_PER_WAVE) {
             int ii[ROWS_PER_WAVE];
-            double d[ROWS_PER_WAVE];
+            double e[ROWS_PER_WAVE];
 #pragma unroll
             for (int u = 0; u < ROWS_PER_WAVE; ++u) {
                 ii[u] = i0 + u < rows ? i0 + u : rows - 1;
-                d[u] = 0.0;
+                e[u] = 0.0;
             }
-            for (int c = lane; c < n; c += WAVE) {
+            for (int c = lane; c < d; c += WAVE) {
                 double tv[ROWS_PER_WAVE], cv[ROWS_PER_WAVE];
 #pragma unroll
                 for (int u = 0; u < ROWS_PER_WAVE; ++u) {
@@ -406,15 +409,15 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
                     cv[u] = Ct[(size_t)ii[u] * n + c];
                 }
 #pragma unroll
-                for (int u = 0; u < ROWS_PER_WAVE; ++u) d[u] = fma(tv[u], cv[u], d[u]);
+                for (int u = 0; u < ROWS_PER_WAVE; ++u) e[u] = fma(tv[u], cv[u], e[u]);
             }
 #pragma unroll
             for (int u = 0; u < ROWS_PER_WAVE; ++u) {
-                const double v = wave_sum(d[u]);
+                const double v = wave_sum(e[u]);
                 if (lane == 0 && i0 + u < rows) sh.ev[i0 + u] = v;
             }
         }
-        for (int a = rows + threadIdx.x; a < n; a += NT) sh.ev[a] = sh.skey[a];
+        for (int a = d + threadIdx.x; a < n; a += NT) sh.ev[a] = 0.0;  // padding
         __syncthreads();
         double dmax = 0.0;
         for (int i = threadIdx.x; i < n; i += NT) dmax = fmax(dmax, fabs(sh.ev[i]));
@@ -426,6 +429,7 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
             for (int u = 0; u < ROWS_PER_WAVE; ++u) {
                 ii[u] = i0 + u < k ? i0 + u : k - 1;
                 ei[u] = sh.ev[ii[u]];
+                if (d < n) dmin = fmin(dmin, -ei[u]);  // padding orbitals at 0
             }
             for (int a = lane; a < m; a += WAVE) {
                 const double ea = sh.ev[k + a];
@@ -461,7 +465,7 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
         glbf* Z = M.T + (size_t)k * k;
         gemm_sym<false, true>(k, m, 1.0, Kb, m, Kb, m, X, k, sh.big);
         PD_MARK(sh, 3, tm);
-        gemm<false, false>(k, n, m, 1.0, Kb, m, Cv, n, 0.0, Z, n, sh.big);
+        gemm<false, false>(k, d, m, 1.0, Kb, m, Cv, n, 0.0, Z, n, sh.big);
         PD_MARK(sh, 4, tm);
         double xf = 0.0;
         for (int e = threadIdx.x; e < k * k; e += NT) xf = fma(X[e], X[e], xf);
@@ -485,11 +489,11 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
         glbf* cur = M.F;
         glbf* nxt = M.F + (size_t)k * n;
         // R = sinc(X) C_occ + phi(X) Z
-        wg_axpby((size_t)k * n, ss[J], Ct, ph[J], Z, cur);
+        wg_axpby_rows(k, d, n, ss[J], Ct, ph[J], Z, cur);
         __syncthreads();
         for (int j = J - 1; j >= 0; --j) {
             PD_MARK(sh, 6, tm);
-            gemm_epi(k, n, k, X, k, cur, n, nxt, n, Ct, ss[j], Z, ph[j], sh.big);
+            gemm_epi(k, d, k, X, k, cur, n, nxt, n, Ct, ss[j], Z, ph[j], sh.big);
             PD_MARK(sh, 5, tm);
             glbf* t = cur;
             cur = nxt;
@@ -497,17 +501,17 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
         }
         PD_MARK(sh, 6, tm);
         // C_vir += K^T R
-        gemm<true, false>(m, n, k, 1.0, Kb, m, cur, n, 1.0, Cv, n, sh.big);
+        gemm<true, false>(m, d, k, 1.0, Kb, m, cur, n, 1.0, Cv, n, sh.big);
         PD_MARK(sh, 7, tm);
         // C_occ <- cos(X) C_occ - sinc(X) Z.  The last Horner term is written
         // over C_occ itself: each element of C_occ is read (as E1) and
         // written by the same thread, and no product takes C_occ as an
         // operand, so no copy pass follows
-        wg_axpby((size_t)k * n, cc[J], Ct, -ss[J], Z, J == 0 ? Ct : cur);
+        wg_axpby_rows(k, d, n, cc[J], Ct, -ss[J], Z, J == 0 ? Ct : cur);
         __syncthreads();
         for (int j = J - 1; j >= 0; --j) {
             PD_MARK(sh, 6, tm);
-            gemm_epi(k, n, k, X, k, cur, n, j == 0 ? Ct : nxt, n, Ct, cc[j], Z, -ss[j], sh.big);
+            gemm_epi(k, d, k, X, k, cur, n, j == 0 ? Ct : nxt, n, Ct, cc[j], Z, -ss[j], sh.big);
             PD_MARK(sh, 5, tm);
             glbf* t = cur;
             cur = nxt;
@@ -523,6 +527,80 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
     // the passes spent: good enough for an inexact step (an exact one has
     // returned from its last, measuring pass)
     return 1;
+}
+
+// The padding rows to their place in the whole spectrum, for an eigensolve
+// (no-op if they are there).  T is scratch.
+__device__ __noinline__ void pad_to_spectrum(const Mol& M, const Shared& sh) {
+    Pad& pad = *sh.pad;
+    const int n = M.n, npad = n - pad.nr;
+    if (pad.at == pad.p0) return;
+    const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    auto from = [&](int u) { return u < pad.p0 ? u : (u < pad.p0 + npad ? u - pad.p0 + pad.nr : u - npad); };
+    double e[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        const int u = threadIdx.x + x * NT;
+        e[x] = u < n ? sh.ev[from(u)] : 0.0;
+    }
+    for (int u = w; u < n; u += NWAVE) {
+        const glbf* src = M.Ct + (size_t)from(u) * n;
+        for (int c = lane; c < n; c += WAVE) M.T[(size_t)u * n + c] = src[c];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        const int u = threadIdx.x + x * NT;
+        if (u < n) sh.ev[u] = e[x];
+    }
+    wg_axpby((size_t)n * n, 1.0, M.T, 0.0, nullptr, M.Ct);
+    __syncthreads();
+    pad.at = pad.p0;
+}
+
+// After a sort: sh.sidx and sh.ev for the order that the next step's rows are
+// brought into, the real orbitals ascending, then the padding.  *moved: that
+// moves a row; *kocc: the real orbitals with f > 0, a prefix.
+__device__ __noinline__ void pad_behind(const Shared& sh, int n, bool* moved, int* kocc) {
+    Pad& pad = *sh.pad;
+    const int npad = n - pad.nr, a0 = pad.at, a1 = a0 + npad;
+    double red[3] = {0.0, 0.0, 0.0};
+    int to[2];
+    double e[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+        const int o = threadIdx.x + x * NT;
+        to[x] = -1;
+        if (o >= n) continue;
+        e[x] = sh.ev[o];
+        const double k = e[x] == e[x] ? e[x] : INFINITY;
+        // place among the real orbitals: equal and non-numbers as in wg_sort
+        int r = 0;
+        if (o >= a0 && o < a1) {
+            r = pad.nr + o - a0;
+        } else {
+            for (int i = 0; i < n; ++i) {
+                const double f = sh.ev[i], q = f == f ? f : INFINITY;
+                r += (i < a0 || i >= a1) && (q < k || (q == k && i < o));
+            }
+            if (sh.ftot[o] > 0.0) red[1] = fmax(red[1], (double)(r + 1));
+            if (k < 0.0) red[2] = fmax(red[2], (double)(r + 1));
+        }
+        to[x] = r;
+        if (r != o) red[0] = 1.0;
+    }
+    wg_max_n<3>(red, sh.red);
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+        if (to[x] >= 0) {
+            sh.sidx[to[x]] = threadIdx.x + x * NT;
+            sh.ev[to[x]] = e[x];
+        }
+    __syncthreads();
+    *moved = red[0] != 0.0;
+    *kocc = (int)red[1];
+    pad.p0 = (int)red[2];
+    pad.at = pad.nr;
 }
 
 // ---------------------------------------------------------------------------
@@ -558,11 +636,20 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
         if (ok && ib > 0 && ib < n) ok = sh.skey[ib] - sh.skey[ib - 1] >= need;
         if (ok) { cb_lo = ib; cb_hi = ia; }
     }
-    const size_t nn = (size_t)n * n;
+    // rows and columns of the products: the real orbitals, or all of them when
+    // padding orbitals are among the doubly occupied ones
+    Pad& pad = *sh.pad;
+    const bool trypd = cb_lo >= 0 && cb_lo == cb_hi && o.pd_kmax > 0.0;
+    int d = pad.nr;
+    if (trypd && d < n && pad.p0 < cb_lo) {
+        pad_to_spectrum(M, sh);
+        d = n;
+    }
+    const int d0 = trypd ? d : n;
     // Fock build (scf/base.py:817-859)
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     double t0 = now_us();
-    fock_build(M, vin);
+    fock_build(M, vin, d0);
     {
         const double t = now_us();
         sh.tacc[8] += t - t0;
@@ -578,18 +665,18 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
         // occupations, the energies and W (rotations inside the occupied
         // block leave C^T f C and C_occ^T A_oo C_occ unchanged); only the
         // orbital energies need the diagonalisation inside the two classes.
-        if (cb_lo >= 0 && cb_lo == cb_hi && o.pd_kmax > 0.0) {
-            const int r = pd_step(M, sh, o, cb_lo, 0.0, vin);
+        if (trypd) {
+            const int r = pd_step(M, sh, o, cb_lo, 0.0, vin, d);
             intra = r > 0;
-            if (r != 0) fock_build(M, vin);  // F may have served as scratch
+            if (r != 0 || d0 < n) fock_build(M, vin, n);  // F may have served as scratch
         }
         if (!intra) cb_lo = cb_hi = -1;
         pd = intra && !o.orbitals;
         if (pd && decoupled) *decoupled = cb_lo;
-    } else if (cb_lo >= 0 && cb_lo == cb_hi && o.pd_kmax > 0.0) {
-        const int r = pd_step(M, sh, o, cb_lo, loose, vin);
+    } else if (trypd) {
+        const int r = pd_step(M, sh, o, cb_lo, loose, vin, d);
         pd = r > 0;
-        if (r < 0) fock_build(M, vin);  // F served as scratch
+        if (r < 0 || (r == 0 && d0 < n)) fock_build(M, vin, n);  // F served as scratch
     }
     if (pd) {
         const double dt = now_us() - t0;
@@ -597,9 +684,12 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
         sh.tacc[3] += dt;
         sh.tacc[6] += 1.0;
     } else {
-        // T = F C ; A = C^T T  -> F
-        gemm<false, true>(n, n, n, 1.0, M.F, n, M.Ct, n, 0.0, M.T, n, sh.big);
-        gemm_sym<false, false>(n, n, 1.0, M.Ct, n, M.T, n, M.F, n, sh.big);
+        pad_to_spectrum(M, sh);
+        // T = F C ; A = C^T T  -> F (with the padding in the last rows A's are
+        // F's own zeros)
+        const int da = pad.at == pad.nr ? pad.nr : n;
+        gemm<false, true>(da, da, da, 1.0, M.F, n, M.Ct, n, 0.0, M.T, n, sh.big);
+        gemm_sym<false, false>(da, da, 1.0, M.Ct, n, M.T, n, M.F, n, sh.big);
         double t1 = now_us();
         sw = eig_step(M, sh, o.jacobi_max_sweeps, o.jacobi_tol, loose, o.jacobi_inner, cb_lo, cb_hi, intra);
         sh.tacc[7] = 1.0;  // eigenvalues fresh for the next perturbative step
@@ -627,10 +717,18 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
     // the SCF settles) they are used in place: no gather into F and no copy
     // back, 4 n^2 doubles of traffic less per step
     t0 = now_us();
-    const bool perm = fl.moved;
-    const int kocc = fl.kocc;
+    bool perm = fl.moved;
+    int kocc = fl.kocc;
+    const int held = pad.at == pad.nr ? pad.nr : n;  // rows and columns that move
+    int dp = n;                                      // of the density product
+    if (!last) {
+        dp = pad.nr;
+        if (pad.nr < n) pad_behind(sh, n, &perm, &kocc);
+        else
+            for (int j = threadIdx.x; j < n; j += NT) sh.ev[j] = sh.skey[j];  // in the sorted rows' order
+    }
     if (perm) {
-        gather_occupied(M, sh, M.F, M.T, kocc, false, sort_rows);
+        gather_occupied(M, sh, M.F, M.T, last ? n : held, last ? n : dp, kocc, false, sort_rows);
     } else {
         for (int j0 = w * ROWS_PER_WAVE; j0 < kocc; j0 += NWAVE * ROWS_PER_WAVE) {
             int jj[ROWS_PER_WAVE];
@@ -640,7 +738,7 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
                 jj[u] = j0 + u < kocc ? j0 + u : kocc - 1;
                 f[u] = sh.ftot[jj[u]];
             }
-            for (int c = lane; c < n; c += WAVE) {
+            for (int c = lane; c < dp; c += WAVE) {
                 double cv[ROWS_PER_WAVE];
 #pragma unroll
                 for (int u = 0; u < ROWS_PER_WAVE; ++u) cv[u] = M.Ct[(size_t)jj[u] * n + c];
@@ -657,14 +755,18 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
         // an intermediate step needs the charges, not P: the Mulliken sums
         // a_i = sum_j P_ij S_ij come from the density product's tiles (P is
         // never stored), into q
-        gemm_sym_mull<true, false>(n, kocc, perm ? M.F : M.Ct, n, M.T, n, M.S, n, M.nao, M.q, sh.big);
+        gemm_sym_mull<true, false>(dp, kocc, perm ? M.F : M.Ct, n, M.T, n, M.S, n, M.nao, M.q, sh.big);
     }
 #ifdef XTB_PD_TIMERS
     sh.ptacc[8] += now_us() - t0;
 #endif
     if (sort_rows && perm) {
         // the next step starts from the orbitals in ascending energy order
-        wg_axpby((size_t)n * n, 1.0, M.F, 0.0, nullptr, M.Ct);
+        const int h = last ? n : held;
+        if (h == n) wg_axpby((size_t)n * n, 1.0, M.F, 0.0, nullptr, M.Ct);
+        else
+            for (int r = w; r < h; r += NWAVE)
+                for (int c = lane; c < h; c += WAVE) M.Ct[(size_t)r * n + c] = M.F[(size_t)r * n + c];
     }
     sh.tacc[1] += now_us() - t0;
     const double tm0 = now_us();

@@ -133,6 +133,20 @@ __device__ inline void wg_axpby(size_t len, double a, const glbf* X, double b, c
     for (; e < len; e += NT) Y[e] = Z ? a * X[e] + b * Z[e] : a * X[e];
 }
 
+// The same on rows x cols elements of leading dimension ld.
+__device__ inline void wg_axpby_rows(int rows, int cols, int ld, double a, const glbf* X, double b, const glbf* Z,
+                                     glbf* Y) {
+    if (cols == ld) {
+        wg_axpby((size_t)rows * ld, a, X, b, Z, Y);
+        return;
+    }
+    for (int r = threadIdx.x / WAVE; r < rows; r += NWAVE)
+        for (int c = threadIdx.x % WAVE; c < cols; c += WAVE) {
+            const size_t e = (size_t)r * ld + c;
+            Y[e] = a * X[e] + b * Z[e];
+        }
+}
+
 // ---------------------------------------------------------------------------
 // FP64 matrix cores.  v_mfma_f64_16x16x4_f64: D(16x16) += A(16x4) B(4x16);
 // lane l supplies A[l%16][l/16] and B[l/16][l%16] and holds
@@ -827,17 +841,17 @@ __device__ __noinline__ void ring_vectors_t(glbf* Ct, int ldc, int n, const glbf
             }
 }
 
-// A recorded sweep applied to all n columns of Ct: each wave takes runs of C
+// A recorded sweep applied to ncol columns of Ct: each wave takes runs of C
 // columns.  Up to 64 pairs a lane holds one position, above that two.  C is
-// the wave's share n / 8 rounded up to a compiled size, so that one run covers
-// it (n <= 128) or two even ones do (9 up to n = 144, 12 above; 2 x 16 columns
+// the wave's share ncol / 8 rounded up to a compiled size, so that one run covers
+// it (ncol <= 128) or two even ones do (9 up to n = 144, 12 above; 2 x 16 columns
 // of two positions would not fit the registers).
-__device__ inline void ring_vectors(glbf* Ct, int ldc, int n, const glbf* rot) {
+__device__ inline void ring_vectors(glbf* Ct, int ldc, int n, int ncol, const glbf* rot) {
     const int w = threadIdx.x / WAVE;
-    const int share = (n + NWAVE - 1) / NWAVE;
+    const int share = (ncol + NWAVE - 1) / NWAVE;
 #define XTB_RV(S, C)                                        \
-    for (int c0 = w * (C); c0 < n; c0 += NWAVE * (C))       \
-        ring_vectors_t<S, C>(Ct, ldc, n, rot, c0, n - c0)
+    for (int c0 = w * (C); c0 < ncol; c0 += NWAVE * (C))    \
+        ring_vectors_t<S, C>(Ct, ldc, n, rot, c0, ncol - c0)
     if (ring_pairs(n) <= WAVE) {
         if (share <= 4) { XTB_RV(1, 4); }
         else if (share <= 8) { XTB_RV(1, 8); }
@@ -970,13 +984,13 @@ __device__ __noinline__ void ring_rounds(ldsf* D, int n, int W, glbf* rot, ldsf*
 
 // Diagonalises the symmetric matrix A (full, global, upper triangle read) of
 // order n <= 256 and applies every rotation to the rows of Ct (Ct[k][mu], row
-// k = vector k), i.e. C <- C J; eigenvalues to `ev`.  `D`: LDS of
+// k = vector k, mu < ncol), i.e. C <- C J; eigenvalues to `ev`.  `D`: LDS of
 // ring_doubles(n, W); `cs`: 2 K doubles of LDS (16-byte aligned); `rot`:
 // global scratch of n^2 doubles for a sweep's rotations.  Returns the number
 // of sweeps, or -1 when max_sweeps were spent without reaching `tol`
 // (absolute, largest off-diagonal element of a pair in mode).
-__device__ __noinline__ int wg_jacobi(glbf* A, int n, ldsf* D, int W, glbf* Ct, int ldc, glbf* rot, int max_sweeps,
-                                      double tol, ldsf* cs, ldsf* red, ldsf* ev, int cb_lo, int cb_hi, bool intra) {
+__device__ __noinline__ int wg_jacobi(glbf* A, int n, ldsf* D, int W, glbf* Ct, int ldc, int ncol, glbf* rot,
+                                      int max_sweeps, double tol, ldsf* cs, ldsf* red, ldsf* ev, int cb_lo, int cb_hi, bool intra) {
     const int mode = cb_lo < 0 ? 0 : (intra ? 2 : 1);
     n = __builtin_amdgcn_readfirstlane(n);
     W = __builtin_amdgcn_readfirstlane(W);
@@ -1013,7 +1027,7 @@ __device__ __noinline__ int wg_jacobi(glbf* A, int n, ldsf* D, int W, glbf* Ct, 
         else if (per <= 7) XTB_RR(7);
         else XTB_RR(10);
 #undef XTB_RR
-        ring_vectors(Ct, ldc, n, rot);
+        ring_vectors(Ct, ldc, n, ncol, rot);
         __syncthreads();
         ++sweep;
     }
@@ -1337,7 +1351,8 @@ __device__ __noinline__ void rows_update(glbf* X, int n, size_t ld, int ncol, co
 // Qbuf: global scratch >= (nblocks/2 + 1) * JS * JS doubles.  Returns sweeps
 // or -1 when max_sweeps were spent.
 template <class CAcc>
-__device__ __noinline__ int wg_block_jacobi(glbf* A, int n, CAcc Ct, glbf* Qbuf, int max_sweeps, double tol,
+__device__ __noinline__ int wg_block_jacobi(glbf* A, int n, CAcc Ct, int ncol, int pad0, int pad1, glbf* Qbuf,
+                                            int max_sweeps, double tol,
                                             ldsf* lds, ldsf* red, double* tacc, int inner,
                                             int cb_lo, int cb_hi, bool intra) {
     const int mode = cb_lo < 0 ? 0 : (intra ? 2 : 1);
@@ -1351,7 +1366,13 @@ __device__ __noinline__ int wg_block_jacobi(glbf* A, int n, CAcc Ct, glbf* Qbuf,
     const int nb2 = nb + (nb & 1);
     const int npair = nb2 / 2;
     const int ntile = npair * (npair - 1) / 2;
-    const int nch = (n + WAVE - 1) / WAVE;
+    const int nch = (ncol + WAVE - 1) / WAVE;
+    // pairs of blocks that hold nothing but uncoupled indices (pad0 .. pad1,
+    // or past the end)
+    auto idle = [&](int I, int J) {
+        auto in = [&](int b) { return b * JB >= n || (b * JB >= pad0 && (b * JB + JB < n ? b * JB + JB : n) <= pad1); };
+        return in(I) && in(J);
+    };
     ldsi* ident = reinterpret_cast<ldsi*>(lds + NWAVE * JWAVE_LDS);  // per pair: Q == I
     // symmetrise from the upper triangle
     for (int i = w; i < n; i += NWAVE)
@@ -1388,6 +1409,10 @@ __device__ __noinline__ int wg_block_jacobi(glbf* A, int n, CAcc Ct, glbf* Qbuf,
             for (int k = w; k < npair; k += NWAVE) {
                 int I, J;
                 rr_pair(r, k, nb2, I, J);
+                if (idle(I, J)) {
+                    if (lane == 0) ident[k] = 1;
+                    continue;
+                }
                 unsigned lo_mask = 0u, hi_mask = 0u;
                 if (mode != 0) {
                     // slot classes (slots 0..15 block I, 16..31 block J)
@@ -1436,6 +1461,7 @@ __device__ __noinline__ int wg_block_jacobi(glbf* A, int n, CAcc Ct, glbf* Qbuf,
                     int Ik, Jk, Il, Jl;
                     rr_pair(r, k, nb2, Ik, Jk);
                     rr_pair(r, l, nb2, Il, Jl);
+                    if (idle(Ik, Jk) || idle(Il, Jl)) continue;  // a tile of zeros
                     tile_update(A, n, Qbuf + (size_t)k * JS * JS, Qbuf + (size_t)l * JS * JS, Ik, Jk,
                                 Il, Jl, ident[k], ident[l]);
                 } else {
@@ -1444,7 +1470,7 @@ __device__ __noinline__ int wg_block_jacobi(glbf* A, int n, CAcc Ct, glbf* Qbuf,
                     if (ident[k]) continue;
                     int Ik, Jk;
                     rr_pair(r, k, nb2, Ik, Jk);
-                    rows_update(Ct.a, n, (size_t)Ct.ld, n, Qbuf + (size_t)k * JS * JS, Ik, Jk,
+                    rows_update(Ct.a, n, (size_t)Ct.ld, ncol, Qbuf + (size_t)k * JS * JS, Ik, Jk,
                                 ch * WAVE);
                 }
             }

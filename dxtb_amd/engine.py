@@ -333,7 +333,9 @@ class Pipeline:
         # block the host until the stream (or a busy stream sharing its
         # hardware queue) reaches it, and one copy costs less host time than
         # twenty.  The staging buffer lives as long as the pipeline.
-        order = np.argsort(-layout.n, kind="stable").astype(np.int32)  # largest first
+        # largest first (padded molecules by their real orbitals, which the
+        # kernel's work follows)
+        order = np.lexsort((-layout.nao, -layout.n)).astype(np.int32)
         arrays = dict(layout.arrays)
         arrays["order"] = order
         # the result records start at zero (a warm start reads the previous
