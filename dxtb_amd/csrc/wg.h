@@ -28,6 +28,14 @@ __device__ inline ldsi* to_lds(int* p) { return (ldsi*)p; }
 __device__ inline glbf* to_glb(double* p) { return (glbf*)p; }
 __device__ inline const glbf* to_glb(const double* p) { return (const glbf*)p; }
 
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+template <class T>
+__device__ __forceinline__ T* uniform(T* p) {
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return (T*)(((uint64_t)hi << 32) | lo);
+}
 // DPP move of a double; lanes without a source keep `old`
 template <int CTRL, int ROWS>
 __device__ __forceinline__ double dpp64(double old, double v) {
@@ -199,15 +207,6 @@ __device__ inline v4d v4zero() {
 // 1784 / 1904: n = 136 ran four 128-wide tiles at a quarter of their area.
 // ---------------------------------------------------------------------------
 typedef __attribute__((address_space(1))) char glbc;
-
-__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
-template <class T>
-__device__ __forceinline__ T* uniform(T* p) {
-    const uint64_t v = (uint64_t)p;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (T*)(((uint64_t)hi << 32) | lo);
-}
 
 constexpr int GEMM_KP = 16;             // k-panel depth
 constexpr int GEMM_F = 11;              // fragment rows (columns) of a workgroup tile, at most
@@ -435,34 +434,52 @@ __device__ __forceinline__ void gemm_wg_tile(const GemmOut& g, int m0, int n0, i
         panel(p, 0);
         if (p + 1 < np) panel(p + 1, 1);
     }
-    if constexpr (MODE == GEMM_MULL) {
-        ldsf* rowp = lds;                 // [fn][16 fm] row sums of fragment column c
-        ldsf* colp = lds + 16 * fm * fn;  // [fm][16 fn] column sums of fragment row r
-        __syncthreads();                  // every wave has read the last panel
+    // Epilogue, G fragments at a time so that what it reads is in flight
+    // together, at clamped places without branches.  Per product of a step at
+    // n = 292 with all CUs at it: with two added matrices 75 us (one element
+    // after the other, each waiting for its loads: 105), the Mulliken sums
+    // with their gathers 242 (308)
+    constexpr int G = NF < 4 ? NF : 4;
+    auto live = [&](int t) { return w + NWAVE * t < T; };
+    auto row = [&](int t, int r) { return m0 + 16 * fr[t] + lg + 4 * r; };
+    auto col = [&](int t) { return n0 + 16 * fc[t] + li; };
+    const uint32_t ldc = (uint32_t)g.ldc * 8u;
+    auto fetch = [&](const glbf* X, int M, int N, int t0, double (&x)[G][4]) {
 #pragma unroll
-        for (int t = 0; t < NF; ++t) {
-            if (w + NWAVE * t >= T) break;
-            const int gn = n0 + 16 * fc[t] + li;
-            double cs = 0.0, rs[4];
+        for (int u = 0; u < G; ++u)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int gm = m0 + 16 * fr[t] + lg + 4 * r;
-                rs[r] = 0.0;
-                if (gm < g.nao && gn < g.nao)
-                    rs[r] = g.alpha * acc[t][r] *
-                            *(const glbf*)((const glbc*)g.E1 + ((uint32_t)gm * (uint32_t)g.ldc + (uint32_t)gn) * 8u);
-                cs += rs[r];
+                const int t = t0 + u < NF ? t0 + u : NF - 1;
+                const int gm = row(t, r) < M ? row(t, r) : M - 1, gn = col(t) < N ? col(t) : N - 1;
+                x[u][r] = *(const glbf*)((const glbc*)X + ((uint32_t)gm * ldc + (uint32_t)gn * 8u));
             }
+    };
+    if constexpr (MODE == GEMM_MULL) {
+        ldsf* rowp = lds;                 // [fn][16 fm] row sums of fragment column c
+        ldsf* colp = lds + 16 * fm * fn;  // [4 fm][16 fn] column sums of four rows of fragment row r
+        double x[G][4];
+        fetch(g.E1, g.nao, g.nao, 0, x);
+        __syncthreads();  // every wave has read the last panel
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
+        for (int t0 = 0; t0 < NF; t0 += G) {
+            if (t0 > 0) fetch(g.E1, g.nao, g.nao, t0, x);
 #pragma unroll
-                for (int o = 1; o < 16; o <<= 1) rs[r] += __shfl_xor(rs[r], o, WAVE);
+            for (int u = 0; u < G; ++u) {
+                const int t = t0 + u;
+                if (t >= NF || !live(t)) continue;
+                double cs = 0.0;
 #pragma unroll
-            for (int o = 16; o < WAVE; o <<= 1) cs += __shfl_xor(cs, o, WAVE);
-            if (li == 0)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) rowp[fc[t] * 16 * fm + 16 * fr[t] + lg + 4 * r] = rs[r];
-            if (lg == 0) colp[fr[t] * 16 * fn + 16 * fc[t] + li] = cs;
+                for (int r = 0; r < 4; ++r) {
+                    double v = row(t, r) < g.nao && col(t) < g.nao ? g.alpha * acc[t][r] * x[u][r] : 0.0;
+                    cs += v;
+                    v += dpp64<0x111, 0xf>(0.0, v);
+                    v += dpp64<0x112, 0xf>(0.0, v);
+                    v += dpp64<0x114, 0xf>(0.0, v);
+                    v += dpp64<0x118, 0xf>(0.0, v);
+                    if (li == 15) rowp[fc[t] * 16 * fm + 16 * fr[t] + lg + 4 * r] = v;
+                }
+                colp[(4 * fr[t] + lg) * 16 * fn + 16 * fc[t] + li] = cs;
+            }
         }
         __syncthreads();
         for (int i = threadIdx.x; i < 16 * fm; i += NT) {
@@ -470,41 +487,45 @@ __device__ __forceinline__ void gemm_wg_tile(const GemmOut& g, int m0, int n0, i
             double s = g.C[m0 + i];
             for (int c = diag ? i / 16 : 0; c < fn; ++c) s += rowp[c * 16 * fm + i];
             if (diag)
-                for (int r = 0; r < i / 16; ++r) s += colp[r * 16 * fn + i];
+                for (int r = 0; r < i / 16 * 4; ++r) s += colp[r * 16 * fn + i];
             g.C[m0 + i] = s;
         }
         if (!diag)
             for (int i = threadIdx.x; i < 16 * fn; i += NT) {
                 if (n0 + i >= g.N) continue;
                 double s = g.C[n0 + i];
-                for (int r = 0; r < fm; ++r) s += colp[r * 16 * fn + i];
+                for (int r = 0; r < 4 * fm; ++r) s += colp[r * 16 * fn + i];
                 g.C[n0 + i] = s;
             }
         __syncthreads();
         return;
     }
     glbc* C = (glbc*)g.C;
-    const uint32_t ldc = (uint32_t)g.ldc * 8u;
+    const bool add = MODE == GEMM_PLAIN && !sym && g.beta != 0.0;
 #pragma unroll
-    for (int t = 0; t < NF; ++t) {
-        if (w + NWAVE * t >= T) break;
-        const int gn = n0 + 16 * fc[t] + li;
+    for (int t0 = 0; t0 < NF; t0 += G) {
+        double x[G][4], y[G][4];
+        if (MODE == GEMM_EPI) {
+            fetch(g.E1, g.M, g.N, t0, x);
+            fetch(g.E2, g.M, g.N, t0, y);
+        } else if (add) {
+            fetch(g.C, g.M, g.N, t0, x);
+        }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int gm = m0 + 16 * fr[t] + lg + 4 * r;
-            if (gm < g.M && gn < g.N) {
-                const uint32_t e = (uint32_t)gm * ldc + (uint32_t)gn * 8u;
-                glbf* c0 = (glbf*)(C + e);
-                if (MODE == GEMM_EPI) {
-                    const double e1 = *(const glbf*)((const glbc*)g.E1 + e);
-                    const double e2 = *(const glbf*)((const glbc*)g.E2 + e);
-                    *c0 = fma(g.alpha, acc[t][r], fma(g.s1, e1, g.s2 * e2));
-                } else if (sym) {
-                    const double v = g.alpha * acc[t][r];
-                    *c0 = v;
-                    if (!diag || fr[t] != fc[t]) *(glbf*)(C + ((uint32_t)gn * ldc + (uint32_t)gm * 8u)) = v;
-                } else {
-                    *c0 = g.beta == 0.0 ? g.alpha * acc[t][r] : fma(g.alpha, acc[t][r], g.beta * *c0);
+        for (int u = 0; u < G; ++u) {
+            const int t = t0 + u;
+            if (t >= NF || !live(t)) continue;
+            const int gn = col(t);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int gm = row(t, r);
+                double v = g.alpha * acc[t][r];
+                if (MODE == GEMM_EPI) v = fma(g.alpha, acc[t][r], fma(g.s1, x[u][r], g.s2 * y[u][r]));
+                else if (add) v = fma(g.alpha, acc[t][r], g.beta * x[u][r]);
+                if (gm < g.M && gn < g.N) {
+                    *(glbf*)(C + ((uint32_t)gm * ldc + (uint32_t)gn * 8u)) = v;
+                    if (sym && (!diag || fr[t] != fc[t])) *(glbf*)(C + ((uint32_t)gn * ldc + (uint32_t)gm * 8u)) = v;
                 }
             }
         }
@@ -512,7 +533,8 @@ __device__ __forceinline__ void gemm_wg_tile(const GemmOut& g, int m0, int n0, i
     __syncthreads();
 }
 
-// `tile`: fm | fn << 8 | sym << 16
+// `tile`: fm | fn << 8 | sym << 16 | part << 17; part 1, 2: the diagonal tiles
+// of a symmetric product only, the others only
 template <bool TA, bool TB, int NF, int GE, int MODE>
 __device__ __noinline__ void wg_gemm(int M, int N, int K, int tile, double alpha, const glbf* A, int lda,
                                      const glbf* B, int ldb, double beta, glbf* C, int ldc, ldsf* lds,
@@ -533,15 +555,16 @@ __device__ __noinline__ void wg_gemm(int M, int N, int K, int tile, double alpha
     if (MODE == GEMM_EPI) g.E2 = uniform(E2);
     if (MODE == GEMM_MULL) g.nao = uniform(nao);
     const int fm = tile & 255, fn = (tile >> 8) & 255;
-    const bool sym = MODE == GEMM_MULL || (MODE == GEMM_PLAIN && (tile >> 16));
-    if (MODE == GEMM_MULL) {
+    const bool sym = MODE == GEMM_MULL || (MODE == GEMM_PLAIN && (tile >> 16 & 1));
+    const int part = tile >> 17;
+    if (MODE == GEMM_MULL && part != 2) {
         for (int i = threadIdx.x; i < M; i += NT) g.C[i] = 0.0;
         __syncthreads();
     }
     const int FM = (M + 15) >> 4, FN = (N + 15) >> 4;
     for (int i = 0; i < FM; i += fm)
         for (int j = 0; j < FN; j += fn) {
-            if (sym && j < i) continue;
+            if (sym && (j < i || (part && (i == j) != (part == 1)))) continue;
             gemm_wg_tile<TA, TB, NF, GE, MODE>(g, 16 * i, 16 * j, FM - i < fm ? FM - i : fm, FN - j < fn ? FN - j : fn,
                                                K, A, lda, B, ldb, sym, sym && i == j, lds);
         }
@@ -600,9 +623,14 @@ __device__ inline void gemm_run(int M, int N, int K, double alpha, const glbf* A
         else if (fm > fn) fm = (FM + pm) / (pm + 1), ++pm;
         else fn = (FN + pn) / (pn + 1), ++pn;
     }
-    const int T = sym && fm == FM ? fm * (fm + 1) / 2 : fm * fn;
-    const int nf = (T + 7) >> 3, big = fm > fn ? fm : fn;
-    const int tile = fm | fn << 8 | (sym ? 1 : 0) << 16;
+    // Several tiles of a symmetric product: the diagonal ones, with half the
+    // fragments, and the others in a call each.
+    const int big = fm > fn ? fm : fn, split = sym && fm < FM ? 1 : 0;
+#pragma unroll 1
+    for (int part = split; part <= 2 * split; ++part) {
+        const int T = sym && part < 2 ? fm * (fm + 1) / 2 : fm * fn;
+        const int nf = (T + 7) >> 3;
+        const int tile = fm | fn << 8 | (sym ? 1 : 0) << 16 | part << 17;
 #define XTB_G(NF, GE)                                                                                                \
     wg_gemm<TA, TB, NF, GE, MODE>(M, N, K, tile, alpha, A, lda, B, ldb, beta, C, ldc, lds, E1, E2, s1, s2, nao)
 #define XTB_G23(NF)             \
@@ -614,18 +642,19 @@ __device__ inline void gemm_run(int M, int N, int K, double alpha, const glbf* A
     case NF:           \
         XTB_G(NF, 3);  \
         break;
-    switch (nf) {
-        case 1:
-            if (big <= 4) XTB_G(1, 1);
-            else XTB_G(1, 3);
-            break;
-        case 2:
-            if (big <= 4) XTB_G(2, 1);
-            else XTB_G(2, 3);
-            break;
-        XTB_G23(3) XTB_G23(4) XTB_G23(5) XTB_G23(6) XTB_G23(7) XTB_G23(8)
-        XTB_G3(9) XTB_G3(10) XTB_G3(11) XTB_G3(12) XTB_G3(13) XTB_G3(14) XTB_G3(15)
-        default: XTB_G(16, 3);
+        switch (nf) {
+            case 1:
+                if (big <= 4) XTB_G(1, 1);
+                else XTB_G(1, 3);
+                break;
+            case 2:
+                if (big <= 4) XTB_G(2, 1);
+                else XTB_G(2, 3);
+                break;
+            XTB_G23(3) XTB_G23(4) XTB_G23(5) XTB_G23(6) XTB_G23(7) XTB_G23(8)
+            XTB_G3(9) XTB_G3(10) XTB_G3(11) XTB_G3(12) XTB_G3(13) XTB_G3(14) XTB_G3(15)
+            default: XTB_G(16, 3);
+        }
     }
 #undef XTB_G3
 #undef XTB_G23
