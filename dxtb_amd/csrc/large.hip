@@ -618,12 +618,8 @@ __global__ void __launch_bounds__(NT) k_sort_fermi(int n, int nao, int npow, con
     sh.sidx = reinterpret_cast<ldsi*>(ls + 256 + npow);
     sh.ftot = to_glb(ftot);
     wg_sort(to_glb(ev), sh.skey, sh.sidx, n, npow);
-    Mol M;
-    M.n = n;
-    M.nao = nao;
-    M.nel_a = nel_a;
-    M.nel_b = nel_b;
-    const Filling fl = fill_orbitals(M, sh, kt, thr, maxiter, false, to_glb(occ), to_glb(occ) + n);
+    const Filling fl = fill_orbitals(n, nao, nel_a, nel_b, sh.skey, sh.sidx, sh.ftot, sh.red, kt, thr, maxiter, false,
+                                     to_glb(occ), to_glb(occ) + n);
     for (int j = threadIdx.x; j < n; j += NT) {
         skey_out[j] = sh.skey[j];
         sidx_out[j] = sh.sidx[j];
@@ -746,16 +742,13 @@ __global__ void __launch_bounds__(NT) k_potential(int nsh, const int* sh_ao, con
 __global__ void __launch_bounds__(NT) k_mix(Mixer mx, Broyden bm, int n, xtb_scf_opts o, double* hx, double* hf,
                                             const double* xnew, const double* xold, double* xout, double* ctl,
                                             Post p) {
-    __shared__ double red[256];
-    struct { ldsf* red; } sh{to_lds(red)};
-    Mol M;
-    M.n = n;
-    M.vec0 = 0;
-    M.nvec_total = n;
+    __shared__ double red[RED_DOUBLES];
+    const MixOpts mo{o.x_atol, o.x_atol_max, o.damp, o.damp_init, o.diag_offset};
     double resid = 0.0;
     const bool c = o.mixer == 1
-        ? broyden(bm, M, sh, o, to_glb(hx), to_glb(hf), to_glb(xnew), to_glb(xold), to_glb(xout), &resid)
-        : anderson(mx, M, sh, o, to_glb(hx), to_glb(hf), to_glb(xnew), to_glb(xold), to_glb(xout), &resid);
+        ? broyden(bm, n, n, to_lds(red), mo, o.f_atol, to_glb(hx), to_glb(hf), to_glb(xnew), to_glb(xold),
+                  to_glb(xout), &resid)
+        : anderson(mx, n, n, to_lds(red), mo, to_glb(hx), to_glb(hf), to_glb(xnew), to_glb(xold), to_glb(xout), &resid);
     if (threadIdx.x == 0) {
         ctl[C_CONV] = c ? 1.0 : 0.0;
         ctl[C_RESID] = resid;

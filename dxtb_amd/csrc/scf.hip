@@ -7,11 +7,8 @@
 
 namespace xtb {
 
-__global__ void __launch_bounds__(NT) k_scf(xtb_batch b, xtb_params par, const double* S,
-                                            const double* H0, const double* gam,
-                                            xtb_scf_opts o, xtb_scf_state st, int big_cap) {
+__global__ void __launch_bounds__(NT) k_scf(const ScfArgs args) {
     constexpr bool FUSED = false;
-    const FusedArgs fa{};
 #include "scf_body.inc"
 }
 
@@ -53,8 +50,8 @@ extern "C" int32_t xtb_scf(const xtb_batch* batch, const xtb_params* par, const 
     if (hipFuncSetAttribute((const void*)k_scf, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) !=
         hipSuccess)
         return XTB_EHIP;
-    hipLaunchKernelGGL(k_scf, dim3(batch->nmol + opts->wg_skip), dim3(NT), bytes, (hipStream_t)stream, *batch, *par,
-                       S, H0, gamma, *opts, *state, cap);
+    const ScfArgs args{*batch, *par, S, H0, gamma, *opts, *state, FusedArgs{}, cap};
+    hipLaunchKernelGGL(k_scf, dim3(batch->nmol + opts->wg_skip), dim3(NT), bytes, (hipStream_t)stream, args);
     return hipGetLastError() == hipSuccess ? XTB_OK : XTB_EHIP;
 }
 

@@ -1,56 +1,14 @@
 // Per-molecule SCF pieces shared by the one-workgroup-per-molecule kernel
-// (scf.hip) and the whole-GPU path for one large molecule (large.hip): the
-// molecule view, the LDS view, Fermi smearing and the Anderson mixer.  Every
-// function here is called by all threads of one workgroup.
+// (scf.hip) and the whole-GPU path for one large molecule (large.hip): Fermi
+// smearing, the mixers, Cholesky blocks.  Every function here is called by all
+// threads of one workgroup; uniform arguments come by value (what comes by
+// reference is read from the stack frame, a scratch load, at every use).
 #pragma once
 
 #include "common.h"
 #include "wg.h"
 
 namespace xtb {
-
-struct Mol {
-    int m, n, nao, nsh, nat, vec0, sh0, at0;
-    size_t mat0, gam0;
-    const glbf *S, *H0, *gam;
-    glbf *F, *Ct, *T, *P;
-    glbf *pot, *vnew, *q, *eorb, *emo, *occ, *qsh_out;
-    double nel_a, nel_b;
-    int nvec_total;
-};
-
-struct Shared {
-    ldsf *red, *cs, *skey, *ev, *ftot, *qsh, *vsh, *gq, *qat, *big;
-    ldsi* sidx;
-    int npow, big_cap;
-    double* tacc;  // per-thread stage timers (meaningful on thread 0)
-    // Padding orbitals (padded layout) take no part in the products: see Pad
-    struct Pad* pad;
-#ifdef XTB_PD_TIMERS
-    double* ptacc;  // phases of the perturbative step (instrumented builds only)
-#endif
-};
-
-// The padding orbitals of a padded layout have a unit overlap diagonal, zero
-// H0 and zero potential: they stay exact eigenvectors at energy 0, coupled to
-// nothing.  Between the steps the orbitals' rows are the nr real ones in
-// ascending order, then the padding, so that every product of a step runs
-// over nr rows and columns.  An eigensolve pairs rows by their place in the
-// whole spectrum, padding included (the place decides which rotations
-// precede which); for it the padding rows move to row p0, behind the real
-// ones of negative energy.  Without padding (or when the state is kept for
-// the next call) nr = n.
-struct Pad {
-    int nr;   // real orbitals
-    int at;   // first padding row: nr, or p0
-    int p0;   // where they belong in the whole spectrum
-};
-
-#ifdef XTB_PD_TIMERS
-#define PD_MARK(sh, i, t) do { const double t_ = now_us(); (sh).ptacc[i] += t_ - (t); (t) = t_; } while (0)
-#else
-#define PD_MARK(sh, i, t) do { } while (0)
-#endif
 
 // device wall clock (constant 100 MHz) in microseconds
 __device__ inline double now_us() { return (double)wall_clock64() * 0.01; }
@@ -130,6 +88,9 @@ __device__ __noinline__ bool chol_block(glbf* L, int ld, int nb, glbf* Dg) {
     return ok;
 }
 
+// LDS doubles of the reduction scratch
+constexpr int RED_DOUBLES = 192;
+
 // electronic temperatures below this (0.1 K in Hartree) fill the orbitals
 // by the aufbau principle instead of Fermi smearing
 // (src/dxtb/_src/scf/base.py:888-889)
@@ -142,9 +103,9 @@ constexpr double KT_AUFBAU = 3e-7;
 // KT_AUFBAU the aufbau occupations of the unrounded count instead
 // (filling.py:116-198; base.py:888-889 keeps the initial filling of
 // iterator.py:147-189): orbital j (from 0) is full while j + 1 < nel, the
-// next one takes nel - ceil(nel) + 1.  Sorted eigenvalues in sh.skey, their
-// orbitals in sh.sidx.  Writes the sorted occupations to occ[channel] and
-// the orbitals' sums to sh.ftot.
+// next one takes nel - ceil(nel) + 1.  Sorted eigenvalues in skey, their
+// orbitals in sidx.  Writes the sorted occupations to occ[channel] and
+// the orbitals' sums to ftot.
 //
 // Latency-bound (an exponential and a reduction per Newton step): both
 // channels advance together, and equal ones (closed shells) are one.  With
@@ -159,32 +120,37 @@ struct Filling {
     bool ok;       // every channel converged
 };
 
-template <class SH>
-__device__ __noinline__ Filling fill_orbitals(const Mol& M, const SH& sh, double kt, double thr, int maxiter,
-                                              bool padded, glbf* occ_a, glbf* occ_b) {
-    const int n = M.n;
+template <class F>
+__device__ __noinline__ Filling fill_orbitals(int n, int nao, double nel_a, double nel_b, const ldsf* skey,
+                                              const ldsi* sidx, F* ftot, ldsf* scratch, double kt, double thr,
+                                              int maxiter, bool padded, glbf* occ_a, glbf* occ_b) {
+    n = uniform(n);
+    nao = uniform(nao);
+    nel_a = uniform_copy(nel_a);
+    nel_b = uniform_copy(nel_b);
+    kt = uniform_copy(kt);
     const double eps = 2.220446049250313e-16;
-    const int nch = M.nel_a == M.nel_b ? 1 : 2;
+    const int nch = nel_a == nel_b ? 1 : 2;
     double ef[2] = {0.0, 0.0}, target[2] = {0.0, 0.0};
     bool open[2] = {false, false}, smear[2] = {false, false};
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
-        double nel = c == 0 ? M.nel_a : M.nel_b;
+        double nel = c == 0 ? nel_a : nel_b;
         if (c >= nch || fabs(nel) < eps || kt < KT_AUFBAU) continue;
         nel = rint(nel);
         int homo = (int)ceil(nel - 5e-15) - 1;
         if (homo < 0) homo = 0;
         if (homo > n - 1) homo = n - 1;
         const int lumo = n - 1 <= homo ? homo : homo + 1;
-        ef[c] = 0.5 * (sh.skey[homo] + sh.skey[lumo]);
-        if (padded && (homo >= M.nao || lumo >= M.nao)) ef[c] *= 2.0;  // filling.py:254-264
+        ef[c] = 0.5 * (skey[homo] + skey[lumo]);
+        if (padded && (homo >= nao || lumo >= nao)) ef[c] *= 2.0;  // filling.py:254-264
         target[c] = (double)(homo + 1);
         open[c] = true;
     }
     for (int it = 0; it < maxiter && (open[0] || open[1]); ++it) {
         double acc[4] = {0.0, 0.0, 0.0, 0.0};
         for (int j = threadIdx.x; j < n; j += NT) {
-            const double e = sh.skey[j];
+            const double e = skey[j];
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 if (!open[c]) continue;
@@ -198,7 +164,7 @@ __device__ __noinline__ Filling fill_orbitals(const Mol& M, const SH& sh, double
                 }
             }
         }
-        wg_sum_n<4>(acc, sh.red);
+        wg_sum_n<4>(acc, scratch);
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             if (!open[c]) continue;
@@ -214,11 +180,11 @@ __device__ __noinline__ Filling fill_orbitals(const Mol& M, const SH& sh, double
     const bool ok = !open[0] && !open[1];
     double red[3] = {0.0, 0.0, 0.0};
     for (int j = threadIdx.x; j < n; j += NT) {
-        const double e = sh.skey[j];
+        const double e = skey[j];
         double f[2] = {0.0, 0.0};
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
-            const double nel = c == 0 ? M.nel_a : M.nel_b;
+            const double nel = c == 0 ? nel_a : nel_b;
             if (c >= nch) {
                 f[c] = f[0];
             } else if (smear[c]) {
@@ -232,12 +198,12 @@ __device__ __noinline__ Filling fill_orbitals(const Mol& M, const SH& sh, double
         }
         occ_a[j] = f[0];
         occ_b[j] = f[1];
-        const int o = sh.sidx[j];
-        sh.ftot[o] = f[0] + f[1];
+        const int o = sidx[j];
+        ftot[o] = f[0] + f[1];
         if (f[0] + f[1] > 0.0) red[1] = (double)(j + 1);
         if (o != j) red[2] = 1.0;
     }
-    wg_max_n<3>(red, sh.red);
+    wg_max_n<3>(red, scratch);
     return Filling{{ef[0], nch == 1 ? ef[0] : ef[1]}, red[0], (int)red[1], red[2] != 0.0, ok};
 }
 
@@ -255,14 +221,27 @@ struct Mixer {
     bool soft;  // upstream's soft start; a warm start, already near the fixed point, skips it
 };
 
-template <class SH>
-__device__ __noinline__ bool anderson(Mixer& mx, const Mol& M, const SH& sh, const xtb_scf_opts& o,
-                         glbf* hx, glbf* hf, const glbf* xnew, const glbf* xold,
-                         glbf* xout, double* resid_inf) {
-    const int n = M.n, G = mx.G;
+// what a mixer needs of the options
+struct MixOpts {
+    double x_atol, x_atol_max, damp, damp_init, diag_offset;
+};
+
+// The vectors: n elements; histories hx and hf with `stride` between slots.
+__device__ __noinline__ bool anderson(Mixer& mixer, int n, int stride, ldsf* red, MixOpts o, glbf* hx, glbf* hf,
+                                      const glbf* xnew, const glbf* xold, glbf* xout, double* resid_inf) {
+    n = uniform(n);
+    stride = uniform(stride);
+    o = uniform_copy(o);
+    hx = uniform(hx);
+    hf = uniform(hf);
+    xnew = uniform(xnew);
+    xold = uniform(xold);
+    xout = uniform(xout);
+    Mixer mx = uniform_copy(mixer);
+    const int G = mx.G;
     auto slot = [&](int h) {  // h < G
         const int k = mx.head + h;
-        return (size_t)(k < G ? k : k - G) * M.nvec_total + M.vec0;
+        return (size_t)(k < G ? k : k - G) * stride;
     };
     auto X = [&](int h) { return hx + slot(h); };
     auto Fh = [&](int h) { return hf + slot(h); };
@@ -282,8 +261,8 @@ __device__ __noinline__ bool anderson(Mixer& mx, const Mol& M, const SH& sh, con
         l2 = fma(f, f, l2);
         linf = fmax(linf, fabs(f));
     }
-    l2 = wg_sum(l2, sh.red);
-    linf = wg_max(linf, sh.red + NWAVE);
+    l2 = wg_sum(l2, red);
+    linf = wg_max(linf, red + NWAVE);
     const bool conv = (sqrt(l2) < o.x_atol) && (linf < o.x_atol_max);
     *resid_inf = linf;
     double theta[MIX_MAXG];
@@ -297,7 +276,7 @@ __device__ __noinline__ bool anderson(Mixer& mx, const Mol& M, const SH& sh, con
         // elements: no partial sums to combine
         const int wv = threadIdx.x / WAVE, ln = threadIdx.x % WAVE;
         constexpr int NACC = MIX_MAXG * (MIX_MAXG + 3) / 2, PER = (NACC + NWAVE - 1) / NWAVE;
-        ldsf* tot = sh.red;
+        ldsf* tot = red;
         const int nt = nn * (nn + 3) / 2;
         const glbf *ph[PER], *pj[PER];
         bool rhs[PER];
@@ -360,7 +339,7 @@ __device__ __noinline__ bool anderson(Mixer& mx, const Mol& M, const SH& sh, con
     }
     // new slot for the mixed vector = oldest slot
     const int newhead = (mx.head - 1 + G) % G;
-    glbf* xn = hx + (size_t)newhead * M.nvec_total + M.vec0;
+    glbf* xn = hx + (size_t)newhead * stride;
     for (int i = threadIdx.x; i < n; i += NT) {
         double xm;
         if (nn > 0) {
@@ -381,7 +360,8 @@ __device__ __noinline__ bool anderson(Mixer& mx, const Mol& M, const SH& sh, con
         xn[i] = xm;  // slot newhead may alias X(G-1): element-wise read-before-write
     }
     __syncthreads();
-    mx.head = newhead;
+    mixer.step = mx.step;
+    mixer.head = newhead;
     return conv;
 }
 
@@ -409,10 +389,10 @@ struct Broyden {
 };
 
 // Projections sum_i U_k[i] w_i for k < r, reduced in chunks of 8 and left
-// in LDS at red[128 + k] (red holds 256 doubles; wg_sum_n<8> uses the first
+// in LDS at red[128 + k] (red holds RED_DOUBLES; wg_sum_n<8> uses the first
 // 64).  U_k(i) and w(i) are callables.
-template <class SH, class UK, class W>
-__device__ inline void wg_projections(int r, int n, const SH& sh, UK U, W w, int out0) {
+template <class UK, class W>
+__device__ inline void wg_projections(int r, int n, ldsf* red, UK U, W w, int out0) {
     for (int k0 = 0; k0 < r; k0 += 8) {
         double t[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         for (int i = threadIdx.x; i < n; i += NT) {
@@ -421,39 +401,37 @@ __device__ inline void wg_projections(int r, int n, const SH& sh, UK U, W w, int
             for (int kk = 0; kk < 8; ++kk)
                 if (k0 + kk < r) t[kk] = fma(U(k0 + kk, i), wi, t[kk]);
         }
-        wg_sum_n<8>(t, sh.red);
+        wg_sum_n<8>(t, red);
         if (threadIdx.x == 0) {
 #pragma unroll
             for (int kk = 0; kk < 8; ++kk)
-                if (k0 + kk < r) sh.red[128 + out0 + k0 + kk] = t[kk];
+                if (k0 + kk < r) red[128 + out0 + k0 + kk] = t[kk];
         }
         __syncthreads();
     }
 }
 
-template <class SH>
-__device__ __noinline__ bool broyden(Broyden& bm, const Mol& M, const SH& sh, const xtb_scf_opts& o,
-                                     glbf* hx, glbf* hf, const glbf* fx, const glbf* x, glbf* xout,
-                                     double* resid_inf) {
-    static_assert(128 + 2 * BROYDEN_MAXR <= 256, "projections fit the reduction scratch");
-    const int n = M.n, R = bm.R;
+__device__ __noinline__ bool broyden(Broyden& bm, int n, int stride, ldsf* red, MixOpts o, double f_atol, glbf* hx,
+                                     glbf* hf, const glbf* fx, const glbf* x, glbf* xout, double* resid_inf) {
+    static_assert(128 + 2 * BROYDEN_MAXR <= RED_DOUBLES, "projections fit the reduction scratch");
+    const int R = bm.R;
     constexpr double h0 = 0.5;  // -alpha, alpha = -0.5 (scf/pure/iterator.py:132)
-    auto C = [&](int k) { return hx + (size_t)k * M.nvec_total + M.vec0; };
-    auto D = [&](int k) { return hf + (size_t)k * M.nvec_total + M.vec0; };
+    auto C = [&](int k) { return hx + (size_t)k * stride; };
+    auto D = [&](int k) { return hf + (size_t)k * stride; };
     glbf* xp = C(R);
     glbf* gp = D(R);
-    ldsf* proj = sh.red + 128;  // [0, R): first set, [R, 2R): second set
+    ldsf* proj = red + 128;  // [0, R): first set, [R, 2R): second set
     double g2 = 0.0, ginf = 0.0;
     for (int i = threadIdx.x; i < n; i += NT) {
         const double g = x[i] - fx[i];
         g2 = fma(g, g, g2);
         ginf = fmax(ginf, fabs(g));
     }
-    g2 = wg_sum(g2, sh.red);
-    ginf = wg_max(ginf, sh.red);
+    g2 = wg_sum(g2, red);
+    ginf = wg_max(ginf, red);
     *resid_inf = ginf;
     if (bm.step > 0) {
-        if (bm.dxnorm < o.x_atol && sqrt(g2) < o.f_atol) {
+        if (bm.dxnorm < o.x_atol && sqrt(g2) < f_atol) {
             // the root search stops before it takes x: its result is the
             // previous input (rootsolver.py:200-215 breaks before x = xnew)
             for (int i = threadIdx.x; i < n; i += NT) xout[i] = xp[i];
@@ -465,9 +443,9 @@ __device__ __noinline__ bool broyden(Broyden& bm, const Mol& M, const SH& sh, co
         // (the memory restarts when full)
         const int r = bm.rank;
         const int rr = r >= R ? 0 : r;
-        wg_projections(rr, n, sh, [&](int k, int i) { return C(k)[i]; },
+        wg_projections(rr, n, red, [&](int k, int i) { return C(k)[i]; },
                        [&](int i) { return x[i] - xp[i]; }, 0);
-        wg_projections(rr, n, sh, [&](int k, int i) { return D(k)[i]; },
+        wg_projections(rr, n, red, [&](int k, int i) { return D(k)[i]; },
                        [&](int i) { return (x[i] - fx[i]) - gp[i]; }, R);
         glbf* cn = C(rr);
         glbf* dn = D(rr);
@@ -483,7 +461,7 @@ __device__ __noinline__ bool broyden(Broyden& bm, const Mol& M, const SH& sh, co
             dn[i] = v;
             dyv = fma(dy, v, dyv);
         }
-        dyv = wg_sum(dyv, sh.red);
+        dyv = wg_sum(dyv, red);
         const double sc = 1.0 / dyv;
         for (int i = threadIdx.x; i < n; i += NT) dn[i] *= sc;
         __syncthreads();
@@ -493,7 +471,7 @@ __device__ __noinline__ bool broyden(Broyden& bm, const Mol& M, const SH& sh, co
     }
     // dx = -H g with the updated memory
     const int rk = bm.rank;
-    wg_projections(rk, n, sh, [&](int k, int i) { return D(k)[i]; }, [&](int i) { return x[i] - fx[i]; }, 0);
+    wg_projections(rk, n, red, [&](int k, int i) { return D(k)[i]; }, [&](int i) { return x[i] - fx[i]; }, 0);
     double dn2 = 0.0;
     for (int i = threadIdx.x; i < n; i += NT) {
         const double xi = x[i], g = xi - fx[i];
@@ -505,7 +483,7 @@ __device__ __noinline__ bool broyden(Broyden& bm, const Mol& M, const SH& sh, co
         dn2 = fma(hg, hg, dn2);
         xout[i] = xi - o.damp * hg;  // xout may alias x: element-wise read-before-write
     }
-    bm.dxnorm = sqrt(wg_sum(dn2, sh.red));
+    bm.dxnorm = sqrt(wg_sum(dn2, red));
     bm.step += 1;
     return false;
 }

@@ -25,8 +25,128 @@ namespace xtb {
 
 struct Lay {
     // LDS layout in doubles (offsets), identical on host and device
-    int red, cs, skey, sidx, ev, ftot, qsh, vsh, gq, qat, big, total_fixed;
+    int red, ctx, cs, skey, sidx, ev, ftot, qsh, vsh, gq, qat, big, total_fixed;
 };
+
+typedef __attribute__((address_space(1))) int glbi;
+typedef __attribute__((address_space(3))) uint32_t ldsu;
+
+struct Mol {
+    int m, n, nao, nsh, nat, vec0, sh0, at0;
+    size_t mat0, gam0;
+    const glbf *S, *H0, *gam;
+    glbf *F, *Ct, *T, *P;
+    glbf *pot, *vnew, *q, *eorb, *emo, *occ, *qsh_out;
+    const glbf *n0, *sp_gam3;                 // reference occupations; third-order parameters
+    const glbi *sh_ao, *sh_us, *us_l, *sh_atom, *ao_sh, *atom_sh0, *atom_nsh, *atom_sp;
+    double nel_a, nel_b;
+    int nvec_total;
+};
+
+struct Shared {
+    ldsf *red, *cs, *skey, *ev, *ftot, *qsh, *vsh, *gq, *qat, *big;
+    ldsi* sidx;
+    int npow, big_cap;
+    ldsf* tacc;  // stage timers (thread 0)
+};
+
+// The padding orbitals of a padded layout have a unit overlap diagonal, zero
+// H0 and zero potential: they stay exact eigenvectors at energy 0, coupled to
+// nothing.  Between the steps the orbitals' rows are the nr real ones in
+// ascending order, then the padding, so that every product of a step runs
+// over nr rows and columns.  An eigensolve pairs rows by their place in the
+// whole spectrum, padding included (the place decides which rotations
+// precede which); for it the padding rows move to row p0, behind the real
+// ones of negative energy.  Without padding (or when the state is kept for
+// the next call) nr = n.
+struct Pad {
+    int nr;   // real orbitals
+    int at;   // first padding row: nr, or p0
+    int p0;   // where they belong in the whole spectrum
+};
+
+#ifdef XTB_PD_TIMERS
+// phases of the perturbative step (instrumented builds only)
+#define PD_MARK(sh, i, t)                                                   \
+    do {                                                                    \
+        const double t_ = now_us();                                         \
+        if (threadIdx.x == 0) (sh).red[RED_DOUBLES - 12 + (i)] += t_ - (t); \
+        (t) = t_;                                                           \
+    } while (0)
+#else
+#define PD_MARK(sh, i, t) do { } while (0)
+#endif
+
+struct FusedArgs {
+    const double* pos;
+    double* cn;
+    double* S;
+    double* H0;
+    double* gam;
+    double* dedcn;
+    double* grad;
+};
+
+// The kernels' only argument, at the start of the kernel argument segment:
+// functions read what they need of it by scalar loads from there.
+struct ScfArgs {
+    xtb_batch b;
+    xtb_params par;
+    const double *S, *H0, *gam;
+    xtb_scf_opts o;
+    xtb_scf_state st;
+    FusedArgs fa;
+    int big_cap;
+};
+typedef const __attribute__((address_space(4))) ScfArgs kargs;
+
+// What the out-of-line functions of a molecule share, in LDS; they take it to
+// scalar registers on entry.  By reference it lived in the stack frame, read
+// by scratch loads at every use: a 20-orbital energy took 653 us in the
+// kernel instead of 533, octane's energy and forces 1874 instead of 1725.
+struct Ctx {
+    Mol M;
+    Shared sh;
+    Pad pad;
+    int since;  // perturbative steps since the virtual energies were formed (0: never)
+    kargs* ka;
+    double tacc[12];
+};
+constexpr int CTX_DOUBLES = 64;
+static_assert(sizeof(Ctx) <= 8 * CTX_DOUBLES, "context in LDS");
+
+template <class T>
+__device__ __forceinline__ T ctx_load(const ldsf* ctx, size_t off) {
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    uint32_t v[sizeof(T) / 4];
+    const ldsu* p = (const ldsu*)ctx + off / 4;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 4; ++i) v[i] = __builtin_amdgcn_readfirstlane(p[i]);
+    T y;
+    __builtin_memcpy(&y, v, sizeof(T));
+    return y;
+}
+template <class T>
+__device__ __forceinline__ void ctx_store(ldsf* ctx, size_t off, const T& x) {
+    uint32_t v[sizeof(T) / 4];
+    __builtin_memcpy(v, &x, sizeof(T));
+    ldsu* p = (ldsu*)ctx + off / 4;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 4; ++i) p[i] = v[i];
+}
+#define CTX_GET(ctx, m) ctx_load<decltype(Ctx::m)>(ctx, offsetof(Ctx, m))
+#define CTX_PUT(ctx, m, x) ctx_store<decltype(Ctx::m)>(ctx, offsetof(Ctx, m), x)
+
+template <class T>
+__device__ __forceinline__ T karg_load(const __attribute__((address_space(4))) T* x) {
+    uint32_t v[sizeof(T) / 4];
+    const __attribute__((address_space(4))) uint32_t* p = (const __attribute__((address_space(4))) uint32_t*)x;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 4; ++i) v[i] = p[i];
+    T y;
+    __builtin_memcpy(&y, v, sizeof(T));
+    return y;
+}
 
 __host__ __device__ inline int next_pow2(int v) {
     int p = 1;
@@ -38,7 +158,8 @@ __host__ __device__ inline Lay make_lay(int nmax, int max_nsh, int max_nat) {
     Lay L;
     const int npow = next_pow2(nmax < 2 ? 2 : nmax);
     int o = 0;
-    L.red = o; o += 256;
+    L.red = o; o += RED_DOUBLES;
+    L.ctx = o; o += CTX_DOUBLES;
     L.cs = o; o += 3 * (nmax / 2 + 2);
     L.skey = o; o += npow;
     L.sidx = o; o += (npow + 1) / 2;  // ints
@@ -58,9 +179,14 @@ __host__ __device__ inline Lay make_lay(int nmax, int max_nsh, int max_nat) {
 // eigen step: A (full, in mol.F) -> eigenvalues in sh.ev, rotations applied
 // to mol.Ct.  Returns Jacobi sweeps (-1 on failure).
 // ---------------------------------------------------------------------------
-__device__ __noinline__ int eig_step(const Mol& M, const Shared& sh, int max_sweeps, double rel_tol,
-                                     double loose, int inner, int cb_lo, int cb_hi, bool intra) {
-    const int n = M.n, npad = n - sh.pad->nr;
+__device__ __noinline__ int eig_step(const ldsf* ctx, double loose, int cb_lo, int cb_hi, bool intra) {
+    const Mol M = CTX_GET(ctx, M);
+    const Shared sh = CTX_GET(ctx, sh);
+    const xtb_scf_opts o = karg_load(&CTX_GET(ctx, ka)->o);
+    const Pad pad = CTX_GET(ctx, pad);
+    const int n = M.n, npad = n - pad.nr, max_sweeps = o.jacobi_max_sweeps, inner = o.jacobi_inner;
+    const double rel_tol = o.jacobi_tol;
+    loose = uniform_copy(loose);
     // scale for the absolute tolerance
     double dmax = 0.0;
     for (int i = threadIdx.x; i < n; i += NT) dmax = fmax(dmax, fabs(M.F[(size_t)i * n + i]));
@@ -74,7 +200,7 @@ __device__ __noinline__ int eig_step(const Mol& M, const Shared& sh, int max_swe
                            sh.red, sh.ev, cb_lo, cb_hi, intra);
     } else {
         // block Jacobi; T is free scratch here and holds the subproblem rotations
-        sweeps = wg_block_jacobi(M.F, n, RowsGlobal{M.Ct, n}, M.nao, sh.pad->at, sh.pad->at + npad, M.T, max_sweeps, tol,
+        sweeps = wg_block_jacobi(M.F, n, RowsGlobal{M.Ct, n}, M.nao, pad.at, pad.at + npad, M.T, max_sweeps, tol,
                                  sh.big, sh.red, sh.tacc, inner, cb_lo, cb_hi, intra);
         for (int i = threadIdx.x; i < n; i += NT) sh.ev[i] = M.F[(size_t)i * n + i];
     }
@@ -87,7 +213,9 @@ __device__ __noinline__ int eig_step(const Mol& M, const Shared& sh, int max_swe
 //   Y0 = S/c, Z0 = I;  T = (3I - Z Y)/2;  Y <- Y T;  Z <- T Z
 // Y -> (S/c)^1/2 and Z -> (S/c)^-1/2 quadratically once ||I - S/c|| < 1; c is a
 // Gershgorin bound on the largest eigenvalue of S.  X = Z / sqrt(c).
-__device__ __noinline__ int ortho_setup(const Mol& M, const Shared& sh, int* status) {
+__device__ __noinline__ int ortho_setup(const ldsf* ctx, int* status) {
+    const Mol M = CTX_GET(ctx, M);
+    const Shared sh = CTX_GET(ctx, sh);
     const int n = M.n;
     const size_t nn = (size_t)n * n;
     double rs = 0.0;
@@ -172,7 +300,12 @@ __device__ __noinline__ int ortho_setup(const Mol& M, const Shared& sh, int* sta
 // global scratch; the inverse of block j0's factor goes to Dg + 32 j0
 // (leading dimension its width; n x 32 doubles, n x n for n < 32).  Returns
 // false when a pivot is not positive.
-__device__ __noinline__ bool chol_factor(glbf* L, int n, int ld, glbf* R, glbf* Dg, const Shared& sh) {
+__device__ __noinline__ bool chol_factor(glbf* L, int n, int ld, glbf* R, glbf* Dg, ldsf* big) {
+    L = uniform(L);
+    n = uniform(n);
+    ld = uniform(ld);
+    R = uniform(R);
+    Dg = uniform(Dg);
     constexpr int NB = 32;
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     bool bad = false;
@@ -184,11 +317,11 @@ __device__ __noinline__ bool chol_factor(glbf* L, int n, int ld, glbf* R, glbf* 
         const int mt = n - j0 - nb;
         if (mt > 0) {
             glbf* Pn = L + (size_t)(j0 + nb) * ld + j0;  // panel below the block
-            gemm<false, true>(mt, nb, nb, 1.0, Pn, ld, D, nb, 0.0, R, ld, sh.big);  // b D^-T
+            gemm<false, true>(mt, nb, nb, 1.0, Pn, ld, D, nb, 0.0, R, ld, big);  // b D^-T
             for (int r = w; r < mt; r += NWAVE)
                 for (int c = lane; c < nb; c += WAVE) Pn[(size_t)r * ld + c] = R[(size_t)r * ld + c];
             __syncthreads();
-            gemm<false, true>(mt, mt, nb, -1.0, Pn, ld, Pn, ld, 1.0, Pn + nb, ld, sh.big);
+            gemm<false, true>(mt, mt, nb, -1.0, Pn, ld, Pn, ld, 1.0, Pn + nb, ld, big);
         }
     }
     return !__syncthreads_or(bad);
@@ -197,7 +330,9 @@ __device__ __noinline__ bool chol_factor(glbf* L, int n, int ld, glbf* R, glbf* 
 // Cholesky orthogonaliser: L L^T = S, Ct <- X = L^-1 (rows S-orthonormal).
 // X by block rows, X_i = D_i^-1 (E_i - L_i,<i X_<i), where only the first
 // i0 + nb columns of block row i are non-zero.  L in T, R in F, Dg in P.
-__device__ __noinline__ int chol_setup(const Mol& M, const Shared& sh, int* status) {
+__device__ __noinline__ int chol_setup(const ldsf* ctx, int* status) {
+    const Mol M = CTX_GET(ctx, M);
+    const Shared sh = CTX_GET(ctx, sh);
     constexpr int NB = 32;
     const int n = M.nao, ld = M.n;  // (padding: unit rows and columns)
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
@@ -208,7 +343,7 @@ __device__ __noinline__ int chol_setup(const Mol& M, const Shared& sh, int* stat
     for (int r = w; r < n; r += NWAVE)
         for (int c = lane; c < n; c += WAVE) L[(size_t)r * ld + c] = M.S[(size_t)r * ld + c];
     __syncthreads();
-    if (!chol_factor(L, n, ld, R, Dg, sh)) *status |= XTB_MOL_OVERLAP;
+    if (!chol_factor(L, n, ld, R, Dg, sh.big)) *status |= XTB_MOL_OVERLAP;
     for (int r = w; r < ld; r += NWAVE)
         for (int c = lane; c < ld; c += WAVE) X[(size_t)r * ld + c] = r == c && r >= n ? 1.0 : 0.0;
     __syncthreads();
@@ -232,7 +367,9 @@ __device__ __noinline__ int chol_setup(const Mol& M, const Shared& sh, int* stat
 // P, C S and Dg in T, R in F; the forward substitution C_i <- D_i^-1 (C_i -
 // L_i,<i C_<i) runs in place by block rows.  Returns false (Ct unusable,
 // start cold) when G is not numerically positive definite.
-__device__ __noinline__ bool warm_orthonormalise(const Mol& M, const Shared& sh) {
+__device__ __noinline__ bool warm_orthonormalise(const ldsf* ctx) {
+    const Mol M = CTX_GET(ctx, M);
+    const Shared sh = CTX_GET(ctx, sh);
     constexpr int NB = 32;
     const int n = M.n;
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
@@ -241,7 +378,7 @@ __device__ __noinline__ bool warm_orthonormalise(const Mol& M, const Shared& sh)
     glbf* Dg = M.T;
     gemm<false, false>(n, n, n, 1.0, M.Ct, n, M.S, n, 0.0, M.T, n, sh.big);  // C S
     gemm_sym<false, true>(n, n, 1.0, M.T, n, M.Ct, n, G, n, sh.big);         // C S C^T
-    if (!chol_factor(G, n, n, R, Dg, sh)) return false;
+    if (!chol_factor(G, n, n, R, Dg, sh.big)) return false;
     for (int i0 = 0; i0 < n; i0 += NB) {
         const int nb = n - i0 < NB ? n - i0 : NB;
         glbf* Ci = M.Ct + (size_t)i0 * n;
@@ -262,9 +399,16 @@ __device__ __noinline__ bool warm_orthonormalise(const Mol& M, const Shared& sh)
 // with w = f (or f e when `with_e`).  H may alias Ct: it is written only
 // after every row of G has been gathered.
 // ---------------------------------------------------------------------------
-__device__ __noinline__ void gather_occupied(const Mol& M, const Shared& sh, glbf* G, glbf* H, int rows, int cols, int kocc,
-                                             bool with_e, bool all_rows = false) {
+__device__ __noinline__ void gather_occupied(const ldsf* ctx, glbf* G, glbf* H, int rows, int cols, int kocc, bool with_e,
+                                             bool all_rows = false) {
+    const Mol M = CTX_GET(ctx, M);
+    const Shared sh = CTX_GET(ctx, sh);
     const int n = M.n;
+    G = uniform(G);
+    H = uniform(H);
+    rows = uniform(rows);
+    cols = uniform(cols);
+    kocc = uniform(kocc);
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     for (int j = w; j < (all_rows ? rows : kocc); j += NWAVE) {
         const glbf* src = M.Ct + (size_t)sh.sidx[j] * n;
@@ -334,6 +478,7 @@ __device__ inline void fock_build(const Mol& M, const glbf* vin, int d) {
 // once the next term is below 1e-17, or 1e-13 in inexact steps (||X||_F
 // bounds the spectral norm).  Another pass measures the coupling left and
 // rotates again (pass limits and exits: PD_INEXACT_PASSES, PD_EXACT_PASSES).
+// (pd_applies: the sizes it takes.)
 // Returns 1 when done (rotated, or already decoupled to the tolerance), 0 to
 // ask for the Jacobi eigensolve with Ct and F untouched, -1 to ask for it
 // after F was used as scratch (the caller rebuilds F).  Jacobi is asked for
@@ -362,26 +507,28 @@ struct HornerCoef {
 };
 __constant__ const HornerCoef horner_coef;
 
-__device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_scf_opts& o, int k,
-                                    double loose, const glbf* vin, int d) {
+constexpr int PD_REFRESH = 4;
+__device__ inline bool pd_applies(int n, int k) { return k > 0 && n - k > 0 && 2 * k <= n; }
+
+__device__ __noinline__ int pd_step(const ldsf* ctx, int k, double loose, const glbf* vin, int d, bool refresh) {
+    const Mol M = CTX_GET(ctx, M);
+    const Shared sh = CTX_GET(ctx, sh);
+    const xtb_scf_opts o = karg_load(&CTX_GET(ctx, ka)->o);
+    k = uniform(k);
+    d = uniform(d);
+    loose = uniform_copy(loose);
+    vin = uniform(vin);
     const int n = M.n, m = d - k;  // n: leading dimension
-    if (k <= 0 || n - k <= 0 || 2 * k > n) return 0;
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     glbf* Ct = M.Ct;
     glbf* Cv = M.Ct + (size_t)k * n;
     glbf* Kb = M.P;  // k x m, leading dimension m
     // Virtual orbital energies only scale the amplitudes: an error of a few
     // SCF steps in them leaves a second-order coupling, so they are formed
-    // (all rows of C F) every XTB_PD_REFRESH-th perturbative step only; the
+    // (all rows of C F) every PD_REFRESH-th perturbative step only; the
     // others reuse the last values (sh.ev, in the rows' order) and form
     // the occupied rows of C F.  Every 4th step costs no SCF iterations on
     // 500-orbital molecules; never refreshing them costs two.
-#ifndef XTB_PD_REFRESH
-#define XTB_PD_REFRESH 4
-#endif
-    // sh.tacc[7] counts the steps since the last refresh (>= 1)
-    const bool refresh = sh.tacc[7] == 0.0 || sh.tacc[7] >= XTB_PD_REFRESH;
-    sh.tacc[7] = refresh ? 1.0 : sh.tacc[7] + 1.0;
     const int rows = refresh ? d : k;
     double tm = now_us();
     (void)tm;
@@ -519,7 +666,7 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
         }
         PD_MARK(sh, 6, tm);
 #ifdef XTB_PD_TIMERS
-        sh.ptacc[9] += (double)J;
+        if (threadIdx.x == 0) sh.red[RED_DOUBLES - 12 + 9] += (double)J;
 #endif
         // inexact steps: the second-order estimate of what is left
         if (loose > 0.0 && kmax * aov <= tol) return 1;
@@ -529,12 +676,13 @@ __device__ __noinline__ int pd_step(const Mol& M, const Shared& sh, const xtb_sc
     return 1;
 }
 
-// The padding rows to their place in the whole spectrum, for an eigensolve
-// (no-op if they are there).  T is scratch.
-__device__ __noinline__ void pad_to_spectrum(const Mol& M, const Shared& sh) {
-    Pad& pad = *sh.pad;
+// The padding rows to their place in the whole spectrum, for an eigensolve.
+// T is scratch.
+__device__ __noinline__ void pad_to_spectrum(const ldsf* ctx, Pad pad) {
+    const Mol M = CTX_GET(ctx, M);
+    const Shared sh = CTX_GET(ctx, sh);
+    pad = uniform_copy(pad);
     const int n = M.n, npad = n - pad.nr;
-    if (pad.at == pad.p0) return;
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     auto from = [&](int u) { return u < pad.p0 ? u : (u < pad.p0 + npad ? u - pad.p0 + pad.nr : u - npad); };
     double e[2];
@@ -555,14 +703,19 @@ __device__ __noinline__ void pad_to_spectrum(const Mol& M, const Shared& sh) {
     }
     wg_axpby((size_t)n * n, 1.0, M.T, 0.0, nullptr, M.Ct);
     __syncthreads();
-    pad.at = pad.p0;
 }
 
 // After a sort: sh.sidx and sh.ev for the order that the next step's rows are
-// brought into, the real orbitals ascending, then the padding.  *moved: that
-// moves a row; *kocc: the real orbitals with f > 0, a prefix.
-__device__ __noinline__ void pad_behind(const Shared& sh, int n, bool* moved, int* kocc) {
-    Pad& pad = *sh.pad;
+// brought into, the real orbitals ascending, then the padding.  moved: that
+// moves a row; kocc: the real orbitals with f > 0, a prefix; p0: see Pad.
+struct Behind {
+    int p0, kocc;
+    bool moved;
+};
+__device__ __noinline__ Behind pad_behind(const ldsf* ctx, Pad pad) {
+    const Shared sh = CTX_GET(ctx, sh);
+    pad = uniform_copy(pad);
+    const int n = CTX_GET(ctx, M.n);
     const int npad = n - pad.nr, a0 = pad.at, a1 = a0 + npad;
     double red[3] = {0.0, 0.0, 0.0};
     int to[2];
@@ -597,10 +750,7 @@ __device__ __noinline__ void pad_behind(const Shared& sh, int n, bool* moved, in
             sh.ev[to[x]] = e[x];
         }
     __syncthreads();
-    *moved = red[0] != 0.0;
-    *kocc = (int)red[1];
-    pad.p0 = (int)red[2];
-    pad.at = pad.nr;
+    return Behind{(int)red[2], (int)red[1], red[0] != 0.0};
 }
 
 // ---------------------------------------------------------------------------
@@ -608,11 +758,17 @@ __device__ __noinline__ void pad_behind(const Shared& sh, int n, bool* moved, in
 // leaves q, sorted e/occupations and shell/atom charges behind, and in the
 // last step (`last`) also P and e_orb (the other steps never store P).
 // ---------------------------------------------------------------------------
-__device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_batch& b,
-                        const xtb_params& par, const xtb_scf_opts& o, const glbf* vin,
-                        glbf* vout, int* status, double* ef, double loose, bool allow_bd,
-                        bool sort_rows, bool final_step = false, int* decoupled = nullptr,
-                        bool last = false) {
+__device__ __noinline__ int scf_step(ldsf* ctx, const glbf* vin, glbf* vout, int* status, double* ef, double loose,
+                                     bool allow_bd, bool sort_rows, bool final_step = false,
+                                     int* decoupled = nullptr, bool last = false) {
+    const Mol M = CTX_GET(ctx, M);
+    const Shared sh = CTX_GET(ctx, sh);
+    Pad pad = CTX_GET(ctx, pad);
+    int since = CTX_GET(ctx, since);
+    const xtb_scf_opts o = karg_load(&CTX_GET(ctx, ka)->o);
+    vin = uniform(vin);
+    vout = uniform(vout);
+    loose = uniform_copy(loose);
     const int n = M.n;
     // Occupation classes for this step's eigensolve.  With integer alpha/beta
     // counts and frontier gaps of at least bd_gap_kt x kT in the previous
@@ -638,13 +794,21 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
     }
     // rows and columns of the products: the real orbitals, or all of them when
     // padding orbitals are among the doubly occupied ones
-    Pad& pad = *sh.pad;
-    const bool trypd = cb_lo >= 0 && cb_lo == cb_hi && o.pd_kmax > 0.0;
+    const bool trypd = cb_lo >= 0 && cb_lo == cb_hi && o.pd_kmax > 0.0 && pd_applies(n, cb_lo);
+    auto unpack = [&]() {
+        if (pad.at == pad.p0) return;
+        pad_to_spectrum(ctx, pad);
+        pad.at = pad.p0;
+        if (threadIdx.x == 0) CTX_PUT(ctx, pad, pad);
+        __syncthreads();
+    };
     int d = pad.nr;
     if (trypd && d < n && pad.p0 < cb_lo) {
-        pad_to_spectrum(M, sh);
+        unpack();
         d = n;
     }
+    const bool refresh = since == 0 || since >= PD_REFRESH;
+    if (trypd) since = refresh ? 1 : since + 1;
     const int d0 = trypd ? d : n;
     // Fock build (scf/base.py:817-859)
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
@@ -652,8 +816,10 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
     fock_build(M, vin, d0);
     {
         const double t = now_us();
-        sh.tacc[8] += t - t0;
-        sh.tacc[9] += 1.0;
+        if (threadIdx.x == 0) {
+            sh.tacc[8] += t - t0;
+            sh.tacc[9] += 1.0;
+        }
         t0 = t;
     }
     int sw = 0;
@@ -666,7 +832,7 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
         // block leave C^T f C and C_occ^T A_oo C_occ unchanged); only the
         // orbital energies need the diagonalisation inside the two classes.
         if (trypd) {
-            const int r = pd_step(M, sh, o, cb_lo, 0.0, vin, d);
+            const int r = pd_step(ctx, cb_lo, 0.0, vin, d, refresh);
             intra = r > 0;
             if (r != 0 || d0 < n) fock_build(M, vin, n);  // F may have served as scratch
         }
@@ -674,28 +840,32 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
         pd = intra && !o.orbitals;
         if (pd && decoupled) *decoupled = cb_lo;
     } else if (trypd) {
-        const int r = pd_step(M, sh, o, cb_lo, loose, vin, d);
+        const int r = pd_step(ctx, cb_lo, loose, vin, d, refresh);
         pd = r > 0;
         if (r < 0 || (r == 0 && d0 < n)) fock_build(M, vin, n);  // F served as scratch
     }
     if (pd) {
         const double dt = now_us() - t0;
-        sh.tacc[2] += dt;
-        sh.tacc[3] += dt;
-        sh.tacc[6] += 1.0;
+        if (threadIdx.x == 0) {
+            sh.tacc[2] += dt;
+            sh.tacc[3] += dt;
+            sh.tacc[6] += 1.0;
+        }
     } else {
-        pad_to_spectrum(M, sh);
+        unpack();
         // T = F C ; A = C^T T  -> F (with the padding in the last rows A's are
         // F's own zeros)
         const int da = pad.at == pad.nr ? pad.nr : n;
         gemm<false, true>(da, da, da, 1.0, M.F, n, M.Ct, n, 0.0, M.T, n, sh.big);
         gemm_sym<false, false>(da, da, 1.0, M.Ct, n, M.T, n, M.F, n, sh.big);
         double t1 = now_us();
-        sw = eig_step(M, sh, o.jacobi_max_sweeps, o.jacobi_tol, loose, o.jacobi_inner, cb_lo, cb_hi, intra);
-        sh.tacc[7] = 1.0;  // eigenvalues fresh for the next perturbative step
+        sw = eig_step(ctx, loose, cb_lo, cb_hi, intra);
+        since = 1;  // eigenvalues fresh for the next perturbative step
         double t2 = now_us();
-        sh.tacc[1] += t1 - t0;
-        sh.tacc[2] += t2 - t1;
+        if (threadIdx.x == 0) {
+            sh.tacc[1] += t1 - t0;
+            sh.tacc[2] += t2 - t1;
+        }
     }
     // an intermediate step's eigensolve that ran out of sweeps only slows
     // the SCF down; the final step's results would be unreliable
@@ -706,8 +876,8 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
     // on rotations among near-degenerate orbitals of different occupation:
     // the caller then tightens inexact eigensolves by 2 kT, the bound on
     // |f_i - f_j| / |e_i - e_j| over both channels
-    const Filling fl = fill_orbitals(M, sh, o.kt, o.fermi_thresh, o.fermi_maxiter, o.padded != 0, M.occ,
-                                     M.occ + M.nvec_total);
+    const Filling fl = fill_orbitals(n, M.nao, M.nel_a, M.nel_b, sh.skey, sh.sidx, sh.ftot, sh.red, o.kt,
+                                     o.fermi_thresh, o.fermi_maxiter, o.padded != 0, M.occ, M.occ + M.nvec_total);
     if (!fl.ok) *status |= XTB_MOL_FERMI;
     ef[0] = fl.ef[0];
     ef[1] = fl.ef[1];
@@ -717,18 +887,23 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
     // the SCF settles) they are used in place: no gather into F and no copy
     // back, 4 n^2 doubles of traffic less per step
     t0 = now_us();
-    bool perm = fl.moved;
-    int kocc = fl.kocc;
+    bool perm = uniform((int)fl.moved);
+    int kocc = uniform(fl.kocc);
     const int held = pad.at == pad.nr ? pad.nr : n;  // rows and columns that move
     int dp = n;                                      // of the density product
     if (!last) {
         dp = pad.nr;
-        if (pad.nr < n) pad_behind(sh, n, &perm, &kocc);
-        else
+        if (pad.nr < n) {
+            const Behind bh = pad_behind(ctx, pad);
+            perm = uniform((int)bh.moved);
+            kocc = uniform(bh.kocc);
+            pad.p0 = uniform(bh.p0);
+            pad.at = pad.nr;
+        } else
             for (int j = threadIdx.x; j < n; j += NT) sh.ev[j] = sh.skey[j];  // in the sorted rows' order
     }
     if (perm) {
-        gather_occupied(M, sh, M.F, M.T, last ? n : held, last ? n : dp, kocc, false, sort_rows);
+        gather_occupied(ctx, M.F, M.T, last ? n : held, last ? n : dp, kocc, false, sort_rows);
     } else {
         for (int j0 = w * ROWS_PER_WAVE; j0 < kocc; j0 += NWAVE * ROWS_PER_WAVE) {
             int jj[ROWS_PER_WAVE];
@@ -758,7 +933,7 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
         gemm_sym_mull<true, false>(dp, kocc, perm ? M.F : M.Ct, n, M.T, n, M.S, n, M.nao, M.q, sh.big);
     }
 #ifdef XTB_PD_TIMERS
-    sh.ptacc[8] += now_us() - t0;
+    if (threadIdx.x == 0) sh.red[RED_DOUBLES - 12 + 8] += now_us() - t0;
 #endif
     if (sort_rows && perm) {
         // the next step starts from the orbitals in ascending energy order
@@ -768,12 +943,12 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
             for (int r = w; r < h; r += NWAVE)
                 for (int c = lane; c < h; c += WAVE) M.Ct[(size_t)r * n + c] = M.F[(size_t)r * n + c];
     }
-    sh.tacc[1] += now_us() - t0;
     const double tm0 = now_us();
+    if (threadIdx.x == 0) sh.tacc[1] += tm0 - t0;
     // Mulliken charges and orbital energies (scf/base.py:764-815), one wave
     // per row; the orbital energies only enter the final energy (last step)
     if (!last) {
-        for (int i = threadIdx.x; i < n; i += NT) M.q[i] = (i < M.nao) ? b.n0[M.vec0 + i] - M.q[i] : 0.0;
+        for (int i = threadIdx.x; i < n; i += NT) M.q[i] = (i < M.nao) ? M.n0[i] - M.q[i] : 0.0;
     } else {
         const int w = threadIdx.x / WAVE, l = threadIdx.x % WAVE;
         for (int i0 = w * ROWS_PER_WAVE; i0 < n; i0 += NWAVE * ROWS_PER_WAVE) {
@@ -817,7 +992,7 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
                 const double a = wave_sum(sq[u]), e = wave_sum(se[u]);
                 const int i = i0 + u;
                 if (l == 0 && i < n) {
-                    M.q[i] = (i < M.nao) ? b.n0[M.vec0 + i] - a : 0.0;
+                    M.q[i] = (i < M.nao) ? M.n0[i] - a : 0.0;
                     M.eorb[i] = (i < M.nao) ? e : 0.0;
                 }
             }
@@ -826,15 +1001,15 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
     __syncthreads();
     // shell and atom charges
     for (int s = threadIdx.x; s < M.nsh; s += NT) {
-        const int o0 = b.sh_ao[M.sh0 + s];
-        const int nl = 2 * par.us_l[b.sh_us[M.sh0 + s]] + 1;
+        const int o0 = M.sh_ao[s];
+        const int nl = 2 * M.us_l[M.sh_us[s]] + 1;
         double acc = 0.0;
         for (int x = 0; x < nl; ++x) acc += M.q[o0 + x];
         sh.qsh[s] = acc;
     }
     __syncthreads();
     for (int a = threadIdx.x; a < M.nat; a += NT) {
-        const int s0 = b.atom_sh0[M.at0 + a], ns = b.atom_nsh[M.at0 + a];
+        const int s0 = M.atom_sh0[a], ns = M.atom_nsh[a];
         double acc = 0.0;
         for (int x = 0; x < ns; ++x) acc += sh.qsh[s0 + x];
         sh.qat[a] = acc;
@@ -865,8 +1040,8 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
                 const double v = wave_sum(acc[u]);
                 const int s = s0 + u;
                 if (l == 0 && s < m) {
-                    const int a = b.sh_atom[M.sh0 + s];
-                    const double hd = par.sp_gam3[b.atom_sp[M.at0 + a]];
+                    const int a = M.sh_atom[s];
+                    const double hd = M.sp_gam3[M.atom_sp[a]];
                     sh.gq[s] = v;
                     sh.vsh[s] = v + hd * sh.qat[a] * sh.qat[a];
                 }
@@ -875,36 +1050,31 @@ __device__ __noinline__ int scf_step(const Mol& M, const Shared& sh, const xtb_b
     }
     __syncthreads();
     for (int i = threadIdx.x; i < n; i += NT) {
-        const int s = (i < M.nao) ? b.ao_sh[M.vec0 + i] : -1;
+        const int s = (i < M.nao) ? M.ao_sh[i] : -1;
         vout[i] = (s >= 0) ? sh.vsh[s] : 0.0;
     }
+    if (threadIdx.x == 0) {
+        CTX_PUT(ctx, pad, pad);
+        CTX_PUT(ctx, since, since);
+    }
     __syncthreads();
-    sh.tacc[10] += now_us() - tm0;
+    const double tm1 = now_us();
     // (P, S) reads of this stage in units of 16 n^2 bytes: the last step
     // reads P, S and H0 (orbital energies); the others form q inside the
     // density product (timed with it) and only add the gamma products here
-    sh.tacc[11] += last ? 1.5 : 0.0;
+    if (threadIdx.x == 0) {
+        sh.tacc[10] += tm1 - tm0;
+        sh.tacc[11] += last ? 1.5 : 0.0;
+    }
     return sw < 0 ? 0 : sw;
 }
 
 // Inputs and outputs of the fused single point (k_singlepoint) beyond the
 // SCF's: positions, and the buffers the integral pass and the gradient fill.
-struct FusedArgs {
-    const double* pos;
-    double* cn;
-    double* S;
-    double* H0;
-    double* gam;
-    double* dedcn;
-    double* grad;
-};
-
 // Defined with the fused kernel (singlepoint.hip); the plain SCF kernel
 // never calls them.
-__device__ __noinline__ void molecule_integrals(const Mol& M, const xtb_batch& b, const xtb_params& par,
-                                                const FusedArgs& fa, double* outs, const Shared& sh);
-__device__ __noinline__ void molecule_forces(const Mol& M, const xtb_batch& b, const xtb_params& par,
-                                             const FusedArgs& fa, const Shared& sh);
+__device__ __noinline__ void molecule_integrals(const ldsf* ctx);
+__device__ __noinline__ void molecule_forces(const ldsf* ctx);
 
 }  // namespace xtb
 

@@ -15,8 +15,14 @@ namespace xtb {
 // lanes per atom), S, H0 and gamma over the shell pairs i <= j (a wave per
 // row i), the padding orbitals of a padded layout, and the repulsion energy
 // into the molecule's record.
-__device__ __noinline__ void molecule_integrals(const Mol& M, const xtb_batch& b, const xtb_params& par,
-                                                const FusedArgs& fa, double* outs, const Shared& sh) {
+__device__ __noinline__ void molecule_integrals(const ldsf* ctx) {
+    const Mol M = CTX_GET(ctx, M);
+    const Shared sh = CTX_GET(ctx, sh);
+    kargs* ka = CTX_GET(ctx, ka);
+    const xtb_batch b = karg_load(&ka->b);
+    const xtb_params par = karg_load(&ka->par);
+    const FusedArgs fa = karg_load(&ka->fa);
+    double* outs = ka->st.out;
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     for (int a0 = 0; a0 < M.nat; a0 += NT / CN_PARTS) {
         // every lane of a CN_PARTS group takes part in the butterfly
@@ -62,8 +68,13 @@ __device__ __noinline__ void molecule_integrals(const Mol& M, const xtb_batch& b
 // n^2 >= 4 nat^2 > 5 nat (nat - 1) / 2), then each atom adds its pairs in a
 // fixed order; so the gradient has the same bits on every run.  Then the
 // CN chain rule the same way.  dE/dCN goes to fa.dedcn, dE/dR to fa.grad.
-__device__ __noinline__ void molecule_forces(const Mol& M, const xtb_batch& b, const xtb_params& par,
-                                             const FusedArgs& fa, const Shared& sh) {
+__device__ __noinline__ void molecule_forces(const ldsf* ctx) {
+    const Mol M = CTX_GET(ctx, M);
+    const Shared sh = CTX_GET(ctx, sh);
+    kargs* ka = CTX_GET(ctx, ka);
+    const xtb_batch b = karg_load(&ka->b);
+    const xtb_params par = karg_load(&ka->par);
+    const FusedArgs fa = karg_load(&ka->fa);
     const int w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
     const int nat = M.nat, n = M.n;
     double* scr = (double*)M.F;
@@ -136,12 +147,8 @@ __device__ __noinline__ void molecule_forces(const Mol& M, const xtb_batch& b, c
     __syncthreads();
 }
 
-__global__ void __launch_bounds__(NT) k_singlepoint(xtb_batch b, xtb_params par, xtb_scf_opts o,
-                                                    xtb_scf_state st, int big_cap, FusedArgs fa) {
+__global__ void __launch_bounds__(NT) k_singlepoint(const ScfArgs args) {
     constexpr bool FUSED = true;
-    const double* S = fa.S;
-    const double* H0 = fa.H0;
-    const double* gam = fa.gam;
 #include "scf_body.inc"
 }
 
@@ -165,8 +172,7 @@ extern "C" int32_t xtb_singlepoint(const xtb_batch* batch, const xtb_params* par
     if (hipFuncSetAttribute((const void*)k_singlepoint, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) !=
         hipSuccess)
         return XTB_EHIP;
-    const FusedArgs fa{positions, cn, S, H0, gamma, dedcn, grad};
-    hipLaunchKernelGGL(k_singlepoint, dim3(batch->nmol + opts->wg_skip), dim3(NT), bytes, (hipStream_t)stream,
-                       *batch, *par, *opts, *state, cap, fa);
+    const ScfArgs args{*batch, *par, S, H0, gamma, *opts, *state, {positions, cn, S, H0, gamma, dedcn, grad}, cap};
+    hipLaunchKernelGGL(k_singlepoint, dim3(batch->nmol + opts->wg_skip), dim3(NT), bytes, (hipStream_t)stream, args);
     return hipGetLastError() == hipSuccess ? XTB_OK : XTB_EHIP;
 }

@@ -36,6 +36,20 @@ __device__ __forceinline__ T* uniform(T* p) {
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
     return (T*)(((uint64_t)hi << 32) | lo);
 }
+// A uniform value or struct of them as scalars (arguments of an out-of-line
+// call arrive in vector registers, which are spilled around the next call).
+template <class T>
+__device__ __forceinline__ T uniform_copy(const T& x) {
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    uint32_t v[sizeof(T) / 4];
+    __builtin_memcpy(v, &x, sizeof(T));
+#pragma unroll
+    for (uint32_t& u : v) u = __builtin_amdgcn_readfirstlane(u);
+    T y;
+    __builtin_memcpy(&y, v, sizeof(T));
+    return y;
+}
+
 // DPP move of a double; lanes without a source keep `old`
 template <int CTRL, int ROWS>
 __device__ __forceinline__ double dpp64(double old, double v) {
@@ -1382,7 +1396,7 @@ __device__ __noinline__ void rows_update(glbf* X, int n, size_t ld, int ncol, co
 template <class CAcc>
 __device__ __noinline__ int wg_block_jacobi(glbf* A, int n, CAcc Ct, int ncol, int pad0, int pad1, glbf* Qbuf,
                                             int max_sweeps, double tol,
-                                            ldsf* lds, ldsf* red, double* tacc, int inner,
+                                            ldsf* lds, ldsf* red, ldsf* tacc, int inner,
                                             int cb_lo, int cb_hi, bool intra) {
     const int mode = cb_lo < 0 ? 0 : (intra ? 2 : 1);
     // mode 2 skips pairs of pure blocks of different classes; every block then
@@ -1505,8 +1519,10 @@ __device__ __noinline__ int wg_block_jacobi(glbf* A, int n, CAcc Ct, int ncol, i
             }
             __syncthreads();
             const double t2 = (double)wall_clock64() * 0.01;
-            tacc[4] += t1 - t0;
-            tacc[5] += t2 - t1;
+            if (threadIdx.x == 0) {
+                tacc[4] += t1 - t0;
+                tacc[5] += t2 - t1;
+            }
         }
         ++sweep;
     }
