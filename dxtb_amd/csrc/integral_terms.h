@@ -80,107 +80,147 @@ __device__ inline void gamma_pair(const xtb_batch& b, const xtb_params& par,
 // On-site blocks: S = identity on the shell's own orbitals, H0 = h on the
 // diagonal, zero between different shells of the same atom.
 // ---------------------------------------------------------------------------
-__device__ inline void shell_pair_s_h0(const xtb_batch& b, const xtb_params& par,
-                                       const double* __restrict__ pos, double* __restrict__ S,
-                                       double* __restrict__ H0, int m, int i, int j, double cni,
-                                       double cnj, const double* s_alpha, const double* s_coeff) {
+// shells i (angular momentum LI) <= j (LJ) of molecule m
+template <int LI, int LJ>
+__device__ inline void shell_pair_s_h0_t(const xtb_batch& b, const xtb_params& par,
+                                         const double* __restrict__ pos, double* __restrict__ S,
+                                         double* __restrict__ H0, int m, int i, int j, double cni,
+                                         double cnj, const double* s_alpha, const double* s_coeff) {
     const int n = b.mol_n[m];
     const int sh0 = b.mol_sh0[m], at0 = b.mol_atom0[m];
     const size_t mat0 = (size_t)b.mol_mat0[m];
     const int usi = b.sh_us[sh0 + i], usj = b.sh_us[sh0 + j];
     const int ati = b.sh_atom[sh0 + i], atj = b.sh_atom[sh0 + j];
-    const int li = par.us_l[usi], lj = par.us_l[usj];
-    const int ni = 2 * li + 1, nj = 2 * lj + 1;
     const int oi = b.sh_ao[sh0 + i], oj = b.sh_ao[sh0 + j];
     const double hi = par.us_level[usi] - par.us_kcn[usi] * cni;
     const double hj = par.us_level[usj] - par.us_kcn[usj] * cnj;
-    (void)ni;
-    (void)nj;
-    dispatch_l(li, lj, [&](auto LIc, auto LJc) {
-        constexpr int LI = decltype(LIc)::value, LJ = decltype(LJc)::value;
-        constexpr int NI = 2 * LI + 1, NJ = 2 * LJ + 1;
-        double blk[NI][NJ], hblk[NI][NJ];
+    constexpr int NI = 2 * LI + 1, NJ = 2 * LJ + 1;
+    double blk[NI][NJ], hblk[NI][NJ];
 #pragma unroll
-        for (int x = 0; x < NI; ++x)
+    for (int x = 0; x < NI; ++x)
 #pragma unroll
-            for (int y = 0; y < NJ; ++y) { blk[x][y] = 0.0; hblk[x][y] = 0.0; }
-        if (ati == atj) {
-            if constexpr (LI == LJ) {
-                if (i == j)
+        for (int y = 0; y < NJ; ++y) { blk[x][y] = 0.0; hblk[x][y] = 0.0; }
+    if (ati == atj) {
+        if constexpr (LI == LJ) {
+            if (i == j)
 #pragma unroll
-                    for (int x = 0; x < NI; ++x) { blk[x][x] = 1.0; hblk[x][x] = hi; }
-            }
-        } else {
-            const int ga = at0 + ati, gb = at0 + atj;
-            double R[3] = {pos[3 * ga] - pos[3 * gb], pos[3 * ga + 1] - pos[3 * gb + 1],
-                           pos[3 * ga + 2] - pos[3 * gb + 2]};
-            const double dist = sqrt(R[0] * R[0] + R[1] * R[1] + R[2] * R[2]);
-            if (dist < par.int_cutoff && dist > 0.1) {
-                double dummy[3][NI][NJ];
-                shell_overlap_t<false, LI, LJ>(par.us_nprim[usi], s_alpha + usi * XTB_MAXPRIM,
-                                               s_coeff + usi * XTB_MAXPRIM, par.us_nprim[usj],
-                                               s_alpha + usj * XTB_MAXPRIM, s_coeff + usj * XTB_MAXPRIM, R,
-                                               blk, dummy);
-                const double rab = par.sp_rad[b.atom_sp[ga]] + par.sp_rad[b.atom_sp[gb]];
-                double pi, dpi;
-                dist_poly(dist, rab, par.us_shpoly[usi], par.us_shpoly[usj], pi, dpi);
-                const double fac = 0.5 * (hi + hj) * par.us_K[usi * par.nus + usj] * pi;
-#pragma unroll
-                for (int x = 0; x < NI; ++x)
-#pragma unroll
-                    for (int y = 0; y < NJ; ++y) hblk[x][y] = blk[x][y] * fac;
-            }
+                for (int x = 0; x < NI; ++x) { blk[x][x] = 1.0; hblk[x][x] = hi; }
         }
+    } else {
+        const int ga = at0 + ati, gb = at0 + atj;
+        double R[3] = {pos[3 * ga] - pos[3 * gb], pos[3 * ga + 1] - pos[3 * gb + 1],
+                       pos[3 * ga + 2] - pos[3 * gb + 2]};
+        const double dist = sqrt(R[0] * R[0] + R[1] * R[1] + R[2] * R[2]);
+        if (dist < par.int_cutoff && dist > 0.1) {
+            double dummy[3][NI][NJ];
+            shell_overlap_t<false, LI, LJ>(par.us_nprim[usi], s_alpha + usi * XTB_MAXPRIM,
+                                           s_coeff + usi * XTB_MAXPRIM, par.us_nprim[usj],
+                                           s_alpha + usj * XTB_MAXPRIM, s_coeff + usj * XTB_MAXPRIM, R,
+                                           blk, dummy);
+            const double rab = par.sp_rad[b.atom_sp[ga]] + par.sp_rad[b.atom_sp[gb]];
+            double pi, dpi;
+            dist_poly(dist, rab, par.us_shpoly[usi], par.us_shpoly[usj], pi, dpi);
+            const double fac = 0.5 * (hi + hj) * par.us_K[usi * par.nus + usj] * pi;
 #pragma unroll
-        for (int x = 0; x < NI; ++x)
+            for (int x = 0; x < NI; ++x)
 #pragma unroll
-            for (int y = 0; y < NJ; ++y) {
-                const size_t e1 = mat0 + (size_t)(oi + x) * n + (oj + y);
-                const size_t e2 = mat0 + (size_t)(oj + y) * n + (oi + x);
-                S[e1] = blk[x][y];
-                H0[e1] = hblk[x][y];
-                S[e2] = blk[x][y];
-                H0[e2] = hblk[x][y];
-            }
+                for (int y = 0; y < NJ; ++y) hblk[x][y] = blk[x][y] * fac;
+        }
+    }
+#pragma unroll
+    for (int x = 0; x < NI; ++x)
+#pragma unroll
+        for (int y = 0; y < NJ; ++y) {
+            const size_t e1 = mat0 + (size_t)(oi + x) * n + (oj + y);
+            const size_t e2 = mat0 + (size_t)(oj + y) * n + (oi + x);
+            S[e1] = blk[x][y];
+            H0[e1] = hblk[x][y];
+            S[e2] = blk[x][y];
+            H0[e2] = hblk[x][y];
+        }
+}
+
+__device__ inline void shell_pair_s_h0(const xtb_batch& b, const xtb_params& par,
+                                       const double* __restrict__ pos, double* __restrict__ S,
+                                       double* __restrict__ H0, int m, int i, int j, double cni,
+                                       double cnj, const double* s_alpha, const double* s_coeff) {
+    const int sh0 = b.mol_sh0[m];
+    dispatch_l(par.us_l[b.sh_us[sh0 + i]], par.us_l[b.sh_us[sh0 + j]], [&](auto LIc, auto LJc) {
+        shell_pair_s_h0_t<decltype(LIc)::value, decltype(LJc)::value>(b, par, pos, S, H0, m, i, j, cni, cnj, s_alpha,
+                                                                      s_coeff);
     });
+}
+
+// Element e of the upper triangle (diagonal included) of n rows, rows d and
+// n - 1 - d joined into runs of n + 1: r <= c.
+__device__ inline void triangle(int n, int e, int& r, int& c) {
+    const int d = (int)((uint32_t)e / (uint32_t)(n + 1)), t = e - d * (n + 1);
+    const bool lo = t < n - d;
+    r = lo ? d : n - 1 - d;
+    c = lo ? d + t : t - 1;
 }
 
 // ---------------------------------------------------------------------------
 // repulsion energy (repulsion/base.py:269-334, rep.py:65-98):
 //   E = sum_{A<B, R<=25} Z_A Z_B exp(-sqrt(a_A a_B) R^kexp) / R
-// of molecule m by one workgroup, written (not added): thread t < REP_LANES
-// takes the atom pairs t, t + REP_LANES, ... of the upper triangle in order
-// and the partial sums are added in a fixed order, so the energy has the
-// same bits on every run and in every kernel that calls this (workgroups of
-// 256 threads in the integral pass, 512 in the fused single point).
+// of molecule m by one workgroup of T threads, written (not added): lane l <
+// REP_LANES takes the atom pairs l, l + REP_LANES, ... of the upper triangle
+// in order, a thread REP_LANES / T lanes, and the lanes' sums are added in a
+// fixed order, so the energy has the same bits on every run and in every
+// kernel that calls this (workgroups of 256 threads in the integral pass,
+// 512 in the fused single point).  One workgroup's latency bounds it, hence
+// several pairs per thread in flight.
+// red: REP_LANES / 64 doubles of LDS.
 // ---------------------------------------------------------------------------
+constexpr int REP_LANES = 1024;
+
+template <int T>
 __device__ inline void repulsion_molecule(const xtb_batch& b, const xtb_params& par,
-                                   const double* __restrict__ pos, double* out, int m,
-                                   double* red) {
-    constexpr int REP_LANES = 256;  // <= blockDim.x of every caller
+                                          const double* __restrict__ pos, double* out, int m, double* red) {
+    constexpr int Q = REP_LANES / T;
     const int na = b.mol_nat[m], a0 = b.mol_atom0[m];
     const long np = (long)na * (na - 1) / 2;
-    double e = 0.0;
-    for (long p = threadIdx.x; p < np && (int)threadIdx.x < REP_LANES; p += REP_LANES) {
-        // row A of the upper triangle holding pair index p (row A starts at
-        // A (2 na - A - 1) / 2)
-        int A = (int)((2.0 * na - 1.0 - sqrt((2.0 * na - 1.0) * (2.0 * na - 1.0) - 8.0 * (double)p)) * 0.5);
-        if (A < 0) A = 0;
-        while (A > 0 && (long)A * (2 * na - A - 1) / 2 > p) --A;
-        while ((long)(A + 1) * (2 * na - A - 2) / 2 <= p) ++A;
-        const int B = A + 1 + (int)(p - (long)A * (2 * na - A - 1) / 2);
-        const int ga = a0 + A, gb = a0 + B;
-        const double dx = pos[3 * ga] - pos[3 * gb], dy = pos[3 * ga + 1] - pos[3 * gb + 1],
-                     dz = pos[3 * ga + 2] - pos[3 * gb + 2];
-        const double r = sqrt(dx * dx + dy * dy + dz * dz);
-        if (r <= par.rep_cutoff) {
-            const int sa = b.atom_sp[ga], sb = b.atom_sp[gb];
+    double e[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) e[q] = 0.0;
+    for (long p0 = threadIdx.x; p0 < np; p0 += REP_LANES) {
+        double r[Q];
+        int ga[Q], gb[Q];
+        bool near[Q], any = false;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const long p = p0 + (long)T * q < np ? p0 + (long)T * q : np - 1;
+            // row A of the upper triangle holding pair index p (row A starts at
+            // A (2 na - A - 1) / 2)
+            int A = (int)((2.0 * na - 1.0 - sqrt((2.0 * na - 1.0) * (2.0 * na - 1.0) - 8.0 * (double)p)) * 0.5);
+            if (A < 0) A = 0;
+            while (A > 0 && (long)A * (2 * na - A - 1) / 2 > p) --A;
+            while ((long)(A + 1) * (2 * na - A - 2) / 2 <= p) ++A;
+            ga[q] = a0 + A;
+            gb[q] = a0 + A + 1 + (int)(p - (long)A * (2 * na - A - 1) / 2);
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const double dx = pos[3 * ga[q]] - pos[3 * gb[q]], dy = pos[3 * ga[q] + 1] - pos[3 * gb[q] + 1],
+                         dz = pos[3 * ga[q] + 2] - pos[3 * gb[q] + 2];
+            r[q] = sqrt(dx * dx + dy * dy + dz * dz);
+            near[q] = p0 + (long)T * q < np && r[q] <= par.rep_cutoff;
+            any = any || near[q];
+        }
+        if (!any) continue;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int sa = b.atom_sp[ga[q]], sb = b.atom_sp[gb[q]];
             const double alpha = sqrt(par.sp_arep[sa] * par.sp_arep[sb] + 2.2250738585072014e-308);
-            e += par.sp_zeff[sa] * par.sp_zeff[sb] * exp(-alpha * pow(r, par.kexp)) / r;
+            const double v = par.sp_zeff[sa] * par.sp_zeff[sb] * exp(-alpha * pow(r[q], par.kexp)) / r[q];
+            if (near[q]) e[q] += v;
         }
     }
-    for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
-    if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = e;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        for (int o = 32; o > 0; o >>= 1) e[q] += __shfl_xor(e[q], o, 64);
+        if (threadIdx.x % 64 == 0) red[threadIdx.x / 64 + q * (T / 64)] = e[q];
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
         double tot = 0.0;

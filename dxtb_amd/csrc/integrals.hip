@@ -85,17 +85,17 @@ __global__ void __launch_bounds__(256) k_gamma(xtb_batch b, xtb_params par,
 
 __global__ void __launch_bounds__(256) k_repulsion_mol(xtb_batch b, xtb_params par,
                                                        const double* __restrict__ pos, double* out) {
-    __shared__ double red[4];
-    repulsion_molecule(b, par, pos, out, blockIdx.x, red);
+    __shared__ double red[REP_LANES / 64];
+    repulsion_molecule<256>(b, par, pos, out, blockIdx.x, red);
 }
 
 // ---------------------------------------------------------------------------
-// The whole integral pass in one launch: workgroups [0, ntile_sh) are the
-// shell-pair tiles of k_s_h0 (S, H0 and gamma), each first forming the
-// coordination numbers of its tile's atoms in LDS (the same summation as
+// The whole integral pass in one launch: the first nmol workgroups each write
+// one molecule's repulsion energy (the longest work, so first); the others
+// are the shell-pair tiles of k_s_h0 (S, H0 and gamma), each first forming
+// the coordination numbers of its tile's atoms in LDS (the same summation as
 // k_cn, so the same bits; the diagonal tile holding an atom's first shell
-// also stores it); workgroups [ntile_sh, ntile_sh + nmol) each write one
-// molecule's repulsion energy.  One launch instead of four (CN, S/H0/gamma,
+// also stores it).  One launch instead of four (CN, S/H0/gamma,
 // zeroing, repulsion): under a busy serving loop every launch waits for
 // free compute units.
 // ---------------------------------------------------------------------------
@@ -107,11 +107,11 @@ __global__ void __launch_bounds__(256) k_integrals(xtb_batch b, xtb_params par,
     __shared__ double s_alpha[XTB_MAX_US_LDS * XTB_MAXPRIM];
     __shared__ double s_coeff[XTB_MAX_US_LDS * XTB_MAXPRIM];
     __shared__ double s_cn[32];
-    if ((int)blockIdx.x >= b.ntile_sh) {
-        repulsion_molecule(b, par, pos, out, blockIdx.x - b.ntile_sh, s_cn);
+    if ((int)blockIdx.x < b.nmol) {
+        repulsion_molecule<256>(b, par, pos, out, blockIdx.x, s_cn);
         return;
     }
-    const int* tl = b.tile_sh + 3 * blockIdx.x;
+    const int* tl = b.tile_sh + 3 * (blockIdx.x - b.nmol);
     const int m = tl[0], i0 = tl[1], j0 = tl[2];
     const int nsh = b.mol_nsh[m];
     const int sh0 = b.mol_sh0[m], at0 = b.mol_atom0[m];
