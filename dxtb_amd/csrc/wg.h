@@ -1127,8 +1127,9 @@ __device__ __forceinline__ double row_down(double v, double last) { return dpp64
 // two of the 120 2 x 2 blocks each, and Q stays in registers, 8 columns per
 // row of 16 lanes, its rows moving around the ring by row shifts of the lanes.
 // A round is bound by that chain.  With n = 296 on the whole GPU a subproblem
-// takes 27 us; looking up a schedule, packed triangle indices and Q's rows in
-// LDS took 62 us.
+// takes 22 us, 4 of them saved by staging with all loads in flight; looking up
+// a schedule, packed triangle indices and Q's rows in LDS took 62 us.  (Q's
+// update a round late, to fill the rotation's latency, changed nothing.)
 __device__ __noinline__ int wave_jacobi_sub(ldsf* D, ldsf* cs, glbf* qg, double tol, int max_sweeps, int mode,
                                             unsigned lo_mask, unsigned hi_mask) {
     constexpr int K = JB, m = JS - 1, E = K * JW;
@@ -1253,25 +1254,40 @@ __device__ __noinline__ int wave_jacobi_sub(ldsf* D, ldsf* cs, glbf* qg, double 
 // read): staged into D (slots beyond n zero), and its diagonalised form
 // written back (every element).
 __device__ inline void sub_stage(const glbf* A, int n, int I, int J, ldsf* D) {
-    const int lane = threadIdx.x % WAVE;
+    const int lane = threadIdx.x % WAVE, j = lane % JS, i0 = lane / JS;
     const Ring G{D, JS, JS - 1, JB, JW};
-    for (int e = lane; e < JS * JS; e += WAVE) {
-        const int i = e / JS, j = e % JS;
-        if (j < i) continue;
-        const int gi = slot_index(I, J, i, n), gj = slot_index(I, J, j, n);
-        double v = 0.0;
-        if (gi >= 0 && gj >= 0) v = A[(size_t)(gi < gj ? gi : gj) * n + (gi < gj ? gj : gi)];
-        D[i == j ? G.diag(i) : G.at(i, j)] = v;
+    const int gj = slot_index(I, J, j, n);
+    // all loads in flight (clamped, without branches), then all stores
+    double v[JS / 2];
+#pragma unroll
+    for (int u = 0; u < JS / 2; ++u) {
+        const int gi = slot_index(I, J, i0 + 2 * u, n);
+        const int a = gi < 0 ? 0 : gi, b = gj < 0 ? 0 : gj;
+        v[u] = A[(uint32_t)(a < b ? a : b) * (uint32_t)n + (uint32_t)(a < b ? b : a)];
+        if (gi < 0 || gj < 0) v[u] = 0.0;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < JS / 2; ++u) {
+        const int i = i0 + 2 * u;
+        if (i <= j) D[i == j ? G.diag(i) : G.at(i, j)] = v[u];
     }
     wave_sync();
 }
 __device__ inline void sub_unstage(glbf* A, int n, int I, int J, ldsf* D) {
-    const int lane = threadIdx.x % WAVE;
+    const int lane = threadIdx.x % WAVE, j = lane % JS, i0 = lane / JS;
     const Ring G{D, JS, JS - 1, JB, JW};
-    for (int e = lane; e < JS * JS; e += WAVE) {
-        const int i = e / JS, j = e % JS;
-        const int gi = slot_index(I, J, i, n), gj = slot_index(I, J, j, n);
-        if (gi >= 0 && gj >= 0) A[(size_t)gi * n + gj] = D[i == j ? G.diag(i) : G.at(i, j)];
+    const int gj = slot_index(I, J, j, n);
+    double v[JS / 2];
+#pragma unroll
+    for (int u = 0; u < JS / 2; ++u) {
+        const int i = i0 + 2 * u;
+        v[u] = D[i == j ? G.diag(i) : G.at(i, j)];
+    }
+#pragma unroll
+    for (int u = 0; u < JS / 2; ++u) {
+        const int gi = slot_index(I, J, i0 + 2 * u, n);
+        if (gi >= 0 && gj >= 0) A[(uint32_t)gi * (uint32_t)n + (uint32_t)gj] = v[u];
     }
 }
 
