@@ -290,7 +290,7 @@ __device__ __noinline__ bool anderson(Mixer& mixer, int n, int stride, ldsf* red
             pj[t] = rhs[t] ? f0 : Fh(h + e);
             s[t] = 0.0;
         }
-#pragma unroll 2
+#pragma unroll 4
         for (int i = ln; i < n; i += WAVE) {
             const double fi = f0[i];
 #pragma unroll

@@ -46,7 +46,7 @@ struct Mol {
 struct Shared {
     ldsf *red, *cs, *skey, *ev, *ftot, *qsh, *vsh, *gq, *qat, *big;
     ldsi* sidx;
-    int npow, big_cap;
+    int big_cap;
     ldsf* tacc;  // stage timers (thread 0)
 };
 
@@ -870,7 +870,7 @@ __device__ __noinline__ int scf_step(ldsf* ctx, const glbf* vin, glbf* vout, int
     // an intermediate step's eigensolve that ran out of sweeps only slows
     // the SCF down; the final step's results would be unreliable
     if (sw < 0 && final_step) *status |= XTB_MOL_JACOBI;
-    wg_sort(sh.ev, sh.skey, sh.sidx, n, sh.npow);
+    wg_sort(sh.ev, sh.skey, sh.sidx, n);
     // Fermi occupations.  ef[2]: the largest f (1 - f).  Above ~1e-6 some
     // levels lie within ~14 kT of the Fermi level, where the density depends
     // on rotations among near-degenerate orbitals of different occupation:

@@ -1550,58 +1550,53 @@ struct RowsGlobal {
     __device__ inline glbf& at(int k, int mu) const { return a[(size_t)k * ld + mu]; }
 };
 
-// Ascending sort of the n keys src[0..n): key[r] = src[idx[r]], in LDS of
-// npow entries each (npow: the next power of two).  src may be key itself.
+// Ascending sort of the n <= 2 NT keys src[0..n): key[r] = src[idx[r]], in LDS
+// of n entries each.  src may be key itself.
 //
-// Up to a key per thread each thread counts the keys below its own (equal
-// ones in index order, NaN as +inf): n LDS broadcasts and two barriers, ~1 us
-// at n = 128 and 3 us at 300, where the bitonic network below, a barrier per
-// stage (28 and 45), takes 3 and 5 us.  It stays for the larger n.
+// Each thread counts the keys below its own (equal ones in index order, NaN
+// as +inf): n LDS broadcasts and four barriers, ~1 us at n = 128 and 3 us at
+// 300, where a bitonic network, a barrier per stage (28 and 45), took 3 and 5
+// us.
 template <class Src>
-__device__ inline void wg_sort(Src src, ldsf* key, ldsi* idx, int n, int npow) {
-    if (n <= NT) {
-        const int j = threadIdx.x, b0 = j - j % WAVE, b1 = b0 + WAVE < n ? b0 + WAVE : n;
-        const double v = j < n ? src[j] : 0.0, e = v == v ? v : INFINITY;
-        __syncthreads();
-        if (j < n) key[j] = e;
-        __syncthreads();
-        int rank = 0;
-        if (b0 < n) {
-#pragma unroll 8
-            for (int i = 0; i < b0; ++i) rank += key[i] <= e;
-#pragma unroll 8
-            for (int i = b0; i < b1; ++i) rank += i < j ? key[i] <= e : key[i] < e;
-#pragma unroll 8
-            for (int i = b1; i < n; ++i) rank += key[i] < e;
-        }
-        __syncthreads();
-        if (j < n) {
-            key[rank] = v;
-            idx[rank] = j;
-        }
-        __syncthreads();
-        return;
-    }
-    for (int j = threadIdx.x; j < npow; j += NT) {
-        key[j] = j < n ? src[j] : INFINITY;
-        idx[j] = j;
+__device__ inline void wg_sort(Src src, ldsf* key, ldsi* idx, int n) {
+    constexpr int Q = 2;
+    double v[Q], e[Q];
+    int rank[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int j = threadIdx.x + NT * q;
+        v[q] = j < n ? src[j] : 0.0;
+        e[q] = v[q] == v[q] ? v[q] : INFINITY;
+        rank[q] = 0;
     }
     __syncthreads();
-    for (int size = 2; size <= npow; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int t = threadIdx.x; t < npow / 2; t += NT) {
-                const int lo = 2 * t - (t & (stride - 1));
-                const int hi = lo + stride;
-                const bool up = ((lo & size) == 0);
-                const double a = key[lo], b = key[hi];
-                if ((a > b) == up) {
-                    key[lo] = b; key[hi] = a;
-                    const int ti = idx[lo]; idx[lo] = idx[hi]; idx[hi] = ti;
-                }
-            }
-            __syncthreads();
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int j = threadIdx.x + NT * q;
+        if (j < n) key[j] = e[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int j = threadIdx.x + NT * q, b0 = j - j % WAVE, b1 = b0 + WAVE < n ? b0 + WAVE : n;
+        if (b0 >= n) continue;
+#pragma unroll 8
+        for (int i = 0; i < b0; ++i) rank[q] += key[i] <= e[q];
+#pragma unroll 8
+        for (int i = b0; i < b1; ++i) rank[q] += i < j ? key[i] <= e[q] : key[i] < e[q];
+#pragma unroll 8
+        for (int i = b1; i < n; ++i) rank[q] += key[i] < e[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const int j = threadIdx.x + NT * q;
+        if (j < n) {
+            key[rank[q]] = v[q];
+            idx[rank[q]] = j;
         }
     }
+    __syncthreads();
 }
 
 }  // namespace xtb
