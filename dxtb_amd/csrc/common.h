@@ -101,31 +101,6 @@ __device__ inline void shell_overlap_t(int npi, const double* ai, const double* 
     }
 }
 
-// Runtime-l form of shell_overlap_t: S and dS are [3][3] (only the leading
-// (2 li + 1) x (2 lj + 1) part is written; the rest is zero).
-template <bool GRAD>
-__device__ inline void shell_overlap(int li, int lj, int npi, const double* ai, const double* ci,
-                                     int npj, const double* aj, const double* cj,
-                                     const double R[3], double S[3][3], double dS[3][3][3]) {
-    for (int x = 0; x < 3; ++x)
-        for (int y = 0; y < 3; ++y) {
-            S[x][y] = 0.0;
-            if (GRAD)
-                for (int k = 0; k < 3; ++k) dS[k][x][y] = 0.0;
-        }
-    dispatch_l(li, lj, [&](auto LIc, auto LJc) {
-        constexpr int LI = decltype(LIc)::value, LJ = decltype(LJc)::value;
-        double s[2 * LI + 1][2 * LJ + 1], ds[3][2 * LI + 1][2 * LJ + 1];
-        shell_overlap_t<GRAD, LI, LJ>(npi, ai, ci, npj, aj, cj, R, s, ds);
-        for (int x = 0; x < 2 * LI + 1; ++x)
-            for (int y = 0; y < 2 * LJ + 1; ++y) {
-                S[x][y] = s[x][y];
-                if (GRAD)
-                    for (int k = 0; k < 3; ++k) dS[k][x][y] = ds[k][x][y];
-            }
-    });
-}
-
 // Distance polynomial Pi(R) = (1 + k_i sqrt(R/Rab)) (1 + k_j sqrt(R/Rab))
 // and (dPi/dR)/R; xtb/base.py:298-312, xtb/gfn1.py:333-345 upstream.
 __device__ inline void dist_poly(double dist, double rab, double ki, double kj, double& pi,

@@ -198,7 +198,11 @@ __global__ void __launch_bounds__(256) k_pgrad_atoms(xtb_batch b, xtb_params par
 // overlaps with the shells' primitives rebuilt at zeta +- h on the host
 // (the tables (alpha, c)+-; `mask` marks the unique shells they change: the
 // shell itself and a shell orthogonalised against it).  One thread per
-// atom pair A < B of a 16 x 16 tile; result to column `col` of `out`.
+// atom pair A < B of a 16 x 16 tile and quarter of its shell pairs (blockIdx.y:
+// even and odd shells of either atom); result to column `col` of `out`.
+// Bound by the latency of a thread's primitive loops: 90 us a launch for 64
+// molecules of 2 to 12 carbons, where a thread with all of its pair's shells,
+// their blocks of run-time size in scratch memory, took 160.
 __global__ void __launch_bounds__(256) k_pgrad_basis(xtb_batch b, xtb_params par,
                                                      const double* __restrict__ ap,
                                                      const double* __restrict__ cp,
@@ -238,31 +242,37 @@ __global__ void __launch_bounds__(256) k_pgrad_basis(xtb_batch b, xtb_params par
             const double rab = par.sp_rad[b.atom_sp[ga]] + par.sp_rad[b.atom_sp[gb]];
             const int sa0 = b.atom_sh0[ga], nsa = b.atom_nsh[ga];
             const int sb0 = b.atom_sh0[gb], nsb = b.atom_nsh[gb];
-            for (int i = sa0; i < sa0 + nsa; ++i) {
-                const int usi = b.sh_us[sh0 + i];
-                const int li = par.us_l[usi], ni = 2 * li + 1, oi = b.sh_ao[sh0 + i];
+            for (int i = sa0 + (int)(blockIdx.y >> 1); i < sa0 + nsa; i += 2) {
+                const int usi = b.sh_us[sh0 + i], oi = b.sh_ao[sh0 + i];
                 const double hi = par.us_level[usi] - par.us_kcn[usi] * cn[ga];
-                for (int j = sb0; j < sb0 + nsb; ++j) {
-                    const int usj = b.sh_us[sh0 + j];
+                for (int j = sb0 + (int)(blockIdx.y & 1); j < sb0 + nsb; j += 2) {
+                    const int usj = b.sh_us[sh0 + j], oj = b.sh_ao[sh0 + j];
                     if (!(((mask >> usi) | (mask >> usj)) & 1u)) continue;
-                    const int lj = par.us_l[usj], nj = 2 * lj + 1, oj = b.sh_ao[sh0 + j];
                     const double hj = par.us_level[usj] - par.us_kcn[usj] * cn[gb];
-                    double Sp[3][3], Sm[3][3], dummy[3][3][3];
-                    shell_overlap<false>(li, lj, par.us_nprim[usi], s_ap + usi * XTB_MAXPRIM,
-                                         s_cp + usi * XTB_MAXPRIM, par.us_nprim[usj],
-                                         s_ap + usj * XTB_MAXPRIM, s_cp + usj * XTB_MAXPRIM, R, Sp, dummy);
-                    shell_overlap<false>(li, lj, par.us_nprim[usi], s_am + usi * XTB_MAXPRIM,
-                                         s_cm + usi * XTB_MAXPRIM, par.us_nprim[usj],
-                                         s_am + usj * XTB_MAXPRIM, s_cm + usj * XTB_MAXPRIM, R, Sm, dummy);
                     double pi, dpi;
                     dist_poly(dist, rab, par.us_shpoly[usi], par.us_shpoly[usj], pi, dpi);
                     const double ht = 0.5 * (hi + hj) * par.us_K[usi * par.nus + usj] * pi;
-                    for (int x = 0; x < ni; ++x)
-                        for (int y = 0; y < nj; ++y) {
-                            const size_t e = (size_t)(oi + x) * n + (oj + y);
-                            const double sval = 2.0 * (P[e] * ht - W[e]) - P[e] * (v[oi + x] + v[oj + y]);
-                            acc += sval * (Sp[x][y] - Sm[x][y]) * inv2h;
-                        }
+                    dispatch_l(par.us_l[usi], par.us_l[usj], [&](auto LIc, auto LJc) {
+                        constexpr int LI = decltype(LIc)::value, LJ = decltype(LJc)::value;
+                        constexpr int NI = 2 * LI + 1, NJ = 2 * LJ + 1;
+                        double Sp[NI][NJ], Sm[NI][NJ], dummy[3][NI][NJ];
+                        shell_overlap_t<false, LI, LJ>(par.us_nprim[usi], s_ap + usi * XTB_MAXPRIM,
+                                                       s_cp + usi * XTB_MAXPRIM, par.us_nprim[usj],
+                                                       s_ap + usj * XTB_MAXPRIM, s_cp + usj * XTB_MAXPRIM, R, Sp,
+                                                       dummy);
+                        shell_overlap_t<false, LI, LJ>(par.us_nprim[usi], s_am + usi * XTB_MAXPRIM,
+                                                       s_cm + usi * XTB_MAXPRIM, par.us_nprim[usj],
+                                                       s_am + usj * XTB_MAXPRIM, s_cm + usj * XTB_MAXPRIM, R, Sm,
+                                                       dummy);
+#pragma unroll
+                        for (int x = 0; x < NI; ++x)
+#pragma unroll
+                            for (int y = 0; y < NJ; ++y) {
+                                const size_t e = (size_t)(oi + x) * n + (oj + y);
+                                const double sval = 2.0 * (P[e] * ht - W[e]) - P[e] * (v[oi + x] + v[oj + y]);
+                                acc += sval * (Sp[x][y] - Sm[x][y]) * inv2h;
+                            }
+                    });
                 }
             }
         }
@@ -315,7 +325,7 @@ extern "C" int32_t xtb_param_grad_basis(const xtb_batch* batch, const xtb_params
     if (!state->P || !state->T || !state->pot) return XTB_EINVAL;
     if (par->nus > PG_MAX_US || batch->nmol <= 0) return XTB_ETOOBIG;
     if (batch->ntile_at > 0)
-        hipLaunchKernelGGL(k_pgrad_basis, dim3(batch->ntile_at), dim3(256), 0, (hipStream_t)stream, *batch,
+        hipLaunchKernelGGL(k_pgrad_basis, dim3(batch->ntile_at, 4), dim3(256), 0, (hipStream_t)stream, *batch,
                            *par, alpha_plus, coeff_plus, alpha_minus, coeff_minus, mask, 0.5 / h,
                            positions, cn, *state, grad, col, ncol);
     return hipGetLastError() == hipSuccess ? XTB_OK : XTB_EHIP;
