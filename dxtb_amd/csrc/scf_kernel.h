@@ -535,35 +535,12 @@ __device__ __noinline__ int pd_step(const ldsf* ctx, int k, double loose, const 
     const int npass = loose > 0.0 ? PD_INEXACT_PASSES : PD_EXACT_PASSES;
     for (int pass = 0; pass < npass; ++pass) {
         if (pass > 0) fock_build(M, vin, d);
-        // T = C F (rows: all, or the occupied ones); A_ov = T_occ C_vir^T
-        gemm<false, false>(rows, d, d, 1.0, Ct, n, M.F, n, 0.0, M.T, n, sh.big);
+        // T = C F (rows: all, or the occupied ones) and the diagonal of T C^T,
+        // the rows' energies; A_ov = T_occ C_vir^T
+        gemm_dot(rows, d, d, Ct, n, M.F, n, M.T, n, Ct, sh.ev, sh.big);
         PD_MARK(sh, 0, tm);
         gemm<false, true>(k, m, d, 1.0, M.T, n, Cv, n, 0.0, Kb, m, sh.big);
         PD_MARK(sh, 1, tm);
-        for (int i0 = w * ROWS_PER_WAVE; i0 < rows; i0 += NWAVE * ROWS_PER_WAVE) {
-            int ii[ROWS_PER_WAVE];
-            double e[ROWS_PER_WAVE];
-#pragma unroll
-            for (int u = 0; u < ROWS_PER_WAVE; ++u) {
-                ii[u] = i0 + u < rows ? i0 + u : rows - 1;
-                e[u] = 0.0;
-            }
-            for (int c = lane; c < d; c += WAVE) {
-                double tv[ROWS_PER_WAVE], cv[ROWS_PER_WAVE];
-#pragma unroll
-                for (int u = 0; u < ROWS_PER_WAVE; ++u) {
-                    tv[u] = M.T[(size_t)ii[u] * n + c];
-                    cv[u] = Ct[(size_t)ii[u] * n + c];
-                }
-#pragma unroll
-                for (int u = 0; u < ROWS_PER_WAVE; ++u) e[u] = fma(tv[u], cv[u], e[u]);
-            }
-#pragma unroll
-            for (int u = 0; u < ROWS_PER_WAVE; ++u) {
-                const double v = wave_sum(e[u]);
-                if (lane == 0 && i0 + u < rows) sh.ev[i0 + u] = v;
-            }
-        }
         for (int a = d + threadIdx.x; a < n; a += NT) sh.ev[a] = 0.0;  // padding
         __syncthreads();
         double dmax = 0.0;

@@ -337,7 +337,7 @@ struct GemmSide {
 // product go to C[i] (0 for i >= nao), from the fragments on and above the
 // diagonal: the row sums of each, and the column sums for the rows of its
 // mirror image, added per row in a fixed order.  A and B must not overlap C.
-enum { GEMM_PLAIN = 0, GEMM_EPI = 1, GEMM_MULL = 2 };
+enum { GEMM_PLAIN = 0, GEMM_EPI = 1, GEMM_MULL = 2, GEMM_DOT = 3 };
 
 struct GemmOut {
     int M, N;
@@ -468,6 +468,43 @@ __device__ __forceinline__ void gemm_wg_tile(const GemmOut& g, int m0, int n0, i
                 x[u][r] = *(const glbf*)((const glbc*)X + ((uint32_t)gm * ldc + (uint32_t)gn * 8u));
             }
     };
+    if constexpr (MODE == GEMM_DOT) {
+        ldsf* rowp = lds;  // [fn][16 fm] row sums of fragment column c
+        ldsf* out = (ldsf*)(uintptr_t)(uint32_t)g.nao;
+        double x[G][4];
+        fetch(g.E1, g.M, g.N, 0, x);
+        __syncthreads();  // every wave has read the last panel
+#pragma unroll
+        for (int t0 = 0; t0 < NF; t0 += G) {
+            if (t0 > 0) fetch(g.E1, g.M, g.N, t0, x);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < G; ++u) {
+                const int t = t0 + u;
+                if (t >= NF || !live(t)) continue;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const bool in = row(t, r) < g.M && col(t) < g.N;
+                    if (in) *(glbf*)((glbc*)g.C + ((uint32_t)row(t, r) * ldc + (uint32_t)col(t) * 8u)) = acc[t][r];
+                    double v = in ? acc[t][r] * x[u][r] : 0.0;
+                    v += dpp64<0x111, 0xf>(0.0, v);
+                    v += dpp64<0x112, 0xf>(0.0, v);
+                    v += dpp64<0x114, 0xf>(0.0, v);
+                    v += dpp64<0x118, 0xf>(0.0, v);
+                    if (li == 15) rowp[fc[t] * 16 * fm + 16 * fr[t] + lg + 4 * r] = v;
+                }
+            }
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < 16 * fm; i += NT) {
+            if (m0 + i >= g.M) continue;
+            double s = n0 > 0 ? out[m0 + i] : 0.0;
+            for (int c = 0; c < fn; ++c) s += rowp[c * 16 * fm + i];
+            out[m0 + i] = s;
+        }
+        __syncthreads();
+        return;
+    }
     if constexpr (MODE == GEMM_MULL) {
         ldsf* rowp = lds;                 // [fn][16 fm] row sums of fragment column c
         ldsf* colp = lds + 16 * fm * fn;  // [4 fm][16 fn] column sums of four rows of fragment row r
@@ -567,7 +604,7 @@ __device__ __noinline__ void wg_gemm(int M, int N, int K, int tile, double alpha
     GemmOut g{M, N, alpha, beta, uniform(C), uniform(ldc), nullptr, nullptr, s1, s2, 0};
     if (MODE != GEMM_PLAIN) g.E1 = uniform(E1);
     if (MODE == GEMM_EPI) g.E2 = uniform(E2);
-    if (MODE == GEMM_MULL) g.nao = uniform(nao);
+    if (MODE == GEMM_MULL || MODE == GEMM_DOT) g.nao = uniform(nao);
     const int fm = tile & 255, fn = (tile >> 8) & 255;
     const bool sym = MODE == GEMM_MULL || (MODE == GEMM_PLAIN && (tile >> 16 & 1));
     const int part = tile >> 17;
@@ -688,6 +725,16 @@ __device__ inline void gemm_epi(int M, int N, int K, const glbf* A, int lda, con
                                 glbf* C, int ldc, const glbf* E1, double s1, const glbf* E2, double s2,
                                 ldsf* lds) {
     gemm_run<false, false, GEMM_EPI>(M, N, K, 1.0, A, lda, B, ldb, 0.0, C, ldc, lds, false, E1, E2, s1, s2, 0);
+}
+
+// C = A B and, with X of C's shape and leading dimension, the diagonal of C
+// X^T: out[i] = sum_j C_ij X_ij (LDS).  A B is not thin (K, N >= 2).  A pass of
+// its own over C and X took 5 us of a step's 68 at n = 68, 43 at n = 289 with
+// all CUs at it; in the product 2 and 15 more.
+__device__ inline void gemm_dot(int M, int N, int K, const glbf* A, int lda, const glbf* B, int ldb, glbf* C, int ldc,
+                                const glbf* X, ldsf* out, ldsf* lds) {
+    gemm_run<false, false, GEMM_DOT>(M, N, K, 1.0, A, lda, B, ldb, 0.0, C, ldc, lds, false, X, nullptr, 0.0, 0.0,
+                                     (int)(uint32_t)(uintptr_t)out);
 }
 
 // C (n x n) = alpha op(A) op(B) for a product known to be symmetric
