@@ -183,38 +183,55 @@ __device__ inline void repulsion_molecule(const xtb_batch& b, const xtb_params& 
     double e[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) e[q] = 0.0;
-    for (long p0 = threadIdx.x; p0 < np; p0 += REP_LANES) {
+    // atoms of pair p: row A of the upper triangle holds it (row A starts at A
+    // (2 na - A - 1) / 2)
+    auto atoms = [&](long p, int& ga, int& gb) {
+        int A = (int)((2.0 * na - 1.0 - sqrt((2.0 * na - 1.0) * (2.0 * na - 1.0) - 8.0 * (double)p)) * 0.5);
+        if (A < 0) A = 0;
+        while (A > 0 && (long)A * (2 * na - A - 1) / 2 > p) --A;
+        while ((long)(A + 1) * (2 * na - A - 2) / 2 <= p) ++A;
+        ga = a0 + A;
+        gb = a0 + A + 1 + (int)(p - (long)A * (2 * na - A - 1) / 2);
+    };
+    auto distance = [&](int ga, int gb) {
+        const double dx = pos[3 * ga] - pos[3 * gb], dy = pos[3 * ga + 1] - pos[3 * gb + 1],
+                     dz = pos[3 * ga + 2] - pos[3 * gb + 2];
+        return sqrt(dx * dx + dy * dy + dz * dz);
+    };
+    auto energy = [&](int ga, int gb, double r) {
+        const int sa = b.atom_sp[ga], sb = b.atom_sp[gb];
+        const double alpha = sqrt(par.sp_arep[sa] * par.sp_arep[sb] + 2.2250738585072014e-308);
+        return par.sp_zeff[sa] * par.sp_zeff[sb] * exp(-alpha * pow(r, par.kexp)) / r;
+    };
+    long p0 = threadIdx.x;
+    for (; p0 - threadIdx.x + REP_LANES <= np; p0 += REP_LANES) {
         double r[Q];
         int ga[Q], gb[Q];
-        bool near[Q], any = false;
+        bool any = false;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) atoms(p0 + (long)T * q, ga[q], gb[q]);
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            const long p = p0 + (long)T * q < np ? p0 + (long)T * q : np - 1;
-            // row A of the upper triangle holding pair index p (row A starts at
-            // A (2 na - A - 1) / 2)
-            int A = (int)((2.0 * na - 1.0 - sqrt((2.0 * na - 1.0) * (2.0 * na - 1.0) - 8.0 * (double)p)) * 0.5);
-            if (A < 0) A = 0;
-            while (A > 0 && (long)A * (2 * na - A - 1) / 2 > p) --A;
-            while ((long)(A + 1) * (2 * na - A - 2) / 2 <= p) ++A;
-            ga[q] = a0 + A;
-            gb[q] = a0 + A + 1 + (int)(p - (long)A * (2 * na - A - 1) / 2);
-        }
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            const double dx = pos[3 * ga[q]] - pos[3 * gb[q]], dy = pos[3 * ga[q] + 1] - pos[3 * gb[q] + 1],
-                         dz = pos[3 * ga[q] + 2] - pos[3 * gb[q] + 2];
-            r[q] = sqrt(dx * dx + dy * dy + dz * dz);
-            near[q] = p0 + (long)T * q < np && r[q] <= par.rep_cutoff;
-            any = any || near[q];
+            r[q] = distance(ga[q], gb[q]);
+            any = any || r[q] <= par.rep_cutoff;
         }
         if (!any) continue;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            const int sa = b.atom_sp[ga[q]], sb = b.atom_sp[gb[q]];
-            const double alpha = sqrt(par.sp_arep[sa] * par.sp_arep[sb] + 2.2250738585072014e-308);
-            const double v = par.sp_zeff[sa] * par.sp_zeff[sb] * exp(-alpha * pow(r[q], par.kexp)) / r[q];
-            if (near[q]) e[q] += v;
+            const double v = energy(ga[q], gb[q], r[q]);
+            if (r[q] <= par.rep_cutoff) e[q] += v;
         }
+    }
+    // the rest, fewer than REP_LANES
+#pragma unroll 1
+    for (int q = 0; q < Q && p0 + (long)T * q < np; ++q) {
+        int ga, gb;
+        atoms(p0 + (long)T * q, ga, gb);
+        const double r = distance(ga, gb);
+        const double v = r <= par.rep_cutoff ? energy(ga, gb, r) : 0.0;
+#pragma unroll
+        for (int x = 0; x < Q; ++x)
+            if (x == q) e[x] += v;
     }
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
