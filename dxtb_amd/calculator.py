@@ -50,8 +50,10 @@ _DISP_WARNED = False
 # GPU (xtb_scf_large); batches use the per-molecule kernel, except for their
 # molecules above its limit (WG_MAX_N orbitals), which take the whole GPU
 # one after the other.  Energy + forces of one molecule alone at a 1e-10
-# threshold, one CU / whole GPU: n = 100: 5.6 / 6.8 ms, 154: 15.0 / 9.0,
-# 236: 19.9 / 11.5, 350: 53 / 16, 460: 99 / 18 (chains; water clusters alike)
+# threshold, one CU / whole GPU: n = 92: 3.0 / 2.9 ms, 124: 4.2 / 2.8, 140:
+# 5.6 / 3.1, 186: 9.5 / 3.5, 348: 34 / 5.1, 468: 73 / 6.8 (chains).  The line
+# lies above the crossing: the paths order their first rotations differently,
+# which at the default threshold moves forces by ~1e-6 Eh/bohr.
 LARGE_N = 128
 
 
