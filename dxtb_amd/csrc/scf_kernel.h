@@ -283,8 +283,8 @@ __device__ __noinline__ int ortho_setup(const ldsf* ctx, int* status) {
 // X = S^-1/2 does (eigenpairs of the generalised problem do not depend on the
 // choice), at about n^3 flops instead of Newton-Schulz's ~10 x 6 n^3.
 // Blocked right-looking factorisation with 32-wide panels in T (lower
-// triangle): each diagonal block is factored and inverted by one wave in
-// LDS; the panel below (x D^T = b, i.e. x = b D^-T) and the trailing update
+// triangle): each diagonal block is factored and inverted by one wave
+// (chol_block); the panel below (x D^T = b, i.e. x = b D^-T) and the trailing update
 // are matrix-core GEMMs.  X follows by block forward substitution L X = I:
 // X_i = D_i^-1 (E_i - L_i,<i X_<i), again with GEMMs.  A block padded beyond
 // n is the identity.  Scratch: F (up to 32 x n, or mt x 32 with stride n),
