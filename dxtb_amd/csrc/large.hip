@@ -26,6 +26,7 @@
 // Upstream runs the same SCF (src/dxtb/_src/scf/unrolling/default.py:71-140)
 // with LAPACK's eigh per step (scf/unrolling/base.py:142-175).
 #include <chrono>
+#include <mutex>
 #include <vector>
 
 #include "scf_core.h"
@@ -878,24 +879,47 @@ Layout make_layout(int n, int nsh, int nat) {
 // workgroup's LDS
 constexpr int LARGE_MAX_N = 8192;
 
-// The calling thread's Box (a call uses it from start to end, so one per
-// thread is enough), kept until the thread ends.
+// Boxes lent to calls, one each from start to end (a call returns only when
+// nothing can post to its box any more).  At most MAILS_KEPT idle ones stay
+// for later calls: allocating pinned memory synchronises the whole device,
+// which other streams' work would feel at every call.
 struct Mail {
-    Box* box = nullptr;
-    unsigned long long seq = 0;  // of the last post asked for
+    Box* box;
+    unsigned long long seq;  // of the last post asked for
+};
+constexpr size_t MAILS_KEPT = 16;
+std::mutex mails_mutex;
+Mail mails_idle[MAILS_KEPT];
+size_t mails_count = 0;
+
+struct MailLease {
+    Mail mail{nullptr, 0};
     hipError_t open() {
-        if (box) return hipSuccess;
-        const hipError_t e = hipHostMalloc((void**)&box, sizeof(Box),
+        {
+            std::lock_guard<std::mutex> lock(mails_mutex);
+            if (mails_count > 0) {
+                mail = mails_idle[--mails_count];
+                return hipSuccess;
+            }
+        }
+        const hipError_t e = hipHostMalloc((void**)&mail.box, sizeof(Box),
                                            hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);
-        if (e == hipSuccess) box->seq = 0;
-        else box = nullptr;
+        if (e == hipSuccess) mail.box->seq = 0;
+        else mail.box = nullptr;
         return e;
     }
-    ~Mail() {
-        if (box) (void)hipHostFree(box);
+    ~MailLease() {
+        if (!mail.box) return;
+        {
+            std::lock_guard<std::mutex> lock(mails_mutex);
+            if (mails_count < MAILS_KEPT) {
+                mails_idle[mails_count++] = mail;
+                return;
+            }
+        }
+        (void)hipHostFree(mail.box);
     }
 };
-thread_local Mail thread_mail;
 
 struct Ctx {
     hipStream_t s;
@@ -1461,8 +1485,9 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
     const double tstart = now_s();
     Ctx c;
     c.s = (hipStream_t)stream;
-    c.mail = &thread_mail;
-    if (c.mail->open() != hipSuccess) return XTB_EHIP;
+    MailLease lease;
+    if (lease.open() != hipSuccess) return XTB_EHIP;
+    c.mail = &lease.mail;
     c.b = batch;
     c.par = par;
     c.o = *opts;
@@ -1518,7 +1543,7 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
         rec.v[slot] = v;
         rec.mask |= 1u << slot;
     };
-    // nothing may post to this thread's box after the call
+    // nothing may post to the lent box after the call
     auto fail = [&]() {
         (void)hipStreamSynchronize(c.s);
         return XTB_EHIP;

@@ -1,5 +1,5 @@
-"""The whole-GPU path's control values come back through memory of the calling
-thread: calls from several threads and streams at once, and one after another
+"""The whole-GPU path's control values come back through host memory lent to
+each call: calls from several threads and streams at once, and one after another
 on changing streams, give what a single call gives."""
 
 import threading
