@@ -1164,6 +1164,15 @@ __device__ inline int slot_index(int I, int J, int i, int n) {
 __device__ __forceinline__ double row_up(double v, double first) { return dpp64<0x111, 0xf>(first, v); }
 __device__ __forceinline__ double row_down(double v, double last) { return dpp64<0x101, 0xf>(last, v); }
 
+// One element of the rows top and bottom of Q^T at position k, rotated, then
+// the rows move on around the ring
+__device__ __forceinline__ void sub_rotate(double c, double s, int k, double& top, double& bot) {
+    const double t = c * top - s * bot, e = s * top + c * bot;
+    const double up = row_down(t, e);
+    bot = row_up(e, up);
+    top = k == 0 ? t : up;
+}
+
 // Cyclic Jacobi on a 32 x 32 subproblem by one wavefront, in place on its ring
 // storage D (pitch JW; zero rows and columns are never rotated).  The
 // rotations Q, D_final = Q^T D_0 Q, go to qg (Q[i][j] at qg[i JS + j]) if any
@@ -1174,9 +1183,13 @@ __device__ __forceinline__ double row_down(double v, double last) { return dpp64
 // two of the 120 2 x 2 blocks each, and Q stays in registers, 8 columns per
 // row of 16 lanes, its rows moving around the ring by row shifts of the lanes.
 // A round is bound by that chain.  With n = 296 on the whole GPU a subproblem
-// takes 22 us, 4 of them saved by staging with all loads in flight; looking up
-// a schedule, packed triangle indices and Q's rows in LDS took 62 us.  (Q's
-// update a round late, to fill the rotation's latency, changed nothing.)
+// took 22 us so, 4 of them saved by staging with all loads in flight; looking
+// up a schedule, packed triangle indices and Q's rows in LDS took 62 us.  (Q's
+// update a round late, to fill the rotation's latency, changed nothing; left
+// to four waves after the sweep, as on the whole GPU, it comes to 19 us.)
+// With LATER, Q is left to sub_rotations: the rotations of round r go to cs +
+// 2 K r (max_sweeps = 1 then).
+template <bool LATER>
 __device__ __noinline__ int wave_jacobi_sub(ldsf* D, ldsf* cs, glbf* qg, double tol, int max_sweeps, int mode,
                                             unsigned lo_mask, unsigned hi_mask) {
     constexpr int K = JB, m = JS - 1, E = K * JW;
@@ -1250,25 +1263,21 @@ __device__ __noinline__ int wave_jacobi_sub(ldsf* D, ldsf* cs, glbf* qg, double 
             }
             if (lane < K) {
                 const v2d v = {c, s};
-                *(ldsv2*)(cs + 2 * k) = v;
+                *(ldsv2*)(cs + 2 * k + (LATER ? 2 * K * r : 0)) = v;
             }
             wave_sync();
             v2d vp[2], vr[2];
             double x[2][4];
 #pragma unroll
             for (int g = 0; g < 2; ++g) {
-                vp[g] = *(ldsv2*)cp[g];
-                vr[g] = *(ldsv2*)cr[g];
+                vp[g] = *(ldsv2*)(cp[g] + (LATER ? 2 * K * r : 0));
+                vr[g] = *(ldsv2*)(cr[g] + (LATER ? 2 * K * r : 0));
 #pragma unroll
                 for (int u = 0; u < 4; ++u) x[g][u] = *ad[g][u];
             }
+            if (!LATER) {
 #pragma unroll
-            for (int y = 0; y < 8; ++y) {
-                const double a = top[y], b = bot[y];
-                const double t = c * a - s * b, e = s * a + c * b;
-                const double up = row_down(t, e);
-                bot[y] = row_up(e, up);
-                top[y] = k == 0 ? t : up;
+                for (int y = 0; y < 8; ++y) sub_rotate(c, s, k, top[y], bot[y]);
             }
 #pragma unroll
             for (int g = 0; g < 2; ++g) {
@@ -1287,7 +1296,7 @@ __device__ __noinline__ int wave_jacobi_sub(ldsf* D, ldsf* cs, glbf* qg, double 
             wave_sync();
         }
     }
-    if (rotated) {
+    if (!LATER && rotated) {
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
             qg[(g0 + c) * JS + rt] = top[c];
@@ -1300,40 +1309,45 @@ __device__ __noinline__ int wave_jacobi_sub(ldsf* D, ldsf* cs, glbf* qg, double 
 // The subproblem of block pair (I, J) of A (full, global, upper triangle
 // read): staged into D (slots beyond n zero), and its diagonalised form
 // written back (every element).
+// By NW waves; with several the caller has a barrier after (before) it.
+template <int NW>
 __device__ inline void sub_stage(const glbf* A, int n, int I, int J, ldsf* D) {
-    const int lane = threadIdx.x % WAVE, j = lane % JS, i0 = lane / JS;
+    const int t = threadIdx.x % (WAVE * NW), j = t % JS, i0 = t / JS;
+    constexpr int U = JS / (2 * NW);
     const Ring G{D, JS, JS - 1, JB, JW};
     const int gj = slot_index(I, J, j, n);
     // all loads in flight (clamped, without branches), then all stores
-    double v[JS / 2];
+    double v[U];
 #pragma unroll
-    for (int u = 0; u < JS / 2; ++u) {
-        const int gi = slot_index(I, J, i0 + 2 * u, n);
+    for (int u = 0; u < U; ++u) {
+        const int gi = slot_index(I, J, i0 + 2 * NW * u, n);
         const int a = gi < 0 ? 0 : gi, b = gj < 0 ? 0 : gj;
         v[u] = A[(uint32_t)(a < b ? a : b) * (uint32_t)n + (uint32_t)(a < b ? b : a)];
         if (gi < 0 || gj < 0) v[u] = 0.0;
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < JS / 2; ++u) {
-        const int i = i0 + 2 * u;
+    for (int u = 0; u < U; ++u) {
+        const int i = i0 + 2 * NW * u;
         if (i <= j) D[i == j ? G.diag(i) : G.at(i, j)] = v[u];
     }
     wave_sync();
 }
+template <int NW>
 __device__ inline void sub_unstage(glbf* A, int n, int I, int J, ldsf* D) {
-    const int lane = threadIdx.x % WAVE, j = lane % JS, i0 = lane / JS;
+    const int t = threadIdx.x % (WAVE * NW), j = t % JS, i0 = t / JS;
+    constexpr int U = JS / (2 * NW);
     const Ring G{D, JS, JS - 1, JB, JW};
     const int gj = slot_index(I, J, j, n);
-    double v[JS / 2];
+    double v[U];
 #pragma unroll
-    for (int u = 0; u < JS / 2; ++u) {
-        const int i = i0 + 2 * u;
+    for (int u = 0; u < U; ++u) {
+        const int i = i0 + 2 * NW * u;
         v[u] = D[i == j ? G.diag(i) : G.at(i, j)];
     }
 #pragma unroll
-    for (int u = 0; u < JS / 2; ++u) {
-        const int gi = slot_index(I, J, i0 + 2 * u, n);
+    for (int u = 0; u < U; ++u) {
+        const int gi = slot_index(I, J, i0 + 2 * NW * u, n);
         if (gi >= 0 && gj >= 0) A[(uint32_t)gi * (uint32_t)n + (uint32_t)gj] = v[u];
     }
 }
@@ -1546,11 +1560,11 @@ __device__ __noinline__ int wg_block_jacobi(glbf* A, int n, CAcc Ct, int ncol, i
                         continue;
                     }
                 }
-                sub_stage(A, n, I, J, D);
+                sub_stage<1>(A, n, I, J, D);
                 const int rot =
-                    wave_jacobi_sub(D, cs, Qbuf + (size_t)k * JS * JS, tol, inner, mode, lo_mask, hi_mask);
+                    wave_jacobi_sub<false>(D, cs, Qbuf + (size_t)k * JS * JS, tol, inner, mode, lo_mask, hi_mask);
                 if (lane == 0) ident[k] = rot ? 0 : 1;
-                if (rot) sub_unstage(A, n, I, J, D);
+                if (rot) sub_unstage<1>(A, n, I, J, D);
                 wave_sync();
             }
             __syncthreads();
