@@ -969,10 +969,30 @@ __device__ inline double fast_rsq(double x) {
     return fma(fma(-h * y, y, 0.5), y, y);
 }
 
+// 2 x 2 block of the pairs P < R in round 0, the t-th of run d (rows P = d and
+// K - 2 - d of the strict triangle joined into runs of K): its elements (p, a),
+// (p, b), (q, a), (q, b) lie at D[row + col], and col moves on by one a round,
+// around the ring of m.  With one pair only (K = 1) there is no block; the
+// answer is then a place inside D that is read and not written.
+struct RingBlock {
+    int P, R;
+    int row[4], col[4];
+};
+__host__ __device__ constexpr RingBlock ring_block(int K, int W, int d, int t) {
+    const int m = 2 * K - 1, E = K * W;
+    const bool lo = t < K - 1 - d;
+    const int P = lo ? d : (K > 1 ? K - 2 - d : 0), R = lo ? d + 1 + t : t;
+    const int p = P, q = P > 0 ? m - P : 0, a = R, b = R > 0 ? m - R : 0;
+    const int dm = R - P, dp = R + P;
+    const bool fold = dp >= K;
+    const int row = (fold ? m - dp : dp) * W;
+    return {P, R, {P == 0 ? E : dm * W, P == 0 ? E : row, row, dm * W},
+            {P == 0 ? a : p, P == 0 ? b : (fold ? p : b), fold ? a : q, b}};
+}
+
 // The rounds of one sweep on D, every thread holding NB of the K (K - 1) / 2
-// 2 x 2 blocks P < R (rows P and K - 2 - P of the strict triangle joined into
-// runs of K).  A block's four addresses and the rounds in which they wrap
-// around the ring stay in registers.
+// 2 x 2 blocks P < R.  A block's four addresses and the rounds in which they
+// wrap around the ring stay in registers.
 template <int NB>
 __device__ __noinline__ void ring_rounds(ldsf* D, int n, int W, glbf* rot, ldsf* cs, double skip, int mode, int cb_lo,
                                          int cb_hi) {
@@ -987,22 +1007,16 @@ __device__ __noinline__ void ring_rounds(ldsf* D, int n, int W, glbf* rot, ldsf*
 #pragma unroll
     for (int g = 0; g < NB; ++g) {
         const int e0 = threadIdx.x + g * NT, e = e0 < nblk ? e0 : (nblk > 0 ? nblk - 1 : 0);
-        const int d = (int)(((uint32_t)e * inv) >> 22), t = e - d * K;
-        const bool lo = t < K - 1 - d;
-        const int P = lo ? d : K - 2 - d, R = lo ? d + 1 + t : t;
-        const int p = P, q = G.wrap(-P), a = R, b = G.wrap(-R);
-        const int dm = R - P, dp = R + P;
-        const bool fold = dp >= K;
-        const int row = (fold ? m - dp : dp) * W;
-        const int s1 = P == 0 ? b : (fold ? p : b), s2 = fold ? a : q;
-        ad[g][0] = D + (P == 0 ? E + a : dm * W + p);  // (p, a)
-        ad[g][1] = D + ((P == 0 ? E : row) + s1);      // (p, b)
-        ad[g][2] = D + (row + s2);                     // (q, a)
-        ad[g][3] = D + (dm * W + b);                   // (q, b)
-        rw[g] = (uint32_t)(m - 1 - (P == 0 ? a : p)) | (uint32_t)(m - 1 - s1) << 8 | (uint32_t)(m - 1 - s2) << 16 |
-                (uint32_t)(m - 1 - b) << 24;
-        cp[g] = cs + 2 * P;
-        cr[g] = cs + 2 * R;
+        const int d = (int)(((uint32_t)e * inv) >> 22);
+        const RingBlock x = ring_block(K, W, d, e - d * K);
+        rw[g] = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            ad[g][u] = D + x.row[u] + x.col[u];
+            rw[g] |= (uint32_t)(m - 1 - x.col[u]) << (8 * u);
+        }
+        cp[g] = cs + 2 * x.P;
+        cr[g] = cs + 2 * x.R;
     }
     for (int r = 0; r < m; ++r) {
         // rotation parameters, and the pairs' own diagonal blocks: with

@@ -1,0 +1,54 @@
+"""The eigensolvers on matrices at their edges, handed to the SCF entry points
+as H0 with S = 1 and no charge-dependent terms, so that the orbital energies
+are H0's eigenvalues."""
+
+import ctypes as ct
+
+import numpy as np
+import pytest
+import torch
+
+from dxtb_amd import _lib, workloads
+from dxtb_amd.engine import ScfOptions
+from dxtb_amd.large import LargeSystem
+from helpers import run_native
+
+pytestmark = pytest.mark.gpu
+
+
+def _levels(numbers, positions, h0, large=False, **opt):
+    """(orbital energies, status, C) with `h0` in place of the molecule's H0."""
+    if large:
+        ls = LargeSystem(numbers, "cuda:0")
+        ls.run(positions, forces=False)
+        pipe = ls.pipe
+    else:
+        pipe = run_native([(np.asarray(numbers), positions)])
+    n = int(pipe.L.n[0])
+    dev = pipe.device
+    pipe.matrix(pipe.S, 0).copy_(torch.eye(n, dtype=torch.float64, device=dev))
+    pipe.matrix(pipe.H0, 0).copy_(torch.as_tensor(h0, device=dev))
+    pipe.gamma.zero_()
+    par = _lib.XtbParams.from_buffer_copy(pipe.dt.s)
+    gam3 = torch.zeros(int(par.nsp), dtype=torch.float64, device=dev)
+    par.sp_gam3 = gam3.data_ptr()
+    o = ScfOptions(orbital_energies=True, **opt).to_struct(want_w=False, padded=False)
+    args = [ct.byref(pipe.batch), ct.byref(par), pipe.S.data_ptr(), pipe.H0.data_ptr(), pipe.gamma.data_ptr(),
+            ct.byref(o), ct.byref(pipe.state)]
+    s = ct.c_void_p(torch.cuda.current_stream().cuda_stream)
+    if large:
+        _lib.check(pipe.lib.xtb_scf_large(*args, pipe.work.data_ptr(), pipe.work.numel(), s), "xtb_scf_large")
+    else:
+        _lib.check(pipe.lib.xtb_scf(*args, s), "xtb_scf")
+    torch.cuda.synchronize()
+    return (pipe.emo[:n].cpu().numpy(), int(pipe.records()[0, _lib.OUT_STATUS].item()),
+            pipe.matrix(pipe.C, 0).cpu().numpy())
+
+
+def test_two_orbitals():
+    """One pair and no 2 x 2 block: a coupled hydrogen atom."""
+    h = np.array([[-0.4, 0.1], [0.1, -0.2]])
+    e, status, c = _levels([1], np.zeros((1, 3)), h)
+    assert status == 0
+    assert np.abs(e - np.linalg.eigvalsh(h)).max() < 1e-14
+    assert np.abs(c @ c.T - np.eye(2)).max() < 1e-14
