@@ -1271,7 +1271,7 @@ int eig(Ctx& c, double rel_tol, double loose) {
         chk_launch(c);
         finish(c, rb, 1, C_OFF, next_post(c));
         if (!read_ctl(c)) return -1;
-        if (sweep == 0) tol = fmax(rel_tol * fmax(c.h[C_DMAX], 1.0), loose);
+        if (sweep == 0) tol = fmax(fmax(rel_tol * fmax(c.h[C_DMAX], 1.0), loose), JACOBI_TOL_MIN);
         if (c.h[C_OFF] <= tol) break;
         if (sweep >= c.o.jacobi_max_sweeps) {
             sweep = -1;

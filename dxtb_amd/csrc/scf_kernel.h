@@ -191,7 +191,7 @@ __device__ __noinline__ int eig_step(const ldsf* ctx, double loose, int cb_lo, i
     double dmax = 0.0;
     for (int i = threadIdx.x; i < n; i += NT) dmax = fmax(dmax, fabs(M.F[(size_t)i * n + i]));
     dmax = wg_max(dmax, sh.red);
-    const double tol = fmax(rel_tol * fmax(dmax, 1.0), loose);
+    const double tol = fmax(fmax(rel_tol * fmax(dmax, 1.0), loose), JACOBI_TOL_MIN);
     const int npk = n * (n + 1) / 2;
     int sweeps;
     if (npk <= sh.big_cap) {

@@ -954,6 +954,11 @@ __device__ inline void ring_vectors(glbf* Ct, int ldc, int n, int ncol, const gl
 #undef XTB_RV
 }
 
+// Smallest tolerance of a Jacobi eigensolve, whatever is asked for: a pivot is
+// rotated from 1e-3 of it on, so that the sum of squares under the rotation's
+// root stays a normal number.
+constexpr double JACOBI_TOL_MIN = 1e-140;
+
 // 1 / x and 1 / sqrt(x) for normal positive x: the hardware estimates with
 // Newton steps to full precision (the rotations need no correctly rounded
 // division, whose scaling and fix-up steps double the dependent chain)

@@ -52,3 +52,19 @@ def test_two_orbitals():
     assert status == 0
     assert np.abs(e - np.linalg.eigvalsh(h)).max() < 1e-14
     assert np.abs(c @ c.T - np.eye(2)).max() < 1e-14
+
+
+@pytest.mark.parametrize("path", ["lds", "blocks", "whole-gpu"])
+def test_pivots_whose_square_underflows(path):
+    """jacobi_tol = 0 with equal diagonal elements: off-diagonal elements far
+    below 1e-154, whose squares are zero, change no level and no orbital."""
+    z, p = (np.array([1, 1]), np.array([[0.0, 0.0, 0.0], [0.0, 0.0, 1.5]])) if path == "lds" else \
+        workloads.water_cluster(np.random.default_rng(3), 30)
+    n = 4 if path == "lds" else 240
+    h = -0.5 * np.eye(n)
+    for i, j in ((0, 1), (1, n - 1)):
+        h[i, j] = h[j, i] = 1e-200
+    e, status, c = _levels(z, p, h, large=path == "whole-gpu", jacobi_tol=0.0, eig_inexact=0.0)
+    assert status == 0
+    assert np.abs(e + 0.5).max() < 1e-15
+    assert np.abs(c @ c.T - np.eye(n)).max() < 1e-15
