@@ -19,7 +19,7 @@ using namespace xtb;
 extern "C" int32_t xtb_scf_lds_bytes(const xtb_batch* batch, int32_t* bytes, int32_t* big_cap) {
     if (!batch || !bytes || !big_cap) return XTB_EINVAL;
     const Lay L = make_lay(batch->max_n, batch->max_nsh, batch->max_nat);
-    const int budget = 160 * 1024 / 8;
+    const int budget = LDS_DOUBLES;
     const int n = batch->max_n;
     const int want_a = n * (n + 1) / 2;
     const int avail = budget - L.total_fixed;
@@ -29,7 +29,7 @@ extern "C" int32_t xtb_scf_lds_bytes(const xtb_batch* batch, int32_t* bytes, int
         const int ring = ring_doubles(n, ring_pitch(n, avail));
         cap = std::max(cap, std::max(want_a, ring));
     } else {
-        cap = NMIXED_LDS;  // block Jacobi for the largest
+        cap = NMIXED_LDS <= avail ? NMIXED_LDS : NMIXED_LDS_MIN;  // block Jacobi for the largest
     }
     if (L.total_fixed + cap > budget) return XTB_ETOOBIG;
     *big_cap = cap;

@@ -154,13 +154,18 @@ __host__ __device__ inline int next_pow2(int v) {
     return p;
 }
 
+constexpr int LDS_DOUBLES = 160 * 1024 / 8;  // of a CU
+static_assert((RING_MAX_N + 1) * (RING_MAX_N + 2) / 2 > LDS_DOUBLES, "a matrix that fits the LDS fits the rounds");
+
+// (skey and sidx are rounded up to a power of two: between 184 and 202 orbitals
+// the slack is part of the line between the LDS and the block Jacobi)
 __host__ __device__ inline Lay make_lay(int nmax, int max_nsh, int max_nat) {
     Lay L;
     const int npow = next_pow2(nmax < 2 ? 2 : nmax);
     int o = 0;
     L.red = o; o += RED_DOUBLES;
     L.ctx = o; o += CTX_DOUBLES;
-    L.cs = o; o += 3 * (nmax / 2 + 2);
+    L.cs = o; o += 3 * ((nmax < RING_MAX_N ? nmax : RING_MAX_N) / 2 + 2);  // (LDS Jacobi only)
     L.skey = o; o += npow;
     L.sidx = o; o += (npow + 1) / 2;  // ints
     L.ev = o; o += nmax;

@@ -814,12 +814,17 @@ struct Ring {
     __device__ inline int diag(int i) const { return i == m ? K * W + m : i; }
 };
 
+// The largest n that the rounds cover: 10 of the K (K - 1) / 2 2 x 2 blocks for
+// each thread.
+constexpr int RING_MAX_N = 202;
+
 // doubles that Ring needs for n with row pitch W (the row of the fixed index
 // exists for even n only; it is a dummy otherwise)
 __host__ __device__ constexpr int ring_pairs(int n) { return (n + 1) / 2; }
 __host__ __device__ constexpr int ring_doubles(int n, int W) {
     return ring_pairs(n) * W + (n % 2 == 0 ? n : 0);
 }
+static_assert(ring_pairs(RING_MAX_N) * (ring_pairs(RING_MAX_N) - 1) / 2 <= 10 * NT, "ring_rounds<10>");
 // row pitch: the next W = 2 mod 4 if the matrix then fits in cap doubles
 __host__ __device__ inline int ring_pitch(int n, int cap) {
     const int m = 2 * ring_pairs(n) - 1;
@@ -1092,7 +1097,7 @@ __device__ __noinline__ void ring_rounds(ldsf* D, int n, int W, glbf* rot, ldsf*
 }
 
 // Diagonalises the symmetric matrix A (full, global, upper triangle read) of
-// order n <= 256 and applies every rotation to the rows of Ct (Ct[k][mu], row
+// order n <= RING_MAX_N and applies every rotation to the rows of Ct (Ct[k][mu], row
 // k = vector k, mu < ncol), i.e. C <- C J; eigenvalues to `ev`.  `D`: LDS of
 // ring_doubles(n, W); `cs`: 2 K doubles of LDS (16-byte aligned); `rot`:
 // global scratch of n^2 doubles for a sweep's rotations.  Returns the number
@@ -1161,9 +1166,11 @@ constexpr int JD = ring_doubles(JS, JW);
 constexpr int JWAVE_LDS = JD + JS;       // D, (c, s)
 constexpr int NBLOCK_LDS = NWAVE * JWAVE_LDS + 64;  // + flags
 // The LDS share of a launch whose largest matrix does not fit: matrices up to
-// 161 orbitals among its molecules still take the LDS Jacobi.
+// 161 orbitals among its molecules still take the LDS Jacobi.  Where a large
+// molecule's vectors leave less, what its GEMMs and subproblems need will do.
 constexpr int NMIXED_LDS = 13052;
-static_assert(NBLOCK_LDS <= NMIXED_LDS && NGEMM_MFMA_LDS <= NMIXED_LDS, "LDS of the mixed launches");
+constexpr int NMIXED_LDS_MIN = NGEMM_MFMA_LDS > NBLOCK_LDS ? NGEMM_MFMA_LDS : NBLOCK_LDS;
+static_assert(NMIXED_LDS_MIN <= NMIXED_LDS, "LDS of the mixed launches");
 
 __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
