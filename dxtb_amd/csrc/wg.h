@@ -640,6 +640,18 @@ __device__ __noinline__ void wg_gemm_thin(int M, int N, int K, double alpha, con
             for (int j = 0; j < nao && i < nao; ++j) a = fma(dot(i, j), E1[(size_t)i * ldc + j], a);
             C[i] = a;
         }
+    } else if (MODE == GEMM_DOT) {
+        ldsf* out = (ldsf*)(uintptr_t)(uint32_t)nao;
+        for (int i = threadIdx.x; i < M; i += NT) {
+            double a = 0.0;
+            for (int j = 0; j < N; ++j) {
+                const size_t x = (size_t)i * ldc + j;
+                const double d = dot(i, j);
+                C[x] = d;
+                a = fma(d, E1[x], a);
+            }
+            out[i] = a;
+        }
     } else {
         for (int e = threadIdx.x; e < M * N; e += NT) {
             const int i = e / N, j = e - i * N;
@@ -728,9 +740,9 @@ __device__ inline void gemm_epi(int M, int N, int K, const glbf* A, int lda, con
 }
 
 // C = A B and, with X of C's shape and leading dimension, the diagonal of C
-// X^T: out[i] = sum_j C_ij X_ij (LDS).  A B is not thin (K, N >= 2).  A pass of
-// its own over C and X took 5 us of a step's 68 at n = 68, 43 at n = 289 with
-// all CUs at it; in the product 2 and 15 more.
+// X^T: out[i] = sum_j C_ij X_ij (LDS).  A pass of its own over C and X took 5
+// us of a step's 68 at n = 68, 43 at n = 289 with all CUs at it; in the product
+// 2 and 15 more.
 __device__ inline void gemm_dot(int M, int N, int K, const glbf* A, int lda, const glbf* B, int ldb, glbf* C, int ldc,
                                 const glbf* X, ldsf* out, ldsf* lds) {
     gemm_run<false, false, GEMM_DOT>(M, N, K, 1.0, A, lda, B, ldb, 0.0, C, ldc, lds, false, X, nullptr, 0.0, 0.0,
