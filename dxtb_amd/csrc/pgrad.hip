@@ -198,11 +198,16 @@ __global__ void __launch_bounds__(256) k_pgrad_atoms(xtb_batch b, xtb_params par
 // overlaps with the shells' primitives rebuilt at zeta +- h on the host
 // (the tables (alpha, c)+-; `mask` marks the unique shells they change: the
 // shell itself and a shell orthogonalised against it).  One thread per
-// atom pair A < B of a 16 x 16 tile and quarter of its shell pairs (blockIdx.y:
-// even and odd shells of either atom); result to column `col` of `out`.
-// Bound by the latency of a thread's primitive loops: 90 us a launch for 64
-// molecules of 2 to 12 carbons, where a thread with all of its pair's shells,
-// their blocks of run-time size in scratch memory, took 160.
+// atom pair A < B of a 16 x 16 tile and quarter of its shell pairs (even and
+// odd shells of either atom); result to column `col` of `out`.  An
+// off-diagonal tile takes four workgroups (blockIdx.y: the quarter), a diagonal
+// one, with 120 pairs, two, and the only tile of a molecule of up to 16 atoms
+// one, two quarters a thread: such a molecule gets one addition and the same
+// bits on every run.  The sums of larger ones arrive in any order.
+// Bound by the latency of a thread's primitive loops: 92 us a launch for 64
+// molecules of 2 to 12 carbons.  With four workgroups for every tile it takes
+// 89, but then no gradient has the same bits twice; with all shell pairs in a
+// thread, their blocks of run-time size in scratch memory, 160.
 __global__ void __launch_bounds__(256) k_pgrad_basis(xtb_batch b, xtb_params par,
                                                      const double* __restrict__ ap,
                                                      const double* __restrict__ cp,
@@ -223,9 +228,24 @@ __global__ void __launch_bounds__(256) k_pgrad_basis(xtb_batch b, xtb_params par
     __syncthreads();
     const int* tl = b.tile_at + 3 * blockIdx.x;
     const int m = tl[0];
-    const int A = tl[1] + threadIdx.x / 16;
-    const int B = tl[2] + threadIdx.x % 16;
     const int nat = b.mol_nat[m];
+    const bool diag = tl[1] == tl[2], alone = nat <= 16;
+    if (diag && (int)blockIdx.y > (alone ? 0 : 1)) return;
+    int A = threadIdx.x / 16, B = threadIdx.x % 16, q0 = blockIdx.y, q1 = -1;
+    if (diag) {
+        // the 120 pairs row by row, twice: quarters 0 and 3, 1 and 2
+        int p = threadIdx.x % 128;
+        for (A = 0; A < 15 && p >= 15 - A; ++A) p -= 15 - A;
+        B = A < 15 ? A + 1 + p : A;
+        q0 = threadIdx.x / 128;
+        q1 = 3 - q0;
+        if (!alone) {
+            if (blockIdx.y > 0) q0 = q1;
+            q1 = -1;
+        }
+    }
+    A += tl[1];
+    B += tl[2];
     double acc = 0.0;
     if (A < nat && B < nat && B > A) {
         const int n = b.mol_n[m];
@@ -242,37 +262,39 @@ __global__ void __launch_bounds__(256) k_pgrad_basis(xtb_batch b, xtb_params par
             const double rab = par.sp_rad[b.atom_sp[ga]] + par.sp_rad[b.atom_sp[gb]];
             const int sa0 = b.atom_sh0[ga], nsa = b.atom_nsh[ga];
             const int sb0 = b.atom_sh0[gb], nsb = b.atom_nsh[gb];
-            for (int i = sa0 + (int)(blockIdx.y >> 1); i < sa0 + nsa; i += 2) {
-                const int usi = b.sh_us[sh0 + i], oi = b.sh_ao[sh0 + i];
-                const double hi = par.us_level[usi] - par.us_kcn[usi] * cn[ga];
-                for (int j = sb0 + (int)(blockIdx.y & 1); j < sb0 + nsb; j += 2) {
-                    const int usj = b.sh_us[sh0 + j], oj = b.sh_ao[sh0 + j];
-                    if (!(((mask >> usi) | (mask >> usj)) & 1u)) continue;
-                    const double hj = par.us_level[usj] - par.us_kcn[usj] * cn[gb];
-                    double pi, dpi;
-                    dist_poly(dist, rab, par.us_shpoly[usi], par.us_shpoly[usj], pi, dpi);
-                    const double ht = 0.5 * (hi + hj) * par.us_K[usi * par.nus + usj] * pi;
-                    dispatch_l(par.us_l[usi], par.us_l[usj], [&](auto LIc, auto LJc) {
-                        constexpr int LI = decltype(LIc)::value, LJ = decltype(LJc)::value;
-                        constexpr int NI = 2 * LI + 1, NJ = 2 * LJ + 1;
-                        double Sp[NI][NJ], Sm[NI][NJ], dummy[3][NI][NJ];
-                        shell_overlap_t<false, LI, LJ>(par.us_nprim[usi], s_ap + usi * XTB_MAXPRIM,
-                                                       s_cp + usi * XTB_MAXPRIM, par.us_nprim[usj],
-                                                       s_ap + usj * XTB_MAXPRIM, s_cp + usj * XTB_MAXPRIM, R, Sp,
-                                                       dummy);
-                        shell_overlap_t<false, LI, LJ>(par.us_nprim[usi], s_am + usi * XTB_MAXPRIM,
-                                                       s_cm + usi * XTB_MAXPRIM, par.us_nprim[usj],
-                                                       s_am + usj * XTB_MAXPRIM, s_cm + usj * XTB_MAXPRIM, R, Sm,
-                                                       dummy);
+            for (int q = q0; q >= 0; q = q == q0 ? q1 : -1) {
+                for (int i = sa0 + (q >> 1); i < sa0 + nsa; i += 2) {
+                    const int usi = b.sh_us[sh0 + i], oi = b.sh_ao[sh0 + i];
+                    const double hi = par.us_level[usi] - par.us_kcn[usi] * cn[ga];
+                    for (int j = sb0 + (q & 1); j < sb0 + nsb; j += 2) {
+                        const int usj = b.sh_us[sh0 + j], oj = b.sh_ao[sh0 + j];
+                        if (!(((mask >> usi) | (mask >> usj)) & 1u)) continue;
+                        const double hj = par.us_level[usj] - par.us_kcn[usj] * cn[gb];
+                        double pi, dpi;
+                        dist_poly(dist, rab, par.us_shpoly[usi], par.us_shpoly[usj], pi, dpi);
+                        const double ht = 0.5 * (hi + hj) * par.us_K[usi * par.nus + usj] * pi;
+                        dispatch_l(par.us_l[usi], par.us_l[usj], [&](auto LIc, auto LJc) {
+                            constexpr int LI = decltype(LIc)::value, LJ = decltype(LJc)::value;
+                            constexpr int NI = 2 * LI + 1, NJ = 2 * LJ + 1;
+                            double Sp[NI][NJ], Sm[NI][NJ], dummy[3][NI][NJ];
+                            shell_overlap_t<false, LI, LJ>(par.us_nprim[usi], s_ap + usi * XTB_MAXPRIM,
+                                                           s_cp + usi * XTB_MAXPRIM, par.us_nprim[usj],
+                                                           s_ap + usj * XTB_MAXPRIM, s_cp + usj * XTB_MAXPRIM, R, Sp,
+                                                           dummy);
+                            shell_overlap_t<false, LI, LJ>(par.us_nprim[usi], s_am + usi * XTB_MAXPRIM,
+                                                           s_cm + usi * XTB_MAXPRIM, par.us_nprim[usj],
+                                                           s_am + usj * XTB_MAXPRIM, s_cm + usj * XTB_MAXPRIM, R, Sm,
+                                                           dummy);
 #pragma unroll
-                        for (int x = 0; x < NI; ++x)
+                            for (int x = 0; x < NI; ++x)
 #pragma unroll
-                            for (int y = 0; y < NJ; ++y) {
-                                const size_t e = (size_t)(oi + x) * n + (oj + y);
-                                const double sval = 2.0 * (P[e] * ht - W[e]) - P[e] * (v[oi + x] + v[oj + y]);
-                                acc += sval * (Sp[x][y] - Sm[x][y]) * inv2h;
-                            }
-                    });
+                                for (int y = 0; y < NJ; ++y) {
+                                    const size_t e = (size_t)(oi + x) * n + (oj + y);
+                                    const double sval = 2.0 * (P[e] * ht - W[e]) - P[e] * (v[oi + x] + v[oj + y]);
+                                    acc += sval * (Sp[x][y] - Sm[x][y]) * inv2h;
+                                }
+                        });
+                    }
                 }
             }
         }

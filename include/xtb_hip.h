@@ -412,8 +412,10 @@ int32_t xtb_param_grad(const xtb_batch* batch, const xtb_params* par,
  * bit u of `mask` marks the unique shells they change.  Needs P, W (state.T
  * of an xtb_scf with want_w) and the potential of the same batch.  dS/dzeta
  * is the central difference of the contracted overlaps; the contraction with
- * the energy's derivative in S is that of xtb_forces.  Replaces autograd
- * with differentiable "slater" entries (examples/optim/param.py). */
+ * the energy's derivative in S is that of xtb_forces.  Up to 16 atoms the
+ * result has the same bits on every run; the sums of larger molecules are
+ * added in any order.  Replaces autograd with differentiable "slater" entries
+ * (examples/optim/param.py). */
 int32_t xtb_param_grad_basis(const xtb_batch* batch, const xtb_params* par,
                              const double* alpha_plus, const double* coeff_plus,
                              const double* alpha_minus, const double* coeff_minus,
