@@ -720,12 +720,11 @@ __global__ void __launch_bounds__(256) k_scale_rows(int n, const double* X, cons
     }
 }
 
-// A'_ij = (f_i + f_j)/2 A_ij for the k x k occupied block, f of row i =
-// ftot[sidx[i]] (sidx null: ftot[i])
-__global__ void __launch_bounds__(256) k_scale_pairs(int k, double* A, const int* sidx, const double* ftot) {
+// A'_ij = (f_i + f_j)/2 A_ij for the k x k occupied block, f of row i = ftot[i]
+__global__ void __launch_bounds__(256) k_scale_pairs(int k, double* A, const double* ftot) {
     const int i = blockIdx.x;
-    const double fi = ftot[sidx ? sidx[i] : i];
-    for (int j = threadIdx.x; j < k; j += 256) A[(size_t)i * k + j] *= 0.5 * (fi + ftot[sidx ? sidx[j] : j]);
+    const double fi = ftot[i];
+    for (int j = threadIdx.x; j < k; j += 256) A[(size_t)i * k + j] *= 0.5 * (fi + ftot[j]);
 }
 
 // Mulliken (scf/base.py:764-815): q_i = n0_i - (P S)_ii, eorb_i = (P H0)_ii
@@ -1660,7 +1659,7 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
         fock(c, state->vnew);
         gemm_t<false, false, false>(c, k, n, n, 1.0, c.Ct, n, c.F, n, 0.0, c.T, n, false);
         gemm_t<false, true, false>(c, k, k, n, 1.0, c.T, n, c.Ct, n, 0.0, c.F, k, false);
-        hipLaunchKernelGGL(k_scale_pairs, dim3(k), dim3(256), 0, c.s, k, c.F, (const int*)nullptr, c.ftot);
+        hipLaunchKernelGGL(k_scale_pairs, dim3(k), dim3(256), 0, c.s, k, c.F, c.ftot);
         chk_launch(c);
         double* R = c.F + (size_t)k * k;
         gemm_t<false, false, false>(c, k, n, k, 1.0, c.F, k, c.Ct, n, 0.0, R, n, false);

@@ -942,31 +942,18 @@ __device__ __noinline__ int scf_step(ldsf* ctx, const glbf* vin, glbf* vout, int
                 sq[u] = 0.0;
                 se[u] = 0.0;
             }
-            if (last) {
-                for (int j = l; j < M.nao; j += WAVE) {
-                    double pv[ROWS_PER_WAVE], sv[ROWS_PER_WAVE], hv[ROWS_PER_WAVE];
+            for (int j = l; j < M.nao; j += WAVE) {
+                double pv[ROWS_PER_WAVE], sv[ROWS_PER_WAVE], hv[ROWS_PER_WAVE];
 #pragma unroll
-                    for (int u = 0; u < ROWS_PER_WAVE; ++u) {
-                        pv[u] = M.P[(size_t)ii[u] * n + j];
-                        sv[u] = M.S[(size_t)ii[u] * n + j];
-                        hv[u] = M.H0[(size_t)ii[u] * n + j];
-                    }
-#pragma unroll
-                    for (int u = 0; u < ROWS_PER_WAVE; ++u) {
-                        sq[u] = fma(pv[u], sv[u], sq[u]);
-                        se[u] = fma(pv[u], hv[u], se[u]);
-                    }
+                for (int u = 0; u < ROWS_PER_WAVE; ++u) {
+                    pv[u] = M.P[(size_t)ii[u] * n + j];
+                    sv[u] = M.S[(size_t)ii[u] * n + j];
+                    hv[u] = M.H0[(size_t)ii[u] * n + j];
                 }
-            } else {
-                for (int j = l; j < M.nao; j += WAVE) {
-                    double pv[ROWS_PER_WAVE], sv[ROWS_PER_WAVE];
 #pragma unroll
-                    for (int u = 0; u < ROWS_PER_WAVE; ++u) {
-                        pv[u] = M.P[(size_t)ii[u] * n + j];
-                        sv[u] = M.S[(size_t)ii[u] * n + j];
-                    }
-#pragma unroll
-                    for (int u = 0; u < ROWS_PER_WAVE; ++u) sq[u] = fma(pv[u], sv[u], sq[u]);
+                for (int u = 0; u < ROWS_PER_WAVE; ++u) {
+                    sq[u] = fma(pv[u], sv[u], sq[u]);
+                    se[u] = fma(pv[u], hv[u], se[u]);
                 }
             }
 #pragma unroll
