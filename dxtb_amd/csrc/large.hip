@@ -7,16 +7,16 @@
 // stream ordered; a few control scalars come back once or twice per step
 // through host memory that the kernels write (read_ctl):
 //
-//   setup   Loewdin orthogonaliser X = S^-1/2 by the coupled Newton-Schulz
-//           iteration on matrix-core GEMMs; the orbitals start as the rows
-//           of X
+//   setup   Cholesky orthogonaliser X = L^-1, S = L L^T (or Loewdin's S^-1/2
+//           by the coupled Newton-Schulz iteration), on matrix-core GEMMs;
+//           the orbitals start as the rows of X
 //   step    Fock build F = H0 - 1/2 S o (v_i + v_j)  (scf/base.py:817-859)
 //           -> gapped closed shell: perturbative occupied-virtual rotation
-//              of the previous step's orbitals (GEMMs), as in scf.hip
+//              of the previous step's orbitals (GEMMs), as in scf_kernel.h
 //           -> otherwise A = C F C^T and parallel-ordered block Jacobi: one
-//              launch solves the 32 x 32 subproblems of a round (a wave
-//              each), one applies their rotations to A and to the orbitals
-//              on matrix cores
+//              launch solves the 32 x 32 subproblems of a round (a workgroup
+//              of four waves each), one applies their rotations to A and to
+//              the orbitals on matrix cores
 //           -> sort, Fermi smearing (filling.py:201-366), density
 //              P = C^T diag(f) C, Mulliken charges, ES2/ES3 potential,
 //              Anderson mixing (mixer/anderson.py:163-317), all on device
@@ -506,7 +506,7 @@ __global__ void __launch_bounds__(NT) k_dev_identity(int n, const double* T, dou
 
 // ---------------------------------------------------------------------------
 // Cholesky orthogonaliser X = L^-1, S = L L^T (the per-workgroup version is
-// chol_setup in scf.hip), 32-wide panels.  k_chol_diag: one wave factors the
+// chol_setup in scf_kernel.h), 32-wide panels.  k_chol_diag: one wave factors the
 // diagonal block j0 of the lower triangle of L in place and writes its
 // inverse to Dg (nb x nb, leading dimension nb); a non-positive pivot sets
 // ctl[C_ERR].
@@ -533,15 +533,15 @@ __global__ void k_set_slot(double* ctl, int slot, double v) {
 // ---------------------------------------------------------------------------
 // Block Jacobi on the whole GPU (the per-workgroup version is
 // wg_block_jacobi).  Round r of the round-robin order pairs the 16-index
-// blocks; k_jsub solves each pair's 32 x 32 subproblem with one wave
-// (wave_jacobi_sub), stores its rotation Q_k and the rotated diagonal
+// blocks; k_jsub solves each pair's 32 x 32 subproblem (wave_jacobi_sub and
+// sub_rotate), stores its rotation Q_k and the rotated diagonal
 // block, and flags Q_k == I; k_japply then applies every Q_k of the round
 // to the off-diagonal tiles of A (Q_k^T A_kl Q_l) and to the orbital rows.
 // ---------------------------------------------------------------------------
 // One workgroup per block pair k of round r.  The first wave runs the rounds of
 // a sweep on the subproblem and records the rotations; all four stage it and
 // apply the sweep to Q, two columns of Q^T a lane: 18.7 us a launch at n = 296
-// and 12.2 at 4800 (everything in one wave 22.5 and 14.3).
+// and 10.2 at 4800 (everything in one wave 22.5 and 14.3).
 constexpr int JSUB_WAVES = 4;
 __global__ void __launch_bounds__(JSUB_WAVES * WAVE) k_jsub(double* A_, int n, int r, int nb2, double* Qbuf, int* ident,
                                                             double tol, int inner) {
@@ -1080,7 +1080,7 @@ void axpby(Ctx& c, size_t len, double a, const double* X, double b, const double
 }
 
 // Loewdin orthogonaliser by coupled Newton-Schulz (as ortho_setup in
-// scf.hip): Ct <- X = S^-1/2.  Returns false when the iteration did not
+// scf_kernel.h): Ct <- X = S^-1/2.  Returns false when the iteration did not
 // converge (S numerically singular).
 bool ortho(Ctx& c) {
     const int n = c.n;
@@ -1195,7 +1195,7 @@ bool warm_orthonormalise(Ctx& c, const double* pot) {
     return true;
 }
 
-// Cholesky orthogonaliser (as chol_setup in scf.hip): S = L L^T by
+// Cholesky orthogonaliser (as chol_setup in scf_kernel.h): S = L L^T by
 // right-looking 32-wide panels (a wave factors each diagonal block, the panel
 // solve and the trailing update are grid GEMMs), then X = L^-1 by the
 // right-looking triangular inverse: block row j of X <- D_j^-1 X_j, rows
@@ -1248,7 +1248,7 @@ bool ortho_chol(Ctx& c) {
 }
 
 // Block Jacobi on A = F (full symmetric); rotations applied to the orbital
-// rows.  Tolerance as eig_step in scf.hip.  Eigenvalue estimates -> ev.
+// rows.  Tolerance as eig_step in scf_kernel.h.  Eigenvalue estimates -> ev.
 // Returns sweeps, or -1 when max_sweeps were spent.
 int eig(Ctx& c, double rel_tol, double loose) {
     const double t0 = now_s();
@@ -1294,7 +1294,7 @@ int eig(Ctx& c, double rel_tol, double loose) {
 }
 
 // Perturbative occupied-virtual rotation of a closed shell with k doubly
-// occupied rows first (pd_step in scf.hip, with grid GEMMs).  Returns 1
+// occupied rows first (pd_step in scf_kernel.h, with grid GEMMs).  Returns 1
 // when done, 0 to ask for Jacobi with Ct and F untouched, -1 to ask for it
 // after F served as scratch.
 int pd(Ctx& c, int k, double loose, const double* vin) {
@@ -1396,7 +1396,7 @@ void scaled_occupied(Ctx& c, const double* ev, double* H) {
     chk_launch(c);
 }
 
-// one SCF map vin -> vout (scf_step in scf.hip); the sort's control values
+// one SCF map vin -> vout (scf_step in scf_kernel.h); the sort's control values
 // are posted (!sort_rows) or left for the mixing step's post
 int step(Ctx& c, const double* vin, double* vout, int& status, double loose, bool allow_bd, bool sort_rows,
          bool final_step, int* decoupled, bool last) {
@@ -1627,7 +1627,7 @@ extern "C" int32_t xtb_scf_large(const xtb_batch* batch, const xtb_params* par, 
     bool converged = false;
     for (int it = 0; it < o.maxiter && c.err == hipSuccess; ++it) {
         // fractional occupations near the Fermi level tighten the inexact
-        // eigensolve by 2 kT (as in scf.hip)
+        // eigensolve by 2 kT (as in scf_kernel.h)
         const double soft = c.h[C_FSOFT] > 1e-6 ? fmin(1.0, 2.0 * o.kt) : 1.0;
         sweeps += step(c, state->pot, state->vnew, status, o.eig_inexact * resid * soft, o.eig_inexact > 0.0,
                        true, false, nullptr, false);

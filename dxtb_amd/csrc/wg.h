@@ -1225,8 +1225,8 @@ __device__ __forceinline__ void sub_rotate(double c, double s, int k, double& to
 // up a schedule, packed triangle indices and Q's rows in LDS took 62 us.  (Q's
 // update a round late, to fill the rotation's latency, changed nothing; left
 // to four waves after the sweep, as on the whole GPU, it comes to 19 us.)
-// With LATER, Q is left to sub_rotations: the rotations of round r go to cs +
-// 2 K r (max_sweeps = 1 then).
+// With LATER, Q is left to the caller (sub_rotate): the rotations of round r go
+// to cs + 2 K r (max_sweeps = 1 then).
 template <bool LATER>
 __device__ __noinline__ int wave_jacobi_sub(ldsf* D, ldsf* cs, glbf* qg, double tol, int max_sweeps, int mode,
                                             unsigned lo_mask, unsigned hi_mask) {

@@ -8,12 +8,13 @@ gradients come from the same kernels as for a batch, and the SCF from
 and mixer as the per-molecule kernel, with every stage a grid kernel that
 spreads over all CUs and the SCF loop on the host:
 
-* Loewdin orthogonaliser X = S^-1/2 by coupled Newton-Schulz on matrix-core
-  GEMMs (128 x 128 tiles per workgroup, XCD-aware tile order);
+* Cholesky orthogonaliser L^-1, or Loewdin's S^-1/2 by coupled Newton-Schulz,
+  on matrix-core GEMMs (16- to 96-wide tiles with their operands loaded
+  straight to registers, XCD-aware tile order);
 * per SCF step, for gapped closed shells, the perturbative
   occupied-virtual rotation of the previous step's orbitals (GEMMs);
-  otherwise A = C F C^T and parallel-ordered block Jacobi (a wave per 32 x 32
-  subproblem, the rotations applied to A and the orbitals on matrix cores),
+  otherwise A = C F C^T and parallel-ordered block Jacobi (a workgroup per 32 x
+  32 subproblem, the rotations applied to A and the orbitals on matrix cores),
   which gives the eigenpairs upstream's eigh does
   (src/dxtb/_src/scf/unrolling/base.py:142-175);
 * sort and Fermi smearing (src/dxtb/_src/wavefunction/filling.py:201-366),
